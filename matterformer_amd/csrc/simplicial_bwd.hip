@@ -162,10 +162,6 @@ struct Params {
   int NP;       // N rounded up to 64: LDS list capacity
   int OB;       // workgroups per (b, h, role)
   int vec;      // q/k/v/go/out rows 4-element loads are aligned (D % 4 == 0, aligned bases)
-  const int* served;  // [B] nonzero: the pair kernel computed this molecule's gradients (or NULL)
-  const int* unserved;  // the number of molecules the pair kernel left over (with `served`)
-  int blocks;         // 3 B H OB work blocks; the grid may be smaller and loop over them
-  int served_lds;     // byte offset of the LDS copy of `served` (after the role's layout)
   // low-rank terms (LR instantiations): factors [B*H, N, N, R] fp32, gates [B*H, N], basis [H, Rm, D]
   const float* al;
   const float* ar;
@@ -980,25 +976,14 @@ __device__ __forceinline__ void run_role(const Params& p, unsigned char* smem, i
 template <int DP, bool M16, bool BIAS, bool LR>
 __global__ void __launch_bounds__((Shape<DP, M16, LR>::kThreads), (Shape<DP, M16, LR>::kMinBlocks)) simplicial_bwd_kernel(Params p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  if (p.served != nullptr && *p.unserved == 0) return;  // the pair kernel served every molecule
   const int G = p.B * p.H * p.OB;
-  const int* served = reinterpret_cast<const int*>(smem + p.served_lds);
-  if (p.served != nullptr) {
-    for (int i = threadIdx.x; i < p.B; i += Shape<DP, M16, LR>::kThreads)
-      const_cast<int*>(served)[i] = p.served[i];
-    __syncthreads();
-  }
-  for (int w = blockIdx.x; w < p.blocks; w += gridDim.x) {
-    const int role = w / G;
-    const int blk = w - role * G;
-    const int bh = blk / p.OB;
-    const int ob = blk - bh * p.OB;
-    if (p.served != nullptr && served[bh / p.H] != 0) continue;  // uniform: the pair kernel's molecule
-    if (w != int(blockIdx.x)) __syncthreads();  // the previous block's LDS reads are done
-    if (role == kRoleQ) run_role<DP, kRoleQ, M16, BIAS, LR>(p, smem, bh, ob);
-    else if (role == kRoleJ) run_role<DP, kRoleJ, M16, BIAS, LR>(p, smem, bh, ob);
-    else run_role<DP, kRoleK, M16, BIAS, LR>(p, smem, bh, ob);
-  }
+  const int role = int(blockIdx.x) / G;
+  const int blk = int(blockIdx.x) - role * G;
+  const int bh = blk / p.OB;
+  const int ob = blk - bh * p.OB;
+  if (role == kRoleQ) run_role<DP, kRoleQ, M16, BIAS, LR>(p, smem, bh, ob);
+  else if (role == kRoleJ) run_role<DP, kRoleJ, M16, BIAS, LR>(p, smem, bh, ob);
+  else run_role<DP, kRoleK, M16, BIAS, LR>(p, smem, bh, ob);
 }
 
 // dc[row][r] = basis[h][r] . go[row] for every row of [B*H, N] (message term), and coeff[row][r] = 0:
@@ -1106,8 +1091,6 @@ template <int DP, bool M16, bool LR = false>
 int launch(Params prm, bool has_pv, bool has_bias, hipStream_t stream) {
   size_t lds = Lay<DP, M16, LR>::bytes(prm.NP, has_pv, has_bias, (LR && prm.ml && prm.coeff) ? prm.RmP : 0);
   lds = (lds + 15) & ~size_t(15);
-  prm.served_lds = int(lds);
-  if (prm.served != nullptr) lds += size_t(prm.B) * 4;
   DeviceInfo dev;
   int st = device_info(&dev);
   if (st != MF_OK) return st;
@@ -1126,10 +1109,7 @@ int launch(Params prm, bool has_pv, bool has_bias, hipStream_t stream) {
   prm.OB = int(std::max(1LL, std::min<long long>(want, (prm.N + kW - 1) / kW)));
   const long long blocks = 3 * bh * prm.OB;
   if (blocks > 0x7fffffffLL) return fail(MF_ERR_UNSUPPORTED, "mf_simplicial_bwd: grid too large");
-  prm.blocks = int(blocks);
-  // after the pair kernel most blocks are skipped: a grid of a few workgroups per CU loops over them
-  const long long grid = prm.served != nullptr ? std::min<long long>(blocks, 2LL * dev.num_cus) : blocks;
-  hipLaunchKernelGGL(kerns[has_bias], dim3(unsigned(grid)), dim3(Shape<DP, M16, LR>::kThreads), lds, stream, prm);
+  hipLaunchKernelGGL(kerns[has_bias], dim3(unsigned(blocks)), dim3(Shape<DP, M16, LR>::kThreads), lds, stream, prm);
   MF_HIP_CHECK(hipGetLastError());
   return MF_OK;
 }
@@ -1271,12 +1251,14 @@ extern "C" int mf_simplicial_bwd(const mf_simplicial_bwd_args* a, void* stream) 
     }
     return MF_OK;
   }
-  // bf16 operands and a bf16 grad_out: bf16 MFMA (K steps of 32 d), which stages grad_out rows as bf16 (exact
-  // only for a bf16 grad_out).  Everything else -- fp16 operands, or a grad_out of another dtype -- takes the
-  // fp32 path, which reads every operand in its own dtype.
+  // bf16 operands and grad_out with head_dim 64 take the pair formulation (simplicial_pair_bwd.hip, which also
+  // writes the zero rows of 16-bit gradients)
+  const bool pair = simplicial_pair_bwd_serves(a);
   if (gout16) {
-    hipLaunchKernelGGL(zero_rows_kernel, dim3(unsigned(a->batch * a->heads)), dim3(256), 0, s, prm);
-    MF_HIP_CHECK(hipGetLastError());
+    if (!pair) {
+      hipLaunchKernelGGL(zero_rows_kernel, dim3(unsigned(a->batch * a->heads)), dim3(256), 0, s, prm);
+      MF_HIP_CHECK(hipGetLastError());
+    }
     if (has_bias && (a->du || a->dv_bias || a->dw || a->dgate)) {
       const size_t gates = size_t(a->batch) * a->heads * a->tokens, plane = gates * a->tokens;
       const size_t grid = std::min<size_t>((plane / 8 + 255) / 256, 4096);
@@ -1285,15 +1267,11 @@ extern "C" int mf_simplicial_bwd(const mf_simplicial_bwd_args* a, void* stream) 
       MF_HIP_CHECK(hipGetLastError());
     }
   }
+  if (pair) return simplicial_pair_bwd_launch(a, s);
+  // other bf16 operands with a bf16 grad_out: bf16 MFMA (K steps of 32 d), which stages grad_out rows as bf16
+  // (exact only for a bf16 grad_out).  Everything else -- fp16 operands, or a grad_out of another dtype -- takes
+  // the fp32 path, which reads every operand in its own dtype.
   if (a->dtype == MF_DTYPE_BF16 && a->grad_dtype == MF_DTYPE_BF16) {
-    // molecules of at most 80 valid atoms take the pair formulation; the ownership kernel below takes the rest
-    if (simplicial_pair_bwd_serves(a)) {
-      const int st = simplicial_pair_bwd_launch(a, s);
-      if (st != MF_OK) return st;
-      if (a->tokens <= simplicial_pair_bwd_max_tokens()) return MF_OK;
-      prm.served = simplicial_pair_bwd_served(a);
-      prm.unserved = simplicial_pair_bwd_unserved_count(a);
-    }
     if (D <= 32) return launch<32, true>(prm, has_pv, has_bias, s);
     if (D <= 64) return launch<64, true>(prm, has_pv, has_bias, s);
     return launch<128, true>(prm, has_pv, has_bias, s);
@@ -1310,6 +1288,6 @@ extern "C" uint64_t mf_simplicial_bwd_workspace_size(int32_t batch, int32_t head
   // the message term's coefficients, or (head_dim 64) the pair kernel's plan and partial sums; one call uses
   // at most one of them
   const uint64_t msg = message_rank > 0 ? message_workspace_bytes(batch, heads, tokens, message_rank) : 0;
-  const uint64_t pair = head_dim == 64 ? uint64_t(simplicial_pair_bwd_workspace_bytes(batch, heads)) : 0;
+  const uint64_t pair = head_dim == 64 ? uint64_t(simplicial_pair_bwd_workspace_bytes(batch, heads, tokens)) : 0;
   return std::max(msg, pair);
 }

@@ -1,7 +1,6 @@
 // 2-simplicial attention backward, pair formulation, for bf16 operands and
-// head_dim 64 on gfx950 (CDNA4): molecules of at most 80 valid queries and 80
-// valid keys, one or two workgroups per (molecule, head), deterministic (no
-// floating-point atomics).
+// head_dim 64 on gfx950 (CDNA4), molecules of any size up to 512 tokens,
+// deterministic (no floating-point atomics).
 //
 // The gradient of simplicial_attention.py:206-344 (the quantities of
 // triton_simplicial_attention.py:332-782) with the key pairs p = (j, k) as
@@ -15,40 +14,59 @@
 // Five products of n^3 D multiply-adds, against eleven when every index
 // recomputes the scores it owns (simplicial_bwd.hip).
 //
-// Work split.  The keys are cut into 16-key tiles k0 .. k0 + 15 (outer loop,
-// the four waves in step); inside a tile each wave takes the pairs of keys
-// (j, j + 1) = (2 jp, 2 jp + 1), jp = wave, wave + 4, ..., and for each pair
-// tile (2 j x 16 k = 32 pairs) every 16-query tile:
+// Units.  lse and go . out are given, so every (query block, j block, k block)
+// of a molecule is independent work.  A unit (one workgroup of four waves) is
+// a run of the j keys of one (molecule, head); it walks its j in blocks of at
+// most 24, and for each the query and k blocks of at most 64 rows (48 with a
+// bias; one of each for most molecules).  A block triple is staged in LDS
+// (78 KB, so two workgroups share a CU and each SIMD holds two waves: with one
+// wave a SIMD issued an instruction every ~7 cycles, and one unit's staging
+// latency was another's idle time), then
+//   for each 16-key tile k0 .. k0 + 15, each wave takes the key pairs
+//   (j, j + 1) = (2 jp, 2 jp + 1), jp = wave, wave + 4, ..., in three steps:
 //   S, dP   C[i][k] = sum_d A[i][d] B[d][k]   A = q / go rows (LDS), B = W / Z
-//           of the tile, formed in registers (MFMA 16x16x32 bf16)
-//   dq_i   += dS[i][p] W[p][d]   K = the 32 pairs, dS turned through a
-//           per-wave LDS scratch (transposed read)
-//   G^T, H^T (key x d) += dS^T / P^T [k][i] q / go [i][d]: the S accumulators
-//           of two query tiles are the A operand as they are (K = 32 queries)
-// then dk1_j / dv1_j (sums over the tile's keys: in-lane over 4 keys, then
-// across the four lane groups) go to the wave's own LDS rows of j, and
-// dk2 / dv2 of the tile's keys accumulate over the wave's j in registers; at
-// the end of the key tile the four waves' partials are added in a fixed
-// order.  dq accumulates over every pair in registers and the four waves'
-// rows are added in a fixed order at the end.  Every sum has a fixed order:
-// two calls give identical bits.
+//           of (j, the tile), formed in registers (MFMA 16x16x32 f16), for
+//           every 16-query tile; P and dS are kept as packed fp16
+//   G^T, H^T (key x d) += dS^T / P^T [k][i] q / go [i][d], 16 d at a time: the
+//           S accumulators of two query tiles are the A operand as they are
+//           (K = 32 queries), the B operand (transposed reads) serves both j
+//   dq_i   += dS[i][p] W[p][d], K = the 32 pairs, dS turned through a per-wave
+//           LDS scratch (transposed read).
+// The steps keep a wave's registers under 256 (two waves per SIMD) although
+// both j share every row read from LDS.
+// dk1_j / dv1_j (sums over the tile's keys) are added to the wave's own LDS
+// rows of j: each lane sums 4 keys, and the four lane groups' partials of the
+// four 16-d tiles meet in a transposing reduction (3 lane swaps and 3 adds per
+// four values) that leaves d = lane in every lane, so a row is updated by one
+// full-wave read and write.  dk2 / dv2 of the tile's keys accumulate over the
+// wave's j in registers, dq over every pair; the four waves' partials are
+// added in a fixed order.  Every sum has a fixed order: two calls give
+// identical bits.
 //
-// Schedule.  A one-workgroup planning kernel counts every molecule's valid
-// keys and queries, marks the molecules this kernel serves (for the
-// ownership kernel to skip), and writes the unit list longest first (cost
-// ~ j pairs x key tiles x query tiles, the LPT order): molecules with more
-// than 40 valid keys run as two units that take alternate key pairs
-// (jp = part, part + 2, ...), the others as one.  Workgroup w runs unit w.
-// The two halves of a molecule own their dk1 / dv1 rows and hold partial
-// sums of dq, dk2 and dv2: part 0 writes its partials to the fp32 gradient
-// rows (to its own slab of the workspace when the gradients are bf16), part 1
-// to its slab, and a third launch writes part 0 + part 1 in that order.  (Handing the sums over inside the kernel would need
-// a device-scope release and acquire per half, which on this part write back
-// and invalidate the whole L2 of the XCD and held each workgroup's CU for
-// tens of microseconds.)
+// Measured (64 GEOM-like molecules of mean 44 atoms, 8 heads, kernel time):
+// 109 us without a bias (191 us when one wave per SIMD held both j, the
+// products' operands and all query tiles in 470 registers, and a unit had a
+// whole CU: 0.29 PFLOP/s of the five products now), 278 us with a fp32 or
+// bf16 bias (1.88 ms and 365 us on the kernels that served them before); four
+// molecules of 192 atoms, 12 heads, bf16 bias: 1.16 ms (5.47 ms on the
+// ownership kernel).  A variant with more spilled registers than the 8 of the
+// staging code doubled the loop's time: a spill waits on memory that two
+// waves per SIMD cannot cover.
+//
+// Schedule.  The prepare launch's first workgroup counts every molecule's
+// valid keys and queries, picks the j per unit (24, 12 or 6, with a bias 16, 8 or 4: fewer when more
+// leaves the chip without two units per CU) and writes the unit list longest
+// first (LPT); its other workgroups write the zero rows of 16-bit gradients.
+// The units of a molecule own their dk1 / dv1 rows; where a molecule has more
+// than one block triple, dq, dk2 and dv2 are summed in the unit's slab of the
+// workspace (read back by the thread that wrote it) and a combine launch adds
+// the slabs in unit order.  (Handing the sums over inside the kernel would
+// need a device-scope release and acquire per unit, which on this part write
+// back and invalidate the whole L2 of the XCD and held each workgroup's CU
+// for tens of microseconds.)
 //
 // Precision.  The rows are staged as fp16 scaled by powers of two, one per
-// operand and unit, that bring each operand's largest magnitude into [1, 2)
+// operand and block, that bring each operand's largest magnitude into [1, 2)
 // (bf16 values convert exactly; entries below 2^-14 of the largest lose low
 // bits as fp16 subnormals, which moves a dot product by at most 2^-24 of its
 // largest term), so that one v_pk_mul_f16 forms two pair products and the
@@ -61,8 +79,14 @@
 //     (the reference's dP contraction is fp32, :611-645);
 //   dS (scaled by 2^-es, es chosen from the operand scales so that
 //     |dS| < 2^15 always) and P as MFMA operands: rounded once to fp16;
-//   softmax, dS and every accumulator fp32; the scales are undone, exactly,
-//   when the gradients are written.
+//   softmax, dS, every accumulator and every bias sum fp32; the scales are
+//   undone, exactly, before block triples are added.
+//
+// Factorized bias (BIAS 1: bf16, 2: fp32 terms): S += gate_i (u_ij + v_ik +
+// w_jk) with u staged transposed in LDS as fp32, v read per key tile into
+// registers, w per pair (fetched one pair ahead).  du (sum over the tile's
+// keys, a transposing reduction over 16 lanes), dv_bias (registers over the
+// wave's j), dgate and dw all come from the fp32 dS.
 #include <algorithm>
 #include <cmath>
 
@@ -73,12 +97,13 @@ namespace pbwd {
 
 constexpr int kWaves = 4;
 constexpr int kThreads = kWaves * 64;
-constexpr int DP = 64;           // head_dim
-constexpr int KS = DP + 8;       // bf16 row stride of the staged rows (144 B)
-constexpr int kMaxN = 80;        // valid queries and valid keys per molecule
-constexpr int NT = kMaxN / 16;   // 16-row tiles
-constexpr int SS = 16 + 4;       // bf16 row stride of the dS scratch (40 B)
-constexpr int kSlot = 2 * 16 * DP;  // floats of one wave's dk2 / dv2 partial of a key tile
+constexpr int DP = 64;            // head_dim
+constexpr int KS = DP + 8;        // fp16 row stride of the staged rows (144 B)
+constexpr int SS = 16 + 4;        // fp16 row stride of the dS scratch (40 B)
+constexpr int PS = DP + 4;        // fp32 row stride of the waves' partial sums
+constexpr int kMaxTokens = 512;
+constexpr int kMaxPlanBatch = 2048;
+constexpr int kPlanThreads = 1024;
 
 struct Params {
   const __bf16* q;
@@ -89,8 +114,6 @@ struct Params {
   const __bf16* go;
   const float* out;
   const float* lse;
-  const uint8_t* qv;
-  const uint8_t* pkv;
   const uint8_t* pv;
   void* dq;               // gradients, fp32 or (gout16) bf16
   void* dk1;
@@ -98,106 +121,120 @@ struct Params {
   void* dk2;
   void* dv2;
   int gout16;
-  const int* total;       // plan: units in the list
-  const uint32_t* units;  // plan: (b H + h) << 1 | part, longest first
+  const int* head;        // plan: [0] units in the list, [1] j per unit
+  const uint32_t* units;  // plan: (b H + h) << 6 | part, longest first
   const int2* counts;     // plan: [B] valid keys, valid queries
-  const uint16_t* lists;  // plan: [B][2][kMaxN] their atoms
-  float* slab;            // [B*H][2 parts][5][kMaxN][DP] partial dq, dk2, dv2 of split molecules and (bias)
-                          // the dk1, dv1 sums of the unit's keys (compacted rows)
-  // factorized bias (BIAS kernels): S += gate_i (u_ij + v_ik + w_jk), u / v / w [B*H, N, N], gate [B*H, N]
-  // bf16; gradients fp32 or (gout16) bf16, NULL = not wanted
-  const uint16_t* bu;
-  const uint16_t* bv;
-  const uint16_t* bw;
-  const uint16_t* bg;
+  const uint16_t* lists;  // plan: [B][2][N] their atoms
+  float* slab;            // [B*H][cap parts][3][N][DP] partial dq, dk2, dv2 (compacted rows)
+  // factorized bias (BIAS kernels): S += gate_i (u_ij + v_ik + w_jk), u / v / w [B*H, N, N], gate [B*H, N],
+  // bf16 or fp32; gradients fp32 or (gout16) bf16, NULL = not wanted
+  const void* bu;
+  const void* bv;
+  const void* bw;
+  const void* bg;
   void* du;
   void* dvb;
   void* dw;
   void* dgate;
-  float* dwpart;          // [B*H][kMaxN j][kMaxN k] dw of the earlier query passes (compacted)
-  float* dupart;          // [B*H][kMaxN / 16 key tiles][kMaxN i][kMaxN j] per-key-tile sums over k of dS 2^-es
-  float* dvbpart;         // [B*H][2 parts][kMaxN i][kMaxN k] sums over the part's j of dS 2^-es
-  float* dgpart;          // [B*H][2 parts][kMaxN i] sums over the part's (j, k) of dS 2^-es (u + v + w)
-  float* fds;             // [B*H] 2^es of the unit (dS is carried as dS 2^-es)
-  int H, N;
+  float* dwpart;          // [B*H][N j][N k] dw of the earlier query blocks (compacted)
+  float* dvpart;          // [B*H][cap parts][N i][N k] sums over the part's j of dS
+  float* dgpart;          // [B*H][cap parts][N i] sums over the part's (j, k) of dS (u + v + w)
+  int H, N, cap;
 };
-
-// Units per molecule: two halves (alternate key pairs) above 40 valid keys.
-__device__ __forceinline__ int parts_of(int nk) { return nk > 40 ? 2 : 1; }
-
-// Relative cost of one unit: j pairs x key tiles x MFMA per (pair tile, all queries).
-__device__ __forceinline__ uint32_t unit_cost(int nk, int nq) {
-  const int nqt = (nq + 15) / 16;
-  return uint32_t((nk + 1) / 2) * uint32_t((nk + 15) / 16) * uint32_t(28 * nqt + 16 * ((nqt + 1) / 2)) /
-         uint32_t(parts_of(nk));
-}
 
 // Workspace of the pair path (16-byte aligned regions).
+constexpr size_t kWsTarget = size_t(16) << 30;  // bytes; calls past kWsLimit take the ownership kernel
+constexpr size_t kWsLimit = size_t(48) << 30;
 struct Ws {
-  size_t units, served, counts, lists, slab, dupart, dvbpart, dgpart, fds, dwpart, bytes;
-  Ws(int B, int H) {
-    const size_t bh = size_t(B) * H;
-    units = 16;  // [0, 4): units in the list, [4, 8): molecules the pair kernel does not serve
-    served = units + ((bh * 2 * 4 + 15) & ~size_t(15));
-    counts = served + ((size_t(B) * 4 + 15) & ~size_t(15));
+  int cap;  // units per (molecule, head) at most
+  size_t units, counts, lists, slab, dvpart, dgpart, dwpart, bytes;
+  Ws(int B, int H, int N) {
+    const size_t bh = size_t(B) * H, n = size_t(N);
+    // a few units per CU are enough: large batches get three per (molecule, head), small ones as many as give
+    // 2048 units (4 j each at the least); fewer where the partial sums would pass kWsTarget
+    cap = int(std::min<size_t>(std::min<size_t>(std::max<size_t>(3, 2048 / bh), (n + 3) / 4), 64));
+    while (layout(B, bh, n) > kWsTarget && cap > 1) --cap;
+  }
+  size_t layout(int B, size_t bh, size_t n) {
+    units = 16;
+    counts = units + ((bh * cap * 4 + 15) & ~size_t(15));
     lists = counts + size_t(B) * 8;
-    slab = (lists + size_t(B) * 2 * kMaxN * 2 + 255) & ~size_t(255);
-    dupart = slab + bh * 2 * 5 * kMaxN * DP * 4;
-    dvbpart = dupart + bh * (kMaxN / 16) * kMaxN * kMaxN * 4;
-    dgpart = dvbpart + bh * 2 * kMaxN * kMaxN * 4;
-    fds = dgpart + bh * 2 * kMaxN * 4;
-    dwpart = (fds + bh * 4 + 15) & ~size_t(15);
-    bytes = dwpart + bh * kMaxN * kMaxN * 4;
+    slab = (lists + size_t(B) * 2 * n * 2 + 255) & ~size_t(255);
+    dvpart = slab + bh * cap * 3 * n * DP * 4;
+    dgpart = dvpart + bh * cap * n * n * 4;
+    dwpart = (dgpart + bh * cap * n * 4 + 15) & ~size_t(15);
+    bytes = dwpart + bh * n * n * 4;
+    return bytes;
   }
 };
-constexpr int kPlanThreads = 1024;
-constexpr int kMaxPlanBatch = 2048;
-constexpr int kMaxTokens = 512;  // mask rows the plan reads in one pass of 8 x 64 bytes
 
 struct PlanParams {
   const uint8_t* qv;
   const uint8_t* pkv;
-  int* total;       // total[0] units, total[1] unserved molecules
+  int* head;        // [0] units, [1] j per unit
   uint32_t* units;
-  int* served;
   int2* counts;     // [B] (valid keys, valid queries)
-  uint16_t* lists;  // [B][2][kMaxN] valid key atoms, valid query atoms (when they fit)
-  int B, H, N;
+  uint16_t* lists;  // [B][2][N] valid key atoms, valid query atoms
+  void* dq;         // 16-bit gradients: zero rows are written here (NULL: fp32 gradients, filled by the caller)
+  void* dk1;
+  void* dv1;
+  void* dk2;
+  void* dv2;
+  int B, H, N, cap;
+  int jm;           // j per unit at most
 };
 
-// LDS layout (bytes).  BIAS: no dk1 / dv1 sums (they run in the workspace) but the bias terms u^T [j][i],
-// v^T [k][i] (bf16 as given) and the gates.
-constexpr int KU = kMaxN + 8;  // bf16 row stride of u^T, v^T (176 B)
+// LDS layout (bytes).  A block has at most QM query, JM j and KM k rows: 64, 24 and 64 without a bias; the bias
+// terms leave LDS and registers for 48, 16 and 48.  The scratch of the main loop, and between key tiles and at a triple's end the partial
+// sums of dk2, dv2 and dq, share one region.
 template <bool BIAS>
 struct Lay {
-  static constexpr size_t rows = 0;                                            // q, go, k1, k2, v1, v2: [80][KS] fp16
-  static constexpr size_t acc1 = rows + size_t(6) * kMaxN * KS * 2;            // dk1, dv1 of the wave's j: [2][80][64] f32
-  static constexpr size_t slot = acc1 + (BIAS ? 0 : size_t(2) * kMaxN * DP * 4);  // [4 waves][kSlot] f32
-  static constexpr size_t dvb = slot + size_t(kWaves) * kSlot * 4;             // BIAS: [4 waves][5][16 k][16 i] f32
-  static constexpr size_t scr = dvb + (BIAS ? size_t(kWaves) * NT * 256 * 4 : 0);  // [4 waves][2][32][SS] fp16
-  static constexpr size_t ut = scr + size_t(kWaves) * 2 * 32 * SS * 2;         // BIAS: [80][KU] bf16
-  static constexpr size_t vt = ut + (BIAS ? size_t(kMaxN) * KU * 2 : 0);      // BIAS: [80][KU] bf16
-  static constexpr size_t gt = vt + (BIAS ? size_t(kMaxN) * KU * 2 : 0);      // BIAS: [2][80] f32 gate, gate log2 e
-  static constexpr size_t lse2 = gt + (BIAS ? 2 * kMaxN * 4 : 0);              // [80] f32
-  static constexpr size_t dlt = lse2 + kMaxN * 4;                              // [80] f32
-  static constexpr size_t pvb = dlt + kMaxN * 4;                               // [80][3] u32 pair bits
-  static constexpr size_t kidx = pvb + kMaxN * 3 * 4;                          // [80] i32
-  static constexpr size_t qidx = kidx + kMaxN * 4;                             // [80] i32
-  static constexpr size_t cnt = qidx + kMaxN * 4;                              // [4] i32
-  static constexpr size_t red = cnt + 16;                                      // [4 waves][8] u32 operand maxima
-  static constexpr size_t con = red + kWaves * 8 * 4;                          // [8] f32 unit constants (kC*)
-  static constexpr size_t bytes = con + 8 * 4;
-  static_assert(bytes <= 160 * 1024, "one workgroup per CU");
-  // BIAS passes of at most 3 query tiles: the four waves' dq partials in slot + dvb
-  static_assert(!BIAS || size_t(kWaves) * 48 * DP * 4 <= scr - slot, "dq partials of a pass fit slot + dvb");
-  static_assert(size_t(kWaves) * kMaxN * DP * 4 <= scr, "dq partials reuse rows + acc1 / slot");
-  static_assert(size_t(kMaxN) * 16 <= size_t(kSlot), "a wave's dv_bias partials of a key tile fit its slot");
-  static_assert(48 * 4 <= 2 * 32 * SS * 2, "a wave's dgate partials of a pass fit its scratch");
+  static constexpr int QM = BIAS ? 48 : 64;
+  static constexpr int JM = BIAS ? 16 : 24;
+  static constexpr int KM = BIAS ? 48 : 64;
+  static constexpr int KU = QM + 4;                                             // fp32 row stride of u^T, v^T, du
+  static constexpr int KW = KM + 4;                                             // fp32 row stride of w / dw
+  static constexpr int kRows = 2 * QM + 2 * JM + 2 * KM;                        // q, go, k1, v1, k2, v2
+  static constexpr size_t rows = 0;                                             // [kRows][KS] fp16
+  static constexpr size_t acc1 = rows + size_t(kRows) * KS * 2;                 // [2][JM][64] f32 dk1, dv1
+  static constexpr size_t scr = acc1 + size_t(2) * JM * DP * 4;                 // [4 waves][16][PS] f32 / scratch
+  static constexpr size_t scr_bytes = size_t(kWaves) * (QM / 16 * 32 * SS * 2 > 16 * PS * 4 ? QM / 16 * 32 * SS * 2 : 16 * PS * 4);
+  static constexpr size_t ut = scr + scr_bytes;                                 // BIAS: [JM][KU] f32 u^T
+  static constexpr size_t dut = ut + (BIAS ? size_t(JM) * KU * 4 : 0);          // BIAS: [JM][KU] f32 sums of dS over k
+  static constexpr size_t wd = dut + (BIAS ? size_t(JM) * KU * 4 : 0);          // BIAS: [JM][KW] f32 w, then dw
+  static constexpr size_t vt = wd + (BIAS ? size_t(JM) * KW * 4 : 0);           // BIAS: [KM][KU] f32 v^T
+  static constexpr size_t gt = vt + (BIAS ? size_t(KM) * KU * 4 : 0);           // BIAS: [QM] f32 gate log2 e
+  static constexpr size_t lse2 = gt + (BIAS ? QM * 4 : 0);                      // [QM] f32
+  static constexpr size_t dlt = lse2 + QM * 4;                                  // [QM] f32 go . out
+  static constexpr size_t dls = dlt + QM * 4;                                   // [QM] f32 go . out 2^-es
+  static constexpr size_t pvb = dls + QM * 4;                                   // [JM][8] bytes: pair bits
+  static constexpr size_t jidx = pvb + JM * 8;                                  // [JM] i32
+  static constexpr size_t kidx = jidx + JM * 4;                                 // [KM] i32
+  static constexpr size_t qidx = kidx + KM * 4;                                 // [QM] i32
+  static constexpr size_t red = qidx + QM * 4;                                  // [4 waves][8] u32 operand maxima
+  static constexpr size_t bytes = red + kWaves * 8 * 4;
+  static_assert(bytes <= 80 * 1024, "two workgroups per CU");
+  static_assert(!BIAS || size_t(kWaves) * QM * 16 * 4 <= scr_bytes, "the waves' dv_bias partials of a key tile fit");
 };
 
-// Unit constants in LDS: S log2 e = S_c cS; dS 2^-es = P (dP_c cP - delta 2^-es); the written gradients are
-// the accumulated sums times fDq, fDk1, fDk2, fDv1, fDv2.
-enum { kCS = 0, kCP, kFDq, kFDk1, kFDk2, kFDv1, kFDv2, kFDs };
+// j keys per unit and units of a molecule: `jt` j per unit, at most `cap` units, whole key pairs.
+__device__ __forceinline__ int parts_of(int nk, int jt, int cap) {
+  const int pairs = (nk + 1) / 2, most = min(cap, (nk + jt - 1) / jt);
+  const int per = (pairs + most - 1) / most;
+  return (pairs + per - 1) / per;
+}
+__device__ __forceinline__ int unit_rows(int nk, int parts) { return 2 * (((nk + 1) / 2 + parts - 1) / parts); }
+// Blocks of a run of n rows, at most m rows (a multiple of 16) each, cut at multiples of 16.
+__device__ __forceinline__ int blocks_of(int n, int m) { return (n + m - 1) / m; }
+__device__ __forceinline__ int block_rows(int n, int blocks) { return 16 * (((n + 15) / 16 + blocks - 1) / blocks); }
+
+// Relative cost of one unit: rounds of key pairs x key tiles x (fixed work per query block + query tiles), and
+// the staging.
+__device__ __forceinline__ uint32_t unit_cost(int nk, int nq, int jt, int cap) {
+  const int jr = unit_rows(nk, parts_of(nk, jt, cap));
+  const int nqt = (nq + 15) / 16, nkt = (nk + 15) / 16, nqb = blocks_of(nq, 64);
+  return uint32_t((jr / 2 + kWaves - 1) / kWaves) * uint32_t(nkt) * uint32_t(6 * nqb + 2 * nqt) + 24u;
+}
 
 typedef __attribute__((__vector_size__(4 * sizeof(_Float16)))) _Float16 mf_f16x4;
 
@@ -234,15 +271,6 @@ __device__ __forceinline__ uint4 to_f16x8(const uint4 r, float scale) {
                __builtin_bit_cast(uint32_t, p3)};
 }
 
-// Eight fp32 rounded (toward zero) to fp16.
-__device__ __forceinline__ mf_f16x8 pack_f16x8(const float* f) {
-  const uint4 w{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(f[0], f[1])),
-               __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(f[2], f[3])),
-               __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(f[4], f[5])),
-               __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(f[6], f[7]))};
-  return __builtin_bit_cast(mf_f16x8, w);
-}
-
 __device__ __forceinline__ mf_f16x8 cat8(const mf_f16x4 a, const mf_f16x4 b) {
   return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
 }
@@ -260,12 +288,13 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 // DPP lane moves within rows of 16 (VALU, no LDS): quad_perm [1,0,3,2], quad_perm [2,3,0,1], row_half_mirror,
-// row_mirror.
+// row_mirror, row_ror 4 and 8.
 template <int CTRL>
 __device__ __forceinline__ uint32_t dpp(uint32_t v) {
   return uint32_t(__builtin_amdgcn_update_dpp(0, int(v), CTRL, 0xf, 0xf, false));
 }
 constexpr int kDppXor1 = 0xb1, kDppXor2 = 0x4e, kDppHalfMirror = 0x141, kDppMirror = 0x140;
+constexpr int kDppRor4 = 0x124, kDppRor8 = 0x128;
 
 // Maximum over the wave in every lane: within rows by DPP, across the four rows by the gfx950 lane swaps.
 __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
@@ -286,13 +315,18 @@ __device__ __forceinline__ float sum8(float x) {
   return x + __uint_as_float(dpp<kDppHalfMirror>(__float_as_uint(x)));
 }
 
-// Sum over each 16-lane row, in every lane of the row.
-__device__ __forceinline__ float row16_sum(float x) {
-  x = sum8(x);
-  return x + __uint_as_float(dpp<kDppMirror>(__float_as_uint(x)));
+// Sums over the four 16-lane groups of four values at once: lane group g returns the sum of x[g], added as
+// (g0 + g2) + (g1 + g3).  Each lane swap leaves two values' halves where one add joins both.
+__device__ __forceinline__ float sum_groups4(const float x0, const float x1, const float x2, const float x3) {
+  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x0), __float_as_uint(x2), false, false);
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x1), __float_as_uint(x3), false, false);
+  const float y = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  const float z = __uint_as_float(b[0]) + __uint_as_float(b[1]);
+  const auto c = __builtin_amdgcn_permlane16_swap(__float_as_uint(y), __float_as_uint(z), false, false);
+  return __uint_as_float(c[0]) + __uint_as_float(c[1]);
 }
 
-// Sum over the four 16-lane groups, (g0 + g2) + (g1 + g3) in every lane: the gfx950 lane swaps (VALU, no LDS).
+// Sum over the four lane groups, in every lane.
 __device__ __forceinline__ float sum_groups(float x) {
   const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
   const float y = __uint_as_float(a[0]) + __uint_as_float(a[1]);
@@ -300,17 +334,69 @@ __device__ __forceinline__ float sum_groups(float x) {
   return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
-// The unit list (one workgroup).  Mask rows r = 2 b (valid keys of molecule b) and 2 b + 1 (valid queries)
-// are read four per wave at a time, every byte load issued before the first ballot; each row's count and, when
-// it is at most kMaxN, its list of atoms go to the workspace.  Then the LPT rank of each served molecule (unit
-// cost descending, ties by index) and its list positions = prefix sums of the units ranked before it.
-__global__ void __launch_bounds__(kPlanThreads) pair_bwd_plan(PlanParams pp) {
+// Sum over each 16-lane row, in every lane of the row.
+__device__ __forceinline__ float row16_sum(float x) {
+  x = sum8(x);
+  return x + __uint_as_float(dpp<kDppMirror>(__float_as_uint(x)));
+}
+
+// Sums over each 16-lane row of four values: lane r16 returns the sum of v[r16 & 3].  Two exchange steps leave that
+// value in the lane, two rotations finish the sum.
+__device__ __forceinline__ float row16_sum4(const float (&v)[4], int r16) {
+  const bool o1 = (r16 & 1) != 0, o2 = (r16 & 2) != 0;
+  float w[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const float keep = o1 ? v[2 * h + 1] : v[2 * h], send = o1 ? v[2 * h] : v[2 * h + 1];
+    w[h] = keep + __uint_as_float(dpp<kDppXor1>(__float_as_uint(send)));
+  }
+  const float keep = o2 ? w[1] : w[0], send = o2 ? w[0] : w[1];
+  float x = keep + __uint_as_float(dpp<kDppXor2>(__float_as_uint(send)));
+  x += __uint_as_float(dpp<kDppRor4>(__float_as_uint(x)));
+  return x + __uint_as_float(dpp<kDppRor8>(__float_as_uint(x)));
+}
+
+// One bias element as fp32 (BIAS 1: bf16, 2: fp32).
+template <int BIAS>
+__device__ __forceinline__ float load_bias(const void* p, size_t i) {
+  if constexpr (BIAS == 2) return static_cast<const float*>(p)[i];
+  else return bf_u16(static_cast<const uint16_t*>(p)[i]);
+}
+
+// The prepare launch.  Workgroup 0 makes the unit list: mask rows r = 2 b (valid keys of molecule b) and
+// 2 b + 1 (valid queries) are read four per wave at a time, every byte load issued before the first ballot; each
+// row's count and its list of atoms go to the workspace.  Then the j per unit, the LPT rank of each molecule
+// (unit cost descending, ties by index) and its list positions = prefix sums of the units ranked before it.
+// Workgroups 1 .. B H (16-bit gradients): the zero rows of one (molecule, head) each -- padded queries (dq) and
+// keys (dk1, dv1, dk2, dv2), and every row of a molecule without a valid query or key.
+__global__ void __launch_bounds__(kPlanThreads) pair_bwd_prepare(PlanParams pp) {
   __shared__ uint32_t s_cost[kMaxPlanBatch];
   __shared__ int s_units[kMaxPlanBatch];
   __shared__ int s_count[2 * kMaxPlanBatch];
-  __shared__ int s_total, s_unserved;
+  __shared__ int s_total, s_level[3];
   const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
   const int B = pp.B, H = pp.H, N = pp.N;
+  if (blockIdx.x > 0) {
+    const int bh = int(blockIdx.x) - 1, b = bh / H;
+    const uint8_t* mq = pp.qv + size_t(b) * N;
+    const uint8_t* mk = pp.pkv + size_t(b) * N;
+    const int any_q = __syncthreads_or(tid < N && mq[min(tid, N - 1)] != 0);
+    const int any_k = __syncthreads_or(tid < N && mk[min(tid, N - 1)] != 0);
+    const bool empty = !any_q || !any_k;
+    const size_t base = size_t(bh) * N * (DP / 8);
+    const uint4 z{0u, 0u, 0u, 0u};
+    for (int u = tid; u < N * (DP / 8); u += kPlanThreads) {
+      const int row = u / (DP / 8);
+      if (empty || mq[row] == 0) static_cast<uint4*>(pp.dq)[base + u] = z;
+      if (empty || mk[row] == 0) {
+        static_cast<uint4*>(pp.dk1)[base + u] = z;
+        static_cast<uint4*>(pp.dv1)[base + u] = z;
+        static_cast<uint4*>(pp.dk2)[base + u] = z;
+        static_cast<uint4*>(pp.dv2)[base + u] = z;
+      }
+    }
+    return;
+  }
   constexpr int kRows = 4;
   for (int r0 = kRows * wave; r0 < 2 * B; r0 += kRows * (kPlanThreads / 64)) {
     uint8_t v[kRows][kMaxTokens / 64];
@@ -331,35 +417,39 @@ __global__ void __launch_bounds__(kPlanThreads) pair_bwd_plan(PlanParams pp) {
     for (int rr = 0; rr < kRows; ++rr) {
       const int r = r0 + rr;
       if (r >= 2 * B) break;  // uniform
-      uint16_t* list = pp.lists + size_t(r >> 1) * 2 * kMaxN + (r & 1) * kMaxN;
+      uint16_t* list = pp.lists + size_t(r) * N;
       int count = 0;
 #pragma unroll
       for (int sg = 0; sg < kMaxTokens / 64; ++sg) {
         const bool on = v[rr][sg] != 0;
         const unsigned long long bal = __ballot(on);
-        const int at = count + __popcll(bal & ((1ull << lane) - 1ull));
-        if (on && at < kMaxN) list[at] = uint16_t(64 * sg + lane);
+        if (on) list[count + __popcll(bal & ((1ull << lane) - 1ull))] = uint16_t(64 * sg + lane);
         count += __popcll(bal);
       }
       if (lane == 0) s_count[r] = count;
     }
   }
-  if (tid == 0) {
-    s_total = 0;
-    s_unserved = 0;
-  }
+  if (tid == 0) s_total = 0;
+  if (tid < 3) s_level[tid] = 0;
   lds_barrier();
+  // units at jm, jm / 2 and jm / 4 j per unit; the largest j that still gives two units per CU (512), else jm / 4
   for (int b = tid; b < B; b += kPlanThreads) {
     const int nk = s_count[2 * b], nq = s_count[2 * b + 1];
-    const bool served = nk > 0 && nq > 0 && nk <= kMaxN && nq <= kMaxN;
-    s_cost[b] = served ? unit_cost(nk, nq) : 0u;
-    s_units[b] = served ? H * parts_of(nk) : 0;
-    pp.served[b] = served ? 1 : 0;
-    if (!served && nk > 0 && nq > 0) atomicAdd(&s_unserved, 1);
+    if (nk <= 0 || nq <= 0) continue;
+#pragma unroll
+    for (int l = 0; l < 3; ++l) atomicAdd(&s_level[l], H * parts_of(nk, pp.jm >> l, pp.cap));
+  }
+  lds_barrier();
+  const int jt = s_level[0] >= 512 ? pp.jm : (s_level[1] >= 512 ? pp.jm / 2 : pp.jm / 4);
+  for (int b = tid; b < B; b += kPlanThreads) {
+    const int nk = s_count[2 * b], nq = s_count[2 * b + 1];
+    const bool work = nk > 0 && nq > 0;
+    s_cost[b] = work ? unit_cost(nk, nq, jt, pp.cap) : 0u;
+    s_units[b] = work ? H * parts_of(nk, jt, pp.cap) : 0;
     pp.counts[b] = int2{nk, nq};
   }
   lds_barrier();
-  // rank: kTpm threads per molecule, each over every kTpm-th other molecule, partial sums added over the
+  // rank: tpm threads per molecule, each over every tpm-th other molecule, partial sums added over the
   // thread group (adjacent lanes) by shuffles
   const int tpm = B >= kPlanThreads ? 1 : (B > kPlanThreads / 2 ? 2 : (B > kPlanThreads / 4 ? 4 : (B > kPlanThreads / 8 ? 8 : 16)));
   for (int t0 = 0; t0 < B * tpm; t0 += kPlanThreads) {
@@ -372,905 +462,874 @@ __global__ void __launch_bounds__(kPlanThreads) pair_bwd_plan(PlanParams pp) {
         if (s_cost[o] > cb || (s_cost[o] == cb && o < b)) pre += s_units[o];
     }
     for (int off = 1; off < tpm; off <<= 1) pre += __shfl_xor(pre, off, 64);
-    if (b < B && sub == 0) {
-      const int parts = parts_of(s_count[2 * b]);
-      for (int u = 0; u < s_units[b]; ++u)
-        pp.units[pre + u] = (uint32_t(b * H + u / parts) << 1) | uint32_t(u % parts);
-      atomicAdd(&s_total, s_units[b]);
+    if (b < B && s_units[b] > 0) {
+      const int parts = s_units[b] / H;
+      for (int u = sub; u < s_units[b]; u += tpm)
+        pp.units[pre + u] = (uint32_t(b * H + u / parts) << 6) | uint32_t(u % parts);
+      if (sub == 0) atomicAdd(&s_total, s_units[b]);
     }
   }
   lds_barrier();
   if (tid == 0) {
-    pp.total[0] = s_total;
-    pp.total[1] = s_unserved;
+    pp.head[0] = s_total;
+    pp.head[1] = jt;
   }
 }
 
-// The unit's main loop (key tiles x key pairs x NQT query tiles from tile qt0), its dk1 / dv1 rows, dq, and
-// for a split molecule the combination of the two halves.  LDS as staged by the kernel.  A unit may run its
-// query tiles in passes (first .. last): every key-side sum is linear in the queries, so a later pass adds to
-// what the earlier ones left (dk2 / dv2 partials in the unit's slab rows, the dk1 / dv1 sums and dw in the
-// workspace, each read back by the thread that wrote it); dq and the query-side bias sums belong to the pass.
-template <int NQT, bool BIAS>
-__device__ __forceinline__ void unit_body(const Params& p, unsigned char* smem, int nq, int nk, int part, int parts,
-                                          int bh, bool has_pv, int qt0, bool first, bool last) {
-  using Ly = Lay<BIAS>;
-  const int q0 = qt0 * 16;
-  const int tid = threadIdx.x;
-  const int lane = lane_id();
-  const int wave = wave_id();
+// The thread index, opaque to the compiler: what is computed from it stays inside the loop that asks, instead of
+// being hoisted out of the block loops into registers (and from there into scratch) held throughout.
+__device__ __forceinline__ int opaque_tid() {
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
+// One block triple of a unit as the kernel staged it: nq queries from q0, nj j keys from j0, nk keys from k0
+// (compacted positions), the scale exponents of its operands.
+struct Triple {
+  int bh, part, q0, nq, j0, nj, k0, nk;
+  int eq, eg, e1, e2, f1, f2;       // exponents of q, go, k1, k2, v1, v2
+  bool direct;                      // the molecule's only triple: gradients written here, not to the slab
+  bool first_q, first_k;            // the unit's first triple with these queries (dq) / these keys (dk2, dv2)
+  bool first_t;                     // the unit's first triple with these (queries, keys): dv_bias
+};
+
+// Row `row`, columns d4 .. d4 + 3 of the four waves' partial sums, added in wave order, times f.
+__device__ __forceinline__ float4 sum_partials(const float* slot, int row, int d4, float f) {
+  float4 s = *reinterpret_cast<const float4*>(slot + row * PS + d4);
+#pragma unroll
+  for (int w = 1; w < kWaves; ++w) {
+    const float4 x = *reinterpret_cast<const float4*>(slot + (w * 16 + row) * PS + d4);
+    s.x += x.x; s.y += x.y; s.z += x.z; s.w += x.w;
+  }
+  return float4{s.x * f, s.y * f, s.z * f, s.w * f};
+}
+
+// Four gradient elements, fp32 or rounded to bf16 (16-byte aligned tensors, whole rows of 64).
+__device__ __forceinline__ void store_grad4(void* base, size_t i, const float4 v, int bf16) {
+  if (bf16) {
+    const uint2 w{__builtin_bit_cast(uint32_t, mf_bf16x2{__bf16(v.x), __bf16(v.y)}),
+                  __builtin_bit_cast(uint32_t, mf_bf16x2{__bf16(v.z), __bf16(v.w)})};
+    *reinterpret_cast<uint2*>(static_cast<__bf16*>(base) + i) = w;
+  } else {
+    *reinterpret_cast<float4*>(static_cast<float*>(base) + i) = v;
+  }
+}
+
+// A unit's running sum of a slab row (this thread wrote what it reads back).
+__device__ __forceinline__ void add_slab(float* p, float4 s, bool first) {
+  if (!first) {
+    const float4 o = *reinterpret_cast<const float4*>(p);
+    s.x += o.x; s.y += o.y; s.z += o.z; s.w += o.w;
+  }
+  *reinterpret_cast<float4*>(p) = s;
+}
+
+// The main loop over one triple and its sums.
+template <int NQT, int BIAS>
+__device__ __forceinline__ void triple_body(const Params& p, unsigned char* smem, const Triple& c) {
+  using Ly = Lay<BIAS != 0>;
+  constexpr int QM = Ly::QM, JM = Ly::JM, KM = Ly::KM, KU = Ly::KU, KW = Ly::KW;
+  const int tid = opaque_tid();
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4;
   const int r16 = lane & 15;
-  const size_t rbase = size_t(bh) * p.N;
-  // split molecules: part 1's partial dq, dk2, dv2 go to its slab, and part 0's too when the gradients are
-  // 16-bit (fp32 ones hold part 0's partials in the gradient rows until the combine launch)
-  const bool to_slab = parts == 2 && (part == 1 || p.gout16 != 0);
-  float* slab = p.slab + (size_t(bh) * 2 + part) * 5 * kMaxN * DP;
+  const int N = p.N;
+  const size_t rbase = size_t(c.bh) * N;
+  float* slab = p.slab + (size_t(c.bh) * p.cap + c.part) * 3 * N * DP;
   _Float16* Qs = reinterpret_cast<_Float16*>(smem + Ly::rows);
-  _Float16* Gs = Qs + kMaxN * KS;
-  _Float16* K1s = Gs + kMaxN * KS;
-  _Float16* K2s = K1s + kMaxN * KS;
-  _Float16* V1s = K2s + kMaxN * KS;
-  _Float16* V2s = V1s + kMaxN * KS;
+  _Float16* Gs = Qs + QM * KS;
+  _Float16* K1s = Gs + QM * KS;
+  _Float16* V1s = K1s + JM * KS;
+  _Float16* K2s = V1s + JM * KS;
+  _Float16* V2s = K2s + KM * KS;
   float* dk1a = reinterpret_cast<float*>(smem + Ly::acc1);
-  float* dv1a = dk1a + kMaxN * DP;
-  float* slot = reinterpret_cast<float*>(smem + Ly::slot);
-  _Float16* scr = reinterpret_cast<_Float16*>(smem + Ly::scr) + wave * 2 * 32 * SS;
-  const float* con = reinterpret_cast<const float*>(smem + Ly::con);
-  const float cS = con[kCS], cP = con[kCP];
-  const float* lse2 = reinterpret_cast<const float*>(smem + Ly::lse2) + q0;  // the pass's queries
-  const float* dlt = reinterpret_cast<const float*>(smem + Ly::dlt) + q0;
-  const _Float16* Qp = Qs + q0 * KS;
-  const _Float16* Gp = Gs + q0 * KS;
+  float* dv1a = dk1a + JM * DP;
+  float* slot = reinterpret_cast<float*>(smem + Ly::scr);
+  _Float16* scr = reinterpret_cast<_Float16*>(smem + Ly::scr) + wave * (QM / 16) * 32 * SS;
+  const float* uT = reinterpret_cast<const float*>(smem + Ly::ut);
+  const float* vT = reinterpret_cast<const float*>(smem + Ly::vt);
+  float* dut = reinterpret_cast<float*>(smem + Ly::dut);
+  float* wd = reinterpret_cast<float*>(smem + Ly::wd);
+  const float* cg = reinterpret_cast<const float*>(smem + Ly::gt);
+  const float* lse2 = reinterpret_cast<const float*>(smem + Ly::lse2);
+  const float* dls = reinterpret_cast<const float*>(smem + Ly::dls);
   const uint32_t* pvb = reinterpret_cast<const uint32_t*>(smem + Ly::pvb);
   const int* kidx = reinterpret_cast<const int*>(smem + Ly::kidx);
   const int* qidx = reinterpret_cast<const int*>(smem + Ly::qidx);
-  // BIAS: the staged bias terms, and the dk1 / dv1 sums of the unit's keys in the workspace (slab rows 3, 4)
-  const uint16_t* uT = reinterpret_cast<const uint16_t*>(smem + Ly::ut) + q0;
-  const uint16_t* vT = reinterpret_cast<const uint16_t*>(smem + Ly::vt) + q0;
-  const float* cg = reinterpret_cast<const float*>(smem + Ly::gt) + q0;
-  float* sk1 = slab + 3 * kMaxN * DP;
-  float* sv1 = slab + 4 * kMaxN * DP;
-  const int N = p.N;
-  // BIAS: the B operand that sums dS over the keys of each j of a pair tile (column c = pair j index)
-  const mf_f16x8 jsum = r16 == (g >> 1) ? mf_f16x8{1, 1, 1, 1, 1, 1, 1, 1} : mf_f16x8{0, 0, 0, 0, 0, 0, 0, 0};
+  // dS is carried as dS 2^-es, |dS 2^-es| < 2^15:  S log2 e = S_c cS,  dS 2^-es = P (dP_c cP - delta 2^-es)
+  const int es = c.eg + c.f1 + c.f2 - 5;
+  const float cS = ldexpf(kLog2e, c.eq + c.e1 + c.e2);
+  constexpr float cP = 32.0f;  // 2^(eg + f1 + f2 - es)
+  const float uD = ldexpf(1.0f, es);
+  const float fk1 = ldexpf(1.0f, c.e2 + es + c.eq), fv1 = ldexpf(1.0f, c.f2 + c.eg);
 
-  const int nkt = (nk + 15) / 16;
-  const int njp = (nk + 1) / 2;
-  // BIAS: dgate partial of queries qt 16 + 4 g + r over the lane's (j, k)
-  float accg[NQT][4];
-#pragma unroll
-  for (int t = 0; t < NQT; ++t)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) accg[t][r] = 0.0f;
+  const int nkt = (c.nk + 15) / 16;
+  const int njp = (c.nj + 1) / 2;
 
   mf_f32x4 dqa[NQT][4];
 #pragma unroll
   for (int t = 0; t < NQT; ++t)
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt) dqa[t][dt] = mf_f32x4{0.f, 0.f, 0.f, 0.f};
-
+  // BIAS: dgate partial of queries 16 t + 4 g + r over the lane's (j, k)
+  float accg[BIAS ? NQT : 1][4];
+#pragma unroll
+  for (int t = 0; t < (BIAS ? NQT : 1); ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) accg[t][r] = 0.0f;
   for (int kt = 0; kt < nkt; ++kt) {
     const int k0 = kt * 16;
-    // key k0 + r16 at d = 32 s + 8 g + e: the B operands of S and dP
-    mf_f16x8 k2c[2], v2c[2];
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      k2c[s] = *reinterpret_cast<const mf_f16x8*>(K2s + (k0 + r16) * KS + 32 * s + 8 * g);
-      v2c[s] = *reinterpret_cast<const mf_f16x8*>(V2s + (k0 + r16) * KS + 32 * s + 8 * g);
-    }
-    // keys k0 + 8 (g & 1) + e at d = 16 dt + r16: the dq B operand (transposed reads; lane 4 e' + a of a group
-    // addresses row e' (+4), columns 4 a .. 4 a + 3)
-    mf_f16x8 kcol[4];
-    // keys k0 + 4 g + r at d = 16 dt + r16: the dk1 / dv1 sums (BIAS: read in each pair tile's epilogue, which
-    // leaves the registers to the bias sums)
-    float kk2[4][4], kv2[4][4];
-    auto read_kv2 = [&](int dt) {
-      const int roff = (k0 + 4 * g + (r16 >> 2)) * KS + 16 * dt + 4 * (r16 & 3);
-      const auto a4 = read_tr16(K2s + roff);
-      const auto b4 = read_tr16(V2s + roff);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        kk2[dt][r] = float(a4[r]);
-        kv2[dt][r] = float(b4[r]);
-      }
-    };
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt) {
-      const _Float16* pc = K2s + (k0 + 8 * (g & 1) + (r16 >> 2)) * KS + 16 * dt + 4 * (r16 & 3);
-      kcol[dt] = cat8(read_tr16(pc), read_tr16(pc + 4 * KS));
-      if constexpr (!BIAS) read_kv2(dt);
-    }
-    // BIAS: this wave's dv_bias partials of the key tile (LDS, [qt][key r16][query 4 g + r])
-    float* dvl = reinterpret_cast<float*>(smem + Ly::dvb) + wave * NT * 256;
-    if constexpr (BIAS) {
-#pragma unroll
-      for (int qt = 0; qt < NQT; ++qt)
-        *reinterpret_cast<float4*>(dvl + (qt * 16 + r16) * 16 + 4 * g) = float4{0.f, 0.f, 0.f, 0.f};
-    }
     mf_f32x4 dk2a[4], dv2a[4];  // key k0 + 4 g + r, d = 16 dt + r16
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt) {
       dk2a[dt] = mf_f32x4{0.f, 0.f, 0.f, 0.f};
       dv2a[dt] = mf_f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    const bool kvalid = k0 + r16 < nk;
+    float dva[BIAS ? NQT : 1][4];  // dv_bias partial of the lane's (query, key) over the wave's j
+#pragma unroll
+    for (int t = 0; t < (BIAS ? NQT : 1); ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) dva[t][r] = 0.0f;
 
-    for (int jp = part + parts * wave; jp < njp; jp += parts * kWaves) {
+    for (int jp = wave; jp < njp; jp += kWaves) {
       const int ja = 2 * jp;
-      // BIAS: w of pairs (ja + jn, k0 + r16) (clamped indices, unconditional loads), and dw partials
-      float wv[2] = {0.0f, 0.0f}, dwa[2] = {0.0f, 0.0f};
-      if constexpr (BIAS) {
-        const int kc = kidx[min(k0 + r16, nk - 1)];
-#pragma unroll
-        for (int jn = 0; jn < 2; ++jn) wv[jn] = bf_u16(p.bw[(rbase + kidx[min(ja + jn, nk - 1)]) * N + kc]);
-      }
-      // the epilogue's LDS operands, read now so that their latency hides under the query loop:
-      // k1 / v1 of j = ja + jn at d = 16 dt + r16, and the dk1 / dv1 sums of j so far
-      _Float16 k1h[2][4];
-      float k1p[2][4], v1p[2][4], d1k[2][4], d1v[2][4];
-#pragma unroll
-      for (int jn = 0; jn < 2; ++jn)
-#pragma unroll
-        for (int dt = 0; dt < 4; ++dt) {
-          k1h[jn][dt] = K1s[(ja + jn) * KS + 16 * dt + r16];
-          if constexpr (!BIAS) {
-            k1p[jn][dt] = float(k1h[jn][dt]);
-            v1p[jn][dt] = float(V1s[(ja + jn) * KS + 16 * dt + r16]);
-          }
-          if constexpr (BIAS) {
-            d1k[jn][dt] = sk1[(ja + jn) * DP + 16 * dt + r16];
-            d1v[jn][dt] = sv1[(ja + jn) * DP + 16 * dt + r16];
-          } else {
-            d1k[jn][dt] = dk1a[(ja + jn) * DP + 16 * dt + r16];
-            d1v[jn][dt] = dv1a[(ja + jn) * DP + 16 * dt + r16];
-          }
-        }
-      if constexpr (BIAS) {  // the workspace rows hold sums only after the first key tile (read back by the
-                             // g = 0 lanes that wrote them: the same thread, so in order)
-        if (kt == 0 && first) {
-#pragma unroll
-          for (int jn = 0; jn < 2; ++jn)
-#pragma unroll
-            for (int dt = 0; dt < 4; ++dt) {
-              d1k[jn][dt] = 0.0f;
-              d1v[jn][dt] = 0.0f;
-            }
-        }
-      }
-      // ---- the pair tile's operands: W, Z (hi, lo) of pairs (ja + jn, k0 + r16), d = 32 s + 8 g + e ----
-      mf_f16x8 wb[2][2], zh[2][2], zl[2][2];
-#pragma unroll
-      for (int jn = 0; jn < 2; ++jn)
+      // (BIAS: the LDS addresses are formed again for each pair, a few VALU, instead of living in scratch)
+      int ol = lane;
+      if constexpr (BIAS != 0) asm volatile("" : "+v"(ol));
+      const int g = ol >> 4, r16 = ol & 15;
+      mf_f16x8 wb[2][2], zh[2][2], zl[2][2];  // W, Z (hi, lo) of pairs (ja + jn, k0 + r16), d = 32 s + 8 g + e
+      bool ok[2];
+      auto form = [&](int jn) {
+        const int j = ja + jn;
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
-          const mf_f16x8 a = *reinterpret_cast<const mf_f16x8*>(K1s + (ja + jn) * KS + 32 * s + 8 * g);
-          const mf_f16x8 c = *reinterpret_cast<const mf_f16x8*>(V1s + (ja + jn) * KS + 32 * s + 8 * g);
-          wb[jn][s] = a * k2c[s];
-          zh[jn][s] = c * v2c[s];
-          zl[jn][s] = __builtin_elementwise_fma(c, v2c[s], -zh[jn][s]);
+          const mf_f16x8 a = *reinterpret_cast<const mf_f16x8*>(K1s + j * KS + 32 * s + 8 * g);
+          const mf_f16x8 b = *reinterpret_cast<const mf_f16x8*>(V1s + j * KS + 32 * s + 8 * g);
+          const mf_f16x8 k2c = *reinterpret_cast<const mf_f16x8*>(K2s + (k0 + r16) * KS + 32 * s + 8 * g);
+          const mf_f16x8 v2c = *reinterpret_cast<const mf_f16x8*>(V2s + (k0 + r16) * KS + 32 * s + 8 * g);
+          wb[jn][s] = a * k2c;
+          zh[jn][s] = b * v2c;
+          zl[jn][s] = __builtin_elementwise_fma(b, v2c, -zh[jn][s]);
         }
-      // W of pairs (ja + (g >> 1), k0 + 8 (g & 1) + e) at d = 16 dt + r16: the dq B operand
-      mf_f16x8 wc[4];
+        ok[jn] = ((pvb[j * 2 + ((k0 + r16) >> 5)] >> ((k0 + r16) & 31)) & 1u) != 0u;
+      };
+      // P and dS of (j, query tile) as packed fp16: word r / 2 of query 16 t + 4 g + r, key k0 + r16
+      uint2 dsw[2][NQT], pw[2][NQT];
+      auto score = [&](int jn, int t, const mf_f16x8 (&aq)[2], const mf_f16x8 (&ag)[2], float wj, float& dwj,
+                       float (&dsv)[4]) {
+        mf_f32x4 sacc = mf_f32x4{0.f, 0.f, 0.f, 0.f}, pacc = mf_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int dt = 0; dt < 4; ++dt) wc[dt] = kcol[dt] * ((g >> 1) ? k1h[1][dt] : k1h[0][dt]);
-      bool pok[2];
-#pragma unroll
-      for (int jn = 0; jn < 2; ++jn) {
-        const int j = ja + jn;
-        pok[jn] = kvalid && j < nk && (!has_pv || ((pvb[j * 3 + ((k0 + r16) >> 5)] >> ((k0 + r16) & 31)) & 1u));
-      }
-
-      mf_f32x4 gt[2][4], ht[2][4];  // G^T, H^T of the pair tile: key k0 + 4 g + r, d = 16 dt + r16
-#pragma unroll
-      for (int jn = 0; jn < 2; ++jn)
-#pragma unroll
-        for (int dt = 0; dt < 4; ++dt) {
-          gt[jn][dt] = mf_f32x4{0.f, 0.f, 0.f, 0.f};
-          ht[jn][dt] = mf_f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int s = 0; s < 2; ++s) {
+          sacc = mma(aq[s], wb[jn][s], sacc);
+          pacc = mma(ag[s], zh[jn][s], pacc);
+          pacc = mma(ag[s], zl[jn][s], pacc);
         }
-
+        const float4 l2 = *reinterpret_cast<const float4*>(lse2 + t * 16 + 4 * g);
+        const float4 dl = *reinterpret_cast<const float4*>(dls + t * 16 + 4 * g);
+        const float l2v[4] = {l2.x, l2.y, l2.z, l2.w};
+        const float dlv[4] = {dl.x, dl.y, dl.z, dl.w};
+        float cl[4], base[4], pp[4];
+        if constexpr (BIAS != 0) {  // gate_i (u_ij + v_ik + w_jk) of the lane's queries and pair
+          const float4 c4 = *reinterpret_cast<const float4*>(cg + t * 16 + 4 * g);
+          const float4 u4 = *reinterpret_cast<const float4*>(uT + (ja + jn) * KU + t * 16 + 4 * g);
+          const float4 v4 = *reinterpret_cast<const float4*>(vT + (k0 + r16) * KU + t * 16 + 4 * g);
+          cl[0] = c4.x; cl[1] = c4.y; cl[2] = c4.z; cl[3] = c4.w;
+          base[0] = (u4.x + v4.x) + wj;
+          base[1] = (u4.y + v4.y) + wj;
+          base[2] = (u4.z + v4.z) + wj;
+          base[3] = (u4.w + v4.w) + wj;
+        }
 #pragma unroll
-      for (int qb = 0; qb < NQT; qb += 2) {
-        // The block's two query tiles side by side (independent chains): S and dP, softmax, dS through the
-        // wave's scratch (one slot per tile) for dq.  A tile past NQT carries zeros.
-        const int NH = qb + 1 < NQT ? 2 : 1;
-        float dsv[2][2][4], pvv[2][2][4];  // [half][jn][r]: query (qb + half) 16 + 4 g + r, key k0 + r16
-        mf_f32x4 sacc[2][2], pacc[2][2];
-#pragma unroll
-        for (int h = 0; h < NH; ++h)
-#pragma unroll
-          for (int jn = 0; jn < 2; ++jn) {
-            sacc[h][jn] = mf_f32x4{0.f, 0.f, 0.f, 0.f};
-            pacc[h][jn] = mf_f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int r = 0; r < 4; ++r) {
+          float s2 = fmaf(sacc[r], cS, -l2v[r]);
+          if constexpr (BIAS != 0) s2 = fmaf(cl[r], base[r], s2);
+          pp[r] = ok[jn] ? fast_exp2(s2) : 0.0f;
+          dsv[r] = pp[r] * fmaf(pacc[r], cP, -dlv[r]);
+          if constexpr (BIAS != 0) {
+            accg[t][r] = fmaf(dsv[r], base[r], accg[t][r]);
+            dwj = fmaf(cl[r], dsv[r], dwj);
+            dva[t][r] += dsv[r];
           }
+        }
+        dsw[jn][t] = uint2{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(dsv[0], dsv[1])),
+                           __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(dsv[2], dsv[3]))};
+        pw[jn][t] = uint2{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(pp[0], pp[1])),
+                          __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(pp[2], pp[3]))};
+        // dS [pair (jn, key)][query] into the tile's slot of the wave's scratch
+        *reinterpret_cast<uint2*>(scr + t * 32 * SS + (jn * 16 + r16) * SS + 4 * g) = dsw[jn][t];
+      };
+      auto rows_of = [&](const _Float16* base, int t, mf_f16x8 (&a)[2]) {
 #pragma unroll
         for (int s = 0; s < 2; ++s)
+          a[s] = *reinterpret_cast<const mf_f16x8*>(base + (t * 16 + r16) * KS + 32 * s + 8 * g);
+      };
+      if constexpr (BIAS == 0 && NQT < 4) {  // both j share the rows of a query tile
+        form(0);
+        form(1);
 #pragma unroll
-          for (int h = 0; h < NH; ++h) {
-            const int qt = qb + h;
-            const mf_f16x8 aq = *reinterpret_cast<const mf_f16x8*>(Qp + (qt * 16 + r16) * KS + 32 * s + 8 * g);
-            const mf_f16x8 ag = *reinterpret_cast<const mf_f16x8*>(Gp + (qt * 16 + r16) * KS + 32 * s + 8 * g);
-#pragma unroll
-            for (int jn = 0; jn < 2; ++jn) {
-              sacc[h][jn] = mma(aq, wb[jn][s], sacc[h][jn]);
-              pacc[h][jn] = mma(ag, zh[jn][s], pacc[h][jn]);
-            }
-#pragma unroll
-            for (int jn = 0; jn < 2; ++jn) pacc[h][jn] = mma(ag, zl[jn][s], pacc[h][jn]);
-          }
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          if (h >= NH) {
-#pragma unroll
-            for (int jn = 0; jn < 2; ++jn)
-#pragma unroll
-              for (int r = 0; r < 4; ++r) {
-                dsv[h][jn][r] = 0.0f;
-                pvv[h][jn][r] = 0.0f;
-              }
-            continue;
-          }
-          const int qt = qb + h;
-          const float4 l2 = *reinterpret_cast<const float4*>(lse2 + qt * 16 + 4 * g);
-          const float4 dl = *reinterpret_cast<const float4*>(dlt + qt * 16 + 4 * g);
-          const float l2v[4] = {l2.x, l2.y, l2.z, l2.w};
-          const float dlv[4] = {dl.x, dl.y, dl.z, dl.w};
-          // BIAS: gate_i (u_ij + v_ik + w_jk) of the lane's queries and pairs (natural units)
-          float cl[4] = {0.f, 0.f, 0.f, 0.f}, base[2][4];
-          if constexpr (BIAS) {
-            // (the offset is opaque to the compiler, so these loads stay here instead of being hoisted out of
-            // the loops into registers held throughout)
-            int qo = qt * 16 + 4 * g;
-            asm volatile("" : "+v"(qo));
-            const float4 l4 = *reinterpret_cast<const float4*>(cg + kMaxN + qo);
-            cl[0] = l4.x; cl[1] = l4.y; cl[2] = l4.z; cl[3] = l4.w;
-            const uint2 v4 = *reinterpret_cast<const uint2*>(vT + (k0 + r16) * KU + qo);
-            const float vv[4] = {bf_lo(v4.x), bf_hi(v4.x), bf_lo(v4.y), bf_hi(v4.y)};
-#pragma unroll
-            for (int jn = 0; jn < 2; ++jn) {
-              const uint2 u4 = *reinterpret_cast<const uint2*>(uT + (ja + jn) * KU + qo);
-              const float uu[4] = {bf_lo(u4.x), bf_hi(u4.x), bf_lo(u4.y), bf_hi(u4.y)};
-#pragma unroll
-              for (int r = 0; r < 4; ++r) base[jn][r] = (uu[r] + vv[r]) + wv[jn];
-            }
-          }
-#pragma unroll
-          for (int jn = 0; jn < 2; ++jn)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              float s2 = fmaf(sacc[h][jn][r], cS, -l2v[r]);
-              if constexpr (BIAS) s2 = fmaf(cl[r], base[jn][r], s2);
-              const float pp = pok[jn] ? fast_exp2(s2) : 0.0f;
-              pvv[h][jn][r] = pp;
-              dsv[h][jn][r] = pp * fmaf(pacc[h][jn][r], cP, -dlv[r]);
-              if constexpr (BIAS) {
-                accg[qt][r] = fmaf(dsv[h][jn][r], base[jn][r], accg[qt][r]);
-                dwa[jn] = fmaf(cl[r], dsv[h][jn][r], dwa[jn]);
-              }
-            }
-          if constexpr (BIAS) {
-            int vo = (qt * 16 + r16) * 16 + 4 * g;
-            asm volatile("" : "+v"(vo));
-            float4* pv = reinterpret_cast<float4*>(dvl + vo);
-            float4 a = *pv;
-            a.x += dsv[h][0][0] + dsv[h][1][0];
-            a.y += dsv[h][0][1] + dsv[h][1][1];
-            a.z += dsv[h][0][2] + dsv[h][1][2];
-            a.w += dsv[h][0][3] + dsv[h][1][3];
-            *pv = a;
-          }
-          // dS [pair (jn, key)][query] into slot h of the wave's scratch
-#pragma unroll
-          for (int jn = 0; jn < 2; ++jn) {
-            const uint2 v{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(dsv[h][jn][0], dsv[h][jn][1])),
-                          __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(dsv[h][jn][2], dsv[h][jn][3]))};
-            *reinterpret_cast<uint2*>(scr + h * 32 * SS + (jn * 16 + r16) * SS + 4 * g) = v;
-          }
+        for (int t = 0; t < NQT; ++t) {
+          mf_f16x8 aq[2], ag[2];
+          rows_of(Qs, t, aq);
+          rows_of(Gs, t, ag);
+          float ds[4], none = 0.0f;
+          score(0, t, aq, ag, 0.0f, none, ds);
+          score(1, t, aq, ag, 0.0f, none, ds);
         }
-        __builtin_amdgcn_wave_barrier();
-        // dq of queries qt 16 + r16: A = dS [query][pairs (jn = g >> 1, keys 8 (g & 1) + e)] by transposed reads
-        mf_f16x8 ads[2];
-#pragma unroll
-        for (int h = 0; h < NH; ++h) {
-          const _Float16* ps = scr + h * 32 * SS + ((g >> 1) * 16 + 8 * (g & 1) + (r16 >> 2)) * SS + 4 * (r16 & 3);
-          ads[h] = cat8(read_tr16(ps), read_tr16(ps + 4 * SS));
-        }
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int h = 0; h < NH; ++h)
-#pragma unroll
-          for (int dt = 0; dt < 4; ++dt) dqa[qb + h][dt] = mma(ads[h], wc[dt], dqa[qb + h][dt]);
-        // BIAS: du partial of (query, j) over the tile's 16 keys: column c < 2 of dS x jsum is the sum for
-        // j = ja + c (lanes r16 < 2), written once per key tile
-        if constexpr (BIAS) {
-          if (p.du != nullptr) {
-#pragma unroll
-            for (int h = 0; h < NH; ++h) {
-              const mf_f32x4 su = mma(ads[h], jsum, mf_f32x4{0.f, 0.f, 0.f, 0.f});
-              if (r16 < 2) {
-                float* dst = p.dupart + ((size_t(bh) * (kMaxN / 16) + kt) * kMaxN + q0 + (qb + h) * 16 + 4 * g) * kMaxN +
-                             ja + r16;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) dst[r * kMaxN] = su[r];
-              }
-            }
-          }
-        }
-        // G^T and H^T: A = dS^T / P^T of the two query tiles as the lane holds them (K slot 4 h + r is query
-        // (qb + h) 16 + 4 g + r), B = q / go at those queries and d = 16 dt + r16 (transposed reads)
-        mf_f16x8 dsb[2], pb[2];
+        __builtin_amdgcn_sched_barrier(0);
+      } else if constexpr (BIAS == 0) {
 #pragma unroll
         for (int jn = 0; jn < 2; ++jn) {
-          float t8[8], u8[8];
+          form(jn);
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            t8[r] = dsv[0][jn][r];
-            t8[4 + r] = dsv[1][jn][r];
-            u8[r] = pvv[0][jn][r];
-            u8[4 + r] = pvv[1][jn][r];
+          for (int t = 0; t < NQT; ++t) {
+            mf_f16x8 aq[2], ag[2];
+            rows_of(Qs, t, aq);
+            rows_of(Gs, t, ag);
+            float ds[4], none = 0.0f;
+            score(jn, t, aq, ag, 0.0f, none, ds);
           }
-          dsb[jn] = pack_f16x8(t8);
-          pb[jn] = pack_f16x8(u8);
+          __builtin_amdgcn_sched_barrier(0);
         }
-        // the second tile's rows when it exists, else the first's again (its K slots carry zeros)
-        const int off2 = (qb + 1 < NQT ? 16 : 0) * KS;
+      } else {  // one j at a time: the bias sums leave no registers for two
 #pragma unroll
-        for (int dt = 0; dt < 4; ++dt) {
-          const int off = (qb * 16 + 4 * g + (r16 >> 2)) * KS + 16 * dt + 4 * (r16 & 3);
-          const mf_f16x8 bq = cat8(read_tr16(Qp + off), read_tr16(Qp + off + off2));
-          const mf_f16x8 bg = cat8(read_tr16(Gp + off), read_tr16(Gp + off + off2));
+        for (int jn = 0; jn < 2; ++jn) {
+          const int j = ja + jn;
+          form(jn);
+          const float wj = wd[j * KW + k0 + r16];  // its place takes dw below (each pair belongs to one wave)
+          // su: the sum over the tile's keys of dS of (j, query 16 (r16 >> 2) + 4 g + (r16 & 3))
+          float dwj = 0.0f, su = 0.0f;
 #pragma unroll
-          for (int jn = 0; jn < 2; ++jn) {
-            gt[jn][dt] = mma(dsb[jn], bq, gt[jn][dt]);
-            ht[jn][dt] = mma(pb[jn], bg, ht[jn][dt]);
+          for (int t = 0; t < NQT; ++t) {
+            mf_f16x8 aq[2], ag[2];
+            float dsv[4];
+            rows_of(Qs, t, aq);
+            rows_of(Gs, t, ag);
+            score(jn, t, aq, ag, wj, dwj, dsv);
+            const float st = row16_sum4(dsv, r16);
+            su = (r16 >> 2) == t ? st : su;
           }
+          const int i = 16 * (r16 >> 2) + 4 * g + (r16 & 3);
+          if (r16 < 4 * NQT) dut[j * KU + i] = fmaf(su, uD, dut[j * KU + i]);
+          // dw of (j, the lane's key): dwj sums gate log2 e dS 2^-es
+          const float x = sum_groups(dwj) * (uD * (1.0f / kLog2e));
+          if (g == 0) wd[j * KW + k0 + r16] = x;
+          __builtin_amdgcn_sched_barrier(0);
         }
       }
 
-      // BIAS: dw of the pair tile (sum over the four query groups; each pair belongs to one wave of one unit)
-      if constexpr (BIAS) {
-        if (p.dw != nullptr) {
-          const float fds = con[kFDs] * (1.0f / kLog2e);  // dwa holds sums of gate log2 e dS 2^-es
+      // ---- G^T, H^T (key k0 + 4 g + r, d = 16 dt + r16) and the pairs' key-side gradients, 16 d at a time.  A =
+      // dS^T / P^T of two query tiles as the lane holds them (K slot 4 h + r is query (qb + h) 16 + 4 g + r), B =
+      // q / go at those queries (transposed reads; the second tile's rows when it exists, else the first's
+      // again: its K slots carry zeros) ----
+      float x[2][4], y[2][4];
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt) {
+        mf_f32x4 gt[2], ht[2];
+#pragma unroll
+        for (int jn = 0; jn < 2; ++jn) {
+          gt[jn] = mf_f32x4{0.f, 0.f, 0.f, 0.f};
+          ht[jn] = mf_f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+#pragma unroll
+        for (int qb = 0; qb < NQT; qb += 2) {
+          const bool two = qb + 1 < NQT;
+          const int off = (qb * 16 + 4 * g + (r16 >> 2)) * KS + 16 * dt + 4 * (r16 & 3);
+          const int off2 = off + (two ? 16 * KS : 0);
+          const mf_f16x8 bq = cat8(read_tr16(Qs + off), read_tr16(Qs + off2));
+          const mf_f16x8 bg = cat8(read_tr16(Gs + off), read_tr16(Gs + off2));
 #pragma unroll
           for (int jn = 0; jn < 2; ++jn) {
-            float x = sum_groups(dwa[jn]) * fds;
-            if (g == 0 && ja + jn < nk && kvalid) {
-              // earlier passes keep their sum in the workspace (read back by the thread that wrote it)
-              float* o = p.dwpart + (size_t(bh) * kMaxN + ja + jn) * kMaxN + k0 + r16;
-              if (!first) x += *o;
-              if (!last) *o = x;
-              else store_grad(p.dw, (rbase + kidx[ja + jn]) * N + kidx[k0 + r16], x, p.gout16);
-            }
+            const uint2 d2 = two ? dsw[jn][two ? qb + 1 : qb] : uint2{0u, 0u};
+            const uint2 p2 = two ? pw[jn][two ? qb + 1 : qb] : uint2{0u, 0u};
+            gt[jn] = mma(__builtin_bit_cast(mf_f16x8, uint4{dsw[jn][qb].x, dsw[jn][qb].y, d2.x, d2.y}), bq, gt[jn]);
+            ht[jn] = mma(__builtin_bit_cast(mf_f16x8, uint4{pw[jn][qb].x, pw[jn][qb].y, p2.x, p2.y}), bg, ht[jn]);
+          }
+        }
+        // k2 / v2 of keys k0 + 4 g + r at d = 16 dt + r16 (transposed reads), k1 / v1 of j
+        const int roff = (k0 + 4 * g + (r16 >> 2)) * KS + 16 * dt + 4 * (r16 & 3);
+        const auto k2t = read_tr16(K2s + roff);
+        const auto v2t = read_tr16(V2s + roff);
+#pragma unroll
+        for (int jn = 0; jn < 2; ++jn) {
+          const float k1p = float(K1s[(ja + jn) * KS + 16 * dt + r16]);
+          const float v1p = float(V1s[(ja + jn) * KS + 16 * dt + r16]);
+          x[jn][dt] = 0.0f;
+          y[jn][dt] = 0.0f;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            dk2a[dt][r] = fmaf(k1p, gt[jn][r], dk2a[dt][r]);
+            dv2a[dt][r] = fmaf(v1p, ht[jn][r], dv2a[dt][r]);
+            x[jn][dt] = fmaf(float(k2t[r]), gt[jn][r], x[jn][dt]);
+            y[jn][dt] = fmaf(float(v2t[r]), ht[jn][r], y[jn][dt]);
           }
         }
       }
-      // ---- the pair tile's key-side gradients ----
-      if constexpr (BIAS) {
-#pragma unroll
-        for (int dt = 0; dt < 4; ++dt) read_kv2(dt);
-#pragma unroll
-        for (int jn = 0; jn < 2; ++jn)
-#pragma unroll
-          for (int dt = 0; dt < 4; ++dt) {
-            k1p[jn][dt] = float(k1h[jn][dt]);
-            v1p[jn][dt] = float(V1s[(ja + jn) * KS + 16 * dt + r16]);
-          }
-      }
+      // dk1_j / dv1_j at d = lane: rows of j belong to this wave
 #pragma unroll
       for (int jn = 0; jn < 2; ++jn) {
-        const int j = ja + jn;
-        if (j >= nk) continue;  // uniform
-#pragma unroll
-        for (int dt = 0; dt < 4; ++dt) {
-          // dk2 / dv2 of keys k0 + 4 g + r: + k1_j / v1_j (.) G^T / H^T
-          // dk1_j / dv1_j at d = 16 dt + r16: sum over the 16 keys (4 in the lane, then the four groups)
-          float x = 0.0f, y = 0.0f;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            dk2a[dt][r] = fmaf(k1p[jn][dt], gt[jn][dt][r], dk2a[dt][r]);
-            dv2a[dt][r] = fmaf(v1p[jn][dt], ht[jn][dt][r], dv2a[dt][r]);
-            x = fmaf(kk2[dt][r], gt[jn][dt][r], x);
-            y = fmaf(kv2[dt][r], ht[jn][dt][r], y);
-          }
-          x = sum_groups(x);
-          y = sum_groups(y);
-          if (g == 0) {  // rows of j belong to this wave
-            if constexpr (BIAS) {
-              if (kt + 1 < nkt || !last) {
-                sk1[j * DP + 16 * dt + r16] = d1k[jn][dt] + x;
-                sv1[j * DP + 16 * dt + r16] = d1v[jn][dt] + y;
-              } else {  // the last key tile: the gradient rows
-                const size_t o = (rbase + kidx[j]) * DP + 16 * dt + r16;
-                store_grad(p.dk1, o, (d1k[jn][dt] + x) * con[kFDk1], p.gout16);
-                store_grad(p.dv1, o, (d1v[jn][dt] + y) * con[kFDv1], p.gout16);
-              }
-            } else {
-              dk1a[j * DP + 16 * dt + r16] = d1k[jn][dt] + x;
-              dv1a[j * DP + 16 * dt + r16] = d1v[jn][dt] + y;
-            }
-          }
-        }
+        const int o = (ja + jn) * DP + lane;
+        const float xs = sum_groups4(x[jn][0], x[jn][1], x[jn][2], x[jn][3]);
+        const float ys = sum_groups4(y[jn][0], y[jn][1], y[jn][2], y[jn][3]);
+        dk1a[o] = fmaf(xs, fk1, dk1a[o]);
+        dv1a[o] = fmaf(ys, fv1, dv1a[o]);
       }
+      // ---- dq of queries 16 t + r16: A = dS [query][pairs (ja + (g >> 1), keys 8 (g & 1) + e)] by transposed
+      // reads (lane 4 e' + a of a group addresses row e' (+4), columns 4 a .. 4 a + 3), B = W of those pairs at
+      // d = 16 dt + r16 ----
+      __builtin_amdgcn_wave_barrier();
+      mf_f16x8 wc[4];
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt) {
+        const _Float16* pc = K2s + (k0 + 8 * (g & 1) + (r16 >> 2)) * KS + 16 * dt + 4 * (r16 & 3);
+        wc[dt] = cat8(read_tr16(pc), read_tr16(pc + 4 * KS)) * K1s[(ja + (g >> 1)) * KS + 16 * dt + r16];
+      }
+#pragma unroll
+      for (int t = 0; t < NQT; ++t) {
+        const _Float16* ps = scr + t * 32 * SS + ((g >> 1) * 16 + 8 * (g & 1) + (r16 >> 2)) * SS + 4 * (r16 & 3);
+        const mf_f16x8 ads = cat8(read_tr16(ps), read_tr16(ps + 4 * SS));
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) dqa[t][dt] = mma(ads, wc[dt], dqa[t][dt]);
+      }
+      __builtin_amdgcn_wave_barrier();
     }
 
-    // ---- dk2 / dv2 of the key tile: the four waves' partials in wave order ----
-    {
-      float* sl = slot + wave * kSlot;
+    // ---- dk2, then dv2 of the key tile: the four waves' partials in wave order ----
+    lds_barrier();  // every wave is done with its scratch
+#pragma unroll
+    for (int which = 0; which < 2; ++which) {
 #pragma unroll
       for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          sl[(4 * g + r) * DP + 16 * dt + r16] = dk2a[dt][r];
-          sl[16 * DP + (4 * g + r) * DP + 16 * dt + r16] = dv2a[dt][r];
+        for (int r = 0; r < 4; ++r)
+          slot[(wave * 16 + 4 * g + r) * PS + 16 * dt + r16] = which ? dv2a[dt][r] : dk2a[dt][r];
+      lds_barrier();
+      const int kk = tid / 16, d4 = 4 * (tid % 16);
+      if (k0 + kk < c.nk) {
+        const float4 s = sum_partials(slot, kk, d4, which ? ldexpf(1.0f, c.f1 + c.eg) : ldexpf(1.0f, c.e1 + es + c.eq));
+        if (c.direct) {
+          store_grad4(which ? p.dv2 : p.dk2, (rbase + kidx[k0 + kk]) * DP + d4, s, p.gout16);
+        } else {
+          add_slab(slab + (size_t(1 + which) * N + c.k0 + k0 + kk) * DP + d4, s, c.first_k);
         }
-    }
-    lds_barrier();
-    for (int u = tid; u < kSlot; u += kThreads) {
-      const int which = u / (16 * DP);
-      const int kk = (u / DP) % 16;
-      const int d = u % DP;
-      if (k0 + kk < nk) {
-        float s = slot[u] + slot[kSlot + u];
-        s += slot[2 * kSlot + u];
-        s += slot[3 * kSlot + u];
-        s *= which ? con[kFDv2] : con[kFDk2];
-        float* ps = slab + size_t(1 + which) * kMaxN * DP + (k0 + kk) * DP + d;
-        if (!first) s += *ps;  // an earlier pass's partial (this thread wrote it)
-        if (to_slab || !last) *ps = s;
-        else store_grad(which ? p.dv2 : p.dk2, (rbase + kidx[k0 + kk]) * DP + d, s, p.gout16);
       }
+      lds_barrier();
     }
-    // BIAS: dv_bias partial of the key tile (sum over the part's j), the four waves' partials in wave order
-    if constexpr (BIAS) {
+    // BIAS: dv_bias partial of the key tile: [t][key r16][query 4 g + r] per wave, a query tile at a time per slot
+    if constexpr (BIAS != 0) {
       if (p.dvb != nullptr) {
-        const float* dv0 = reinterpret_cast<const float*>(smem + Ly::dvb);
-        for (int u = tid; u < NQT * 256; u += kThreads) {  // key fastest: 64-byte runs of the global rows
-          const int kk = u % 16, i16 = (u / 16) % 16, qt = u / 256;
-          const int i = q0 + qt * 16 + i16, l = (qt * 16 + kk) * 16 + i16;
-          if (i < nq && k0 + kk < nk)
-            p.dvbpart[((size_t(bh) * 2 + part) * kMaxN + i) * kMaxN + k0 + kk] =
-                ((dv0[l] + dv0[NT * 256 + l]) + dv0[2 * NT * 256 + l]) + dv0[3 * NT * 256 + l];
+#pragma unroll
+        for (int t = 0; t < NQT; ++t)
+          *reinterpret_cast<float4*>(slot + (wave * NQT + t) * 256 + r16 * 16 + 4 * g) =
+              float4{dva[t][0], dva[t][1], dva[t][2], dva[t][3]};
+        lds_barrier();
+        for (int u = tid; u < NQT * 256; u += kThreads) {  // key fastest: 64-byte runs of the rows
+          const int kk = u % 16, i16 = (u / 16) % 16, t = u / 256;
+          const int i = t * 16 + i16, l = t * 256 + kk * 16 + i16;
+          if (i < c.nq && k0 + kk < c.nk) {
+            float s = (((slot[l] + slot[NQT * 256 + l]) + slot[2 * NQT * 256 + l]) + slot[3 * NQT * 256 + l]) * uD;
+            float* o = p.dvpart + ((size_t(c.bh) * p.cap + c.part) * N + c.q0 + i) * N + c.k0 + k0 + kk;
+            *o = c.first_t ? s : s + *o;
+          }
         }
+        lds_barrier();
       }
     }
-    lds_barrier();
   }
 
-  if constexpr (BIAS) {
-    // dgate partials of the pass: sums over each lane's keys into the wave's own scratch (other waves may still
-    // be using theirs), then the four waves in order
-    float* gs = reinterpret_cast<float*>(scr);
+  // ---- dq: the four waves' partials in wave order, a query tile at a time ----
 #pragma unroll
-    for (int qt = 0; qt < NQT; ++qt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float x = row16_sum(accg[qt][r]);
-        if (r16 == 0) gs[qt * 16 + 4 * g + r] = x;
-      }
-  } else {
-    // ---- dk1 / dv1 rows of the unit's keys j (key pairs jp = j / 2 with jp % parts == part) ----
-    for (int u = tid; u < nk * DP; u += kThreads) {
-      if (((u / DP) >> 1) % parts != part) continue;
-      const size_t o = (rbase + kidx[u / DP]) * DP + (u % DP);
-      store_grad(p.dk1, o, dk1a[u] * con[kFDk1], p.gout16);
-      store_grad(p.dv1, o, dv1a[u] * con[kFDv1], p.gout16);
-    }
-  }
-  lds_barrier();  // rows and acc1 are free for the dq partials
-  if constexpr (BIAS) {
-    if (p.dgate != nullptr) {
-      const float* gs = reinterpret_cast<const float*>(smem + Ly::scr);
-      constexpr int kW = 2 * 32 * SS / 2;  // floats per wave's scratch
-      for (int i = tid; i < min(nq - q0, NQT * 16); i += kThreads)
-        p.dgpart[(size_t(bh) * 2 + part) * kMaxN + q0 + i] =
-            ((gs[i] + gs[kW + i]) + gs[2 * kW + i]) + gs[3 * kW + i];
-    }
-  }
-  // ---- dq: the four waves' partials in wave order ----
-  // (BIAS: in slot + dvb, since a later pass still needs the rows)
-  float* dqs = reinterpret_cast<float*>(smem + (BIAS ? Ly::slot : 0));
-  constexpr int kDqs = NQT * 16 * DP;  // one wave's partials
-#pragma unroll
-  for (int qt = 0; qt < NQT; ++qt) {
+  for (int t = 0; t < NQT; ++t) {
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        dqs[wave * kDqs + (qt * 16 + 4 * g + r) * DP + 16 * dt + r16] = dqa[qt][dt][r];
-  }
-  lds_barrier();
-  for (int u = tid; u < min(nq - q0, NQT * 16) * DP; u += kThreads) {
-    float s = dqs[u] + dqs[kDqs + u];
-    s += dqs[2 * kDqs + u];
-    s += dqs[3 * kDqs + u];
-    s *= con[kFDq];
-    if (to_slab) slab[q0 * DP + u] = s;
-    else store_grad(p.dq, (rbase + qidx[q0 + u / DP]) * DP + (u % DP), s, p.gout16);
-  }
-  if (!last) lds_barrier();  // slot, dvb and the scratch are the next pass's
-}
-
-template <bool BIAS>
-__global__ void __launch_bounds__(kThreads, 1) pair_bwd_kernel(Params p) {
-  using Lk = Lay<BIAS>;
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  if (int(blockIdx.x) >= *p.total) return;
-  const uint32_t unit = p.units[blockIdx.x];
-  const int bh = int(unit >> 1);
-  const int part = int(unit & 1u);
-  const int b = bh / p.H;
-  const int N = p.N;
-  const int tid = threadIdx.x;
-  _Float16* Qs = reinterpret_cast<_Float16*>(smem + Lk::rows);  // q, go, k1, k2, v1, v2 rows in this order
-  const int lane = lane_id();
-  const int wave = wave_id();
-  float* lse2 = reinterpret_cast<float*>(smem + Lk::lse2);
-  float* dlt = reinterpret_cast<float*>(smem + Lk::dlt);
-  uint32_t* pvb = reinterpret_cast<uint32_t*>(smem + Lk::pvb);
-  int* kidx = reinterpret_cast<int*>(smem + Lk::kidx);
-  int* qidx = reinterpret_cast<int*>(smem + Lk::qidx);
-
-  // ---- valid keys and queries of molecule b, from the plan (which lists only molecules with 1 .. kMaxN) ----
-  const int2 nkq = p.counts[b];
-  const int nk = nkq.x, nq = nkq.y;
-  if (tid < 2 * kMaxN) {
-    const int at = tid < kMaxN ? tid : tid - kMaxN;
-    if (at < (tid < kMaxN ? nk : nq)) (tid < kMaxN ? kidx : qidx)[at] = p.lists[size_t(b) * 2 * kMaxN + tid];
-  }
-  lds_barrier();
-  const int parts = parts_of(nk);
-  const size_t rbase = size_t(bh) * N;
-  // ---- stage q, go, k1, k2, v1, v2 rows (compacted, zero past the counts) as fp16 scaled by 2^-e per operand
-  // (e = the exponent of the operand's largest magnitude over the unit), and lse log2 e and
-  // delta 2^-es = go . out 2^-es of each query (+inf / 0 on the padding rows: P = 0 there).  Every global
-  // load is issued before the first LDS store. ----
-  {
-    constexpr int kChunks = 6 * kMaxN * 8 / kThreads;  // 16-byte pieces per thread (15)
-    constexpr int kDl = (kMaxN * 8 + kThreads - 1) / kThreads;  // (query, 8-d chunk) items per thread (3)
-    static_assert(kChunks * kThreads == 6 * kMaxN * 8, "whole passes");
-    const __bf16* srcs[6] = {p.q, p.go, p.k1, p.k2, p.v1, p.v2};
-    uint4 buf[kChunks];
-#pragma unroll
-    for (int i = 0; i < kChunks; ++i) {
-      const int u = tid + kThreads * i;
-      const int t = u / (kMaxN * 8);
-      const int rr = (u / 8) % kMaxN;
-      const int c = u % 8;
-      // rows past the count load row 0 (cached) and are zeroed after: no branch around the loads
-      const int rrc = rr < (t < 2 ? nq : nk) ? rr : 0;
-      const int idx = t < 2 ? qidx[rrc] : kidx[rrc];
-      buf[i] = *reinterpret_cast<const uint4*>(srcs[t] + (rbase + idx) * DP + 8 * c);
-    }
-#pragma unroll
-    for (int i = 0; i < kChunks; ++i) {
-      const int u = tid + kThreads * i;
-      const int t = u / (kMaxN * 8);
-      if ((u / 8) % kMaxN >= (t < 2 ? nq : nk)) buf[i] = uint4{0u, 0u, 0u, 0u};
-    }
-    uint4 gr[kDl];
-    float4 o0[kDl], o1[kDl];
-    float lv[kDl];
-#pragma unroll
-    for (int i = 0; i < kDl; ++i) {
-      const int u = tid + kThreads * i;
-      const int rr = u / 8, c = u % 8;
-      const bool ok = u < kMaxN * 8 && rr < nq;
-      const size_t row = rbase + qidx[ok ? rr : 0];
-      gr[i] = *reinterpret_cast<const uint4*>(p.go + row * DP + 8 * c);
-      o0[i] = *reinterpret_cast<const float4*>(p.out + row * DP + 8 * c);
-      o1[i] = *reinterpret_cast<const float4*>(p.out + row * DP + 8 * c + 4);
-      lv[i] = p.lse[row] * kLog2e;
-      if (!ok) {
-        gr[i] = uint4{0u, 0u, 0u, 0u};
-        lv[i] = INFINITY;
-      }
-    }
-    // largest magnitude of each operand: per thread, per wave, then over the four waves
-    uint32_t mx[6] = {0u, 0u, 0u, 0u, 0u, 0u};
-#pragma unroll
-    for (int i = 0; i < kChunks; ++i) {
-      const int t = (tid + kThreads * i) / (kMaxN * 8);
-      const uint32_t m = absmax_bits8(buf[i]);
-#pragma unroll
-      for (int tt = 0; tt < 6; ++tt) mx[tt] = t == tt ? max(mx[tt], m) : mx[tt];
-    }
-    uint32_t* red = reinterpret_cast<uint32_t*>(smem + Lk::red);
-#pragma unroll
-    for (int tt = 0; tt < 6; ++tt) {
-      mx[tt] = wave_max_u32(mx[tt]);
-      if (lane == 0) red[wave * 8 + tt] = mx[tt];
+      for (int r = 0; r < 4; ++r) slot[(wave * 16 + 4 * g + r) * PS + 16 * dt + r16] = dqa[t][dt][r];
+    lds_barrier();
+    const int ii = t * 16 + tid / 16, d4 = 4 * (tid % 16);
+    if (ii < c.nq) {
+      const float4 s = sum_partials(slot, tid / 16, d4, ldexpf(1.0f, es + c.e1 + c.e2));
+      if (c.direct) store_grad4(p.dq, (rbase + qidx[ii]) * DP + d4, s, p.gout16);
+      else add_slab(slab + (size_t(c.q0) + ii) * DP + d4, s, c.first_q);
     }
     lds_barrier();
-    int ex[6];
-#pragma unroll
-    for (int tt = 0; tt < 6; ++tt)
-      ex[tt] = scale_exp(max(max(red[tt], red[8 + tt]), max(red[16 + tt], red[24 + tt])));
-    // operands q, go, k1, k2, v1, v2 = 0 .. 5; dS is carried as dS 2^-es, |dS| < 2^(eg + ev1 + ev2 + 10)
-    const int es = ex[1] + ex[4] + ex[5] - 5;
-#pragma unroll
-    for (int i = 0; i < kChunks; ++i) {
-      const int u = tid + kThreads * i;
-      const int t = u / (kMaxN * 8);
-      const int rr = (u / 8) % kMaxN;
-      const int c = u % 8;
-      int e = ex[0];
-#pragma unroll
-      for (int tt = 1; tt < 6; ++tt) e = t == tt ? ex[tt] : e;
-      *reinterpret_cast<uint4*>(Qs + size_t(t) * kMaxN * KS + rr * KS + 8 * c) = to_f16x8(buf[i], ldexpf(1.0f, -e));
-    }
-    if (tid == 0) {
-      float* con = reinterpret_cast<float*>(smem + Lk::con);
-      con[kCS] = ldexpf(kLog2e, ex[0] + ex[2] + ex[3]);
-      con[kCP] = ldexpf(1.0f, ex[1] + ex[4] + ex[5] - es);
-      con[kFDq] = ldexpf(1.0f, es + ex[2] + ex[3]);
-      con[kFDk1] = ldexpf(1.0f, ex[3] + es + ex[0]);
-      con[kFDk2] = ldexpf(1.0f, ex[2] + es + ex[0]);
-      con[kFDv1] = ldexpf(1.0f, ex[5] + ex[1]);
-      con[kFDv2] = ldexpf(1.0f, ex[4] + ex[1]);
-      con[kFDs] = ldexpf(1.0f, es);
-      if (BIAS && part == 0) p.fds[bh] = con[kFDs];
-    }
-    const float dscale = ldexpf(1.0f, -es);
-#pragma unroll
-    for (int i = 0; i < kDl; ++i) {
-      const int u = tid + kThreads * i;
-      if (kThreads * i >= kMaxN * 8) break;  // whole waves: kMaxN * 8 is a multiple of 64
-      const int rr = u / 8, c = u % 8;
-      float s = bf_lo(gr[i].x) * o0[i].x;
-      s = fmaf(bf_hi(gr[i].x), o0[i].y, s); s = fmaf(bf_lo(gr[i].y), o0[i].z, s);
-      s = fmaf(bf_hi(gr[i].y), o0[i].w, s); s = fmaf(bf_lo(gr[i].z), o1[i].x, s);
-      s = fmaf(bf_hi(gr[i].z), o1[i].y, s); s = fmaf(bf_lo(gr[i].w), o1[i].z, s);
-      s = fmaf(bf_hi(gr[i].w), o1[i].w, s);
-      s = sum8(s);
-      if (u < kMaxN * 8 && c == 0) {
-        dlt[rr] = rr < nq ? s * dscale : 0.0f;
-        lse2[rr] = lv[i];
-      }
-    }
   }
-  // ---- pair bits of the compacted keys (pair_valid), 3 words per j ----
-  const bool has_pv = p.pv != nullptr;
-  if (has_pv) {
-    for (int u = tid; u < kMaxN * 3; u += kThreads) {
-      const int j = u / 3, w = u % 3;
-      uint32_t bits = 0u;
-      if (j < nk) {
-        const uint8_t* row = p.pv + (size_t(b) * N + kidx[j]) * N;
-        for (int t = 0; t < 32; ++t) {
-          const int k = 32 * w + t;
-          if (k < nk && row[kidx[k]] != 0) bits |= 1u << t;
+  // BIAS: dgate partials: sums over each lane row's keys, then the four waves in order
+  if constexpr (BIAS != 0) {
+    if (p.dgate != nullptr) {
+#pragma unroll
+      for (int t = 0; t < NQT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float x = row16_sum(accg[t][r]);
+          if (r16 == 0) slot[wave * QM + t * 16 + 4 * g + r] = x;
         }
+      lds_barrier();
+      if (tid < c.nq) {
+        const float s = (((slot[tid] + slot[QM + tid]) + slot[2 * QM + tid]) + slot[3 * QM + tid]) * uD;
+        float* o = p.dgpart + (size_t(c.bh) * p.cap + c.part) * N + c.q0 + tid;
+        *o = c.first_q ? s : s + *o;
       }
-      pvb[u] = bits;
-    }
-  }
-  if constexpr (BIAS) {
-    // ---- u^T [j][i] = u[i][j] and v^T [k][i] = v[i][k] of the compacted atoms (bf16 as given, zero past the
-    // counts), the gates and gate log2 e (zero past nq).  Loads from clamped indices, then the selects. ----
-    uint16_t* ut = reinterpret_cast<uint16_t*>(smem + Lk::ut);
-    uint16_t* vt = reinterpret_cast<uint16_t*>(smem + Lk::vt);
-    float* cgs = reinterpret_cast<float*>(smem + Lk::gt);
-    constexpr int kPer = 25;  // every load issued before the first LDS store
-    static_assert(kMaxN * kMaxN % (kThreads * kPer) == 0, "whole passes");
-    for (int u0 = 0; u0 < kMaxN * kMaxN; u0 += kThreads * kPer) {
-      uint16_t a[kPer], c[kPer];
-#pragma unroll
-      for (int t = 0; t < kPer; ++t) {
-        const int u = u0 + tid + kThreads * t;
-        const int i = u / kMaxN, j = u % kMaxN;
-        const size_t o = (rbase + qidx[min(i, nq - 1)]) * N + kidx[min(j, nk - 1)];
-        a[t] = p.bu[o];
-        c[t] = p.bv[o];
-      }
-#pragma unroll
-      for (int t = 0; t < kPer; ++t) {
-        const int u = u0 + tid + kThreads * t;
-        const int i = u / kMaxN, j = u % kMaxN;
-        const bool ok = i < nq && j < nk;
-        ut[j * KU + i] = ok ? a[t] : uint16_t(0);
-        vt[j * KU + i] = ok ? c[t] : uint16_t(0);
-      }
-    }
-    if (tid < kMaxN) {
-      const float gv = bf_u16(p.bg[rbase + qidx[min(tid, nq - 1)]]);
-      cgs[tid] = tid < nq ? gv : 0.0f;
-      cgs[kMaxN + tid] = tid < nq ? gv * kLog2e : 0.0f;
-    }
-  } else {
-    for (int u = tid; u < 2 * kMaxN * DP / 4; u += kThreads)
-      reinterpret_cast<float4*>(smem + Lk::acc1)[u] = float4{0.f, 0.f, 0.f, 0.f};
-  }
-  lds_barrier();
-
-  if constexpr (BIAS) {  // at most three query tiles per pass (the bias sums leave no registers for more)
-    switch ((nq + 15) / 16) {
-      case 1: unit_body<1, true>(p, smem, nq, nk, part, parts, bh, has_pv, 0, true, true); break;
-      case 2: unit_body<2, true>(p, smem, nq, nk, part, parts, bh, has_pv, 0, true, true); break;
-      case 3: unit_body<3, true>(p, smem, nq, nk, part, parts, bh, has_pv, 0, true, true); break;
-      case 4:
-        unit_body<2, true>(p, smem, nq, nk, part, parts, bh, has_pv, 0, true, false);
-        unit_body<2, true>(p, smem, nq, nk, part, parts, bh, has_pv, 2, false, true);
-        break;
-      default:
-        unit_body<3, true>(p, smem, nq, nk, part, parts, bh, has_pv, 0, true, false);
-        unit_body<2, true>(p, smem, nq, nk, part, parts, bh, has_pv, 3, false, true);
-        break;
-    }
-  } else {
-    switch ((nq + 15) / 16) {
-      case 1: unit_body<1, false>(p, smem, nq, nk, part, parts, bh, has_pv, 0, true, true); break;
-      case 2: unit_body<2, false>(p, smem, nq, nk, part, parts, bh, has_pv, 0, true, true); break;
-      case 3: unit_body<3, false>(p, smem, nq, nk, part, parts, bh, has_pv, 0, true, true); break;
-      case 4: unit_body<4, false>(p, smem, nq, nk, part, parts, bh, has_pv, 0, true, true); break;
-      default: unit_body<NT, false>(p, smem, nq, nk, part, parts, bh, has_pv, 0, true, true); break;
+      lds_barrier();
     }
   }
 }
 
-// Split molecules: part 0's partial dq, dk2, dv2 are in the fp32 gradient rows (or, 16-bit gradients, in its
-// slab), part 1's in its slab; write part 0 + part 1 (in that order).  One workgroup per (molecule, head); a
-// separate launch, so the stream orders it after both halves without any cross-workgroup fence.
-__global__ void __launch_bounds__(kThreads) pair_bwd_combine(Params p) {
+template <int BIAS>
+__global__ void __launch_bounds__(kThreads, 2) pair_bwd_kernel(Params p) {
+  using Lk = Lay<BIAS != 0>;
+  constexpr int QM = Lk::QM, JM = Lk::JM, KM = Lk::KM, KU = Lk::KU, KW = Lk::KW;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  if (int(blockIdx.x) >= p.head[0]) return;
+  const uint32_t unit = p.units[blockIdx.x];
+  const int jt = p.head[1];
+  const int N = p.N;
+  Triple c;
+  c.bh = int(unit >> 6);
+  c.part = int(unit & 63u);
+  const int b = c.bh / p.H;
+  const int2 nkq = p.counts[b];
+  const int nk = nkq.x, nq = nkq.y;
+  const int parts = parts_of(nk, jt, p.cap);
+  const int jr = unit_rows(nk, parts);
+  const int ju0 = c.part * jr, ju1 = min(nk, ju0 + jr);  // the unit's j
+  const size_t rbase = size_t(c.bh) * N;
+  const uint16_t* klist = p.lists + size_t(2 * b) * N;
+  const uint16_t* qlist = klist + N;
+  const int njb = blocks_of(ju1 - ju0, JM), nqb = blocks_of(nq, QM), nkb = blocks_of(nk, KM);
+  const int jrows = 2 * (((ju1 - ju0 + 1) / 2 + njb - 1) / njb);
+  const int qrows = block_rows(nq, nqb), krows = block_rows(nk, nkb);
+  c.direct = parts == 1 && njb == 1 && nqb == 1 && nkb == 1;
+
+  _Float16* Qs = reinterpret_cast<_Float16*>(smem + Lk::rows);
+  _Float16* Gs = Qs + QM * KS;
+  _Float16* K1s = Gs + QM * KS;
+  _Float16* V1s = K1s + JM * KS;
+  _Float16* K2s = V1s + JM * KS;
+  _Float16* V2s = K2s + KM * KS;
+  float* acc1 = reinterpret_cast<float*>(smem + Lk::acc1);
+  float* lse2 = reinterpret_cast<float*>(smem + Lk::lse2);
+  float* dlt = reinterpret_cast<float*>(smem + Lk::dlt);
+  float* dls = reinterpret_cast<float*>(smem + Lk::dls);
+  float* ut = reinterpret_cast<float*>(smem + Lk::ut);
+  float* dut = reinterpret_cast<float*>(smem + Lk::dut);
+  float* wd = reinterpret_cast<float*>(smem + Lk::wd);
+  float* vt = reinterpret_cast<float*>(smem + Lk::vt);
+  float* cgs = reinterpret_cast<float*>(smem + Lk::gt);
+  int* jidx = reinterpret_cast<int*>(smem + Lk::jidx);
+  int* kidx = reinterpret_cast<int*>(smem + Lk::kidx);
+  int* qidx = reinterpret_cast<int*>(smem + Lk::qidx);
+  uint32_t* red = reinterpret_cast<uint32_t*>(smem + Lk::red);
+
+  for (int jb = 0; jb < njb; ++jb) {
+    c.j0 = ju0 + jb * jrows;
+    c.nj = min(ju1 - c.j0, jrows);
+    for (int qb = 0; qb < nqb; ++qb) {
+      c.q0 = qb * qrows;
+      c.nq = min(nq - c.q0, qrows);
+      for (int kb = 0; kb < nkb; ++kb) {
+        c.k0 = kb * krows;
+        c.nk = min(nk - c.k0, krows);
+        c.first_q = jb == 0 && kb == 0;
+        c.first_k = jb == 0 && qb == 0;
+        c.first_t = jb == 0;
+        // ---- stage the rows that changed (compacted, zero past the counts) as fp16 scaled by 2^-e per
+        // operand, lse log2 e and go . out of each query (+inf / 0 on the padding rows: P = 0 there).  A
+        // thread has a 16-byte piece of row tid / 8 and, for q and k blocks, of row 32 + tid / 8; every
+        // global load is issued before the first LDS store, rows past a count load its last row. ----
+        const bool do_j = qb == 0 && kb == 0, do_q = kb == 0, do_k = nkb > 1 || do_j;
+        const int tid = opaque_tid(), lane = tid & 63, wave = tid >> 6;
+        const int r0 = tid / 8, ch = tid % 8;
+        uint4 bq[2], bg[2], b1 = uint4{0u, 0u, 0u, 0u}, d1 = b1, b2[2], d2[2];
+        float4 o0[2], o1[2];
+        float lv[2];
+        int iq[2], ik[2], ij = 0;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          bq[i] = bg[i] = b2[i] = d2[i] = uint4{0u, 0u, 0u, 0u};
+          o0[i] = o1[i] = float4{0.f, 0.f, 0.f, 0.f};
+          lv[i] = INFINITY;
+          iq[i] = qlist[c.q0 + min(r0 + 32 * i, c.nq - 1)];
+          ik[i] = klist[c.k0 + min(r0 + 32 * i, c.nk - 1)];
+        }
+        ij = klist[c.j0 + min(r0, c.nj - 1)];
+        if (do_j) {
+          b1 = *reinterpret_cast<const uint4*>(p.k1 + (rbase + ij) * DP + 8 * ch);
+          d1 = *reinterpret_cast<const uint4*>(p.v1 + (rbase + ij) * DP + 8 * ch);
+        }
+        if (do_q) {
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            const size_t row = rbase + iq[i];
+            bq[i] = *reinterpret_cast<const uint4*>(p.q + row * DP + 8 * ch);
+            bg[i] = *reinterpret_cast<const uint4*>(p.go + row * DP + 8 * ch);
+            o0[i] = *reinterpret_cast<const float4*>(p.out + row * DP + 8 * ch);
+            o1[i] = *reinterpret_cast<const float4*>(p.out + row * DP + 8 * ch + 4);
+            lv[i] = p.lse[row] * kLog2e;
+          }
+        }
+        if (do_k) {
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            b2[i] = *reinterpret_cast<const uint4*>(p.k2 + (rbase + ik[i]) * DP + 8 * ch);
+            d2[i] = *reinterpret_cast<const uint4*>(p.v2 + (rbase + ik[i]) * DP + 8 * ch);
+          }
+        }
+        // valid pairs (j, k) of the block, eight keys per byte
+        uint32_t bits = 0u;
+        const bool do_bits = do_k && tid < JM * (KM / 8);
+        if (do_bits) {
+          const int j = tid / (KM / 8), k8 = 8 * (tid % (KM / 8));
+          const int left = c.nk - k8;
+          bits = j >= c.nj || left <= 0 ? 0u : (left >= 8 ? 0xffu : (1u << left) - 1u);
+          if (p.pv != nullptr) {
+            const uint8_t* row = p.pv + (size_t(b) * N + klist[c.j0 + min(j, c.nj - 1)]) * N;
+            uint8_t on[8];
+#pragma unroll
+            for (int t = 0; t < 8; ++t) on[t] = row[klist[c.k0 + min(k8 + t, c.nk - 1)]];
+#pragma unroll
+            for (int t = 0; t < 8; ++t) bits &= on[t] != 0 ? 0xffu : ~(1u << t);
+          }
+        }
+        // BIAS: u of (query, j), w of (j, key), v of (query, key) and the gates; thread (tid / 16, tid % 16) of a
+        // 16 x 16 grid of entries
+        constexpr int kT = BIAS ? QM / 16 : 1;
+        static_assert(!BIAS || (JM == 16 && QM == KM), "the 16 x 16 grid covers j; QM / 16 steps cover both others");
+        const int jj = tid % 16, ii = tid / 16;
+        float ul[kT], wl[kT], vl[kT][kT], ga = 0.0f;
+        if constexpr (BIAS != 0) {
+          int qx[kT], kx[kT];
+          const int jx = klist[c.j0 + min(jj, c.nj - 1)], jy = klist[c.j0 + min(ii, c.nj - 1)];
+#pragma unroll
+          for (int t = 0; t < kT; ++t) {
+            qx[t] = qlist[c.q0 + min(ii + 16 * t, c.nq - 1)];
+            kx[t] = klist[c.k0 + min(jj + 16 * t, c.nk - 1)];
+          }
+          if (do_q) ga = load_bias<BIAS>(p.bg, rbase + qlist[c.q0 + min(tid, c.nq - 1)]);
+#pragma unroll
+          for (int t = 0; t < kT; ++t) {
+            ul[t] = do_q ? load_bias<BIAS>(p.bu, (rbase + qx[t]) * N + jx) : 0.0f;
+            wl[t] = load_bias<BIAS>(p.bw, (rbase + jy) * N + kx[t]);
+#pragma unroll
+            for (int u = 0; u < kT; ++u) vl[t][u] = load_bias<BIAS>(p.bv, (rbase + qx[t]) * N + kx[u]);
+          }
+        }
+        const uint4 zero{0u, 0u, 0u, 0u};
+        if (r0 >= c.nj) b1 = d1 = zero;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          if (r0 + 32 * i >= c.nq) {
+            bq[i] = bg[i] = zero;
+            lv[i] = INFINITY;
+          }
+          if (r0 + 32 * i >= c.nk) b2[i] = d2[i] = zero;
+        }
+        // largest magnitude of each operand over the block: per thread, per wave, then over the four waves
+        uint32_t mx[6] = {max(absmax_bits8(bq[0]), absmax_bits8(bq[1])), max(absmax_bits8(bg[0]), absmax_bits8(bg[1])),
+                          absmax_bits8(b1), max(absmax_bits8(b2[0]), absmax_bits8(b2[1])), absmax_bits8(d1),
+                          max(absmax_bits8(d2[0]), absmax_bits8(d2[1]))};
+#pragma unroll
+        for (int t = 0; t < 6; ++t) {
+          mx[t] = wave_max_u32(mx[t]);
+          if (lane == 0) red[wave * 8 + t] = mx[t];
+        }
+        lds_barrier();
+        int ex[6];
+#pragma unroll
+        for (int t = 0; t < 6; ++t)
+          ex[t] = __builtin_amdgcn_readfirstlane(scale_exp(max(max(red[t], red[8 + t]), max(red[16 + t], red[24 + t]))));
+        if (do_q) {
+          c.eq = ex[0];
+          c.eg = ex[1];
+        }
+        if (do_j) {
+          c.e1 = ex[2];
+          c.f1 = ex[4];
+        }
+        if (do_k) {
+          c.e2 = ex[3];
+          c.f2 = ex[5];
+        }
+        const float dscale = ldexpf(1.0f, -(c.eg + c.f1 + c.f2 - 5));
+        if (do_q) {
+          const float sq = ldexpf(1.0f, -ex[0]), sg = ldexpf(1.0f, -ex[1]);
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            const int r = r0 + 32 * i;
+            float s = bf_lo(bg[i].x) * o0[i].x;
+            s = fmaf(bf_hi(bg[i].x), o0[i].y, s); s = fmaf(bf_lo(bg[i].y), o0[i].z, s);
+            s = fmaf(bf_hi(bg[i].y), o0[i].w, s); s = fmaf(bf_lo(bg[i].z), o1[i].x, s);
+            s = fmaf(bf_hi(bg[i].z), o1[i].y, s); s = fmaf(bf_lo(bg[i].w), o1[i].z, s);
+            s = fmaf(bf_hi(bg[i].w), o1[i].w, s);
+            s = sum8(s);
+            if (r < QM) {
+              *reinterpret_cast<uint4*>(Qs + r * KS + 8 * ch) = to_f16x8(bq[i], sq);
+              *reinterpret_cast<uint4*>(Gs + r * KS + 8 * ch) = to_f16x8(bg[i], sg);
+              if (ch == 0) {
+                dlt[r] = r < c.nq ? s : 0.0f;
+                dls[r] = r < c.nq ? s * dscale : 0.0f;
+                lse2[r] = lv[i];
+                qidx[r] = iq[i];
+              }
+            }
+          }
+        } else if (ch == 0) {  // the scale of dS may have changed
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+            if (r0 + 32 * i < QM) dls[r0 + 32 * i] = dlt[r0 + 32 * i] * dscale;
+        }
+        if (do_j) {
+          if (r0 < JM) {
+            *reinterpret_cast<uint4*>(K1s + r0 * KS + 8 * ch) = to_f16x8(b1, ldexpf(1.0f, -ex[2]));
+            *reinterpret_cast<uint4*>(V1s + r0 * KS + 8 * ch) = to_f16x8(d1, ldexpf(1.0f, -ex[4]));
+            if (ch == 0) jidx[r0] = ij;
+          }
+          static_assert(2 * JM * DP / 4 % kThreads == 0, "whole passes");
+          static_assert(JM <= 32 && QM <= 64 && KM <= 64, "rows of a thread");
+#pragma unroll
+          for (int u = 0; u < 2 * JM * DP / 4 / kThreads; ++u)
+            reinterpret_cast<float4*>(acc1)[tid + kThreads * u] = float4{0.f, 0.f, 0.f, 0.f};
+        }
+        if (do_bits) (smem + Lk::pvb)[(tid / (KM / 8)) * 8 + tid % (KM / 8)] = uint8_t(bits);
+        if constexpr (BIAS != 0) {
+          if (do_q && tid < QM) cgs[tid] = tid < c.nq ? ga * kLog2e : 0.0f;
+#pragma unroll
+          for (int t = 0; t < kT; ++t) {
+            if (do_q) {
+              ut[jj * KU + ii + 16 * t] = ii + 16 * t < c.nq && jj < c.nj ? ul[t] : 0.0f;
+              dut[jj * KU + ii + 16 * t] = 0.0f;
+            }
+            wd[ii * KW + jj + 16 * t] = wl[t];
+#pragma unroll
+            for (int u = 0; u < kT; ++u) vt[(jj + 16 * u) * KU + ii + 16 * t] = vl[t][u];
+          }
+        }
+        if (do_k) {
+          const float s2 = ldexpf(1.0f, -ex[3]), t2 = ldexpf(1.0f, -ex[5]);
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            const int r = r0 + 32 * i;
+            if (r < KM) {
+              *reinterpret_cast<uint4*>(K2s + r * KS + 8 * ch) = to_f16x8(b2[i], s2);
+              *reinterpret_cast<uint4*>(V2s + r * KS + 8 * ch) = to_f16x8(d2[i], t2);
+              if (ch == 0) kidx[r] = ik[i];
+            }
+          }
+        }
+        lds_barrier();
+        switch ((c.nq + 15) / 16) {
+          case 1: triple_body<1, BIAS>(p, smem, c); break;
+          case 2: triple_body<2, BIAS>(p, smem, c); break;
+          case 3: triple_body<3, BIAS>(p, smem, c); break;
+          default:
+            if constexpr (BIAS == 0) triple_body<4, BIAS>(p, smem, c);
+            break;
+        }
+        if constexpr (BIAS != 0) {  // dw of the triple's (j, k), summed over the query blocks
+          if (p.dw != nullptr) {
+            const int tid = opaque_tid();
+            for (int u = tid; u < c.nj * KM; u += kThreads) {
+              const int j = u / KM, k = u % KM;
+              if (k >= c.nk) continue;
+              float x = wd[j * KW + k];
+              // earlier query blocks keep their sum in the workspace (read back by the thread that wrote it)
+              float* o = p.dwpart + (rbase + c.j0 + j) * N + c.k0 + k;
+              if (qb > 0) x += *o;
+              if (qb + 1 < nqb) *o = x;
+              else store_grad(p.dw, (rbase + jidx[j]) * N + kidx[k], x, p.gout16);
+            }
+          }
+          if (kb + 1 < nkb) lds_barrier();
+        }
+      }
+      if constexpr (BIAS != 0) {  // du of the block's (query, j): every key is in
+        if (p.du != nullptr) {
+          for (int u = opaque_tid(); u < c.nq * JM; u += kThreads) {
+            const int i = u / JM, j = u % JM;
+            if (j < c.nj)
+              store_grad(p.du, (rbase + qidx[i]) * N + jidx[j], cgs[i] * (1.0f / kLog2e) * dut[j * KU + i], p.gout16);
+          }
+        }
+        if (qb + 1 < nqb) lds_barrier();
+      }
+    }
+    // ---- dk1 / dv1 rows of the block's j (the barriers that end the body order the waves' rows) ----
+    for (int u = opaque_tid(); u < c.nj * (DP / 4); u += kThreads) {
+      const int j = u / (DP / 4), d4 = 4 * (u % (DP / 4));
+      const size_t o = (rbase + jidx[j]) * DP + d4;
+      store_grad4(p.dk1, o, *reinterpret_cast<const float4*>(acc1 + j * DP + d4), p.gout16);
+      store_grad4(p.dv1, o, *reinterpret_cast<const float4*>(acc1 + (JM + j) * DP + d4), p.gout16);
+    }
+    if (jb + 1 < njb) lds_barrier();
+  }
+}
+
+// Molecules of more than one block triple: dq, dk2, dv2 are in the units' slabs; add them in unit order.  kCombineSplit
+// workgroups per (molecule, head); a separate launch, so the stream orders it after the units without any
+// cross-workgroup fence.
+constexpr int kCombineSplit = 2;
+__global__ void __launch_bounds__(kThreads) pair_bwd_combine(Params p, int qm, int jm) {
   const int bh = blockIdx.x;
   const int b = bh / p.H;
   const int2 nkq = p.counts[b];
   const int nk = nkq.x, nq = nkq.y;
-  if (nk <= 0 || nq <= 0 || nk > kMaxN || nq > kMaxN || parts_of(nk) == 1) return;
+  if (nk <= 0 || nq <= 0) return;
+  const int parts = parts_of(nk, p.head[1], p.cap);
+  if (parts == 1 && nk <= jm && nq <= qm) return;  // one triple
   const size_t rbase = size_t(bh) * p.N;
-  const float* slab0 = p.slab + size_t(bh) * 2 * 5 * kMaxN * DP;
-  const float* slab = slab0 + 5 * kMaxN * DP;  // part 1
-  const uint16_t* lists = p.lists + size_t(b) * 2 * kMaxN;
-  const bool g16 = p.gout16 != 0;
-  // rows: dq of the nq queries, then dk2 and dv2 of the nk keys, 16 float4 each; 8 per thread at a time
-  const int nrows = nq + 2 * nk;
-  for (int u0 = 0; u0 < nrows * 16; u0 += 8 * kThreads) {
-    float4 a[8], c[8];
-    size_t dst[8];
-    void* base[8];
+  const size_t pstride = size_t(3) * p.N * DP;
+  const float* slab = p.slab + size_t(bh) * p.cap * pstride;
+  const uint16_t* klist = p.lists + size_t(2 * b) * p.N;
+  const uint16_t* qlist = klist + p.N;
+  // rows: dq of the nq queries, then dk2 and dv2 of the nk keys, 16 float4 each; kAt per thread at a time
+  constexpr int kAt = 4;
+  const int total = (nq + 2 * nk) * 16;
+  for (int u0 = blockIdx.y * kAt * kThreads; u0 < total; u0 += kCombineSplit * kAt * kThreads) {
+    float4 a[kAt];
+    size_t so[kAt], dst[kAt];
+    void* base[kAt];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int u = min(u0 + int(threadIdx.x) + kThreads * i, nrows * 16 - 1);  // clamped: no branch around loads
+    for (int i = 0; i < kAt; ++i) {
+      const int u = min(u0 + int(threadIdx.x) + kThreads * i, total - 1);  // clamped: no branch around loads
       const int row = u / 16, q4 = u % 16;
       const int which = row < nq ? 0 : (row < nq + nk ? 1 : 2);
       const int rr = which == 0 ? row : (which == 1 ? row - nq : row - nq - nk);
-      const int idx = which == 0 ? lists[kMaxN + rr] : lists[rr];
       base[i] = which == 0 ? p.dq : (which == 1 ? p.dk2 : p.dv2);
-      dst[i] = (rbase + idx) * DP + 4 * q4;
-      const size_t so = size_t(which) * kMaxN * DP + rr * DP + 4 * q4;
-      a[i] = g16 ? *reinterpret_cast<const float4*>(slab0 + so)
-                 : *reinterpret_cast<const float4*>(static_cast<const float*>(base[i]) + dst[i]);
-      c[i] = *reinterpret_cast<const float4*>(slab + so);
+      dst[i] = (rbase + (which == 0 ? qlist[rr] : klist[rr])) * DP + 4 * q4;
+      so[i] = (size_t(which) * p.N + rr) * DP + 4 * q4;
+      a[i] = *reinterpret_cast<const float4*>(slab + so[i]);
+    }
+    for (int part = 1; part < parts; ++part) {
+#pragma unroll
+      for (int i = 0; i < kAt; ++i) {
+        const float4 s = *reinterpret_cast<const float4*>(slab + part * pstride + so[i]);
+        a[i].x += s.x; a[i].y += s.y; a[i].z += s.z; a[i].w += s.w;
+      }
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      if (u0 + int(threadIdx.x) + kThreads * i >= nrows * 16) continue;
-      const float4 v{a[i].x + c[i].x, a[i].y + c[i].y, a[i].z + c[i].z, a[i].w + c[i].w};
-      if (g16) {
-        const uint2 w{__builtin_bit_cast(uint32_t, mf_bf16x2{__bf16(v.x), __bf16(v.y)}),
-                      __builtin_bit_cast(uint32_t, mf_bf16x2{__bf16(v.z), __bf16(v.w)})};
-        *reinterpret_cast<uint2*>(static_cast<__bf16*>(base[i]) + dst[i]) = w;
-      } else {
-        *reinterpret_cast<float4*>(static_cast<float*>(base[i]) + dst[i]) = v;
-      }
+    for (int i = 0; i < kAt; ++i) {
+      if (u0 + int(threadIdx.x) + kThreads * i < total) store_grad4(base[i], dst[i], a[i], p.gout16);
     }
   }
 }
 
-// The factorized bias gradients of every served molecule from the units' partial sums (dS 2^-es):
-//   du_ij = gate_i 2^es sum_kt dupart[kt][i][j],  dv_ik = gate_i 2^es (part 0 + part 1),
-//   dgate_i = 2^es (part 0 + part 1); dw was written by the units.  kFinishSplit workgroups per (molecule,
-// head), each thread kFinishBatch entries at a time with every load issued before the first store.
-constexpr int kFinishSplit = 4, kFinishBatch = 4;
+// dv_ik = gate_i sum of the parts and dgate_i = sum of the parts, in part order (du and dw are written by the
+// units).  kFinishSplit workgroups per (molecule, head), each thread kFinishAt entries at a time.
+constexpr int kFinishSplit = 4, kFinishAt = 4;
+template <int BIAS>
 __global__ void __launch_bounds__(kThreads) pair_bwd_bias_finish(Params p) {
-  __shared__ float s_gate[kMaxN];
-  __shared__ int s_q[kMaxN], s_k[kMaxN];
   const int bh = blockIdx.x;
   const int b = bh / p.H;
   const int2 nkq = p.counts[b];
   const int nk = nkq.x, nq = nkq.y;
-  if (nk <= 0 || nq <= 0 || nk > kMaxN || nq > kMaxN) return;
+  if (nk <= 0 || nq <= 0) return;
   const int tid = threadIdx.x;
-  const size_t rbase = size_t(bh) * p.N;
-  const uint16_t* lists = p.lists + size_t(b) * 2 * kMaxN;
-  const float fds = p.fds[bh];
-  const bool two = parts_of(nk) == 2;
-  if (tid < kMaxN) {
-    s_k[tid] = lists[min(tid, nk - 1)];
-    s_q[tid] = lists[kMaxN + min(tid, nq - 1)];
-    s_gate[tid] = bf_u16(p.bg[rbase + lists[kMaxN + min(tid, nq - 1)]]);
-  }
-  __syncthreads();
-  const float* dvp = p.dvbpart + size_t(bh) * 2 * kMaxN * kMaxN;
-  const float* dup = p.dupart + size_t(bh) * (kMaxN / 16) * kMaxN * kMaxN;
-  const int n = nq * nk, nkt = (nk + 15) / 16;
-  const int step = kThreads * kFinishSplit;
-  for (int u0 = blockIdx.y * kThreads + tid; u0 < n; u0 += kFinishBatch * step) {
-    float su[kFinishBatch], sv[kFinishBatch];
+  const int N = p.N;
+  const size_t rbase = size_t(bh) * N;
+  const uint16_t* klist = p.lists + size_t(2 * b) * N;
+  const uint16_t* qlist = klist + N;
+  const int parts = parts_of(nk, p.head[1], p.cap);
+  if (p.dvb != nullptr) {
+    const float* dvp = p.dvpart + size_t(bh) * p.cap * N * N;
+    const int n = nq * nk, step = kThreads * kFinishSplit;
+    for (int u0 = blockIdx.y * kThreads + tid; u0 < n; u0 += kFinishAt * step) {
+      float sv[kFinishAt], gate[kFinishAt];
+      size_t e[kFinishAt], o[kFinishAt];
 #pragma unroll
-    for (int t = 0; t < kFinishBatch; ++t) {
-      const int u = min(u0 + t * step, n - 1);  // clamped: loads without branches
-      const int e = (u / nk) * kMaxN + u % nk;
-      su[t] = 0.0f;
-#pragma unroll
-      for (int kt = 0; kt < kMaxN / 16; ++kt) {
-        const float x = dup[size_t(kt) * kMaxN * kMaxN + e];
-        su[t] += kt < nkt ? x : 0.0f;  // tiles past nkt hold stale workspace bytes
+      for (int t = 0; t < kFinishAt; ++t) {
+        const int u = min(u0 + t * step, n - 1), i = u / nk, k = u % nk;  // clamped: loads without branches
+        const int qi = qlist[i];
+        e[t] = size_t(i) * N + k;
+        o[t] = (rbase + qi) * N + klist[k];
+        gate[t] = load_bias<BIAS>(p.bg, rbase + qi);
+        sv[t] = dvp[e[t]];
       }
-      const float v1 = dvp[kMaxN * kMaxN + e];
-      sv[t] = dvp[e] + (two ? v1 : 0.0f);
-    }
+      for (int part = 1; part < parts; ++part)
 #pragma unroll
-    for (int t = 0; t < kFinishBatch; ++t) {
-      const int u = u0 + t * step;
-      if (u >= n) break;
-      const int i = u / nk, j = u % nk;
-      const size_t o = (rbase + s_q[i]) * p.N + s_k[j];
-      const float c = s_gate[i] * fds;
-      if (p.du != nullptr) store_grad(p.du, o, c * su[t], p.gout16);
-      if (p.dvb != nullptr) store_grad(p.dvb, o, c * sv[t], p.gout16);
+        for (int t = 0; t < kFinishAt; ++t) sv[t] += dvp[size_t(part) * N * N + e[t]];
+#pragma unroll
+      for (int t = 0; t < kFinishAt; ++t)
+        if (u0 + t * step < n) store_grad(p.dvb, o[t], gate[t] * sv[t], p.gout16);
     }
   }
   if (p.dgate != nullptr && blockIdx.y == 0) {
-    const float* gp = p.dgpart + size_t(bh) * 2 * kMaxN;
-    for (int i = tid; i < nq; i += kThreads)
-      store_grad(p.dgate, rbase + s_q[i], fds * (two ? gp[i] + gp[kMaxN + i] : gp[i]), p.gout16);
+    const float* gp = p.dgpart + size_t(bh) * p.cap * N;
+    for (int i = tid; i < nq; i += kThreads) {
+      float s = gp[i];
+      for (int part = 1; part < parts; ++part) s += gp[size_t(part) * N + i];
+      store_grad(p.dgate, rbase + qlist[i], s, p.gout16);
+    }
   }
 }
 
 }  // namespace pbwd
 
+size_t simplicial_pair_bwd_workspace_bytes(int batch, int heads, int tokens) {
+  if (batch <= 0 || heads <= 0 || tokens <= 0 || batch > pbwd::kMaxPlanBatch || tokens > pbwd::kMaxTokens) return 0;
+  const size_t bytes = pbwd::Ws(batch, heads, tokens).bytes;
+  return bytes <= pbwd::kWsLimit ? bytes : 0;
+}
+
 bool simplicial_pair_bwd_serves(const mf_simplicial_bwd_args* a) {
   if (a->dtype != MF_DTYPE_BF16 || a->grad_dtype != MF_DTYPE_BF16 || a->head_dim != pbwd::DP) return false;
-  if (a->batch > pbwd::kMaxPlanBatch || a->tokens > pbwd::kMaxTokens || a->workspace == nullptr ||
-      reinterpret_cast<uintptr_t>(a->workspace) % 256 != 0 ||
-      a->workspace_bytes < pbwd::Ws(a->batch, a->heads).bytes)
+  const size_t need = simplicial_pair_bwd_workspace_bytes(a->batch, a->heads, a->tokens);
+  if (need == 0 || a->workspace == nullptr || reinterpret_cast<uintptr_t>(a->workspace) % 256 != 0 ||
+      a->workspace_bytes < need)
     return false;
+  if (int64_t(a->batch) * a->heads >= (1 << 26)) return false;  // unit codes are 32 bits
   if (a->angle_left != nullptr || a->message_left != nullptr) return false;
-  if (a->bias_u != nullptr) {  // bf16 bias terms (staged as they are)
-    if (a->bias_dtype != MF_DTYPE_BF16 || !a->bias_v || !a->bias_w || !a->bias_gate) return false;
+  if (a->bias_u != nullptr) {
+    if (a->bias_dtype != MF_DTYPE_BF16 && a->bias_dtype != MF_DTYPE_F32) return false;
+    if (!a->bias_v || !a->bias_w || !a->bias_gate) return false;
   }
   if (!a->dq || !a->dk1 || !a->dv1 || !a->dk2 || !a->dv2) return false;
   for (const void* ptr : {(const void*)a->q, (const void*)a->k1, (const void*)a->v1, (const void*)a->k2,
-                          (const void*)a->v2, (const void*)a->grad_out, (const void*)a->out})
+                          (const void*)a->v2, (const void*)a->grad_out, (const void*)a->out, (const void*)a->dq,
+                          (const void*)a->dk1, (const void*)a->dv1, (const void*)a->dk2, (const void*)a->dv2})
     if (reinterpret_cast<uintptr_t>(ptr) % 16 != 0) return false;
   return true;
 }
 
-int simplicial_pair_bwd_max_tokens() { return pbwd::kMaxN; }
-
-size_t simplicial_pair_bwd_workspace_bytes(int batch, int heads) {
-  if (batch <= 0 || heads <= 0 || batch > pbwd::kMaxPlanBatch) return 0;
-  return pbwd::Ws(batch, heads).bytes;
-}
-
-const int* simplicial_pair_bwd_served(const mf_simplicial_bwd_args* a) {
-  const pbwd::Ws ws(a->batch, a->heads);
-  return reinterpret_cast<const int*>(static_cast<const unsigned char*>(a->workspace) + ws.served);
-}
-
-const int* simplicial_pair_bwd_unserved_count(const mf_simplicial_bwd_args* a) {
-  return static_cast<const int*>(a->workspace) + 1;
+template <int BIAS>
+static int launch_units(const pbwd::Params& p, int blocks, int bh, hipStream_t stream) {
+  using namespace pbwd;
+  constexpr size_t lds = Lay<BIAS != 0>::bytes;
+  const int st = ensure_dynamic_lds(reinterpret_cast<const void*>(pair_bwd_kernel<BIAS>), int(lds));
+  if (st != MF_OK) return st;
+  hipLaunchKernelGGL(pair_bwd_kernel<BIAS>, dim3(unsigned(blocks)), dim3(kThreads), lds, stream, p);
+  MF_HIP_CHECK(hipGetLastError());
+  hipLaunchKernelGGL(pair_bwd_combine, dim3(unsigned(bh), kCombineSplit), dim3(kThreads), 0, stream, p,
+                     Lay<BIAS != 0>::QM, Lay<BIAS != 0>::JM);
+  MF_HIP_CHECK(hipGetLastError());
+  if constexpr (BIAS != 0) {
+    if (p.dvb != nullptr || p.dgate != nullptr) {
+      hipLaunchKernelGGL(pair_bwd_bias_finish<BIAS>, dim3(unsigned(bh), kFinishSplit), dim3(kThreads), 0, stream, p);
+      MF_HIP_CHECK(hipGetLastError());
+    }
+  }
+  return MF_OK;
 }
 
 int simplicial_pair_bwd_launch(const mf_simplicial_bwd_args* a, hipStream_t stream) {
   using namespace pbwd;
-  if (a->batch > kMaxPlanBatch) return fail(MF_ERR_UNSUPPORTED, "mf_simplicial_bwd: pair plan batch too large");
-  const Ws ws(a->batch, a->heads);
+  const Ws ws(a->batch, a->heads, a->tokens);
   unsigned char* wsp = static_cast<unsigned char*>(a->workspace);
+  const bool g16 = a->grads_dtype == MF_DTYPE_BF16;
   PlanParams pp{};
   pp.qv = a->query_valid;
   pp.pkv = a->pair_key_valid;
-  pp.total = reinterpret_cast<int*>(wsp);
+  pp.head = reinterpret_cast<int*>(wsp);
   pp.units = reinterpret_cast<uint32_t*>(wsp + ws.units);
-  pp.served = reinterpret_cast<int*>(wsp + ws.served);
   pp.counts = reinterpret_cast<int2*>(wsp + ws.counts);
   pp.lists = reinterpret_cast<uint16_t*>(wsp + ws.lists);
+  pp.dq = a->dq; pp.dk1 = a->dk1; pp.dv1 = a->dv1; pp.dk2 = a->dk2; pp.dv2 = a->dv2;
   pp.B = a->batch;
   pp.H = a->heads;
   pp.N = a->tokens;
+  pp.cap = ws.cap;
+  pp.jm = a->bias_u != nullptr ? Lay<true>::JM : Lay<false>::JM;
   Params p{};
-  p.total = pp.total;
+  p.head = pp.head;
   p.units = pp.units;
   p.counts = pp.counts;
   p.lists = pp.lists;
@@ -1283,55 +1342,28 @@ int simplicial_pair_bwd_launch(const mf_simplicial_bwd_args* a, hipStream_t stre
   p.go = static_cast<const __bf16*>(a->grad_out);
   p.out = a->out;
   p.lse = a->lse;
-  p.qv = a->query_valid;
-  p.pkv = a->pair_key_valid;
   p.pv = a->pair_valid;
   p.dq = a->dq; p.dk1 = a->dk1; p.dv1 = a->dv1; p.dk2 = a->dk2; p.dv2 = a->dv2;
-  p.gout16 = a->grads_dtype == MF_DTYPE_BF16 ? 1 : 0;
-  const bool bias = a->bias_u != nullptr;
-  if (bias) {
-    p.bu = static_cast<const uint16_t*>(a->bias_u);
-    p.bv = static_cast<const uint16_t*>(a->bias_v);
-    p.bw = static_cast<const uint16_t*>(a->bias_w);
-    p.bg = static_cast<const uint16_t*>(a->bias_gate);
-    p.du = a->du;
-    p.dvb = a->dv_bias;
-    p.dw = a->dw;
-    p.dgate = a->dgate;
-    p.dupart = reinterpret_cast<float*>(wsp + ws.dupart);
-    p.dvbpart = reinterpret_cast<float*>(wsp + ws.dvbpart);
-    p.dgpart = reinterpret_cast<float*>(wsp + ws.dgpart);
-    p.fds = reinterpret_cast<float*>(wsp + ws.fds);
-    p.dwpart = reinterpret_cast<float*>(wsp + ws.dwpart);
-  }
+  p.gout16 = g16 ? 1 : 0;
   p.H = a->heads;
   p.N = a->tokens;
-  DeviceInfo dev;
-  int st = device_info(&dev);
-  if (st != MF_OK) return st;
-  const size_t lds = bias ? Lay<true>::bytes : Lay<false>::bytes;
-  const void* kern = bias ? reinterpret_cast<const void*>(pair_bwd_kernel<true>)
-                          : reinterpret_cast<const void*>(pair_bwd_kernel<false>);
-  if (lds > size_t(dev.max_lds_per_block))
-    return fail(MF_ERR_UNSUPPORTED, "mf_simplicial_bwd: the pair kernel needs " + std::to_string(lds) +
-                                        " bytes of LDS per workgroup");
-  st = ensure_dynamic_lds(kern, int(lds));
-  if (st != MF_OK) return st;
-  const long long blocks = 2LL * a->batch * a->heads;  // the most units a plan can list
-  if (blocks > 0x7fffffffLL) return fail(MF_ERR_UNSUPPORTED, "mf_simplicial_bwd: grid too large");
-  hipLaunchKernelGGL(pair_bwd_plan, dim3(1), dim3(kPlanThreads), 0, stream, pp);
-  MF_HIP_CHECK(hipGetLastError());
-  if (bias) hipLaunchKernelGGL(pair_bwd_kernel<true>, dim3(unsigned(blocks)), dim3(kThreads), lds, stream, p);
-  else hipLaunchKernelGGL(pair_bwd_kernel<false>, dim3(unsigned(blocks)), dim3(kThreads), lds, stream, p);
-  MF_HIP_CHECK(hipGetLastError());
-  hipLaunchKernelGGL(pair_bwd_combine, dim3(unsigned(a->batch * a->heads)), dim3(kThreads), 0, stream, p);
-  MF_HIP_CHECK(hipGetLastError());
+  p.cap = ws.cap;
+  const bool bias = a->bias_u != nullptr;
   if (bias) {
-    hipLaunchKernelGGL(pair_bwd_bias_finish, dim3(unsigned(a->batch * a->heads), kFinishSplit), dim3(kThreads), 0,
-                       stream, p);
-    MF_HIP_CHECK(hipGetLastError());
+    p.bu = a->bias_u; p.bv = a->bias_v; p.bw = a->bias_w; p.bg = a->bias_gate;
+    p.du = a->du; p.dvb = a->dv_bias; p.dw = a->dw; p.dgate = a->dgate;
+    p.dvpart = reinterpret_cast<float*>(wsp + ws.dvpart);
+    p.dgpart = reinterpret_cast<float*>(wsp + ws.dgpart);
+    p.dwpart = reinterpret_cast<float*>(wsp + ws.dwpart);
   }
-  return MF_OK;
+  const int64_t bh = int64_t(a->batch) * a->heads;
+  const int64_t blocks = bh * ws.cap;  // the most units a plan can list
+  if (blocks > 0x7fffffffLL) return fail(MF_ERR_UNSUPPORTED, "mf_simplicial_bwd: grid too large");
+  hipLaunchKernelGGL(pair_bwd_prepare, dim3(unsigned(g16 ? 1 + bh : 1)), dim3(kPlanThreads), 0, stream, pp);
+  MF_HIP_CHECK(hipGetLastError());
+  if (!bias) return launch_units<0>(p, int(blocks), int(bh), stream);
+  if (a->bias_dtype == MF_DTYPE_BF16) return launch_units<1>(p, int(blocks), int(bh), stream);
+  return launch_units<2>(p, int(blocks), int(bh), stream);
 }
 
 }  // namespace mf
