@@ -44,6 +44,10 @@ int simplicial_pair_max_batch(int tokens);
 size_t simplicial_pair_workspace_bytes(int batch, int tokens);
 int simplicial_pair_launch(const mf_simplicial_fwd_args* a, void* claims, int num_cus, hipStream_t stream);
 
+// Pair-formulation forward for fp32 operands of at most 64 tokens (simplicial_pair_f32.hip).
+bool simplicial_pair_f32_serves(const mf_simplicial_fwd_args* a);
+int simplicial_pair_f32_launch(const mf_simplicial_fwd_args* a, hipStream_t stream);
+
 // Pair-formulation backward for bf16 operands and head_dim 64
 // (simplicial_pair_bwd.hip): every molecule of a call it serves, given
 // simplicial_pair_bwd_workspace_bytes() of 256-byte aligned workspace (a plan

@@ -1,0 +1,73 @@
+"""The fp32 pair-formulation kernels at the edges of their tiles and of the range they serve (forward at most 64
+tokens and head_dim 64, backward 32 and 32; larger calls run the general kernels), with and without a factorized
+bias, against float64 on the same inputs.
+
+Bar, normwise per result: products and sums are fp32 over at most n^2 = 4096 terms in short chains; 2^-24 per
+rounding with random signs over the chains (about 20 roundings a term) gives below 1e-6, and the hardware exp2's
+1 ulp of arguments up to 30 another 1e-6: 4e-6.  With offsets near 300 (log2 units) the argument itself is rounded
+to 2^-24 * 300 = 2e-5 of P: 4e-5 there."""
+
+import pytest
+import torch
+
+from matterformer_amd.hip_simplicial_attention import hip_simplicial_attention_forward
+from matterformer_amd.workloads import random_simplicial
+from test_gpu_simplicial_bwd import GRAD_NAMES, fp64_grads, hip_grads, logit_std, rel_err
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [([1, 2, 15], 4), ([16, 17, 9], 32), ([31, 32, 5], 32), ([29, 32], 20), ([32, 16], 64), ([33, 48], 32),
+          ([49, 64], 36), ([65, 12], 32)]
+
+
+@pytest.mark.parametrize("bias_dtype", [None, torch.float32, torch.bfloat16], ids=["none", "fp32", "bf16"])
+@pytest.mark.parametrize("counts,D", SHAPES, ids=lambda v: "-".join(map(str, v)) if isinstance(v, list) else f"D{v}")
+def test_fp32_tile_edges(cuda, counts, D, bias_dtype):
+    B, H, N = len(counts), 2, max(counts)
+    holes = [(b, 2) for b, n in enumerate(counts) if n > 8]
+    q, k1, v1, k2, v2, qv, pkv, pv = random_simplicial(B, H, N, D, seed=N + D, counts=counts, holes=holes,
+                                                       pair_drop=0.1, std=logit_std(D))
+    pv = pv | (torch.arange(N) < 2)[None, None, :]  # every query has valid pairs
+    gen = torch.Generator().manual_seed(N * 3 + D)
+    go = torch.randn(B, H, N, D, generator=gen)
+    bias = None
+    if bias_dtype is not None:
+        bias = [(torch.randn(B, H, N, N, generator=gen) * 0.5).to(bias_dtype) for _ in range(3)] + \
+               [torch.randn(B, H, N, generator=gen).to(bias_dtype)]
+    ops = [q, k1, v1, k2, v2]
+    out, got = hip_grads([t.to(cuda) for t in ops], qv.to(cuda), pkv.to(cuda), pv.to(cuda), go.to(cuda), "ieee_fp32",
+                         bias=None if bias is None else [t.to(cuda) for t in bias])
+    want, ref = fp64_grads(ops, qv, pkv, pv, go, bias=bias)
+    assert rel_err(out.cpu().numpy(), want) <= 4e-6
+    for name, g, r in zip(GRAD_NAMES, got, ref):
+        # a bf16 bias gets bf16 gradients (rounding 2^-9, 1.7e-3 normwise)
+        bar = 4e-3 if g.dtype == torch.bfloat16 else 4e-6
+        assert rel_err(g.float().cpu().numpy(), r) <= bar, name
+
+
+def test_large_and_masking_scale_logits(cuda):
+    """Logits far past the first tile's maximum in both directions (the offset moves many times) and bias terms of
+    -30000 beside ordinary ones; padded queries, a molecule without keys and one without queries give zeros."""
+    B, H, N, D = 4, 2, 29, 32
+    q, k1, v1, k2, v2, qv, pkv, _ = random_simplicial(B, H, N, D, seed=3, counts=[29, 20, 9, 9], std=logit_std(D))
+    q = q * 60.0
+    qv, pkv = qv.clone(), pkv.clone()
+    pkv[2] = False
+    qv[3] = False
+    gen = torch.Generator().manual_seed(4)
+    u, v, w = (torch.randn(B, H, N, N, generator=gen) for _ in range(3))
+    w[torch.rand(B, H, N, N, generator=gen) < 0.3] = -30000.0
+    bias = [u, v, w, torch.rand(B, H, N, generator=gen) + 0.5]
+    ops = [q, k1, v1, k2, v2]
+    kw = dict(u=bias[0], v_bias=bias[1], w=bias[2], gate=bias[3])
+    out, lse, out32 = hip_simplicial_attention_forward(
+        *[t.to(cuda) for t in ops], query_valid=qv.to(cuda), pair_key_valid=pkv.to(cuda), pair_valid=None,
+        precision="ieee_fp32", **{k: t.to(cuda) for k, t in kw.items()})
+    torch.cuda.synchronize()
+    go = torch.randn(B, H, N, D, generator=gen)
+    sub = slice(0, 2)
+    want, _ = fp64_grads([t[sub] for t in ops], qv[sub], pkv[sub], None, go[sub], bias=[t[sub] for t in bias])
+    assert rel_err(out[sub].cpu().numpy(), want) <= 4e-5
+    assert torch.equal(out, out32)
+    assert not out[2:].any() and not lse[2:].any()
+    assert not out[1, :, 20:].any() and not lse[1, :, 20:].any()
