@@ -1268,6 +1268,7 @@ extern "C" int mf_simplicial_bwd(const mf_simplicial_bwd_args* a, void* stream) 
     }
   }
   if (pair) return simplicial_pair_bwd_launch(a, s);
+  if (simplicial_pair_f32_bwd_serves(a)) return simplicial_pair_f32_bwd_launch(a, s);
   // other bf16 operands with a bf16 grad_out: bf16 MFMA (K steps of 32 d), which stages grad_out rows as bf16
   // (exact only for a bf16 grad_out).  Everything else -- fp16 operands, or a grad_out of another dtype -- takes
   // the fp32 path, which reads every operand in its own dtype.
