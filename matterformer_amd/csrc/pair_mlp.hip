@@ -9,9 +9,9 @@
 // written per head as [B, H, N, N] with the diagonal and the pairs outside
 // the geometry pair mask zero (:711-717).  The reference materialises the
 // [B, N, N, F] features and the [B, N, N, hidden] activations of each MLP;
-// here one wave takes a (molecule b, row i, 64-column group) unit, writes
-// the zeros of its invalid pairs, and for each 16-column chunk with a valid
-// pair runs the 16 pairs (b, i, j0..j0+15) with everything in registers:
+// here a workgroup scans rows (b, i), writes the zeros of their invalid pairs
+// and queues the valid ones in LDS; its waves then take tiles of 32 queued
+// pairs (two MFMA columns of 16) with everything in registers:
 //
 //   layer 1  C1[h][p] = b1[h] + sum_f W1[h][f] X[p][f]    fp32 MFMA 16x16x4,
 //            M = 16 hidden units, N = 16 pairs, K = 4 features per step;
@@ -24,7 +24,13 @@
 //            same order
 //
 // The weights of the three MLPs are staged in LDS once per workgroup (rows
-// padded to an odd stride).  fp32 throughout; the exponentials (rbf features,
+// padded to an odd stride); each is read once for the tile's two columns.
+// The queue makes every tile full whatever the rows hold, and rows are dealt
+// to workgroups in a scrambled order: molecules and rows differ by the number
+// of their valid pairs, and a wave that kept to its own rows had none, one or
+// three of them (64 molecules of mean 44 atoms padded to 181, 8
+// heads: 126 -> 111 us, of which the zeros alone take about 50; compact to 73 columns, where they are few, 256
+// molecules: 389 -> 227 us).  fp32 throughout; the exponentials (rbf features,
 // SiLU) use the hardware exp2 and reciprocal, a few ulp, well inside the
 // rounding of the fp32 sums around them.
 #include <algorithm>
@@ -40,6 +46,16 @@ constexpr int kMaxHidden = 256;
 constexpr int kMaxHeads = 16;
 constexpr int kMaxRbf = 29;  // spoke features 3 + R <= 32
 
+constexpr int kSegGroups = 4;  // 64-column groups of a row scanned at a time, at most
+
+// Size of a workgroup's queue: columns scanned at a time (64 seg_groups, one row per wave) and the pending pairs at
+// which it runs tiles.  The smaller ones are for weights that nearly fill the LDS.
+struct QueueSize {
+  int seg_groups, batch;
+  __host__ __device__ int entries(int waves) const { return batch + waves * 64 * seg_groups; }
+  __host__ __device__ size_t bytes(int waves) const { return (size_t(entries(waves)) * 6 + 15) / 16 * 16; }
+};
+
 struct Params {
   const float* delta;
   const float* dnorm;
@@ -51,7 +67,8 @@ struct Params {
   const float* w2[3];
   const float* b2[3];
   float* out[3];
-  int B, N, R, hidden, heads, groups;
+  QueueSize queue;
+  int B, N, R, hidden, heads;
   // periodic features (PER instantiations): nf Fourier frequencies, the molecule's 6 global features
   int nf;
   const float* freqs;
@@ -69,48 +86,98 @@ __device__ __forceinline__ float silu(float x) {
   return x * __builtin_amdgcn_rcpf(1.0f + e);
 }
 
-// One MLP over the 16 pairs of a chunk: layer 1 (K steps of 4 features, x[t] = feature 4 t + g of pair r16),
-// SiLU, layer 2; lane (g, r16) returns outputs 4 g .. 4 g + 3 of pair r16.  Two 16-unit hidden slices are
-// in flight at a time so one slice's SiLU overlaps the other's MFMA chain.
+// One MLP over the two 16-pair columns of a tile: layer 1 (K steps of 4 features, x[c][t] = feature 4 t + g of
+// pair r16 of column c), SiLU, layer 2; lane (g, r16) returns outputs 4 g .. 4 g + 3 of pair r16 of each column.
 template <int K>
-__device__ __forceinline__ mf_f32x4 mlp16(const float (&x)[K], const float* W1, const float* B1, const float* W2,
-                                          const float* B2, int s1, int s2, int HT, int g, int r16) {
-  mf_f32x4 o2;
+__device__ __forceinline__ void mlp32(const float (&x)[2][K], const float* W1, const float* B1, const float* W2,
+                                      const float* B2, int s1, int s2, int HT, int g, int r16, mf_f32x4 (&o2)[2]) {
 #pragma unroll
-  for (int r = 0; r < 4; ++r) o2[r] = B2[4 * g + r];
+  for (int r = 0; r < 4; ++r) o2[0][r] = o2[1][r] = B2[4 * g + r];
   const float* w2row = W2 + r16 * s2 + 4 * g;
-  int ht = 0;
-  for (; ht + 2 <= HT; ht += 2) {
+  const float* w1row = W1 + r16 * s1 + g;
+  const float* b1row = B1 + 4 * g;
+  for (int ht = 0; ht < HT; ++ht) {
     mf_f32x4 ca, cb;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      ca[r] = B1[16 * ht + 4 * g + r];
-      cb[r] = B1[16 * ht + 16 + 4 * g + r];
-    }
-    const float* wa = W1 + (16 * ht + r16) * s1 + g;
-    const float* wb = wa + 16 * s1;
+    for (int r = 0; r < 4; ++r) ca[r] = cb[r] = b1row[16 * ht + r];
 #pragma unroll
     for (int t = 0; t < K; ++t) {
-      ca = mma(wa[4 * t], x[t], ca);
-      cb = mma(wb[4 * t], x[t], cb);
+      const float w = w1row[16 * ht * s1 + 4 * t];
+      ca = mma(w, x[0][t], ca);
+      cb = mma(w, x[1][t], cb);
     }
 #pragma unroll
-    for (int r = 0; r < 4; ++r) o2 = mma(w2row[16 * ht + r], silu(ca[r]), o2);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) o2 = mma(w2row[16 * ht + 16 + r], silu(cb[r]), o2);
+    for (int r = 0; r < 4; ++r) {
+      const float w = w2row[16 * ht + r];
+      o2[0] = mma(w, silu(ca[r]), o2[0]);
+      o2[1] = mma(w, silu(cb[r]), o2[1]);
+    }
   }
-  if (ht < HT) {
-    mf_f32x4 ca;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) ca[r] = B1[16 * ht + 4 * g + r];
-    const float* wa = W1 + (16 * ht + r16) * s1 + g;
-#pragma unroll
-    for (int t = 0; t < K; ++t) ca = mma(wa[4 * t], x[t], ca);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) o2 = mma(w2row[16 * ht + r], silu(ca[r]), o2);
-  }
-  return o2;
 }
+
+// Rows as the workgroups take them: row s of the scan is row i of molecule b, molecules fastest and shifted by a
+// hash of i, so that a workgroup's rows (s, s + stride, ...) come from many molecules and heights.
+__device__ __forceinline__ void scan_row(long long s, int B, int& b, int& i) {
+  i = int(s / B);
+  const int r = int(s - (long long)i * B);
+  b = int((unsigned(r) + (unsigned(i) * 0x9E3779B1u >> 8) % unsigned(B)) % unsigned(B));
+}
+
+// Valid columns of (b, i) from j0: one ballot per 64 columns.
+__device__ __forceinline__ void row_bits(const uint8_t* mask, int N, int b, int i, int j0, int groups, int lane,
+                                         unsigned long long (&bal)[kSegGroups]) {
+  uint8_t v[kSegGroups];
+#pragma unroll
+  for (int c = 0; c < kSegGroups; ++c)
+    v[c] = mask[(size_t(b) * N + i) * N + min(j0 + 64 * c + lane, N - 1)];  // clamped: no branches
+#pragma unroll
+  for (int c = 0; c < kSegGroups; ++c) {
+    const int j = j0 + 64 * c + lane;
+    bal[c] = __ballot(c < groups && j < N && j != i && v[c] != 0);
+  }
+}
+
+// Queued pairs: row b N + i and column j, 6 bytes each.  Past 65535 columns the rows are below 2^21 (the entry points'
+// limit), and the column's high bits take the row word's upper ones.
+struct Queue {
+  uint32_t* row;
+  uint16_t* col;
+  int shift;
+  __device__ Queue(void* lds, int entries, int N)
+      : row(static_cast<uint32_t*>(lds)), col(reinterpret_cast<uint16_t*>(static_cast<uint32_t*>(lds) + entries)),
+        shift(N > 65535 ? 21 : 31) {}
+  __device__ __forceinline__ void get(int at, uint32_t& r, uint32_t& j) const {
+    const uint32_t w = row[at];
+    r = w & ((1u << shift) - 1u);
+    j = col[at] | (w >> shift) << 16;
+  }
+  // appends a wave's valid pairs from `at` (the counts of the waves before it are in)
+  __device__ __forceinline__ void append(int at, uint32_t r, int j0, int lane, const unsigned long long (&bal)[kSegGroups]) {
+#pragma unroll
+    for (int c = 0; c < kSegGroups; ++c) {
+      if ((bal[c] >> lane) & 1ull) {
+        const int o = at + __popcll(bal[c] & ((1ull << lane) - 1ull));
+        const uint32_t j = uint32_t(j0 + 64 * c + lane);
+        row[o] = r | (j >> 16) << shift;
+        col[o] = uint16_t(j);
+      }
+      at += __popcll(bal[c]);
+    }
+  }
+  // moves the entries n .. pending - 1 (fewer than the workgroup's threads) to the front; all threads call it
+  __device__ __forceinline__ void drop(int n, int pending, int tid) {
+    __syncthreads();
+    const bool on = tid < pending - n;
+    const uint32_t r = on ? row[n + tid] : 0u;
+    const uint16_t c = on ? col[n + tid] : uint16_t(0);
+    __syncthreads();
+    if (on) {
+      row[tid] = r;
+      col[tid] = c;
+    }
+    __syncthreads();
+  }
+};
 
 // Spoke feature f of a pair under PER (transformer.py:641-652; geometry_bias's _periodic_terms): the delta,
 // rbf, then for each delta component c the sines and cosines of (2 pi delta_c) freq_k, then the 6 global
@@ -190,108 +257,131 @@ __global__ void __launch_bounds__(kThreads, PER ? 1 : 4) pair_mlp_kernel(Params 
     const int f = 4 * t + g;
     cp[t] = f < p.R ? p.centers[f] : 0.0f;
   }
-  // unit u = (cg * N + i) * B + b: molecule b, row i, 64-column group cg.  Each lane owns one pair (b, i, j)
-  // of the unit and writes the zeros of all outputs when the pair is invalid (256-byte row pieces per
-  // store); the 16-column chunks with a valid pair then run the MLPs and write their valid pairs.  Waves
-  // take units round-robin, the next unit's (cg, i, b) following by carries (wave-uniform scalar
-  // arithmetic), and its pair-mask byte is fetched one unit ahead.
-  const int nwaves = gridDim.x * (kThreads / 64);
-  const int db = nwaves % B, di = (nwaves / B) % N, dc = (nwaves / B) / N;
-  int b, i, cg;
-  {
-    const int u0 = blockIdx.x * (kThreads / 64) + (tid >> 6);
-    b = u0 % B;
-    i = (u0 / B) % N;
-    cg = (u0 / B) / N;
-  }
-  auto mask_byte = [&](int bb, int ii, int cc) -> unsigned {
-    const int j = cc * 64 + lane;
-    if (cc >= p.groups || j >= N) return 0u;
-    return p.mask[(size_t(bb) * N + ii) * N + j];
-  };
-  unsigned mbyte = mask_byte(b, i, cg);
-  while (cg < p.groups) {
-    int nb = b + db;
-    int carry = nb >= B;
-    nb -= carry ? B : 0;
-    int ni = i + di + carry;
-    carry = ni >= N;
-    ni -= carry ? N : 0;
-    const int ncg = cg + dc + carry;
-    const unsigned next = mask_byte(nb, ni, ncg);
-
-    const size_t prow = (size_t(b) * N + i) * N;
-    // output element (o, b, i, j): ((b * H + o) * N + i) * N + j
-    const size_t obase = size_t(b) * H * plane + size_t(i) * N;
-    const int j = cg * 64 + lane;
-    const bool in = j < N;
-    const bool valid = in && j != i && mbyte != 0u;
-    if (in && !valid) {
-      for (int m = 0; m < 3; ++m) {
-        float* dst = p.out[m] + obase + j;
-        for (int o = 0; o < H; ++o) dst[size_t(o) * plane] = 0.0f;
-      }
-    }
-    const unsigned long long bal = __ballot(valid);
-    for (int c = 0; c < 4; ++c) {
-      const unsigned bits = unsigned(bal >> (16 * c)) & 0xffffu;
-      if (bits == 0u) continue;  // wave-uniform
-      const int jc = cg * 64 + 16 * c + r16;
-      const bool jvalid = (bits >> r16) & 1u;
-      const size_t pair = prow + (jvalid ? jc : 0);
-      const float dn = jvalid ? p.dnorm[pair] : 0.0f;
-      float xs[KS], xp[KP];
-      if constexpr (PER) {
-        const float d0 = jvalid ? p.delta[3 * pair] : 0.0f;
-        const float d1 = jvalid ? p.delta[3 * pair + 1] : 0.0f;
-        const float d2 = jvalid ? p.delta[3 * pair + 2] : 0.0f;
+  constexpr int kWaves = kThreads / 64, kTile = 32, kBatch = kWaves * kTile;
+  Queue queue(lds + off[2][3] + 16, p.queue.entries(kWaves), N);
+  __shared__ int counts[kWaves];
+  const int wave = tid >> 6;
+  const int sw = 64 * p.queue.seg_groups;  // columns scanned at a time
+  const long long rows = (long long)B * N;
+  const long long stride = (long long)gridDim.x * kWaves;
+  int pending = 0;
+  // the first `tiles` tiles of the queue (the last one may be short): features, MLPs, stores
+  auto run_tiles = [&](int n) {
+    for (int t0 = wave * kTile; t0 < n; t0 += kBatch) {
+      bool pv[2];
+      float xs[2][KS], xp[2][KP];
+      size_t obase[2];
 #pragma unroll
-        for (int t = 0; t < KS; ++t) {
-          const float d = dn - cs[t];
-          xs[t] = periodic_spoke(p, 4 * t + g, d0, d1, d2, __builtin_amdgcn_exp2f(kexp * (d * d)), b);
-        }
+      for (int c = 0; c < 2; ++c) {
+        pv[c] = t0 + 16 * c + r16 < n;
+        const int at = pv[c] ? t0 + 16 * c + r16 : t0;
+        uint32_t row, j;
+        queue.get(at, row, j);
+        const int b = int(row / uint32_t(N));
+        obase[c] = size_t(b) * H * plane + size_t(row - uint32_t(b) * uint32_t(N)) * N + j;
+        const size_t pair = size_t(row) * N + j;
+        const float dn = p.dnorm[pair];
+        const float* dl = p.delta + 3 * pair;
+        if constexpr (PER) {
+          const float d0 = dl[0], d1 = dl[1], d2 = dl[2];
 #pragma unroll
-        for (int t = 0; t < KP; ++t) {
-          const int f = 4 * t + g;
-          const float d = dn - cp[t];
-          xp[t] = f < p.R ? __builtin_amdgcn_exp2f(kexp * (d * d))
-                          : (f < p.R + 6 ? p.glob[size_t(b) * 6 + (f - p.R)] : 0.0f);
-        }
-      } else {
+          for (int t = 0; t < KS; ++t) {
+            const float d = dn - cs[t];
+            xs[c][t] = periodic_spoke(p, 4 * t + g, d0, d1, d2, __builtin_amdgcn_exp2f(kexp * (d * d)), b);
+          }
 #pragma unroll
-        for (int t = 0; t < KS; ++t) {
-          const int f = 4 * t + g;
-          const float d = dn - cs[t];
-          const float rbf = __builtin_amdgcn_exp2f(kexp * (d * d));
-          xs[t] = f < 3 ? (jvalid ? p.delta[3 * pair + f] : 0.0f) : (f < 3 + p.R ? rbf : 0.0f);
-        }
+          for (int t = 0; t < KP; ++t) {
+            const int f = 4 * t + g;
+            const float d = dn - cp[t];
+            xp[c][t] = f < p.R ? __builtin_amdgcn_exp2f(kexp * (d * d))
+                               : (f < p.R + 6 ? p.glob[size_t(b) * 6 + (f - p.R)] : 0.0f);
+          }
+        } else {
+          const float d0 = dl[min(g, 2)];
 #pragma unroll
-        for (int t = 0; t < KP; ++t) {
-          const int f = 4 * t + g;
-          const float d = dn - cp[t];
-          xp[t] = f < p.R ? __builtin_amdgcn_exp2f(kexp * (d * d)) : 0.0f;
+          for (int t = 0; t < KS; ++t) {
+            const int f = 4 * t + g;
+            const float d = dn - cs[t];
+            const float rbf = __builtin_amdgcn_exp2f(kexp * (d * d));
+            xs[c][t] = f < 3 ? d0 : (f < 3 + p.R ? rbf : 0.0f);
+          }
+#pragma unroll
+          for (int t = 0; t < KP; ++t) {
+            const int f = 4 * t + g;
+            const float d = dn - cp[t];
+            xp[c][t] = f < p.R ? __builtin_amdgcn_exp2f(kexp * (d * d)) : 0.0f;
+          }
         }
       }
+#pragma unroll 1
       for (int m = 0; m < 3; ++m) {
-        const mf_f32x4 o2 = m < 2 ? mlp16<KS>(xs, lds + off[m][0], lds + off[m][1], lds + off[m][2],
-                                               lds + off[m][3], s1s, s2, HT, g, r16)
-                                  : mlp16<KP>(xp, lds + off[m][0], lds + off[m][1], lds + off[m][2],
-                                              lds + off[m][3], s1p, s2, HT, g, r16);
-        if (jvalid) {
-          float* dst = p.out[m] + obase + jc;
+        mf_f32x4 o2[2];
+        if (m < 2)
+          mlp32<KS>(xs, lds + off[m][0], lds + off[m][1], lds + off[m][2], lds + off[m][3], s1s, s2, HT, g, r16, o2);
+        else
+          mlp32<KP>(xp, lds + off[m][0], lds + off[m][1], lds + off[m][2], lds + off[m][3], s1p, s2, HT, g, r16, o2);
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          if (!pv[c]) continue;
+          float* dst = p.out[m] + obase[c];
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const int o = 4 * g + r;
-            if (o < H) dst[size_t(o) * plane] = o2[r];
+            if (o < H) dst[size_t(o) * plane] = o2[c][r];
           }
         }
       }
     }
-    b = nb;
-    i = ni;
-    cg = ncg;
-    mbyte = next;
+  };
+  for (long long s0 = (long long)blockIdx.x; s0 < rows; s0 += stride) {
+    const long long s = s0 + (long long)wave * gridDim.x;
+    const bool on = s < rows;
+    int b = 0, i = 0;
+    if (on) scan_row(s, B, b, i);
+    for (int j0 = 0; j0 < N; j0 += sw) {
+      unsigned long long bal[kSegGroups];
+#pragma unroll
+      for (int c = 0; c < kSegGroups; ++c) bal[c] = 0ull;
+      int mine = 0;
+      if (on) {
+        row_bits(p.mask, N, b, i, j0, p.queue.seg_groups, lane, bal);
+#pragma unroll
+        for (int c = 0; c < kSegGroups; ++c) mine += __popcll(bal[c]);
+      }
+      if (lane == 0) counts[wave] = mine;
+      __syncthreads();
+      int at = pending, total = 0;
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) {
+        const int n = counts[w];
+        at += w < wave ? n : 0;
+        total += n;
+      }
+      queue.append(at, uint32_t(b) * uint32_t(N) + uint32_t(i), j0, lane, bal);
+      pending += total;
+      // the zeros of the row's invalid pairs (whole row pieces per store)
+      if (on) {
+        const size_t obase = size_t(b) * H * plane + size_t(i) * N;
+        for (int m = 0; m < 3; ++m)
+          for (int o = 0; o < H; ++o) {
+            float* dst = p.out[m] + obase + size_t(o) * plane + j0;
+#pragma unroll
+            for (int c = 0; c < kSegGroups; ++c) {
+              const int j = 64 * c + lane;
+              if (c < p.queue.seg_groups && j0 + j < N && !((bal[c] >> lane) & 1ull)) dst[j] = 0.0f;
+            }
+          }
+      }
+      __syncthreads();
+      if (pending >= p.queue.batch) {  // whole batches: every wave has the same number of full tiles
+        const int n = pending / p.queue.batch * p.queue.batch;
+        run_tiles(n);
+        queue.drop(n, pending, tid);
+        pending -= n;
+      }
+    }
   }
+  run_tiles(pending);
 }
 
 size_t lds_bytes(int ks, int kp, int hidden) {
@@ -305,15 +395,22 @@ size_t lds_bytes(int ks, int kp, int hidden) {
 }
 
 template <int KS, int KP, bool PER>
-int launch(const Params& p, int num_cus, int max_lds, hipStream_t s) {
-  const size_t lds = lds_bytes(KS, KP, p.hidden);
-  if (lds > size_t(max_lds))
+int launch(Params p, int num_cus, int max_lds, hipStream_t s) {
+  constexpr int kWaves = kThreads / 64;
+  const size_t weights = (lds_bytes(KS, KP, p.hidden) + 15) / 16 * 16;
+  p.queue = QueueSize{kSegGroups, 32 * kWaves};
+  const size_t room = size_t(max_lds) - sizeof(int) * kWaves;  // (beside the static counts)
+  if (weights + p.queue.bytes(kWaves) > room) p.queue = QueueSize{1, 32 * kWaves};
+  if (weights + p.queue.bytes(kWaves) > room) p.queue = QueueSize{1, 32};
+  const size_t lds = weights + p.queue.bytes(kWaves);
+  if (lds > room)
     return fail(MF_ERR_UNSUPPORTED, "mf_pair_mlp_bias: weights exceed the LDS of a workgroup");
   // dynamic LDS above 64 KB needs the attribute (once per kernel and device)
-  const int st = ensure_dynamic_lds(reinterpret_cast<const void*>(pair_mlp_kernel<KS, KP, PER>), 160 * 1024);
+  const int st = ensure_dynamic_lds(reinterpret_cast<const void*>(pair_mlp_kernel<KS, KP, PER>),
+                                    max_lds - int(sizeof(int)) * kWaves);
   if (st != MF_OK) return st;
-  const long long units = (long long)p.B * p.N * p.groups;
-  const int grid = int(std::min<long long>((units + 7) / 8, (long long)num_cus * 2));
+  const long long rows = (long long)p.B * p.N;
+  const int grid = int(std::min<long long>((rows + 7) / 8, (long long)num_cus * 2));
   hipLaunchKernelGGL((pair_mlp_kernel<KS, KP, PER>), dim3(grid), dim3(kThreads), lds, s, p);
   MF_HIP_CHECK(hipGetLastError());
   return MF_OK;
@@ -325,17 +422,22 @@ int launch(const Params& p, int num_cus, int max_lds, hipStream_t s) {
 //   a1 = W1 x + b1,  h = SiLU(a1),  dH = W2^T dY,  dA = dH (.) SiLU'(a1),  SiLU'(a) = s (1 + a (1 - s)),
 //   dW2 += dY h^T,  db2 += dY,  dW1 += dA x^T,  db1 += dA   (db1 as the column of dW1 for a constant-1
 //   feature placed after the last real one).
-// One workgroup of kBwdThreads takes MLP blockIdx.y; its waves take (molecule, row, 64-column group) units
-// as the forward does and, per 16-pair chunk with a valid pair, recompute layer 1 transposed (MFMA 16x16x4
+// One workgroup of kBwdThreads takes MLP blockIdx.y; it queues the valid pairs of its rows as the forward does and
+// its waves take tiles of 16 of them, recompute layer 1 transposed (MFMA 16x16x4
 // fp32, pairs as the rows: lane (g, r16) holds pairs 4 g + r of hidden unit r16), form dH^T the same way,
 // and accumulate dW1^T [f][h] and dW2 [o][h] by MFMA over the pairs (K): accumulator r of h and dA is the B
 // operand of K step r as it is (K index g = pair 4 g + r), so nothing is transposed.  The waves of a workgroup add
 // their sums into LDS in wave order and the workgroup writes them to its workspace slot; a second launch adds
 // the slots in slot order.  Deterministic (no atomics).
 // ---------------------------------------------------------------------------
+//
+// 64 molecules of mean 44 atoms padded to 181, hidden 128, 8 heads: 478 -> 204 us.  The accumulators were indexed by
+// a runtime loop (moves through scratch and relative registers, 115 VALU per hidden tile), and a wave's share was
+// the valid pairs of its own rows.  The MFMA of the valid pairs take 53 us; two waves per SIMD, whose loads of a
+// tile's features and upstream gradients the other one has to cover, are what is left.
 constexpr int kBwdThreads = 256;
 constexpr int kBwdWaves = kBwdThreads / 64;
-constexpr int kBwdGroups = 256;     // workgroups per MLP (about three per CU at ~170 registers per lane)
+constexpr int kBwdGroups = 170;     // workgroups per MLP: two per CU for the three MLPs (~220 registers per lane)
 constexpr int kBwdMaxHidden = 128;  // dW1^T / dW2 accumulators in registers: 2 x HT + HT tiles
 constexpr int kBwdSlots = kBwdGroups;
 
@@ -354,20 +456,20 @@ struct BwdParams {
   float* dw2[3];        // [H, hidden]
   float* db2[3];        // [H]
   float* slots;         // [3][kBwdSlots][48 hidden + 16] per-wave partial sums
-  int B, N, R, hidden, heads, groups;
+  QueueSize queue;
+  int B, N, R, hidden, heads;
 };
 
 __host__ __device__ inline size_t bwd_slot_floats(int hidden) { return size_t(48) * hidden + 16; }
 
-template <int KS, int KP>
-__global__ void __launch_bounds__(kBwdThreads) pair_mlp_bwd_kernel(BwdParams p) {
+template <int K>  // layer-1 K steps (features 4 t + g, the constant 1 included)
+__global__ void __launch_bounds__(kBwdThreads, 2) pair_mlp_bwd_kernel(BwdParams p) {
   extern __shared__ float lds[];
   const int m = blockIdx.y;
-  constexpr int KMAX = KS > KP ? KS : KP;
-  const int K = m < 2 ? KS : KP;          // layer-1 K steps (features 4 t + g)
   const int F = m < 2 ? 3 + p.R : p.R;    // true input width; feature F is the constant 1 (db1)
   const int hidden = p.hidden, H = p.heads, HT = hidden / 16;
-  const int s1 = 4 * K + 1, s2 = hidden + 1;
+  constexpr int s1 = 4 * K + 1;
+  const int s2 = hidden + 1;
   // LDS: W1 [hidden][s1] (columns >= F zero), b1 [hidden], W2 [16][s2] (rows >= H zero), then the
   // workgroup's sums [48 hidden + 16]
   float* W1 = lds;
@@ -401,64 +503,75 @@ __global__ void __launch_bounds__(kBwdThreads) pair_mlp_bwd_kernel(BwdParams p) 
     return f == F ? 1.0f : 0.0f;
   };
 
-  mf_f32x4 aw1[2][kBwdMaxHidden / 16], aw2[kBwdMaxHidden / 16];
+  constexpr int kHT = kBwdMaxHidden / 16;
+  mf_f32x4 aw1[2][kHT], aw2[kHT];  // (indexed by unrolled loops only: a runtime index puts them in scratch)
 #pragma unroll
-  for (int ht = 0; ht < kBwdMaxHidden / 16; ++ht) {
+  for (int ht = 0; ht < kHT; ++ht) {
     aw1[0][ht] = aw1[1][ht] = aw2[ht] = mf_f32x4{0.f, 0.f, 0.f, 0.f};
   }
   float adb2 = 0.0f;
 
-  const long long units = (long long)B * N * p.groups;
-  const int nw = gridDim.x * kBwdWaves;
-  for (long long u = (long long)blockIdx.x * kBwdWaves + wave; u < units; u += nw) {
-    const int b = int(u % B);
-    const int i = int((u / B) % N);
-    const int cg = int(u / ((long long)B * N));
-    const int j = cg * 64 + lane;
-    const bool valid = j < N && j != i && p.mask[(size_t(b) * N + i) * N + min(j, N - 1)] != 0;
-    const unsigned long long bal = __ballot(valid);
-    const size_t prow = (size_t(b) * N + i) * N;
-    for (int c = 0; c < 4; ++c) {
-      const unsigned bits = unsigned(bal >> (16 * c)) & 0xffffu;
-      if (bits == 0u) continue;  // wave-uniform
-      const int j0 = cg * 64 + 16 * c;
+  constexpr int kTile = 16, kBatch = kBwdWaves * kTile;
+  Queue queue(red + 48 * hidden + 16, p.queue.entries(kBwdWaves), N);
+  __shared__ int counts[kBwdWaves];
+  const int sw = 64 * p.queue.seg_groups;  // columns scanned at a time
+  const long long rows = (long long)B * N;
+  const long long stride = (long long)gridDim.x * kBwdWaves;
+  int pending = 0;
+  auto run_tiles = [&](int n) {
+    for (int t0 = wave * kTile; t0 < n; t0 += kBatch) {
       // pair r16 (layer 1, dH): features 4 t + g, upstream gradients of heads 4 s + g
-      const bool v16 = (bits >> r16) & 1u;
-      const size_t pr = prow + (v16 ? j0 + r16 : 0);
-      const float dn16 = v16 ? p.dnorm[pr] : 0.0f;
-      float xf[KMAX];
+      const bool v16 = t0 + r16 < n;
+      const int at16 = v16 ? t0 + r16 : t0;
+      uint32_t row16, j16;
+      queue.get(at16, row16, j16);
+      const int b16 = int(row16 / uint32_t(N));
+      const size_t pr = size_t(row16) * N + j16;
+      const size_t yo16 = size_t(b16) * H * plane + size_t(row16 - uint32_t(b16) * uint32_t(N)) * N + j16;
+      const float dn16 = p.dnorm[pr];
+      float xf[K];
 #pragma unroll
-      for (int t = 0; t < KMAX; ++t) xf[t] = (t < K && v16) ? feature(pr, dn16, 4 * t + g) : 0.0f;
+      for (int t = 0; t < K; ++t) xf[t] = v16 ? feature(pr, dn16, 4 * t + g) : 0.0f;
       float yb[4];
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
         const int o = 4 * s + g;
-        yb[s] = (v16 && o < H) ? gy[(size_t(b) * H + o) * plane + size_t(i) * N + j0 + r16] : 0.0f;
+        yb[s] = (v16 && o < H) ? gy[yo16 + size_t(o) * plane] : 0.0f;
       }
       // pairs 4 g + s (dW1 / dW2 A operands of K step s): features 16 ft + r16, upstream gradient of head r16
       float xw[4][2], ya[4];
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
         const int q = 4 * g + s;
-        const bool vq = (bits >> q) & 1u;
-        const size_t pq = prow + (vq ? j0 + q : 0);
-        const float dnq = vq ? p.dnorm[pq] : 0.0f;
+        const bool vq = t0 + q < n;
+        const int atq = vq ? t0 + q : t0;
+        uint32_t rowq, jq;
+        queue.get(atq, rowq, jq);
+        const int bq = int(rowq / uint32_t(N));
+        const size_t pq = size_t(rowq) * N + jq;
+        const size_t yoq = size_t(bq) * H * plane + size_t(rowq - uint32_t(bq) * uint32_t(N)) * N + jq;
+        const float dnq = p.dnorm[pq];
 #pragma unroll
         for (int ft = 0; ft < 2; ++ft) xw[s][ft] = vq ? feature(pq, dnq, 16 * ft + r16) : 0.0f;
-        ya[s] = (vq && r16 < H) ? gy[(size_t(b) * H + r16) * plane + size_t(i) * N + j0 + q] : 0.0f;
+        ya[s] = (vq && r16 < H) ? gy[yoq + size_t(r16) * plane] : 0.0f;
         adb2 += ya[s];
       }
-      for (int ht = 0; ht < HT; ++ht) {
+#pragma unroll
+      for (int ht = 0; ht < kHT; ++ht) {
+        if (ht >= HT) break;  // uniform
         // layer 1 and dH, transposed: pairs 4 g + r, hidden unit 16 ht + r16
         const float bias1 = B1[16 * ht + r16];
         mf_f32x4 a1 = mf_f32x4{bias1, bias1, bias1, bias1}, dh = mf_f32x4{0.f, 0.f, 0.f, 0.f};
         const float* wa = W1 + (16 * ht + r16) * s1 + g;
 #pragma unroll
-        for (int t = 0; t < KMAX; ++t)
-          if (t < K) a1 = mma(xf[t], wa[4 * t], a1);
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-          if (4 * s < H) dh = mma(yb[s], W2[(4 * s + g) * s2 + 16 * ht + r16], dh);
+        for (int t = 0; t < K; ++t) a1 = mma(xf[t], wa[4 * t], a1);
+        const float* wd = W2 + g * s2 + 16 * ht + r16;  // rows past H are zero
+        dh = mma(yb[0], wd[0], dh);
+        dh = mma(yb[1], wd[4 * s2], dh);
+        if (H > 8) {
+          dh = mma(yb[2], wd[8 * s2], dh);
+          dh = mma(yb[3], wd[12 * s2], dh);
+        }
         float hv[4], dv[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -476,14 +589,52 @@ __global__ void __launch_bounds__(kBwdThreads) pair_mlp_bwd_kernel(BwdParams p) 
         }
       }
     }
+  };
+  for (long long s0 = (long long)blockIdx.x; s0 < rows; s0 += stride) {
+    const long long s = s0 + (long long)wave * gridDim.x;
+    const bool on = s < rows;
+    int b = 0, i = 0;
+    if (on) scan_row(s, B, b, i);
+    for (int j0 = 0; j0 < N; j0 += sw) {
+      unsigned long long bal[kSegGroups];
+#pragma unroll
+      for (int c = 0; c < kSegGroups; ++c) bal[c] = 0ull;
+      int mine = 0;
+      if (on) {
+        row_bits(p.mask, N, b, i, j0, p.queue.seg_groups, lane, bal);
+#pragma unroll
+        for (int c = 0; c < kSegGroups; ++c) mine += __popcll(bal[c]);
+      }
+      if (lane == 0) counts[wave] = mine;
+      __syncthreads();
+      int at = pending, total = 0;
+#pragma unroll
+      for (int w = 0; w < kBwdWaves; ++w) {
+        const int n = counts[w];
+        at += w < wave ? n : 0;
+        total += n;
+      }
+      queue.append(at, uint32_t(b) * uint32_t(N) + uint32_t(i), j0, lane, bal);
+      pending += total;
+      __syncthreads();
+      if (pending >= p.queue.batch) {  // whole batches: every wave has the same number of full tiles
+        const int n = pending / p.queue.batch * p.queue.batch;
+        run_tiles(n);
+        queue.drop(n, pending, tid);
+        pending -= n;
+      }
+    }
   }
+  run_tiles(pending);
   // the waves' sums added into LDS in wave order: dW1^T [32][hidden] (f = 16 ft + 4 g + r, h = 16 ht + r16),
   // dW2 [16][hidden] (o = 4 g + r), db2 [16] (over the four lane groups); then the workgroup's slot
   adb2 += __shfl_xor(adb2, 16, 64);
   adb2 += __shfl_xor(adb2, 32, 64);
   for (int w = 0; w < kBwdWaves; ++w) {
     if (wave == w) {
-      for (int ht = 0; ht < HT; ++ht) {
+#pragma unroll
+      for (int ht = 0; ht < kHT; ++ht) {
+        if (ht >= HT) break;  // uniform
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int h = 16 * ht + r16;
@@ -576,8 +727,7 @@ extern "C" int mf_pair_mlp_bias(const mf_pair_mlp_args* a, void* stream) {
   p.R = a->rbf;
   p.hidden = a->hidden;
   p.heads = a->heads;
-  p.groups = (a->atoms + 63) / 64;
-  if ((long long)a->batch * a->atoms * (p.groups + 1) > 0x7fffffffLL)
+  if ((long long)a->batch * a->atoms * ((a->atoms + 63) / 64 + 1) > 0x7fffffffLL)
     return fail(MF_ERR_UNSUPPORTED, "mf_pair_mlp_bias: batch * atoms * ceil(atoms / 64) must stay below 2^31");
   const bool per = a->n_freqs > 0 || a->global_geom != nullptr;
   if (per) {
@@ -657,13 +807,13 @@ extern "C" int mf_pair_mlp_bias_bwd(const mf_pair_mlp_bwd_args* a, void* stream)
   p.R = f.rbf;
   p.hidden = f.hidden;
   p.heads = f.heads;
-  p.groups = (f.atoms + 63) / 64;
+  p.queue = QueueSize{kSegGroups, 16 * kBwdWaves};
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int ks = (3 + f.rbf + 1 + 3) / 4, kp = (f.rbf + 1 + 3) / 4;  // K steps holding the features (and F)
-  // LDS of the instantiation: W1 rows of 4 KMAX + 1 (the kernel's largest stride), b1, W2, transpose tiles
-  auto go = [&](auto kern, int kmax) -> int {
-    const size_t lds = (size_t(f.hidden) * (4 * kmax + 1) + f.hidden + 16 * size_t(f.hidden + 1) +
-                        bwd_slot_floats(f.hidden)) * sizeof(float);
+  const int ks = (3 + f.rbf + 1 + 3) / 4;  // K steps holding the features (and F)
+  // LDS of the instantiation: W1 rows of 4 K + 1, b1, W2, the workgroup's sums
+  auto go = [&](auto kern, int k) -> int {
+    const size_t lds = (size_t(f.hidden) * (4 * k + 1) + f.hidden + 16 * size_t(f.hidden + 1) +
+                        bwd_slot_floats(f.hidden)) * sizeof(float) + p.queue.bytes(kBwdWaves);
     const int st = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), int(lds));
     if (st != MF_OK) return st;
     hipLaunchKernelGGL(kern, dim3(kBwdGroups, 3), dim3(kBwdThreads), lds, s, p);
@@ -673,6 +823,5 @@ extern "C" int mf_pair_mlp_bias_bwd(const mf_pair_mlp_bwd_args* a, void* stream)
     MF_HIP_CHECK(hipGetLastError());
     return MF_OK;
   };
-  if (ks <= 5 && kp <= 5) return go(pair_mlp_bwd_kernel<5, 5>, 5);
-  return go(pair_mlp_bwd_kernel<8, 8>, 8);
+  return ks <= 5 ? go(pair_mlp_bwd_kernel<5>, 5) : go(pair_mlp_bwd_kernel<8>, 8);
 }

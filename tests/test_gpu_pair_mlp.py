@@ -225,3 +225,36 @@ def test_periodic_features_match_torch(cuda, n_freqs, R):
     torch.cuda.synchronize()
     _check(got, want, feats.pair_mask)
     assert not pair_mlp.serves(module, gfe)  # under autograd: the torch formulation (no periodic backward)
+
+
+@pytest.mark.parametrize("B,N,hidden,H,R", [(1, 2, 16, 1, 4), (2, 65, 48, 8, 16), (2, 257, 256, 4, 29),
+                                            (70, 3, 128, 16, 28)])
+def test_queue_edges_match_torch(cuda, B, N, hidden, H, R):
+    """The queues of valid pairs at their edges: almost no pair, rows of one column past a 64-column group, more than
+    one scan of a row with weights that leave the smaller queue, many tiny molecules; forward and, where it is
+    served, the weight gradients; padded atoms passed beside the pair mask come out zero.  Both sides read the same
+    features (the rbf turn an ulp of d_norm into 1e-4 of a term at 28 centres).  Bar 1e-5 of the largest term of
+    the tensor and 5e-7 beside it: the two pairs of a two-atom molecule may hold one small output, the cancelling
+    sum of up to 256 hidden terms of about 0.2, each rounded to 2^-24 on both sides."""
+    print(f"pair mlp queue B={B} N={N} hidden={hidden} H={H} R={R}", flush=True)
+    module, feats, coords, pad, ups = _trained_module(B, N, hidden, H, R, seed=N + hidden)
+    with torch.no_grad():
+        want = module._compute_factorized_terms(feats, pad)
+    train = hidden <= 128
+    grads = _weight_grads(module, feats, ups) if train else None
+    module = module.to(cuda)
+    full = _to(feats, cuda)
+    full.pair_mask = torch.ones_like(full.pair_mask)  # the padding comes from atom_pad_mask alone
+    with torch.no_grad():
+        got = module._compute_factorized_terms(full, pad.to(cuda))
+    torch.cuda.synchronize()
+    for g, w in zip(got, want):
+        g = g.cpu()
+        assert float((g - w).abs().max()) <= 1e-5 * float(w.abs().max()) + 5e-7
+        assert not g.diagonal(dim1=-2, dim2=-1).any()
+        assert not g.permute(0, 2, 3, 1)[~feats.pair_mask].any()
+    if train:
+        for k, (g, r) in enumerate(zip(_weight_grads(module, _to(feats, cuda), [t.to(cuda) for t in ups]), grads)):
+            g, r = g.cpu().double(), r.double()
+            # both sides fp32: the bar of the float64 comparison above, twice
+            assert float((g - r).norm()) <= 4e-5 * float(r.norm()) + 1e-6, k
