@@ -227,20 +227,23 @@ class SimplicialGeometryBias(_GeometryBiasBase):
         return torch.cat([self._distance_rbf(g.pair_dist_norm)] + self._periodic_terms(g, False), dim=-1)
 
     # -- terms (transformer.py:702-750) ------------------------------------------------------------------------
-    def _compute_factorized_terms(self, geom_features: GeometryFeatures):
+    def _compute_factorized_terms(self, geom_features: GeometryFeatures, atom_pad_mask: torch.Tensor | None = None):
+        """u, v, w; with atom_pad_mask the padded atoms' rows and columns are zero (_mask_atom_pairwise_bias)."""
         if self.spoke_bias_u_mlp is None or self.spoke_bias_v_mlp is None or self.pair_bias_w_mlp is None:
             raise RuntimeError("Factorized simplicial geometry requested without factorized geometry MLPs")
         from matterformer_amd import pair_mlp
 
         if pair_mlp.serves(self, geom_features):
-            return pair_mlp.factorized_terms(self, geom_features)
+            # the kernel takes the padded atoms out of its pair mask: no pass over its [B, H, N, N] outputs (and, under
+            # autograd, over their gradients) follows it
+            return pair_mlp.factorized_terms(self, geom_features, atom_pad_mask)
         spoke = self._build_spoke_features(geom_features)
         pair = self._build_pair_features(geom_features)
         terms = [mlp(feat).permute(0, 3, 1, 2).contiguous()
                  for mlp, feat in ((self.spoke_bias_u_mlp, spoke), (self.spoke_bias_v_mlp, spoke),
                                    (self.pair_bias_w_mlp, pair))]
         mask = geom_features.pair_mask[:, None, :, :].to(dtype=terms[0].dtype)
-        return tuple(self._zero_pairwise_diag(t) * mask for t in terms)
+        return tuple(self._mask_atom_pairwise_bias(self._zero_pairwise_diag(t) * mask, atom_pad_mask) for t in terms)
 
     def _low_rank_factors(self, geom_features: GeometryFeatures, left_mlp: nn.Module, right_mlp: nn.Module,
                           rank: int):
@@ -321,16 +324,14 @@ class SimplicialGeometryBias(_GeometryBiasBase):
                                                          device=gate.device, pad_mask=pad_mask,
                                                          geom_pair_mask=geom_features.pair_mask)
 
-        def pair_terms(parts):
-            return [self._expand_atom_head_bias(self._mask_atom_pairwise_bias(t, atom_pad), seq_len=T) for t in parts]
-
         def rank_terms(parts):
             return [self._expand_atom_head_rank_factor(self._mask_atom_pairwise_rank_factor(t, atom_pad), seq_len=T)
                     for t in parts]
 
         factorized = None
         if self.mode != "none":
-            u, v, w = pair_terms(self._compute_factorized_terms(geom_features))
+            u, v, w = (self._expand_atom_head_bias(t, seq_len=T)
+                       for t in self._compute_factorized_terms(geom_features, atom_pad))
             factorized = SimplicialFactorizedBias(u=u, v=v, w=w, gate=gate)
         message = None
         if self.message_mode == "low_rank":

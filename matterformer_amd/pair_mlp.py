@@ -94,12 +94,18 @@ def _forward_args(module, delta, dnorm, mask, centers, gamma, weights, outs, per
         **fields)
 
 
-def _inputs(module, geom_features):
+def _inputs(module, geom_features, atom_pad):
     g = geom_features
     dev = g.pair_delta.device
     delta = g.pair_delta.detach().contiguous()
     dnorm = g.pair_dist_norm.detach().contiguous()
-    mask = g.pair_mask.to(torch.uint8).contiguous()
+    mask = g.pair_mask
+    if mask.dtype != torch.bool:
+        mask = mask.to(torch.uint8) != 0
+    if atom_pad is not None:
+        keep = ~atom_pad
+        mask = mask & (keep[:, :, None] & keep[:, None, :])
+    mask = mask.contiguous().view(torch.uint8)  # a bool's byte is 0 or 1
     centers = module._edge_rbf_centers.to(device=dev, dtype=torch.float32).contiguous()
     return delta, dnorm, mask, centers, float(module._edge_rbf_gamma_value)
 
@@ -155,10 +161,10 @@ class _PairMlpFunction(torch.autograd.Function):
         return (None, None, None, None, None, None, *grads)
 
 
-def factorized_terms(module, geom_features):
-    """(u, v, w) [B, H, N, N] fp32, diagonal and invalid pairs zero; differentiable in the MLP weights when
-    they take gradients."""
-    delta, dnorm, mask, centers, gamma = _inputs(module, geom_features)
+def factorized_terms(module, geom_features, atom_pad=None):
+    """(u, v, w) [B, H, N, N] fp32, diagonal and invalid pairs zero (the rows and columns of the atoms that
+    atom_pad [B, N] bool marks too); differentiable in the MLP weights when they take gradients."""
+    delta, dnorm, mask, centers, gamma = _inputs(module, geom_features, atom_pad)
     weights = _weights(module)
     if _trains(module, geom_features):
         return _PairMlpFunction.apply(module, delta, dnorm, mask, centers, gamma, *weights)
