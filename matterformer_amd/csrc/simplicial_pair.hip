@@ -26,9 +26,10 @@
 // queries of a static share of (b, h) after its first unit.
 //
 // Per unit the workgroup stages the unit's valid key rows (compacted) into
-// LDS as fp16 scaled by powers of two: K1s, K2s row-major, V1s, V2s as
-// [row][r16][dt] (the ND = DP/16 halves of columns r16, 16+r16, ... side by
-// side), and the group's query rows Qs = q log2(e) 2^sq.  The scales
+// LDS as fp16 scaled by powers of two, row-major (K1s, K2s, V1s, V2s), and the
+// group's query rows Qs = q log2(e) 2^sq.  Row r16 of GEMM2's d tile dt is
+// column d = ND r16 + dt (ND = DP/16), so a lane's ND halves of a V row lie
+// side by side in the row as it is.  The scales
 // normalise max|K1|, max|K2|, max|V1|, max|V2| into [1, 2), so every pair
 // product is a normal fp16 number and one v_pk_mul_f16 forms two of them;
 // sq = -(s1 + s2) keeps S in log2 units.  Keys beyond kCap are taken in
@@ -41,7 +42,7 @@
 //   P      = fp16(2^S)                            (B operand of GEMM2 straight from
 //                                                  the accumulators: keys 4g+r of j0
 //                                                  and of j0+1 are K 8g..8g+7)
-//   Z      = V1s[j] (.) V2s[k0 + 4g + r]          (A operand: d = row, pair = K)
+//   Z      = V1s[j] (.) V2s[k0 + 4g + r]          (A operand: d = ND row + dt, pair = K)
 //   GEMM2  O^T[d][i] += Z^T P                     (MFMA, ND QT per iteration)
 //   L[i]  += 1^T P                                (one MFMA per query tile, A = 1
 //                                                  at the valid keys)
@@ -187,7 +188,8 @@ struct Lay {
   static constexpr int kScal = kG + kWaves * 4 * 4;  // int [8] scale exponents, slow flag, no-shift flag
   static constexpr int kM = kScal + 8 * 4;      // float [kMaxQ] two-pass maxima (log2 units)
   static constexpr int kClaim = kM + kMaxQ * 4;  // ClaimState
-  static constexpr int kTotal = kClaim + int(sizeof(ClaimState));
+  static constexpr int kPM = (kClaim + int(sizeof(ClaimState)) + 7) & ~7;  // uint2 [16] half masks of four pairs by their bits
+  static constexpr int kTotal = kPM + 16 * 8;
   // after the pair loop: partial outputs float [kRedWaves][RQ][RS] and
   // denominators float [kRedWaves][RQ], over K1s .. V2s, Qs and the pair bits
   // (none of them is read after the pair loop)
@@ -196,15 +198,19 @@ struct Lay {
   static constexpr int kRedL = kRed + kRedWaves * RQ * RS * 4;
   static_assert(kRedL + kRedWaves * RQ * 4 <= kInfo, "reduction area must fit in the staging area");
   // BIAS instantiations, after the above: fp16 bias operands of the unit's (j block, k block)
-  //   BU [kCap][kMaxQ]     c_i u_ij (row j, query i)
-  //   BW [kCap][kCap]      w_jk
-  //   BV [kMaxQ][kVS]      c_i v_ik at half k + 2 (halves 0, 1 and past the keys read as masked)
-  //   BG float [kMaxQ]     c_i = log2(e) 2^E gate_i; then per-query |u|, |v| maxima and the block |w| maximum
-  static constexpr int kVS = kCap + 16;
-  static constexpr int kBU = (kTotal + 15) & ~15;
-  static constexpr int kBW = kBU + kCap * kMaxQ * 2;
-  static constexpr int kBV = kBW + kCap * kCap * 2;
-  static constexpr int kBG = kBV + kMaxQ * kVS * 2;
+  //   BU dword [kCap / 2][kUS]   (c_i u_ij, c_i u_i,j+1) of the row pair j, j + 1 and query i (kUS odd: the
+  //                              staging writes run along j)
+  //   BW dword [kCap / 2][kCap]  (w_jk, w_j+1,k) of the row pair
+  //   BV half [kMaxQ][kVS]       c_i v_ik (kVS: the 16-byte reads of 16 rows fall on different banks)
+  //   BT dword [64]              the first dword of each lane's constant part of the A operand
+  //   BG float [kMaxQ]           c_i = log2(e) 2^E gate_i; then per-query |u|, |v| maxima and the block |w| maximum
+  static constexpr int kVS = kCap + 8;
+  static constexpr int kUS = kMaxQ + 1;
+  static constexpr int kBV = (kTotal + 15) & ~15;
+  static constexpr int kBW = kBV + kMaxQ * kVS * 2;
+  static constexpr int kBU = kBW + kCap / 2 * kCap * 4;
+  static constexpr int kBT = kBU + kCap / 2 * kUS * 4;
+  static constexpr int kBG = kBT + 64 * 4;
   static constexpr int kBMax = kBG + kMaxQ * 4;  // float [2][kMaxQ] |u|, |v| maxima, then |w|
   static constexpr int kTotalBias = kBMax + (2 * kMaxQ + 1) * 4;
 };
@@ -433,10 +439,16 @@ __device__ __forceinline__ uint32_t pv_mask(uint32_t bits4, int s) {
 // The first QT of the MQ query tiles held in registers are in use.
 //
 // BIAS: GEMM1 gets one more 32-wide K step per (row, query tile) whose
-// operands carry the factorized bias in log2 units (c_i = log2(e) 2^E gate_i):
-//   A[pair p][K]: K = 0 -> 1, K = 1 -> w[j][k0 + p], K = 2 + t -> (p == t), t < 16
-//   B[K][i]     : K = 0 -> c_i u[i][j], K = 1 -> c_i, K = 2 + t -> c_i v[i][k0 + t]
-// so the accumulator gains c_i (u_ij + w_jk + v_ik) for pair (j, k0 + p).
+// operands carry the factorized bias in log2 units (c_i = log2(e) 2^E gate_i),
+// for the row pair j0, j0 + 1 and its row e (0, 1):
+//   A[pair p][K]: K = t -> (p == t), t < 16; K = 16, 17 -> w[j0][k0 + p], w[j0 + 1][k0 + p]; K = 18 + e -> 1
+//   B[K][i]     : K = t -> c_i v[i][k0 + t]; K = 16 + e -> c_i;  K = 18, 19 -> c_i u[i][j0], c_i u[i][j0 + 1]
+// so the accumulator gains c_i (u_ij + w_jk + v_ik) for pair (j, k0 + p).  A
+// lane's four dwords of an operand hold one that changes with the row pair
+// (w in A, u in B, on the g = 2 lanes): every lane loads it, the others from
+// an address that does not move, so the step needs no select and no branch
+// (selects on g made the compiler branch around the loads, three waits an
+// iteration: 64 molecules of 44 atoms, 8 heads, 67.7 -> 62.9 us without).
 template <int DP, int QT, int MODE, bool HAS_PV, bool BIAS, int MQ>
 __device__ __forceinline__ void pair_loop(const unsigned char* smem, int nkj, int nkk,
                                           const uint4 (&qop)[MQ][DP / 32], float (&negm)[MQ], float sc,
@@ -461,30 +473,23 @@ __device__ __forceinline__ void pair_loop(const unsigned char* smem, int nkj, in
   const bool odd = (nkj & 1) != 0;
   constexpr uint32_t kOne2 = 0x3c003c00u;  // fp16 (1, 1)
   const mf_f32x4 zero4 = mf_f32x4{0.f, 0.f, 0.f, 0.f};
-  // BIAS: the constant part of the A operand (lane (g, r16) holds A[p = r16][K = 8g .. 8g + 7]), the
-  // mask of the B halves that carry v (K in [2, 18)), and c_i as fp16 per query tile
-  uint4 onehot{0u, 0u, 0u, 0u}, vmask{0u, 0u, 0u, 0u};
+  // BIAS: the A operands of the two rows (lane (g, r16) holds A[p = r16][K = 8g .. 8g + 7]) and c_i as fp16
+  // per query tile.  The dword that changes with the row pair is loaded twice, once into each row's operand.
+  uint4 ab_a{0u, 0u, 0u, 0u}, ab_b{0u, 0u, 0u, 0u};
   uint32_t cgh[MQ];
-  const unsigned char* BU = smem + Ly::kBU;
-  const unsigned char* BW = smem + Ly::kBW;
-  const unsigned char* BV = smem + Ly::kBV;
+  const int wstep = g == 2 ? kCap * 4 : 0, ustep = g == 2 ? Ly::kUS * 4 : 0;
   if constexpr (BIAS) {
-    uint32_t oh[4], vm[4];
+    uint32_t oh[4];
 #pragma unroll
     for (int h2 = 0; h2 < 4; ++h2) {
-      uint32_t o = 0u, m = 0u;
-#pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        const int K = 8 * g + 2 * h2 + e;
-        const bool one = K == 0 || (K >= 2 && K < 18 && r16 == K - 2);
-        o |= (one ? 0x3c00u : 0u) << (16 * e);
-        m |= (K >= 2 && K < 18 ? 0xffffu : 0u) << (16 * e);
-      }
-      oh[h2] = o;
-      vm[h2] = m;
+      const int K = 8 * g + 2 * h2;
+      oh[h2] = g < 2 ? (r16 == K ? 0x00003c00u : r16 == K + 1 ? 0x3c000000u : 0u) : 0u;
     }
-    onehot = uint4{oh[0], oh[1], oh[2], oh[3]};
-    vmask = uint4{vm[0], vm[1], vm[2], vm[3]};
+    ab_a = ab_b = uint4{oh[0], oh[1], oh[2], oh[3]};
+    if (g == 2) {
+      ab_a.y = 0x00003c00u;
+      ab_b.y = 0x3c000000u;
+    }
     const float* cg = reinterpret_cast<const float*>(smem + Ly::kBG);
 #pragma unroll
     for (int qt = 0; qt < MQ; ++qt)
@@ -524,13 +529,21 @@ __device__ __forceinline__ void pair_loop(const unsigned char* smem, int nkj, in
         v2p[dt][1] = __builtin_amdgcn_perm(rv[3][dt >> 1], rv[2][dt >> 1], sel);
       }
     }
-    uint4 bvop[MQ];
+    uint4 bb_a[MQ], bb_b[MQ];
+    const unsigned char* wsrc = nullptr;
+    const unsigned char* usrc[MQ];
     if constexpr (BIAS) {
-      // halves k0 + 8g .. k0 + 8g + 7 of the query's BV row are K = 8g .. 8g + 7 (v at k + 2)
+      wsrc = smem + (g == 2 ? Ly::kBW + (jp * kCap + k0 + r16) * 4 : Ly::kBT + (16 * g + r16) * 4);
 #pragma unroll
       for (int qt = 0; qt < QT; ++qt) {
-        const uint4 t = *reinterpret_cast<const uint4*>(BV + ((16 * qt + r16) * Ly::kVS + k0 + 8 * g) * 2);
-        bvop[qt] = uint4{t.x & vmask.x, t.y & vmask.y, t.z & vmask.z, t.w & vmask.w};
+        const int vrow = Ly::kBV + ((16 * qt + r16) * Ly::kVS + k0 + 8 * (g & 1)) * 2;
+        uint4 t = *reinterpret_cast<const uint4*>(smem + vrow);
+        if (g >= 2) t = uint4{g == 2 ? cgh[qt] : 0u, 0u, 0u, 0u};
+        bb_a[qt] = bb_b[qt] = t;
+        if (g == 2) bb_b[qt].x = cgh[qt] << 16;
+        usrc[qt] = smem + (g == 2   ? Ly::kBU + (jp * Ly::kUS + 16 * qt + r16) * 4
+                           : g == 3 ? Ly::kBT + (48 + r16) * 4
+                                    : vrow + 4);
       }
     }
     const int kvalid = nkk - (k0 + 4 * g);  // keys 4g + r valid for r < kvalid
@@ -567,9 +580,18 @@ __device__ __forceinline__ void pair_loop(const unsigned char* smem, int nkj, in
       }
       // valid keys 4g + r of rows j0 (bits_a) and j0 + 1 (bits_b)
       uint32_t bits_a = kmask, bits_b = last_odd ? 0u : kmask;
+      // HAS_PV: their half masks, looked up by the four bits (the staged bits are 0 past the valid keys and
+      // rows; forming the masks took 12 VALU a row)
+      uint2 pm_a{0u, 0u}, pm_b{0u, 0u};
       if constexpr (HAS_PV) {
-        bits_a &= pvb[j0 * Ly::kPVW + pvword] >> pvshift;
-        bits_b &= pvb[(j0 + 1) * Ly::kPVW + pvword] >> pvshift;
+        const uint32_t pv_a = pvb[j0 * Ly::kPVW + pvword], pv_b = pvb[(j0 + 1) * Ly::kPVW + pvword];
+        bits_a &= pv_a >> pvshift;
+        bits_b &= pv_b >> pvshift;
+        if constexpr (MODE != kMax) {
+          const uint2* pm = reinterpret_cast<const uint2*>(smem + Ly::kPM);
+          pm_a = pm[(pv_a >> pvshift) & 15u];
+          pm_b = pm[(pv_b >> pvshift) & 15u];
+        }
       }
       // GEMM1 for rows j0 and j0 + 1
       uint4 wa[NCH], wb[NCH];
@@ -590,20 +612,17 @@ __device__ __forceinline__ void pair_loop(const unsigned char* smem, int nkj, in
         }
       }
       if constexpr (BIAS) {
-        // rows j0, j0 + 1: w of the lane's pair into A (K = 1), c_i u_ij into B (K = 0), both on the g = 0
-        // lanes (the padding row j0 + 1 = nkj reads zeros)
-        const uint32_t w_a = *reinterpret_cast<const uint16_t*>(BW + (j0 * kCap + k0 + r16) * 2);
-        const uint32_t w_b = *reinterpret_cast<const uint16_t*>(BW + ((j0 + 1) * kCap + k0 + r16) * 2);
-        const uint4 ab_a{g == 0 ? (0x3c00u | (w_a << 16)) : onehot.x, onehot.y, onehot.z, onehot.w};
-        const uint4 ab_b{g == 0 ? (0x3c00u | (w_b << 16)) : onehot.x, onehot.y, onehot.z, onehot.w};
+        // (the padding row j0 + 1 = nkj reads zeros)
+        ab_a.x = *reinterpret_cast<const uint32_t*>(wsrc);
+        ab_b.x = *reinterpret_cast<const uint32_t*>(wsrc);
+        wsrc += wstep;
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt) {
-          const uint32_t u_a = *reinterpret_cast<const uint16_t*>(BU + (j0 * Ly::kMaxQ + 16 * qt + r16) * 2);
-          const uint32_t u_b = *reinterpret_cast<const uint16_t*>(BU + ((j0 + 1) * Ly::kMaxQ + 16 * qt + r16) * 2);
-          const uint4 bb_a{g == 0 ? (u_a | (cgh[qt] << 16)) : bvop[qt].x, bvop[qt].y, bvop[qt].z, bvop[qt].w};
-          const uint4 bb_b{g == 0 ? (u_b | (cgh[qt] << 16)) : bvop[qt].x, bvop[qt].y, bvop[qt].z, bvop[qt].w};
-          sa[qt] = mfma(ab_a, bb_a, sa[qt]);
-          sb[qt] = mfma(ab_b, bb_b, sb[qt]);
+          bb_a[qt].y = *reinterpret_cast<const uint32_t*>(usrc[qt]);
+          bb_b[qt].y = *reinterpret_cast<const uint32_t*>(usrc[qt]);
+          usrc[qt] += ustep;
+          sa[qt] = mfma(ab_a, bb_a[qt], sa[qt]);
+          sb[qt] = mfma(ab_b, bb_b[qt], sb[qt]);
         }
       }
       if constexpr (MODE == kMax) {
@@ -676,7 +695,9 @@ __device__ __forceinline__ void pair_loop(const unsigned char* smem, int nkj, in
           pop[qt] = uint4{pack_h2(ea[0], ea[1]), pack_h2(ea[2], ea[3]), pack_h2(eb[0], eb[1]), pack_h2(eb[2], eb[3])};
           // two-pass mode: padded pairs have S = 0, so 2^(0 - m) may exceed
           // the fp16 range; they and the pairs pair_valid clears get P = 0
-          if constexpr (HAS_PV || MODE == kSlow || MODE == kOnline) {
+          if constexpr (HAS_PV) {
+            pop[qt] = uint4{pop[qt].x & pm_a.x, pop[qt].y & pm_a.y, pop[qt].z & pm_b.x, pop[qt].w & pm_b.y};
+          } else if constexpr (MODE == kSlow || MODE == kOnline) {
             pop[qt].x &= pv_mask(bits_a, 0);
             pop[qt].y &= pv_mask(bits_a, 1);
             pop[qt].z &= pv_mask(bits_b, 0);
@@ -900,7 +921,7 @@ __device__ __forceinline__ void unit_body(const Params& p, unsigned char* smem, 
   // ---- factorized bias (BIAS): c_i, then the fp16 operands of a block ------
   float* cgf = reinterpret_cast<float*>(smem + Ly::kBG);
   float* bmax = reinterpret_cast<float*>(smem + Ly::kBMax);  // max |u|, |v|, |w| of the unit's staged values
-  // (j block, k block): BU[j][i] = c_i u_ij, BW[j][k] = w_jk, BV[i][k + 2] = c_i v_ik over the staged rows,
+  // (j block, k block): BU[j][i] = c_i u_ij, BW[j][k] = w_jk, BV[i][k] = c_i v_ik over the staged rows,
   // zero past the valid keys and queries
   auto stage_bias = [&](int jc, int kc, int cE) {
     uint16_t* BU = reinterpret_cast<uint16_t*>(smem + Ly::kBU);
@@ -915,8 +936,8 @@ __device__ __forceinline__ void unit_body(const Params& p, unsigned char* smem, 
     // columns (lane, lane + 64), so a wave's loads of a row are one coalesced run; kRB rows of a
     // wave are loaded before any is converted and stored.  Rows and columns past the valid
     // queries / keys are stored as zero.
-    //   set 0 (U): rows = queries qi < kMaxQ, columns j < rj:  BU[j][qi]     = c_qi u[qa][ka(j0 + j)]
-    //   set 1 (V): rows = queries qi,          columns k < rk:  BV[qi][k + 2] = c_qi v[qa][ka(k0 + k)]
+    //   set 0 (U): rows = queries qi < kMaxQ, columns j < rj:  BU[j][qi] = c_qi u[qa][ka(j0 + j)]
+    //   set 1 (V): rows = queries qi,          columns k < rk:  BV[qi][k] = c_qi v[qa][ka(k0 + k)]
     //   set 2 (W): rows j < rj,                columns k < rk:  BW[j][k]      = w[ka(j0 + j)][ka(k0 + k)]
     // Batches of kRB rows per wave: the U and V rows of a batch, its gates and, in the first batch, the
     // first W rows are loaded before anything is stored (GQ / (kWaves kRB) round trips for U and V);
@@ -989,9 +1010,9 @@ __device__ __forceinline__ void unit_body(const Params& p, unsigned char* smem, 
                           : dt == MF_DTYPE_BF16        ? __uint_as_float(raw << 16)
                                                        : float(__builtin_bit_cast(_Float16, uint16_t(raw)));
           mx[SET] = fmaxf(mx[SET], fabsf(x));
-          if constexpr (SET == 0) BU[c * kMaxQ + r] = half_bits_sat(crow[t] * x);
-          else if constexpr (SET == 1) BV[r * Ly::kVS + c + 2] = half_bits_sat(crow[t] * x);
-          else BW[r * kCap + c] = half_bits_sat(x);
+          if constexpr (SET == 0) BU[((c >> 1) * Ly::kUS + r) * 2 + (c & 1)] = half_bits_sat(crow[t] * x);
+          else if constexpr (SET == 1) BV[r * Ly::kVS + c] = half_bits_sat(crow[t] * x);
+          else BW[((r >> 1) * kCap + c) * 2 + (r & 1)] = half_bits_sat(x);
         }
       }
     };
@@ -1052,23 +1073,14 @@ __device__ __forceinline__ void unit_body(const Params& p, unsigned char* smem, 
     }
   };
   ClaimState* cl = reinterpret_cast<ClaimState*>(smem + Ly::kClaim);
-  // K rows: row-major fp16 scaled by 2^sc_exp
-  auto store_k = [&](unsigned char* dst, const uint4& v, int row, int sc_exp) {
+  // K and V rows: row-major fp16 scaled by 2^sc_exp
+  auto store_row = [&](unsigned char* dst, const uint4& v, int row, int sc_exp) {
     float f[8];
     uint32_t w[4];
     unpack8<T>(v, f);
 #pragma unroll
     for (int e = 0; e < 4; ++e) w[e] = pack_h2(ldexpf(f[2 * e], sc_exp), ldexpf(f[2 * e + 1], sc_exp));
     *reinterpret_cast<uint4*>(dst + row * RB + e0 * 2) = uint4{w[0], w[1], w[2], w[3]};
-  };
-  // V rows: [row][r16][dt]: column d = 16 dt + r16 at half r16 ND + dt
-  auto store_v = [&](unsigned char* dst, const uint4& v, int row, int sc_exp) {
-    float f[8];
-    unpack8<T>(v, f);
-    unsigned char* a = dst + row * RB + ((8 * (cc & 1)) * ND + (cc >> 1)) * 2;
-#pragma unroll
-    for (int e = 0; e < 8; ++e)
-      *reinterpret_cast<_Float16*>(a + e * ND * 2) = _Float16(ldexpf(f[e], sc_exp));
   };
   // bits of pair_valid for rows j of the j block and keys k of the k block
   auto stage_pv = [&](int jc, int kc) {
@@ -1120,10 +1132,10 @@ __device__ __forceinline__ void unit_body(const Params& p, unsigned char* smem, 
         if (i >= nI) break;
         const int row = (tid + kThreads * i) / CPR;
         if (row < rj) {
-          store_k(smem + Ly::kK1, rk1[i], row, 0);
-          store_v(smem + Ly::kV1, rv1[i], row, 0);
-          store_k(smem + Ly::kK2, rk2[i], row, 0);
-          store_v(smem + Ly::kV2, rv2[i], row, 0);
+          store_row(smem + Ly::kK1, rk1[i], row, 0);
+          store_row(smem + Ly::kV1, rv1[i], row, 0);
+          store_row(smem + Ly::kK2, rk2[i], row, 0);
+          store_row(smem + Ly::kV2, rv2[i], row, 0);
         }
       }
       unsigned char* Qs = smem + Ly::kQ;
@@ -1342,12 +1354,12 @@ __device__ __forceinline__ void unit_body(const Params& p, unsigned char* smem, 
         if (i >= nI) break;
         const int row = (tid + kThreads * i) / CPR;
         if (row < rj) {
-          store_k(K1s, rk1[i], row, s1);
-          store_v(V1s, rv1[i], row, t1);
+          store_row(K1s, rk1[i], row, s1);
+          store_row(V1s, rv1[i], row, t1);
         }
         if (row < rk) {
-          store_k(K2s, rk2[i], row, s2);
-          store_v(V2s, rv2[i], row, t2);
+          store_row(K2s, rk2[i], row, s2);
+          store_row(V2s, rv2[i], row, t2);
         }
       }
     } else {
@@ -1361,19 +1373,19 @@ __device__ __forceinline__ void unit_body(const Params& p, unsigned char* smem, 
       load_set(gk1, aj, nkj, t);
 #pragma unroll
       for (int i = 0; i < MAXC; ++i)
-        if ((tid + kThreads * i) / CPR < rj) store_k(K1s, t[i], (tid + kThreads * i) / CPR, s1);
+        if ((tid + kThreads * i) / CPR < rj) store_row(K1s, t[i], (tid + kThreads * i) / CPR, s1);
       load_set(gv1, aj, nkj, t);
 #pragma unroll
       for (int i = 0; i < MAXC; ++i)
-        if ((tid + kThreads * i) / CPR < rj) store_v(V1s, t[i], (tid + kThreads * i) / CPR, t1);
+        if ((tid + kThreads * i) / CPR < rj) store_row(V1s, t[i], (tid + kThreads * i) / CPR, t1);
       load_set(gk2, ak, nkk, t);
 #pragma unroll
       for (int i = 0; i < MAXC; ++i)
-        if ((tid + kThreads * i) / CPR < rk) store_k(K2s, t[i], (tid + kThreads * i) / CPR, s2);
+        if ((tid + kThreads * i) / CPR < rk) store_row(K2s, t[i], (tid + kThreads * i) / CPR, s2);
       load_set(gv2, ak, nkk, t);
 #pragma unroll
       for (int i = 0; i < MAXC; ++i)
-        if ((tid + kThreads * i) / CPR < rk) store_v(V2s, t[i], (tid + kThreads * i) / CPR, t2);
+        if ((tid + kThreads * i) / CPR < rk) store_row(V2s, t[i], (tid + kThreads * i) / CPR, t2);
     }
     if constexpr (BIAS && MULTI) stage_bias(jc, kc, E);
     if constexpr (HAS_PV && (MULTI || BIAS)) stage_pv(jc, kc);
@@ -1553,39 +1565,21 @@ __device__ __forceinline__ void unit_body(const Params& p, unsigned char* smem, 
   __syncthreads();  // every wave is done with K/V (the reduction area aliases them)
   float* red = reinterpret_cast<float*>(smem + Ly::kRed);
   float* redl = reinterpret_cast<float*>(smem + Ly::kRedL);
-  // kRedWaves slots: with 8 waves, wave w + 4 hands its partials to wave w first
-  const int slot = wave & (kRedWaves - 1);
   auto put_partials = [&]() {
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
       if (qt >= nqt) continue;
 #pragma unroll
-      for (int dt = 0; dt < ND; ++dt)
-        *reinterpret_cast<mf_f32x4*>(red + (slot * Ly::RQ + 16 * qt + r16) * Ly::RS + 16 * dt + 4 * g) = O[dt][qt];
-      if (g == 0) redl[slot * Ly::RQ + 16 * qt + r16] = L[qt][0];
+      for (int r = 0; r < 4; ++r) {  // row 4 g + r of the d tiles: columns ND (4 g + r) + dt
+        float* dst = red + (wave * Ly::RQ + 16 * qt + r16) * Ly::RS + ND * (4 * g + r);
+        if constexpr (ND == 4) *reinterpret_cast<float4*>(dst) = float4{O[0][qt][r], O[1][qt][r], O[2][qt][r], O[3][qt][r]};
+        else *reinterpret_cast<float2*>(dst) = float2{O[0][qt][r], O[1][qt][r]};
+      }
+      if (g == 0) redl[wave * Ly::RQ + 16 * qt + r16] = L[qt][0];
     }
   };
-  if constexpr (kWaves > kRedWaves) {
-    static_assert(kWaves == 2 * kRedWaves, "two waves per reduction slot");
-    if (wave >= kRedWaves) put_partials();
-    __syncthreads();
-    if (wave < kRedWaves) {
-#pragma unroll
-      for (int qt = 0; qt < QT; ++qt) {
-        if (qt >= nqt) continue;
-#pragma unroll
-        for (int dt = 0; dt < ND; ++dt) {
-          const mf_f32x4 o2 =
-              *reinterpret_cast<const mf_f32x4*>(red + (slot * Ly::RQ + 16 * qt + r16) * Ly::RS + 16 * dt + 4 * g);
-          O[dt][qt] += o2;
-        }
-        // every lane of a query column holds the same denominator in L[qt][0..3]
-        L[qt][0] += redl[slot * Ly::RQ + 16 * qt + r16];
-      }
-    }
-    __syncthreads();
-  }
-  if (wave < kRedWaves) put_partials();
+  static_assert(kWaves == kRedWaves, "a reduction slot per wave");
+  put_partials();
   __syncthreads();
   constexpr int CPQ = DP / 8;  // 8-column chunks per query
   const float oscale = ldexpf(1.0f, -(t1 + t2));
@@ -1870,6 +1864,15 @@ __global__ void __launch_bounds__(Waves<BIAS>::kCount * 64, 2) simplicial_pair_k
   const int wg = blockIdx.x;
 
   if (tid == 0) cl->claimed = 0;
+  if (tid < 16)
+    reinterpret_cast<uint2*>(smem + Ly::kPM)[tid] = uint2{pv_mask(uint32_t(tid), 0), pv_mask(uint32_t(tid), 1)};
+  if constexpr (BIAS) {
+    // K = 8 g, 8 g + 1 of row r16 of the bias step's A operand (the g = 2 lanes load w instead)
+    if (tid < 64) {
+      const int K = 8 * (tid >> 4), r = tid & 15;
+      reinterpret_cast<uint32_t*>(smem + Ly::kBT)[tid] = r == K ? 0x00003c00u : r == K + 1 ? 0x3c000000u : 0u;
+    }
+  }
   scan_masks<DP, BIAS>(p, smem, s_info);  // ends with a barrier
   rank_molecules<W, Waves<BIAS>::kGroup, Waves<BIAS>::kCap>(p, s_info, s_order, s_pre, reinterpret_cast<uint2*>(smem), wg, &s_first);
   const int total = s_pre[B];
