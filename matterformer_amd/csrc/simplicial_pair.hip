@@ -766,22 +766,14 @@ __device__ __forceinline__ void zero_padded_share(const Params& p, const uint32_
   }
 }
 
-// An element of a bias tensor as float.
-__device__ __forceinline__ float bias_at(const void* t, size_t idx, int dtype) {
-  if (dtype == MF_DTYPE_F32) return static_cast<const float*>(t)[idx];
-  if (dtype == MF_DTYPE_BF16) return float(static_cast<const __bf16*>(t)[idx]);
-  return float(static_cast<const _Float16*>(t)[idx]);
-}
-// fp16 bits of x, saturated to the finite range
-__device__ __forceinline__ uint16_t half_bits_sat(float x) {
-  return __builtin_bit_cast(uint16_t, _Float16(fminf(fmaxf(x, -65504.0f), 65504.0f)));
-}
+// x in the finite range of fp16
+__device__ __forceinline__ float sat_half(float x) { return __builtin_amdgcn_fmed3f(x, -65504.0f, 65504.0f); }
 
 template <typename T, int DP, bool HAS_PV, bool MULTI, bool BIAS, bool STR>
 __device__ __forceinline__ void unit_body(const Params& p, unsigned char* smem, int b, int h, int nk, int q0, int nqg,
                                           bool kpre, bool qpre, bool zero_share) {
   constexpr int GQ = Waves<BIAS>::kGroup;
-  constexpr int QT = GQ / 16;          // query tiles held in registers
+  constexpr int QT = MULTI ? 1 : GQ / 16;  // query tiles held in registers (units of more than kCap keys have one)
   const int nqt = (nqg + 15) >> 4;     // query tiles in use
   constexpr int kWaves = Waves<BIAS>::kCount;
   constexpr int kThreads = kWaves * 64;
@@ -921,150 +913,144 @@ __device__ __forceinline__ void unit_body(const Params& p, unsigned char* smem, 
   // ---- factorized bias (BIAS): c_i, then the fp16 operands of a block ------
   float* cgf = reinterpret_cast<float*>(smem + Ly::kBG);
   float* bmax = reinterpret_cast<float*>(smem + Ly::kBMax);  // max |u|, |v|, |w| of the unit's staged values
-  // (j block, k block): BU[j][i] = c_i u_ij, BW[j][k] = w_jk, BV[i][k] = c_i v_ik over the staged rows,
-  // zero past the valid keys and queries
-  auto stage_bias = [&](int jc, int kc, int cE) {
+  // (j block, k block): BU[j][i] = c_i u_ij, BW[j][k] = w_jk, BV[i][k] = c_i v_ik over the staged keys, zero past
+  // the valid ones (rows of queries past the group are not written: a query's column of S depends on its own
+  // operands alone).  bias_load issues every load of the block, bias_store converts and stores.
+  //
+  // A wave takes whole rows (query rows wv + 4 t of u and v, row pairs wv + 4 t of w) with its lanes along the
+  // first 64 columns: rows and their addresses are wave-uniform (scalar base, one vector offset per column), a
+  // row is one coalesced run, and all rows are in flight together.  Columns 64 .. 79 (larger blocks only) go 16
+  // to a row over all threads.  With per-lane row addresses and batches of four rows, each a round trip, this
+  // stage took a third of a unit (256 molecules of 44 atoms, 8 heads, fp32 bias: 281 -> 247 us; 64 molecules of
+  // bf16 bias 62.9 -> 61.3 us, and 97.8 -> 82.0 us from cold caches).
+  constexpr int kQR = GQ / kWaves;               // u, v rows per wave
+  constexpr int kWP = kCap / 2 / kWaves;         // w row pairs per wave
+  constexpr int kTQ = GQ * 16 / kThreads;        // tail elements per thread: u, v
+  constexpr int kTW = (kCap / 2 * 16 + kThreads - 1) / kThreads;  // ... and w pairs
+  const int wv = __builtin_amdgcn_readfirstlane(wave);
+  struct BiasRegs {
+    uint32_t gate, u[kQR], v[kQR], w[kWP][2];
+    uint32_t tg[kTQ], tu[kTQ], tv[kTQ], tw[kTW][2];
+  };
+  auto query_atom = [&](int r) { return qpre ? q0 + r : int(qidx[q0 + r]); };
+  auto bias_load = [&](int jc, int kc, BiasRegs& R) {
+    const int j0 = jc * kCap, k0 = kc * kCap;
+    const int nkj = min(kCap, nk - j0), nkk = min(kCap, nk - k0);
+    if (nkj <= 0 || nkk <= 0) return;  // nothing to read: bias_store takes no value
+    const int qa = query_atom(min(wv + kWaves * lane, nqg - 1));  // lane t: the wave's query row t
+    const int wa = key_atom(j0 + min(2 * (wv + kWaves * (lane >> 1)) + (lane & 1), nkj - 1));  // lane 2 t + e: row e of pair t
+    const int cj = key_atom(j0 + min(lane, nkj - 1)), ck = key_atom(k0 + min(lane, nkk - 1));
+    auto batch = [&](auto elem) {
+      using E = decltype(elem);
+      const size_t plane = size_t(bh) * N * N;
+      const E* bu = static_cast<const E*>(p.bu) + plane;
+      const E* bv = static_cast<const E*>(p.bv) + plane;
+      const E* bw = static_cast<const E*>(p.bw) + plane;
+      const E* bg = static_cast<const E*>(p.bg) + size_t(bh) * N;
+      auto at = [&](const E* base, int row, int col) { return uint32_t((base + uint32_t(row * N))[uint32_t(col)]); };
+      R.gate = bg[uint32_t(qa)];
+#pragma unroll
+      for (int t = 0; t < kQR; ++t) {
+        const int ra = __builtin_amdgcn_readlane(qa, t);
+        R.u[t] = at(bu, ra, cj);
+        R.v[t] = at(bv, ra, ck);
+      }
+      auto w_rows = [&](auto t0, auto t1) {
+#pragma unroll
+        for (int t = decltype(t0)::value; t < decltype(t1)::value; ++t) {
+          R.w[t][0] = at(bw, __builtin_amdgcn_readlane(wa, 2 * t), ck);
+          R.w[t][1] = at(bw, __builtin_amdgcn_readlane(wa, 2 * t + 1), ck);
+        }
+      };
+      static_assert(!BIAS || kWP == 10, "row groups of 32, 32 and 16 keys");
+      if constexpr (BIAS) {
+        w_rows(std::integral_constant<int, 0>{}, std::integral_constant<int, 4>{});
+        if (nkj > 32) w_rows(std::integral_constant<int, 4>{}, std::integral_constant<int, 8>{});
+        if (nkj > 64) w_rows(std::integral_constant<int, 8>{}, std::integral_constant<int, 10>{});
+      }
+      if (nkj > 64 || nkk > 64) {
+        const int tj = key_atom(j0 + min(64 + r16, nkj - 1)), tk = key_atom(k0 + min(64 + r16, nkk - 1));
+#pragma unroll
+        for (int i = 0; i < kTQ; ++i) {
+          const int ra = query_atom(min((tid + kThreads * i) >> 4, nqg - 1));
+          R.tg[i] = bg[uint32_t(ra)];
+          R.tu[i] = at(bu, ra, tj);
+          R.tv[i] = at(bv, ra, tk);
+        }
+#pragma unroll
+        for (int i = 0; i < kTW; ++i) {
+          const int pr = 2 * ((tid + kThreads * i) >> 4);
+#pragma unroll
+          for (int e = 0; e < 2; ++e) R.tw[i][e] = at(bw, key_atom(j0 + min(pr + e, nkj - 1)), tk);
+        }
+      }
+    };
+    if (p.bias_dtype == MF_DTYPE_F32) batch(uint32_t{});
+    else batch(uint16_t{});
+  };
+  auto bias_store = [&](int jc, int kc, int cE, BiasRegs& R) {
     uint16_t* BU = reinterpret_cast<uint16_t*>(smem + Ly::kBU);
-    uint16_t* BW = reinterpret_cast<uint16_t*>(smem + Ly::kBW);
+    uint32_t* BW = reinterpret_cast<uint32_t*>(smem + Ly::kBW);
     uint16_t* BV = reinterpret_cast<uint16_t*>(smem + Ly::kBV);
     const int j0 = jc * kCap, k0 = kc * kCap;
     const int nkj = min(kCap, nk - j0), nkk = min(kCap, nk - k0);
     const int rj = round16(nkj), rk = round16(nkk);
-    const int dt = p.bias_dtype;
+    const bool any = nkj > 0 && nkk > 0;
     float mx[3] = {0.0f, 0.0f, 0.0f};  // max |u|, |v|, |w| of the staged values
-    // Each set is taken a row per wave (rows wave, wave + kWaves, ...) with the lanes along the
-    // columns (lane, lane + 64), so a wave's loads of a row are one coalesced run; kRB rows of a
-    // wave are loaded before any is converted and stored.  Rows and columns past the valid
-    // queries / keys are stored as zero.
-    //   set 0 (U): rows = queries qi < kMaxQ, columns j < rj:  BU[j][qi] = c_qi u[qa][ka(j0 + j)]
-    //   set 1 (V): rows = queries qi,          columns k < rk:  BV[qi][k] = c_qi v[qa][ka(k0 + k)]
-    //   set 2 (W): rows j < rj,                columns k < rk:  BW[j][k]      = w[ka(j0 + j)][ka(k0 + k)]
-    // Batches of kRB rows per wave: the U and V rows of a batch, its gates and, in the first batch, the
-    // first W rows are loaded before anything is stored (GQ / (kWaves kRB) round trips for U and V);
-    // c_i = log2(e) 2^cE gate_i is formed in registers (and stored to BG).
-    constexpr int kRB = 4;
-    static_assert(GQ % (kWaves * kRB) == 0, "whole batches of query rows");
-    auto set_shape = [&](auto set_tag, int& R, int& C, int& rvalid, int& cvalid, int& cbase, const void*& src) {
-      constexpr int SET = decltype(set_tag)::value;
-      R = SET == 2 ? rj : GQ;
-      C = SET == 0 ? rj : rk;
-      rvalid = SET == 2 ? nkj : nqg;
-      cvalid = SET == 0 ? nkj : nkk;
-      cbase = SET == 0 ? j0 : k0;
-      src = SET == 0 ? p.bu : (SET == 1 ? p.bv : p.bw);
-    };
-    // Loads without branches: a lane's two column atoms are found once, each row's atom once
-    // (wave-uniform), out-of-range rows and columns read a clamped valid element (zeroed when
-    // stored, so no use follows a load and a wave's loads of a batch are in flight together),
-    // and the element width is one uniform choice for the whole batch.
-    auto load_rows = [&](auto set_tag, int r0, uint32_t (&val)[kRB][2]) {
-      constexpr int SET = decltype(set_tag)::value;
-      int R, C, rvalid, cvalid, cbase;
-      const void* src;
-      set_shape(set_tag, R, C, rvalid, cvalid, cbase, src);
-#pragma unroll
-      for (int t = 0; t < kRB; ++t) val[t][0] = val[t][1] = 0u;
-      if (rvalid <= 0 || cvalid <= 0) return;
-      const bool two = kCap > 64 && C > 64;  // a second column per lane (wave-uniform)
-      int ca[2];
-#pragma unroll
-      for (int s = 0; s < 2; ++s) ca[s] = key_atom(cbase + min(lane + 64 * s, cvalid - 1));
-      int ra[kRB];  // row atoms, all found before any load is issued
-#pragma unroll
-      for (int t = 0; t < kRB; ++t) {
-        const int rc = min(r0 + kWaves * t, rvalid - 1);
-        ra[t] = SET == 2 ? key_atom(j0 + rc) : (qpre ? q0 + rc : int(qidx[q0 + rc]));
-      }
-      auto batch = [&](auto wide_tag) {
-        constexpr bool WIDE = decltype(wide_tag)::value;
-#pragma unroll
-        for (int t = 0; t < kRB; ++t) {
-          const size_t rowbase = (size_t(bh) * N + ra[t]) * N;
-#pragma unroll
-          for (int s = 0; s < 2; ++s) {
-            if (s == 1 && !two) continue;  // wave-uniform
-            if constexpr (WIDE) val[t][s] = static_cast<const uint32_t*>(src)[rowbase + ca[s]];
-            else val[t][s] = static_cast<const uint16_t*>(src)[rowbase + ca[s]];
-          }
-        }
+    auto run = [&](auto conv) {  // conv: an element's bits as float
+      const float crow = wv + kWaves * lane < nqg && any ? ldexpf(conv(R.gate) * kLog2e, cE) : 0.0f;
+      if (lane < kQR) cgf[wv + kWaves * lane] = crow;
+      if (!any) return;
+      auto c_of = [&](int t) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(crow), t)); };
+      // (the fp16 conversions saturate to the finite range)
+      auto w_pair = [&](uint32_t lo, uint32_t hi, int pr, int c, bool ok) {
+        const float x0 = ok ? conv(lo) : 0.0f, x1 = ok && pr + 1 < nkj ? conv(hi) : 0.0f;
+        mx[2] = fmaxf(mx[2], fmaxf(fabsf(x0), fabsf(x1)));
+        BW[(pr >> 1) * kCap + c] = pack_h2(sat_half(x0), sat_half(x1));
       };
-      if (dt == MF_DTYPE_F32) batch(std::true_type{});
-      else batch(std::false_type{});
-    };
-    auto store_rows = [&](auto set_tag, int r0, const uint32_t (&val)[kRB][2], const float (&crow)[kRB]) {
-      constexpr int SET = decltype(set_tag)::value;
-      int R, C, rvalid, cvalid, cbase;
-      const void* src;
-      set_shape(set_tag, R, C, rvalid, cvalid, cbase, src);
+      auto u_elem = [&](uint32_t bits, float cr, int r, int c, bool ok) {
+        const float x = ok ? conv(bits) : 0.0f;
+        mx[0] = fmaxf(mx[0], fabsf(x));
+        BU[((c >> 1) * Ly::kUS + r) * 2 + (c & 1)] = __builtin_bit_cast(uint16_t, _Float16(sat_half(cr * x)));
+      };
+      auto v_elem = [&](uint32_t bits, float cr, int r, int c, bool ok) {
+        const float x = ok ? conv(bits) : 0.0f;
+        mx[1] = fmaxf(mx[1], fabsf(x));
+        BV[r * Ly::kVS + c] = __builtin_bit_cast(uint16_t, _Float16(sat_half(cr * x)));
+      };
+      const bool okj = lane < nkj, okk = lane < nkk;
+      if (lane < rj) {
 #pragma unroll
-      for (int t = 0; t < kRB; ++t) {
-        const int r = r0 + kWaves * t;
-        if (r >= R) break;  // wave-uniform
+        for (int t = 0; t < kQR; ++t)
+          if (wv + kWaves * t < nqg) u_elem(R.u[t], c_of(t), wv + kWaves * t, lane, okj);
+      }
+      if (lane < rk) {
 #pragma unroll
-        for (int s = 0; s < (kCap > 64 ? 2 : 1); ++s) {
-          const int c = lane + 64 * s;
-          if (c >= C) continue;
-          const uint32_t raw = val[t][s];
-          const float x = !(r < rvalid && c < cvalid) ? 0.0f
-                          : dt == MF_DTYPE_F32         ? __uint_as_float(raw)
-                          : dt == MF_DTYPE_BF16        ? __uint_as_float(raw << 16)
-                                                       : float(__builtin_bit_cast(_Float16, uint16_t(raw)));
-          mx[SET] = fmaxf(mx[SET], fabsf(x));
-          if constexpr (SET == 0) BU[((c >> 1) * Ly::kUS + r) * 2 + (c & 1)] = half_bits_sat(crow[t] * x);
-          else if constexpr (SET == 1) BV[r * Ly::kVS + c] = half_bits_sat(crow[t] * x);
-          else BW[((r >> 1) * kCap + c) * 2 + (r & 1)] = half_bits_sat(x);
+        for (int t = 0; t < kQR; ++t)
+          if (wv + kWaves * t < nqg) v_elem(R.v[t], c_of(t), wv + kWaves * t, lane, okk);
+#pragma unroll
+        for (int t = 0; t < kWP; ++t)
+          if (2 * (wv + kWaves * t) < nkj) w_pair(R.w[t][0], R.w[t][1], 2 * (wv + kWaves * t), lane, okk);
+      }
+      if (nkj > 64 || nkk > 64) {
+        const int c = 64 + r16;
+#pragma unroll
+        for (int i = 0; i < kTQ; ++i) {
+          const int r = (tid + kThreads * i) >> 4;
+          const float cr = ldexpf(conv(R.tg[i]) * kLog2e, cE);
+          if (r < nqg && c < rj) u_elem(R.tu[i], cr, r, c, c < nkj);
+          if (r < nqg && c < rk) v_elem(R.tv[i], cr, r, c, c < nkk);
+        }
+#pragma unroll
+        for (int i = 0; i < kTW; ++i) {
+          const int pr = 2 * ((tid + kThreads * i) >> 4);
+          if (pr < nkj && c < rk) w_pair(R.tw[i][0], R.tw[i][1], pr, c, c < nkk);
         }
       }
     };
-    using S0 = std::integral_constant<int, 0>;
-    using S1 = std::integral_constant<int, 1>;
-    using S2 = std::integral_constant<int, 2>;
-    const float kNoRow[kRB] = {};
-#pragma unroll 1
-    for (int qb = 0; qb < GQ / (kWaves * kRB); ++qb) {
-      const int r0 = wave + kWaves * kRB * qb;
-      uint32_t vu[kRB][2], vv[kRB][2], vw[kRB][2];
-      float crow[kRB];
-      load_rows(S0{}, r0, vu);
-      load_rows(S1{}, r0, vv);
-      if (qb == 0) load_rows(S2{}, r0, vw);
-      // the gates of query rows wave + kWaves t: all loaded (one uniform width) before any is used
-      uint32_t graw[kRB];
-      int gidx[kRB];
-#pragma unroll
-      for (int t = 0; t < kRB; ++t) {
-        const int rc = min(r0 + kWaves * t, max(nqg - 1, 0));
-        gidx[t] = qpre ? q0 + rc : int(qidx[q0 + rc]);
-      }
-      if (dt == MF_DTYPE_F32) {
-#pragma unroll
-        for (int t = 0; t < kRB; ++t) graw[t] = static_cast<const uint32_t*>(p.bg)[size_t(bh) * N + gidx[t]];
-      } else {
-#pragma unroll
-        for (int t = 0; t < kRB; ++t) graw[t] = static_cast<const uint16_t*>(p.bg)[size_t(bh) * N + gidx[t]];
-      }
-#pragma unroll
-      for (int t = 0; t < kRB; ++t) {
-        const int r = r0 + kWaves * t;
-        const float gte = dt == MF_DTYPE_F32 ? __uint_as_float(graw[t])
-                          : dt == MF_DTYPE_BF16 ? __uint_as_float(graw[t] << 16)
-                                                : float(__builtin_bit_cast(_Float16, uint16_t(graw[t])));
-        crow[t] = r < nqg ? ldexpf(gte * kLog2e, cE) : 0.0f;
-      }
-      store_rows(S0{}, r0, vu, crow);
-      store_rows(S1{}, r0, vv, crow);
-      if (qb == 0) store_rows(S2{}, r0, vw, kNoRow);
-      if (lane == 0) {
-#pragma unroll
-        for (int t = 0; t < kRB; ++t) cgf[r0 + kWaves * t] = crow[t];
-      }
-    }
-    // W rows past the first batch (more than kWaves kRB staged keys)
-    for (int r0 = wave + kWaves * kRB; r0 < rj; r0 += kWaves * kRB) {
-      uint32_t vw[kRB][2];
-      load_rows(S2{}, r0, vw);
-      store_rows(S2{}, r0, vw, kNoRow);
-    }
+    if (p.bias_dtype == MF_DTYPE_F32) run([](uint32_t b) { return __uint_as_float(b); });
+    else if (p.bias_dtype == MF_DTYPE_BF16) run([](uint32_t b) { return __uint_as_float(b << 16); });
+    else run([](uint32_t b) { return float(__builtin_bit_cast(_Float16, uint16_t(b))); });
     // maxima over the wave, into this wave's slots (float order equals bit order for magnitudes)
 #pragma unroll
     for (int e = 0; e < 3; ++e) {
@@ -1082,29 +1068,56 @@ __device__ __forceinline__ void unit_body(const Params& p, unsigned char* smem, 
     for (int e = 0; e < 4; ++e) w[e] = pack_h2(ldexpf(f[2 * e], sc_exp), ldexpf(f[2 * e + 1], sc_exp));
     *reinterpret_cast<uint4*>(dst + row * RB + e0 * 2) = uint4{w[0], w[1], w[2], w[3]};
   };
-  // bits of pair_valid for rows j of the j block and keys k of the k block
-  auto stage_pv = [&](int jc, int kc) {
-    uint32_t* pvb = reinterpret_cast<uint32_t*>(smem + Ly::kPV);
-    const uint8_t* gpv = p.pv + size_t(b) * N * N;
+  // Bits of pair_valid for the rows j of the j block (and the padding row after an odd count, zero) and the keys of
+  // the k block.  A wave takes rows wv + 4 t, its lanes along the keys: a row's bytes are one or two coalesced
+  // loads and its bits a ballot.  pv_load reads the first kPR rows of the wave, pv_store stores them and then
+  // the rows past those (blocks of more than 64 rows).
+  constexpr int kPR = 16;
+  struct PvRegs {
+    uint8_t lo[kPR], hi[kPR];
+  };
+  auto pv_load_rows = [&](int jc, int kc, int t0, PvRegs& R) {
     const int j0 = jc * kCap, k0 = kc * kCap;
     const int nkj = min(kCap, nk - j0), nkk = min(kCap, nk - k0);
-    // a word's bytes are loaded 16 at a time without branches (columns past the block read its last key,
-    // and are masked afterwards), so each 16 loads are in flight together
-    for (int u = tid; u < kCap * Ly::kPVW; u += kThreads) {
-      const int jl = u / Ly::kPVW, wd = u % Ly::kPVW;
-      uint32_t bits = 0;
-      if (jl < nkj && nkk > 0) {
-        const uint8_t* prow = gpv + size_t(key_atom(j0 + jl)) * N;
-#pragma unroll 1
-        for (int h = 0; h < 32; h += 16) {
-          uint8_t v[16];
+    if (nkj <= 0 || nkk <= 0) return;
+    const uint8_t* gpv = p.pv + size_t(b) * N * N;
+    const int ja = key_atom(j0 + min(wv + kWaves * (t0 + lane), nkj - 1));  // lane t: the wave's row t0 + t
+    const uint32_t c0 = uint32_t(key_atom(k0 + min(lane, nkk - 1)));
+    const uint32_t c1 = uint32_t(key_atom(k0 + min(64 + lane, nkk - 1)));
 #pragma unroll
-          for (int t = 0; t < 16; ++t) v[t] = prow[key_atom(k0 + min(wd * 32 + h + t, nkk - 1))];
+    for (int t = 0; t < kPR; ++t) R.lo[t] = (gpv + uint32_t(__builtin_amdgcn_readlane(ja, t) * N))[c0];
+    if (nkk > 64) {
 #pragma unroll
-          for (int t = 0; t < 16; ++t) bits |= (wd * 32 + h + t < nkk && v[t] != 0) ? 1u << (h + t) : 0u;
+      for (int t = 0; t < kPR; ++t) R.hi[t] = (gpv + uint32_t(__builtin_amdgcn_readlane(ja, t) * N))[c1];
+    }
+  };
+  auto pv_load = [&](int jc, int kc, PvRegs& R) { pv_load_rows(jc, kc, 0, R); };
+  auto pv_store = [&](int jc, int kc, PvRegs& R) {
+    uint32_t* pvb = reinterpret_cast<uint32_t*>(smem + Ly::kPV);
+    const int nkj = min(kCap, nk - jc * kCap), nkk = min(kCap, nk - kc * kCap);
+    if (nkj <= 0 || nkk <= 0) return;
+    const int rows = min(kCap, nkj + (nkj & 1));
+    const unsigned long long keep0 = nkk >= 64 ? ~0ull : (1ull << nkk) - 1ull;
+    const unsigned long long keep1 = nkk >= 128 ? ~0ull : nkk > 64 ? (1ull << (nkk - 64)) - 1ull : 0ull;
+    for (int t0 = 0; wv + kWaves * t0 < rows; t0 += kPR) {
+      if (t0 > 0) pv_load_rows(jc, kc, t0, R);
+#pragma unroll
+      for (int t = 0; t < kPR; ++t) {
+        const int jl = wv + kWaves * (t0 + t);
+        if (jl >= rows) break;  // wave-uniform
+        const unsigned long long m0 = jl < nkj ? __ballot(R.lo[t] != 0) & keep0 : 0ull;
+        if (lane == 0) {
+          pvb[jl * Ly::kPVW] = uint32_t(m0);
+          pvb[jl * Ly::kPVW + 1] = uint32_t(m0 >> 32);
+        }
+        if (nkk > 64) {
+          const unsigned long long m1 = jl < nkj ? __ballot(R.hi[t] != 0) & keep1 : 0ull;
+          if (lane == 0) {
+            pvb[jl * Ly::kPVW + 2] = uint32_t(m1);
+            if (Ly::kPVW > 3) pvb[jl * Ly::kPVW + 3] = uint32_t(m1 >> 32);
+          }
         }
       }
-      pvb[u] = bits;
     }
   };
   // GUESS: the unit is staged with unit scales (K, V as they are, Q as q log2(e)) straight from the loads,
@@ -1116,15 +1129,16 @@ __device__ __forceinline__ void unit_body(const Params& p, unsigned char* smem, 
   float ql1 = 0.0f;  // GUESS: the largest ||q'_i||_1 of this wave's query rows
   if constexpr (!MULTI) {
     load_block(0, 0);
-    // without the bias: the pair-valid bits of the unit's one block, while the key rows are in flight (with
-    // the bias they are staged with the block, after the bias: staged here, their waits held up the bias
-    // loads)
-    if constexpr (HAS_PV && !BIAS) stage_pv(0, 0);
+    // the bias operands and the pair-valid bytes, in flight with the key rows
+    BiasRegs br;
+    PvRegs pr;
+    if constexpr (BIAS) bias_load(0, 0, br);
+    if constexpr (HAS_PV) pv_load(0, 0, pr);
     // the workgroup's share of padded query rows, stored while the loads are
     // in flight (first unit only)
     if (zero_share) zero_padded_share<T, DP, STR, Waves<BIAS>::kCount>(p, reinterpret_cast<const uint32_t*>(smem + Ly::kInfo), blockIdx.x, gridDim.x);
-    // the bias operands, loaded while the key rows are in flight (query scale exponent E = 0 assumed)
-    if constexpr (BIAS) stage_bias(0, 0, 0);
+    if constexpr (BIAS) bias_store(0, 0, 0, br);  // (query scale exponent E = 0 assumed)
+    if constexpr (HAS_PV) pv_store(0, 0, pr);
     if constexpr (GUESS) {
       const int rj = round16(nk);
 #pragma unroll
@@ -1288,7 +1302,9 @@ __device__ __forceinline__ void unit_body(const Params& p, unsigned char* smem, 
       // staged with the key rows assuming E = 0; a query scale of its own (E != 0, rare) restages
       if (E != 0) {
         __syncthreads();
-        stage_bias(0, 0, E);
+        BiasRegs br;
+        bias_load(0, 0, br);
+        bias_store(0, 0, E, br);
         __syncthreads();
       }
     } else {
@@ -1347,8 +1363,10 @@ __device__ __forceinline__ void unit_body(const Params& p, unsigned char* smem, 
     unsigned char* V2s = smem + Ly::kV2;
     const int nkj = min(kCap, nk - jc * kCap), nkk = min(kCap, nk - kc * kCap);
     const int rj = round16(nkj), rk = round16(nkk);
-    if constexpr (!MULTI) {
-      // the rows loaded in phase A
+    BiasRegs br;
+    PvRegs pr;
+    (void)br, (void)pr;
+    auto store_rows = [&]() {
 #pragma unroll
       for (int i = 0; i < MAXC; ++i) {
         if (i >= nI) break;
@@ -1362,33 +1380,18 @@ __device__ __forceinline__ void unit_body(const Params& p, unsigned char* smem, 
           store_row(V2s, rv2[i], row, t2);
         }
       }
+    };
+    if constexpr (!MULTI) {
+      store_rows();  // the rows loaded in phase A
     } else {
-      // larger molecules: one tensor at a time, so that few registers are
-      // live next to the accumulators
-      const int j0 = jc * kCap, k0 = kc * kCap;
-      uint4 t[MAXC];
-      int aj[MAXC], ak[MAXC];
-      slot_atoms(j0, nkj, aj);
-      slot_atoms(k0, nkk, ak);
-      load_set(gk1, aj, nkj, t);
-#pragma unroll
-      for (int i = 0; i < MAXC; ++i)
-        if ((tid + kThreads * i) / CPR < rj) store_row(K1s, t[i], (tid + kThreads * i) / CPR, s1);
-      load_set(gv1, aj, nkj, t);
-#pragma unroll
-      for (int i = 0; i < MAXC; ++i)
-        if ((tid + kThreads * i) / CPR < rj) store_row(V1s, t[i], (tid + kThreads * i) / CPR, t1);
-      load_set(gk2, ak, nkk, t);
-#pragma unroll
-      for (int i = 0; i < MAXC; ++i)
-        if ((tid + kThreads * i) / CPR < rk) store_row(K2s, t[i], (tid + kThreads * i) / CPR, s2);
-      load_set(gv2, ak, nkk, t);
-#pragma unroll
-      for (int i = 0; i < MAXC; ++i)
-        if ((tid + kThreads * i) / CPR < rk) store_row(V2s, t[i], (tid + kThreads * i) / CPR, t2);
+      // every load of the block in flight together
+      load_block(jc, kc);
+      if constexpr (BIAS) bias_load(jc, kc, br);
+      if constexpr (HAS_PV) pv_load(jc, kc, pr);
+      store_rows();
     }
-    if constexpr (BIAS && MULTI) stage_bias(jc, kc, E);
-    if constexpr (HAS_PV && (MULTI || BIAS)) stage_pv(jc, kc);
+    if constexpr (BIAS && MULTI) bias_store(jc, kc, E, br);
+    if constexpr (HAS_PV && MULTI) pv_store(jc, kc, pr);
   };
 
   // ---- phase C: pair loop -------------------------------------------------
@@ -1460,7 +1463,8 @@ __device__ __forceinline__ void unit_body(const Params& p, unsigned char* smem, 
     }
   };
   bool slow = false;
-  if (!MULTI && nch == 1) {
+  if constexpr (!MULTI) {
+   if (nch == 1) {
     if (!staged) {
       store_block(0, 0);
       __syncthreads();
@@ -1516,7 +1520,8 @@ __device__ __forceinline__ void unit_body(const Params& p, unsigned char* smem, 
         combine_online();
       }
     }
-  } else if (MULTI && nch > 1 && BIAS) {
+   }
+  } else if constexpr (BIAS) {
     // the bias key-block path (always exact offsets): one pass over the block pairs with running offsets
     __syncthreads();
     slow = true;
@@ -1532,7 +1537,7 @@ __device__ __forceinline__ void unit_body(const Params& p, unsigned char* smem, 
       }
     }
     combine_online();
-  } else if (MULTI && nch > 1) {
+  } else {
     __syncthreads();
     slow = scal[6] != 0;
     load_qop();
