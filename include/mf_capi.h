@@ -251,8 +251,18 @@ typedef struct mf_simplicial_bwd_args {
 
 int mf_simplicial_bwd(const mf_simplicial_bwd_args* args, void* stream);
 
-/* Bytes of workspace mf_simplicial_bwd needs (0 without a message term):   */
-/* per query, the message coefficients dc = basis . go and sum_jk P ML MR.  */
+/* mf_simplicial_bwd for bf16 operands with an fp32 bias, every gradient in */
+/* its leaf's dtype and written in full (zeros where an index is padded):   */
+/* grads_dtype MF_DTYPE_BF16 is that of dq .. dv2, du .. dgate are fp32     */
+/* (bias_dtype MF_DTYPE_F32), all 16-byte aligned.  Serves head_dim 64 and  */
+/* at most 512 tokens with the workspace given; MF_ERR_UNSUPPORTED, with    */
+/* nothing launched, otherwise.                                             */
+int mf_simplicial_bwd_leaf(const mf_simplicial_bwd_args* args, void* stream);
+
+/* Bytes of workspace the backward uses (0: none).  With a message term, per */
+/* query the message coefficients dc = basis . go and sum_jk P ML MR; at     */
+/* head_dim 64, the pair kernel's plan and partial sums (a smaller or NULL   */
+/* workspace there is accepted and the general kernel runs).                 */
 uint64_t mf_simplicial_bwd_workspace_size(int32_t batch, int32_t heads, int32_t tokens,
                                           int32_t head_dim, int32_t message_rank);
 

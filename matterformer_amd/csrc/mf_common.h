@@ -57,7 +57,8 @@ int simplicial_pair_f32_bwd_launch(const mf_simplicial_bwd_args* a, hipStream_t 
 // of units, atom lists and partial sums).
 bool simplicial_pair_bwd_serves(const mf_simplicial_bwd_args* a);
 size_t simplicial_pair_bwd_workspace_bytes(int batch, int heads, int tokens);
-int simplicial_pair_bwd_launch(const mf_simplicial_bwd_args* a, hipStream_t stream);
+// (bias16: the bias gradients are bf16, else fp32)
+int simplicial_pair_bwd_launch(const mf_simplicial_bwd_args* a, bool bias16, hipStream_t stream);
 
 #define MF_HIP_CHECK(expr)                                                     \
   do {                                                                         \

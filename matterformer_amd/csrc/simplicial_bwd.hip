@@ -1070,8 +1070,9 @@ __global__ void __launch_bounds__(256) zero_rows_kernel(Params p) {
   }
 }
 
-// bf16 bias gradients are written in full: the four tensors are cleared first (one flat pass of 16-byte
-// stores, the last n % 8 elements one by one), then the kernels write every valid entry.
+// Bias gradients that are written in full: the four tensors are cleared first (one flat pass of 16-byte
+// stores, the last elements one by one), then the kernels write every valid entry.  plane and gates in 16-bit
+// units (twice the elements of fp32 gradients).
 __global__ void __launch_bounds__(256) zero_bias_kernel(void* du, void* dvb, void* dw, void* dgate, size_t plane,
                                                         size_t gates) {
   void* const ptrs[4] = {du, dvb, dw, dgate};
@@ -1125,7 +1126,9 @@ static uint64_t message_workspace_bytes(int32_t batch, int32_t heads, int32_t to
   return 2ull * uint64_t(batch) * uint64_t(heads) * uint64_t(tokens) * uint64_t(message_rank) * 4ull;
 }
 
-extern "C" int mf_simplicial_bwd(const mf_simplicial_bwd_args* a, void* stream) {
+// bias32: with bf16 gradients of the operands, the bias gradients are fp32 and written in full too (calls that
+// simplicial_pair_bwd_serves; others are refused before anything is launched).
+static int simplicial_bwd_impl(const mf_simplicial_bwd_args* a, bool bias32, void* stream) {
   using namespace mf::sbwd;
   if (a == nullptr) return fail(MF_ERR_INVALID_ARGUMENT, "mf_simplicial_bwd: args is NULL");
   if (!a->q || !a->k1 || !a->v1 || !a->k2 || !a->v2 || !a->grad_out || !a->out || !a->lse)
@@ -1254,20 +1257,21 @@ extern "C" int mf_simplicial_bwd(const mf_simplicial_bwd_args* a, void* stream) 
   // bf16 operands and grad_out with head_dim 64 take the pair formulation (simplicial_pair_bwd.hip, which also
   // writes the zero rows of 16-bit gradients)
   const bool pair = simplicial_pair_bwd_serves(a);
+  if (bias32 && !pair) return fail(MF_ERR_UNSUPPORTED, "mf_simplicial_bwd_leaf: not a call of the pair kernel");
   if (gout16) {
     if (!pair) {
       hipLaunchKernelGGL(zero_rows_kernel, dim3(unsigned(a->batch * a->heads)), dim3(256), 0, s, prm);
       MF_HIP_CHECK(hipGetLastError());
     }
     if (has_bias && (a->du || a->dv_bias || a->dw || a->dgate)) {
-      const size_t gates = size_t(a->batch) * a->heads * a->tokens, plane = gates * a->tokens;
+      const size_t gates = size_t(a->batch) * a->heads * a->tokens * (bias32 ? 2 : 1), plane = gates * a->tokens;
       const size_t grid = std::min<size_t>((plane / 8 + 255) / 256, 4096);
       hipLaunchKernelGGL(zero_bias_kernel, dim3(unsigned(std::max<size_t>(grid, 1))), dim3(256), 0, s, a->du,
                          a->dv_bias, a->dw, a->dgate, plane, gates);
       MF_HIP_CHECK(hipGetLastError());
     }
   }
-  if (pair) return simplicial_pair_bwd_launch(a, s);
+  if (pair) return simplicial_pair_bwd_launch(a, gout16 && !bias32, s);
   if (simplicial_pair_f32_bwd_serves(a)) return simplicial_pair_f32_bwd_launch(a, s);
   // other bf16 operands with a bf16 grad_out: bf16 MFMA (K steps of 32 d), which stages grad_out rows as bf16
   // (exact only for a bf16 grad_out).  Everything else -- fp16 operands, or a grad_out of another dtype -- takes
@@ -1281,6 +1285,16 @@ extern "C" int mf_simplicial_bwd(const mf_simplicial_bwd_args* a, void* stream) 
   if (D <= 32) return launch<32, false>(prm, has_pv, has_bias, s);
   if (D <= 64) return launch<64, false>(prm, has_pv, has_bias, s);
   return launch<128, false>(prm, has_pv, has_bias, s);
+}
+
+extern "C" int mf_simplicial_bwd(const mf_simplicial_bwd_args* a, void* stream) {
+  return simplicial_bwd_impl(a, false, stream);
+}
+
+extern "C" int mf_simplicial_bwd_leaf(const mf_simplicial_bwd_args* a, void* stream) {
+  if (a != nullptr && (a->grads_dtype != MF_DTYPE_BF16 || a->bias_u == nullptr || a->bias_dtype != MF_DTYPE_F32))
+    return mf::fail(MF_ERR_INVALID_ARGUMENT, "mf_simplicial_bwd_leaf: grads_dtype must be MF_DTYPE_BF16 and the bias MF_DTYPE_F32");
+  return simplicial_bwd_impl(a, true, stream);
 }
 
 extern "C" uint64_t mf_simplicial_bwd_workspace_size(int32_t batch, int32_t heads, int32_t tokens, int32_t head_dim,

@@ -120,7 +120,8 @@ struct Params {
   void* dv1;
   void* dk2;
   void* dv2;
-  int gout16;
+  int gout16;             // dq .. dv2 are bf16
+  int bout16;             // du .. dgate are bf16
   const int* head;        // plan: [0] units in the list, [1] j per unit
   const uint32_t* units;  // plan: (b H + h) << 6 | part, longest first
   const int2* counts;     // plan: [B] valid keys, valid queries
@@ -1136,7 +1137,7 @@ __global__ void __launch_bounds__(kThreads, 2) pair_bwd_kernel(Params p) {
               float* o = p.dwpart + (rbase + c.j0 + j) * N + c.k0 + k;
               if (qb > 0) x += *o;
               if (qb + 1 < nqb) *o = x;
-              else store_grad(p.dw, (rbase + jidx[j]) * N + kidx[k], x, p.gout16);
+              else store_grad(p.dw, (rbase + jidx[j]) * N + kidx[k], x, p.bout16);
             }
           }
           if (kb + 1 < nkb) lds_barrier();
@@ -1147,7 +1148,7 @@ __global__ void __launch_bounds__(kThreads, 2) pair_bwd_kernel(Params p) {
           for (int u = opaque_tid(); u < c.nq * JM; u += kThreads) {
             const int i = u / JM, j = u % JM;
             if (j < c.nj)
-              store_grad(p.du, (rbase + qidx[i]) * N + jidx[j], cgs[i] * (1.0f / kLog2e) * dut[j * KU + i], p.gout16);
+              store_grad(p.du, (rbase + qidx[i]) * N + jidx[j], cgs[i] * (1.0f / kLog2e) * dut[j * KU + i], p.bout16);
           }
         }
         if (qb + 1 < nqb) lds_barrier();
@@ -1249,7 +1250,7 @@ __global__ void __launch_bounds__(kThreads) pair_bwd_bias_finish(Params p) {
         for (int t = 0; t < kFinishAt; ++t) sv[t] += dvp[size_t(part) * N * N + e[t]];
 #pragma unroll
       for (int t = 0; t < kFinishAt; ++t)
-        if (u0 + t * step < n) store_grad(p.dvb, o[t], gate[t] * sv[t], p.gout16);
+        if (u0 + t * step < n) store_grad(p.dvb, o[t], gate[t] * sv[t], p.bout16);
     }
   }
   if (p.dgate != nullptr && blockIdx.y == 0) {
@@ -1257,7 +1258,7 @@ __global__ void __launch_bounds__(kThreads) pair_bwd_bias_finish(Params p) {
     for (int i = tid; i < nq; i += kThreads) {
       float s = gp[i];
       for (int part = 1; part < parts; ++part) s += gp[size_t(part) * N + i];
-      store_grad(p.dgate, rbase + qlist[i], s, p.gout16);
+      store_grad(p.dgate, rbase + qlist[i], s, p.bout16);
     }
   }
 }
@@ -1310,7 +1311,7 @@ static int launch_units(const pbwd::Params& p, int blocks, int bh, hipStream_t s
   return MF_OK;
 }
 
-int simplicial_pair_bwd_launch(const mf_simplicial_bwd_args* a, hipStream_t stream) {
+int simplicial_pair_bwd_launch(const mf_simplicial_bwd_args* a, bool bias16, hipStream_t stream) {
   using namespace pbwd;
   const Ws ws(a->batch, a->heads, a->tokens);
   unsigned char* wsp = static_cast<unsigned char*>(a->workspace);
@@ -1345,6 +1346,7 @@ int simplicial_pair_bwd_launch(const mf_simplicial_bwd_args* a, hipStream_t stre
   p.pv = a->pair_valid;
   p.dq = a->dq; p.dk1 = a->dk1; p.dv1 = a->dv1; p.dk2 = a->dk2; p.dv2 = a->dv2;
   p.gout16 = g16 ? 1 : 0;
+  p.bout16 = bias16 ? 1 : 0;
   p.H = a->heads;
   p.N = a->tokens;
   p.cap = ws.cap;

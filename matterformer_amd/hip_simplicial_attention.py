@@ -371,7 +371,7 @@ last_backward_impl: str | None = None
 
 def _kernel_backward(grad_out, q, k1, v1, k2, v2, out, lse, query_valid, pair_key_valid, pair_valid,
                      u, v_bias, w, gate, angle_left, angle_right, angle_gate, message_left, message_right,
-                     message_basis, flags):
+                     message_basis, flags, allow_leaf=True):
     """mf_simplicial_bwd; None when the library reports the shape as beyond its capacity."""
     if not HIP_AVAILABLE:
         raise RuntimeError(f"HIP simplicial attention is unavailable: {_native.load_error()}")
@@ -395,12 +395,16 @@ def _kernel_backward(grad_out, q, k1, v1, k2, v2, out, lse, query_valid, pair_ke
         raise ValueError("query_valid / pair_key_valid must be (B, N) and pair_valid (B, N, N)")
     ext = _prepare_extras(q, B, H, N, D, u, v_bias, w, gate, angle_left, angle_right, angle_gate,
                           message_left, message_right, message_basis)
-    # bf16 operands, grad_out and leaves (bias terms included), no low-rank term: the library writes every
-    # element of bf16 gradients (no fill, no cast); otherwise fp32 gradients, zero-filled here and cast to the
-    # leaves' dtypes
+    # bf16 operands, grad_out and leaves, no low-rank term: the library writes every element of bf16 gradients (no
+    # fill, no cast); so it does for an fp32 bias in the pair kernel's range (64 molecules of 44 atoms padded to
+    # 181, 8 heads: 495 -> 406 us); otherwise fp32 gradients, zero-filled here and cast to the leaves' dtypes
     g16 = (dt == torch.bfloat16 and gdt == torch.bfloat16 and ext.angle is None and ext.message is None
-           and D % 8 == 0 and N <= 4096 and all(t.dtype == torch.bfloat16 for t in (q, k1, v1, k2, v2))
-           and (ext.bias is None or all(t.dtype == torch.bfloat16 for t in (u, v_bias, w, gate))))
+           and D % 8 == 0 and N <= 4096 and all(t.dtype == torch.bfloat16 for t in (q, k1, v1, k2, v2)))
+    leaf = False
+    if g16 and ext.bias is not None and any(t.dtype != torch.bfloat16 for t in (u, v_bias, w, gate)):
+        g16 = leaf = (allow_leaf and D == 64 and N <= 512
+                      and all(t.dtype == torch.float32 for t in (u, v_bias, w, gate)))
+    bdt = torch.float32 if leaf else torch.bfloat16
     if g16:
         grads = [torch.empty(B, H, N, D, device=dev, dtype=torch.bfloat16) for _ in range(5)]
     else:
@@ -410,7 +414,7 @@ def _kernel_backward(grad_out, q, k1, v1, k2, v2, out, lse, query_valid, pair_ke
         for idx, (name, shape) in enumerate((("need_du", (B, H, N, N)), ("need_dv_bias", (B, H, N, N)),
                                              ("need_dw", (B, H, N, N)), ("need_dgate", (B, H, N)))):
             if flags[name]:
-                bias_grads[idx] = (torch.empty(shape, device=dev, dtype=torch.bfloat16) if g16 else
+                bias_grads[idx] = (torch.empty(shape, device=dev, dtype=bdt) if g16 else
                                    torch.zeros(shape, device=dev, dtype=torch.float32))
     # low-rank gradients: (dangle_left, dangle_right, dangle_gate), (dmessage_left, dmessage_right, dmessage_basis)
     lr_grads: list[torch.Tensor | None] = [None] * 6
@@ -454,8 +458,12 @@ def _kernel_backward(grad_out, q, k1, v1, k2, v2, out, lse, query_valid, pair_ke
         workspace=_native.ptr(workspace), workspace_bytes=0 if workspace is None else workspace.numel())
     lib = _native.lib()
     with torch.cuda.device(dev):
-        status = lib.mf_simplicial_bwd(args, _native.current_stream(dev))
+        status = (lib.mf_simplicial_bwd_leaf if leaf else lib.mf_simplicial_bwd)(args, _native.current_stream(dev))
     if status == _native.MF_ERR_UNSUPPORTED:
+        if leaf:  # (beyond the pair kernel's workspace limit: the general kernel, fp32 gradients)
+            return _kernel_backward(grad_out, q, k1, v1, k2, v2, out, lse, query_valid, pair_key_valid, pair_valid,
+                                    u, v_bias, w, gate, angle_left, angle_right, angle_gate, message_left,
+                                    message_right, message_basis, flags, allow_leaf=False)
         return None
     _native.check(status, "mf_simplicial_bwd")
     core = grads if g16 else [g.to(t.dtype) for g, t in zip(grads, (q, k1, v1, k2, v2))]

@@ -62,3 +62,51 @@ def test_queries_and_keys_of_different_counts(cuda):
     for name, g, r in zip(GRAD_NAMES, got, ref):
         bar = 2e-3 if g.dtype == torch.float32 else 4e-3
         assert rel_err(g.float().cpu().numpy(), r) <= bar, (name, rel_err(g.float().cpu().numpy(), r))
+
+
+@pytest.mark.parametrize("wanted", [(True, True, True, True), (False, True, False, False)], ids=["all", "dv"])
+@pytest.mark.parametrize("B,N", [(1, 9), (3, 45), (2, 130)])
+def test_gradients_in_the_leaves_dtypes_are_written_in_full(cuda, B, N, wanted):
+    """bf16 operands with an fp32 bias: the entry that writes every element gives what the zero-filled fp32
+    gradients cast to the leaves' dtypes give, bit for bit (the same sums, rounded once), over buffers that held
+    NaN, padded rows included."""
+    import matterformer_amd.hip_simplicial_attention as hsa
+
+    H, D = 1, 64
+    counts = [max(1, N - 7 * b - 4) for b in range(B)]
+    q, k1, v1, k2, v2, qv, pkv, pv = random_simplicial(B, H, N, D, seed=N, counts=counts, pair_drop=0.1,
+                                                       std=logit_std(D))
+    gen = torch.Generator().manual_seed(N + 1)
+    ops = [t.to(torch.bfloat16).to(cuda) for t in (q, k1, v1, k2, v2)]
+    go = torch.randn(B, H, N, D, generator=gen).to(torch.bfloat16).to(cuda)
+    bias = [(torch.randn(s, generator=gen) * 0.5).to(cuda) for s in [(B, H, N, N)] * 3 + [(B, H, N)]]
+    masks = dict(query_valid=qv.to(cuda), pair_key_valid=pkv.to(cuda), pair_valid=pv.to(cuda))
+    _, lse, out32 = hsa.hip_simplicial_attention_forward(*ops, **masks, u=bias[0], v_bias=bias[1], w=bias[2],
+                                                         gate=bias[3])
+    flags = dict.fromkeys([f"need_d{n}" for n in ("u", "v_bias", "w", "gate", "angle_left", "angle_right", "angle_gate",
+                                                  "message_left", "message_right", "message_basis")], False)
+    flags.update(zip(("need_du", "need_dv_bias", "need_dw", "need_dgate"), wanted))
+    call = (go, *ops, out32, lse, *masks.values(), *bias, *[None] * 6, flags)
+    want = hsa._kernel_backward(*call, allow_leaf=False)
+    poison = [torch.full((1 << 22,), float("nan"), device=cuda) for _ in range(4)]
+    poison += [torch.full((B * H * N * n,), float("nan"), device=cuda) for n in (1, D // 2, N) for _ in range(5)]
+    del poison  # the allocator hands these blocks out again
+    got = hsa._kernel_backward(*call)
+    for g, w in zip(got, want):
+        assert (g is None) == (w is None)
+        if w is not None:
+            assert g.dtype == w.dtype and torch.equal(g, w)
+
+
+def test_leaf_entry_refuses_other_calls():
+    """grads_dtype F32 or a bias of another dtype is refused before anything is read or launched."""
+    from matterformer_amd import _native
+
+    lib = _native.lib()
+    fake = 4096
+    for grads, bias in ((_native.MF_DTYPE_F32, _native.MF_DTYPE_F32), (_native.MF_DTYPE_BF16, _native.MF_DTYPE_BF16)):
+        a = _native.MfSimplicialBwdArgs(q=fake, k1=fake, v1=fake, k2=fake, v2=fake, grad_out=fake, out=fake, lse=fake,
+                                        query_valid=fake, pair_key_valid=fake, bias_u=fake, bias_v=fake, bias_w=fake,
+                                        bias_gate=fake, bias_dtype=bias, grads_dtype=grads, batch=1, heads=1,
+                                        tokens=8, head_dim=64)
+        assert lib.mf_simplicial_bwd_leaf(a, None) == _native.MF_ERR_INVALID_ARGUMENT
