@@ -1653,31 +1653,38 @@ __device__ __forceinline__ uint4 chunk_bytes(int lo, int hi) {
 
 // Valid (nonzero) byte count of bytes [a, e) of a mask row in global memory,
 // and the index of the first zero byte among them (e if none).  The bytes are
-// read as the 16-byte aligned chunks that hold them, eight loads in flight; an
-// aligned chunk that holds a byte of the row lies on that byte's page.  Every
-// chunk is counted whole; the bytes of the first chunk before a are masked
-// there (a compile-time slot), and those of the last chunk from e on are read
-// again once and taken off.  The first zero is looked for from a on; one past
-// e is clamped to e.
-__device__ __forceinline__ void scan_row_global(const uint8_t* row, int a, int e, int& count, int& firstzero) {
+// read as the 16-byte aligned chunks that hold them, sixteen loads in flight
+// (one round trip up to 240 bytes); an aligned chunk that holds a byte of the
+// row lies on that byte's page.  Every chunk is counted whole except for the
+// bytes of the first chunk before a and those of the last from e on.
+// The first zero is looked for from a on; one past e is clamped to e.
+// most: the most chunks of any thread (wave-uniform).
+__device__ __forceinline__ void scan_row_global(const uint8_t* row, int a, int e, int most, int& count,
+                                                int& firstzero) {
+  constexpr int kIn = 16;  // loads in flight
   firstzero = e;
-  if (a >= e) return;
   const uint8_t* begin = row + a;
   const int off = int(reinterpret_cast<uintptr_t>(begin) & 15u);
-  const uint8_t* c0 = begin - off;  // pointer arithmetic keeps the global address space
-  const int span = off + (e - a);   // bytes from c0 to the end of the segment
+  const uint8_t* c0 = begin - off;            // pointer arithmetic keeps the global address space
+  const int span = a < e ? off + (e - a) : 0;  // bytes from c0 to the end of the segment
   const int nch = (span + 15) >> 4;
   const uint4 keep0 = chunk_bytes(off, 16);
   int cnt = 0, zc = -1;
   uint32_t zw[4] = {0u, 0u, 0u, 0u};
-  for (int c = 0; c < nch; c += 8) {
-    uint4 v[8];
+  uint4 vl{0u, 0u, 0u, 0u};  // the last chunk
+  for (int c = 0; c < most; c += kIn) {
+    uint4 v[kIn];
 #pragma unroll
-    for (int t = 0; t < 8; ++t)
-      v[t] = c + t < nch ? *reinterpret_cast<const uint4*>(c0 + 16 * (c + t)) : uint4{0u, 0u, 0u, 0u};
+    for (int t = 0; t < kIn; ++t) {
+      v[t] = uint4{0u, 0u, 0u, 0u};
+      if (c + t < most) {
+        if (c + t < nch) v[t] = *reinterpret_cast<const uint4*>(c0 + 16 * (c + t));
+      }
+    }
     const uint4 m0 = c == 0 ? keep0 : uint4{0x80808080u, 0x80808080u, 0x80808080u, 0x80808080u};
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
+    for (int t = 0; t < kIn; ++t) {
+      if (c + t >= most) break;
       uint32_t n0 = nz_bytes(v[t].x), n1 = nz_bytes(v[t].y), n2 = nz_bytes(v[t].z), n3 = nz_bytes(v[t].w);
       uint32_t z0 = n0 ^ 0x80808080u, z1 = n1 ^ 0x80808080u, z2 = n2 ^ 0x80808080u, z3 = n3 ^ 0x80808080u;
       if (t == 0) {
@@ -1685,6 +1692,7 @@ __device__ __forceinline__ void scan_row_global(const uint8_t* row, int a, int e
         z0 &= m0.x; z1 &= m0.y; z2 &= m0.z; z3 &= m0.w;
       }
       cnt += __popc(n0) + __popc(n1) + __popc(n2) + __popc(n3);
+      if (c + t == nch - 1) vl = v[t];
       if (zc < 0 && (z0 | z1 | z2 | z3) != 0u) {
         zc = c + t;
         zw[0] = z0; zw[1] = z1; zw[2] = z2; zw[3] = z3;
@@ -1692,7 +1700,6 @@ __device__ __forceinline__ void scan_row_global(const uint8_t* row, int a, int e
     }
   }
   if (span & 15) {  // bytes e .. of the last chunk
-    const uint4 vl = *reinterpret_cast<const uint4*>(c0 + 16 * (nch - 1));
     uint4 ml = chunk_bytes(span & 15, 16);
     if (nch == 1) ml = uint4{ml.x & keep0.x, ml.y & keep0.y, ml.z & keep0.z, ml.w & keep0.w};
     cnt -= __popc(nz_bytes(vl.x) & ml.x) + __popc(nz_bytes(vl.y) & ml.y) + __popc(nz_bytes(vl.z) & ml.z) +
@@ -1711,27 +1718,31 @@ __device__ __forceinline__ void scan_row_global(const uint8_t* row, int a, int e
 // Valid key / query counts and prefix flags of every molecule into s_info,
 // straight from the byte masks in global memory.  Rows are taken in passes of
 // whole molecules (row 2m: key mask of molecule m, row 2m + 1: its query
-// mask); TPR adjacent threads scan one row, each a segment of it, and the
+// mask; one row per molecule when both masks are the same bytes, as for plain
+// padding); TPR adjacent threads scan one row, each a segment of it, and the
 // segment counts meet over lanes.
 template <int DP, bool BIAS>
 __device__ __forceinline__ void scan_masks(const Params& p, unsigned char* smem, uint32_t* s_info) {
   constexpr int kThreads = Waves<BIAS>::kCount * 64;
   const int tid = threadIdx.x;
   const int B = p.B, N = p.N;
-  const int rows = 2 * B;
+  const bool same = p.pkv == p.qv;
+  const int sh = same ? 0 : 1;  // rows per molecule: 1 << sh
+  const int rows = B << sh;
   // threads per row: a power of two, <= 8, with rows * tpr <= kThreads when rows allow
   const int tpr = rows > kThreads / 2 ? 1 : rows > kThreads / 4 ? 2 : rows > kThreads / 8 ? 4 : 8;
   const int rpp = kThreads / tpr;  // rows per pass (even)
   int* s_cnt = reinterpret_cast<int*>(smem + Lay<DP, BIAS>::kK2);  // [rpp] counts, then [rpp] first zeros
   static_assert(Lay<DP, BIAS>::kCap * Lay<DP, BIAS>::RB >= kThreads * 2 * 4, "row results must fit in the K2 staging area");
   const int seg = (N + tpr - 1) / tpr;
+  const int most = (seg + 30) >> 4;  // 16-byte chunks of an unaligned segment, at most
   for (int r0 = 0; r0 < rows; r0 += rpp) {
     const int r = r0 + tid / tpr, sg = tid & (tpr - 1);
     int cnt = 0, last = N;  // count and first zero byte of the row
     if (r < rows) {
-      const uint8_t* row = ((r & 1) ? p.qv : p.pkv) + size_t(r >> 1) * N;
+      const uint8_t* row = ((r & sh) ? p.qv : p.pkv) + size_t(r >> sh) * N;
       const int a = min(N, sg * seg);
-      scan_row_global(row, a, min(N, a + seg), cnt, last);
+      scan_row_global(row, a, min(N, a + seg), most, cnt, last);
     }
     // the tpr threads of a row are adjacent lanes of one wave (all active)
     if (tpr >= 2) {
@@ -1751,11 +1762,12 @@ __device__ __forceinline__ void scan_masks(const Params& p, unsigned char* smem,
       s_cnt[rpp + r - r0] = last;
     }
     __syncthreads();
-    const int m0 = r0 >> 1;
-    for (int m = tid; m < rpp / 2 && m0 + m < B; m += kThreads) {
-      const int ck = min(s_cnt[2 * m], N), cq = min(s_cnt[2 * m + 1], N);
+    const int m0 = r0 >> sh;
+    for (int m = tid; m < (rpp >> sh) && m0 + m < B; m += kThreads) {
+      const int rk = m << sh, rq = rk + sh;
+      const int ck = min(s_cnt[rk], N), cq = min(s_cnt[rq], N);
       // the valid bytes are the prefix 0 .. n - 1 exactly when the first zero byte is byte n
-      const int zk = s_cnt[rpp + 2 * m], zq = s_cnt[rpp + 2 * m + 1];
+      const int zk = s_cnt[rpp + rk], zq = s_cnt[rpp + rq];
       s_info[m0 + m] = uint32_t(ck) | (uint32_t(cq) << 11) | (zk == ck ? kKPre : 0u) | (zq == cq ? kQPre : 0u);
     }
     __syncthreads();
@@ -1764,54 +1776,74 @@ __device__ __forceinline__ void scan_masks(const Params& p, unsigned char* smem,
 
 // s_order[rank] = molecule, s_pre[rank] = its first list position
 // (s_pre[B] = attention units in the list), molecules longest first (cost
-// nk^2 x query tiles, ties by index).  A molecule's position is the sum of
-// the units of the molecules ranked before it, so rank and position come
-// from one pass over (cost, units) pairs: 4 threads per molecule, each over
-// every 4th pair.  s_cu holds the pairs (over the staging area).  The
-// molecule whose positions hold position w (when w < s_pre[B]) writes
+// nk^2 x query tiles, ties by index).  The key cost 2^8 + 255 - index (at most
+// 2^31) orders both, so a molecule's rank is the number of larger keys: 4
+// threads per molecule, each over a quarter of the keys.  The first wave then
+// sums the units in rank order, four ranks a lane.  s_key holds the keys and
+// then the units by rank (over the staging area).  The molecule whose
+// positions hold position w (when w < s_pre[B]) gives
 // *s_first = b | (w - its first position) << 16.
+// (Every workgroup scans and ranks for itself before its first unit: 16 -> 12
+// us at 256 molecules of 181 tokens with one comparison a pair, one round trip
+// per scan and one scan for equal masks; two launches of 256 molecules of 44
+// atoms without a bias 252 -> 244 us.)
 template <int W, int GQ, int kCap>
 __device__ __forceinline__ void rank_molecules(const Params& p, const uint32_t* s_info, uint16_t* s_order, int* s_pre,
-                                               uint2* s_cu, int w, int* s_first) {
+                                               uint32_t* s_key, int w, int* s_first) {
   constexpr int kThreads = W * 64;
+  static_assert(kMaxBatch == 256 && kMaxN <= 512, "a key fits 31 bits and its index part 8; four ranks a lane");
   const int tid = threadIdx.x;
   const int B = p.B, H = p.H;
-  const int B4 = (B + 3) & ~3;
-  for (int b = tid; b < B4; b += kThreads) {
-    uint2 cu{0u, 0u};  // padding: cost 0 and index >= B never rank before a molecule
+  const int B16 = (B + 15) & ~15;
+  uint32_t* s_units = s_key + kMaxBatch;
+  for (int b = tid; b < kMaxBatch; b += kThreads) {
+    uint32_t key = 0u;  // past B: no key is smaller
     if (b < B) {
       const uint32_t w = s_info[b];
       const int nk = info_nk(w), nq = info_nq(w);
-      cu.x = uint32_t(nk * nk) * uint32_t((nq + 15) / 16);
-      cu.y = uint32_t(H * num_groups<GQ, kCap>(nk, nq));
+      key = (uint32_t(nk * nk) * uint32_t((nq + 15) / 16)) << 8 | uint32_t(255 - b);
     }
-    s_cu[b] = cu;
+    s_key[b] = key;
+    s_units[b] = 0u;
   }
   __syncthreads();
   for (int t = tid; t < 4 * B; t += kThreads) {
     const int b = t >> 2, part = t & 3;
-    const uint32_t cb = s_cu[b].x;
-    int rank = 0, pre = 0;
-    // pairs part, part + 4, ...: two per 16-byte read
-    const uint4* c4 = reinterpret_cast<const uint4*>(s_cu);
-#pragma unroll 8
-    for (int o = 2 * part; o < B4; o += 8) {
-      const uint4 v = c4[o >> 1];  // pairs o, o + 1
-      const bool f0 = v.x > cb || (v.x == cb && o < b);
-      const bool f1 = v.z > cb || (v.z == cb && o + 1 < b);
-      rank += int(f0) + int(f1);
-      pre += (f0 ? int(v.y) : 0) + (f1 ? int(v.w) : 0);
+    const uint32_t kb = s_key[b];
+    int rank = 0;
+    const uint4* k4 = reinterpret_cast<const uint4*>(s_key);
+#pragma unroll 4
+    for (int o = part; o < B16 / 4; o += 4) {
+      const uint4 v = k4[o];
+      rank += int(v.x > kb) + int(v.y > kb) + int(v.z > kb) + int(v.w > kb);
     }
     // the 4 threads of a molecule are one quad (whole quads are active)
     rank = int(group_reduce<4>(uint32_t(rank), AddI32{}));
-    pre = int(group_reduce<4>(uint32_t(pre), AddI32{}));
     if (part == 0) {
-      const int units = int(s_cu[b].y);
+      const uint32_t w = s_info[b];
       s_order[rank] = uint16_t(b);
-      s_pre[rank] = pre;
-      if (rank == B - 1) s_pre[B] = pre + units;
-      if (w >= pre && w < pre + units) *s_first = b | ((w - pre) << 16);
+      s_units[rank] = uint32_t(H * num_groups<GQ, kCap>(info_nk(w), info_nq(w)));
     }
+  }
+  __syncthreads();
+  if (tid < 64) {
+    const int4 u = reinterpret_cast<const int4*>(s_units)[tid];
+    const int own = u.x + u.y + u.z + u.w;
+    int run = own;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int v = __shfl_up(run, off, 64);
+      run += tid >= off ? v : 0;
+    }
+    const int p0 = run - own, p1 = p0 + u.x, p2 = p1 + u.y, p3 = p2 + u.z;
+    const int r = 4 * tid;
+    const int pre[5] = {p0, p1, p2, p3, run};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (r + e <= B) s_pre[r + e] = pre[e];
+      if (r + e < B && w >= pre[e] && w < pre[e + 1]) *s_first = int(s_order[r + e]) | ((w - pre[e]) << 16);
+    }
+    if (tid == 63 && B == kMaxBatch) s_pre[kMaxBatch] = run;
   }
   __syncthreads();
 }
@@ -1879,7 +1911,7 @@ __global__ void __launch_bounds__(Waves<BIAS>::kCount * 64, 2) simplicial_pair_k
     }
   }
   scan_masks<DP, BIAS>(p, smem, s_info);  // ends with a barrier
-  rank_molecules<W, Waves<BIAS>::kGroup, Waves<BIAS>::kCap>(p, s_info, s_order, s_pre, reinterpret_cast<uint2*>(smem), wg, &s_first);
+  rank_molecules<W, Waves<BIAS>::kGroup, Waves<BIAS>::kCap>(p, s_info, s_order, s_pre, reinterpret_cast<uint32_t*>(smem), wg, &s_first);
   const int total = s_pre[B];
 
   // the rows of padded queries: a static share of (b, h) pairs per
