@@ -275,6 +275,9 @@ int mf_simplicial_fwd_supported(int32_t batch, int32_t heads, int32_t tokens,
 uint64_t mf_simplicial_fwd_workspace_size(int32_t batch, int32_t heads, int32_t tokens,
                                           int32_t head_dim, int32_t dtype);
 
+/* mf_simplicial_fwd that takes operand strides together with pair_valid too. */
+int mf_simplicial_fwd_views(const mf_simplicial_fwd_args* args, void* stream);
+
 /* Allocation-free variant of mf_simplicial_fwd.  It has no counterpart in the
  * reference: it is for callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).

@@ -38,6 +38,7 @@ EXPORTED_SYMBOLS = (
     "mf_simplicial_fwd_supported",
     "mf_simplicial_fwd_workspace_size",
     "mf_simplicial_fwd_noalloc",
+    "mf_simplicial_fwd_views",
     "mf_simplicial_bwd",
     "mf_simplicial_bwd_leaf",
     "mf_simplicial_bwd_workspace_size",
@@ -244,6 +245,7 @@ def _load() -> ctypes.CDLL | None:
     for name, argtype in (
         ("mf_simplicial_fwd", MfSimplicialFwdArgs),
         ("mf_simplicial_fwd_noalloc", MfSimplicialFwdArgs),
+        ("mf_simplicial_fwd_views", MfSimplicialFwdArgs),
         ("mf_simplicial_bwd", MfSimplicialBwdArgs),
         ("mf_simplicial_bwd_leaf", MfSimplicialBwdArgs),
         ("mf_knn", MfKnnArgs),

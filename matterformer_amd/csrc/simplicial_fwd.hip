@@ -875,10 +875,14 @@ static int launch_general(const mf_simplicial_fwd_args* a, size_t lds, int num_c
   return dispatch<0>(a->dtype, DP, prm, lds, grid, s);
 }
 
-static int simplicial_fwd_impl(const mf_simplicial_fwd_args* a, void* stream);
+static int simplicial_fwd_impl(const mf_simplicial_fwd_args* a, bool views, void* stream);
 
 extern "C" int mf_simplicial_fwd(const mf_simplicial_fwd_args* a, void* stream) {
-  return simplicial_fwd_impl(a, stream);
+  return simplicial_fwd_impl(a, false, stream);
+}
+
+extern "C" int mf_simplicial_fwd_views(const mf_simplicial_fwd_args* a, void* stream) {
+  return simplicial_fwd_impl(a, true, stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -940,10 +944,11 @@ extern "C" int mf_simplicial_fwd_noalloc(const mf_simplicial_fwd_args* a, void* 
     sub.workspace = ptr;
     sub.workspace_bytes = kNoAllocScratchBytes;
   }
-  return simplicial_fwd_impl(&sub, stream);
+  return simplicial_fwd_impl(&sub, false, stream);
 }
 
-static int simplicial_fwd_impl(const mf_simplicial_fwd_args* a, void* stream) {
+// views: operand strides are taken together with pair_valid
+static int simplicial_fwd_impl(const mf_simplicial_fwd_args* a, bool views, void* stream) {
   if (a == nullptr) return fail(MF_ERR_INVALID_ARGUMENT, "mf_simplicial_fwd: args is NULL");
   if (!a->q || !a->k1 || !a->v1 || !a->k2 || !a->v2)
     return fail(MF_ERR_INVALID_ARGUMENT, "mf_simplicial_fwd: q, k1, v1, k2 and v2 must be non-NULL");
@@ -977,7 +982,7 @@ static int simplicial_fwd_impl(const mf_simplicial_fwd_args* a, void* stream) {
   // other shapes) run on the general kernel
   const bool bias_only = a->bias_u != nullptr && a->angle_left == nullptr && a->message_left == nullptr;
   if (has_strides(a)) {
-    if (!pair_ok || has_pv || (has_extras(a) && !bias_only))
+    if (!pair_ok || (has_pv && !views) || (has_extras(a) && !bias_only))
       return fail(MF_ERR_UNSUPPORTED,
                   "mf_simplicial_fwd: operand strides other than the contiguous [B*H, N, D] layout are taken by "
                   "the pair kernel only (16-bit operands, head_dim <= 64 and a multiple of 8, tokens <= 512, "

@@ -2020,20 +2020,16 @@ int simplicial_pair_launch(const mf_simplicial_fwd_args* a, void* claims, int nu
   const bool bf = a->dtype == MF_DTYPE_BF16;
   const bool bias = a->bias_u != nullptr;
   // caller strides: their own instantiations (the contiguous ones keep the shape-derived addressing,
-  // which leaves the kernel's scalar registers as they were); none with pair_valid
+  // which leaves the kernel's scalar registers as they were)
   bool strided = false;
   for (const int64_t* st : {a->q_stride, a->kv_stride, a->out_stride})
     strided = strided || st[0] != 0 || st[1] != 0 || st[2] != 0;
-  if (strided && pv)
-    return fail(MF_ERR_UNSUPPORTED, "simplicial pair launch: operand strides are not taken together with pair_valid");
   auto go = [&](auto tag, auto dp, auto has_pv) {
     using T = decltype(tag);
     constexpr int DP = decltype(dp)::value;
     constexpr bool PV = decltype(has_pv)::value;
-    if constexpr (!PV) {
-      if (strided)
-        return bias ? launch<T, DP, false, true, true>(prm, g, stream) : launch<T, DP, false, false, true>(prm, g, stream);
-    }
+    if (strided)
+      return bias ? launch<T, DP, PV, true, true>(prm, g, stream) : launch<T, DP, PV, false, true>(prm, g, stream);
     return bias ? launch<T, DP, PV, true, false>(prm, g, stream) : launch<T, DP, PV, false, false>(prm, g, stream);
   };
   using I32 = std::integral_constant<int, 32>;

@@ -170,8 +170,8 @@ def _operand_views(q, k1, v1, k2, v2, cdt, excluded: bool):
     """The (q, k/v) {batch, head, token} element strides when the five [B, H, N, D] operands can be read
     in place by the pair kernel (views such as the chunks of an in_proj output), else None (the operands
     are then copied to the contiguous layout).  The pair kernel takes 16-bit operands already in the
-    compute dtype, head_dim <= 64 and a multiple of 8, tokens <= 512, no pair_valid and no angle or message
-    term (`excluded`), unit-stride d, strides that are multiples of 8 elements below 2^31 and 16-byte
+    compute dtype, head_dim <= 64 and a multiple of 8, tokens <= 512, no angle or message term
+    (`excluded`), unit-stride d, strides that are multiples of 8 elements below 2^31 and 16-byte
     aligned bases; k1, v1, k2 and v2 share strides."""
     B, H, N, D = q.shape
     if excluded or cdt not in (torch.float16, torch.bfloat16) or D % 8 != 0 or D > 64 or N > 512:
@@ -240,7 +240,7 @@ def hip_simplicial_attention_forward(
 
     cdt = _compute_dtype(q.dtype, precision)
     views = _operand_views(q, k1, v1, k2, v2, cdt,
-                           angle_left is not None or message_left is not None or pair_valid is not None)
+                           angle_left is not None or message_left is not None)
     if views is not None:
         ops = [q, k1, v1, k2, v2]
         q_stride, kv_stride = views
@@ -253,7 +253,7 @@ def hip_simplicial_attention_forward(
 
     out_direct = q.dtype == cdt
     out_stride = (0, 0, 0)
-    if views is not None:
+    if views is not None and pair_valid is None:
         # written in the merged [B, N, H, D] layout that _merge_heads / out_proj read, returned as its
         # [B, H, N, D] view
         out = torch.empty((B, N, H, D), device=q.device, dtype=q.dtype).permute(0, 2, 1, 3)
@@ -288,7 +288,9 @@ def hip_simplicial_attention_forward(
         **ext.fields(),
     )
     with torch.cuda.device(q.device):
-        status = lib.mf_simplicial_fwd(args, _native.current_stream(q.device))
+        # (views with pair_valid: their own entry, the five copies of a small call took a fifth of it)
+        fwd = lib.mf_simplicial_fwd if views is None or pv is None else lib.mf_simplicial_fwd_views
+        status = fwd(args, _native.current_stream(q.device))
     _native.check(status, "mf_simplicial_fwd")
     if out is None:
         out = out_f32.to(q.dtype)

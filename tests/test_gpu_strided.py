@@ -221,3 +221,35 @@ def test_views_with_pair_valid_fall_back_to_copies():
     status = lib.mf_simplicial_fwd(args, _native.current_stream(DEV))
     assert status == _native.MF_ERR_UNSUPPORTED
     assert b"no pair_valid" in lib.mf_last_error()
+
+
+@pytest.mark.parametrize("bias_dtype", [None, torch.float32, torch.bfloat16], ids=["none", "fp32", "bf16"])
+@pytest.mark.parametrize("B,H,N,D", [(1, 1, 2, 64), (3, 4, 45, 64), (2, 2, 90, 32), (2, 2, 130, 64)])
+def test_views_with_pair_valid_match_contiguous_bitwise(B, H, N, D, bias_dtype):
+    """pair_valid beside strided operands, through one and several key blocks; the output stays contiguous."""
+    q, k1, v1, k2, v2 = _views(B, H, N, D, torch.bfloat16, seed=N)
+    qv, pkv = _masks(B, N, seed=N, holes=N > 2)
+    gen = torch.Generator().manual_seed(N + 1)
+    pv = ((torch.rand(B, N, N, generator=gen) < 0.8) | torch.eye(N, dtype=torch.bool)).to(DEV)
+    kw = dict(query_valid=qv, pair_key_valid=pkv, pair_valid=pv, precision="bf16_tc")
+    if bias_dtype is not None:
+        u, vb, w, gate = ((torch.randn(s, generator=gen) * 0.5).to(DEV, bias_dtype)
+                          for s in [(B, H, N, N)] * 3 + [(B, H, N)])
+        kw.update(u=u, v_bias=vb, w=w, gate=gate)
+    out_v, lse_v, o32_v = hip_simplicial_attention_forward(q, k1, v1, k2, v2, **kw)
+    out_c, lse_c, o32_c = hip_simplicial_attention_forward(*(t.contiguous() for t in (q, k1, v1, k2, v2)), **kw)
+    torch.cuda.synchronize()
+    assert out_v.is_contiguous()
+    assert torch.equal(out_v, out_c) and torch.equal(o32_v, o32_c) and torch.equal(lse_v, lse_c)
+
+
+def test_capi_base_entry_still_refuses_strides_with_pair_valid():
+    B, H, N, D = 2, 2, 16, 32
+    q = torch.randn(B, H, N, D, device=DEV).to(torch.bfloat16)
+    out = torch.empty_like(q)
+    lib, args, keep = _capi_args(q, (H * N * D, N * D, D), out, _native.MF_DTYPE_BF16)
+    pv = torch.ones(B, N, N, dtype=torch.bool, device=DEV)
+    args.pair_valid = pv.data_ptr()
+    assert lib.mf_simplicial_fwd(args, _native.current_stream(DEV)) == _native.MF_ERR_UNSUPPORTED
+    assert lib.mf_simplicial_fwd_views(args, _native.current_stream(DEV)) == _native.MF_OK
+    torch.cuda.synchronize()
