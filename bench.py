@@ -752,8 +752,8 @@ def measure_simplicial_extras(lib, w, wd) -> dict:
         "bwd_roofline": {"bound": "mfma", "achieved": round(bwd_flops / (bwd_ms * 1e-3) / 1e12, 3),
                          "peak": BF16_DENSE_PEAK_TFLOPS, "unit": "TFLOP/s",
                          "frac": round(bwd_flops / (bwd_ms * 1e-3) / 1e12 / BF16_DENSE_PEAK_TFLOPS, 5),
-                         "kernel": "mf::pbwd::pair_bwd_kernel (pairs as keys, fp16 operands, LPT plan, large "
-                                   "molecules in two halves) with its plan, combine and zero-rows launches; "
+                         "kernel": "mf::pbwd::pair_bwd_kernel (pairs as keys, fp16 operands, LPT plan, "
+                                   "units of at most 24 j) with its plan, combine and zero-rows launches; "
                                    "deterministic, no atomics",
                          "kernel_ms": round(bwd_ms, 5),
                          "note": "hip_simplicial_attention_backward graph-replayed, bf16 gradients written by the "
@@ -784,7 +784,7 @@ def measure_simplicial_extras(lib, w, wd) -> dict:
     bias_bwd_eager_ms, _ = timed_loop(torch.cuda.current_stream(), bias_bwd_step, 10, 2)
     bias_bwd_ms = _graph_ms(bias_bwd_step, per_graph=10, replays=5)
     res["bias_bwd"] = {"ms": round(bias_bwd_ms, 5), "eager_ms": round(bias_bwd_eager_ms, 5),
-                       "kernel": "mf::pbwd::pair_bwd_kernel<bias=1> (query tiles in passes of at most three) with "
+                       "kernel": "mf::pbwd::pair_bwd_kernel<bias=1> (block triples of 48 / 16 / 48 rows) with "
                                  "its plan, combine, bias finish and clearing launches; dq, dk1, dv1, dk2, dv2, du, "
                                  "dv_bias, dw, dgate in bf16, written in full"}
 
