@@ -259,6 +259,13 @@ int mf_simplicial_bwd(const mf_simplicial_bwd_args* args, void* stream);
 /* nothing launched, otherwise.                                             */
 int mf_simplicial_bwd_leaf(const mf_simplicial_bwd_args* args, void* stream);
 
+/* 1 if mf_simplicial_bwd on these arguments (grads_dtype MF_DTYPE_F32)      */
+/* writes every element of the fp32 gradients itself, zeros where an index   */
+/* is padded, so that the buffers need no fill; 0 if the caller zero-fills   */
+/* them.  Looks at sizes, types and pointers' alignment only; launches       */
+/* nothing.                                                                  */
+int mf_simplicial_bwd_writes_all(const mf_simplicial_bwd_args* args);
+
 /* Bytes of workspace the backward uses (0: none).  With a message term, per */
 /* query the message coefficients dc = basis . go and sum_jk P ML MR; at     */
 /* head_dim 64, the pair kernel's plan and partial sums (a smaller or NULL   */

@@ -1291,6 +1291,10 @@ extern "C" int mf_simplicial_bwd(const mf_simplicial_bwd_args* a, void* stream) 
   return simplicial_bwd_impl(a, false, stream);
 }
 
+extern "C" int mf_simplicial_bwd_writes_all(const mf_simplicial_bwd_args* a) {
+  return a != nullptr && mf::simplicial_pair_f32_bwd_serves(a) ? 1 : 0;
+}
+
 extern "C" int mf_simplicial_bwd_leaf(const mf_simplicial_bwd_args* a, void* stream) {
   if (a != nullptr && (a->grads_dtype != MF_DTYPE_BF16 || a->bias_u == nullptr || a->bias_dtype != MF_DTYPE_F32))
     return mf::fail(MF_ERR_INVALID_ARGUMENT, "mf_simplicial_bwd_leaf: grads_dtype must be MF_DTYPE_BF16 and the bias MF_DTYPE_F32");

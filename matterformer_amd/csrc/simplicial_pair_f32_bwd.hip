@@ -399,6 +399,37 @@ __device__ __forceinline__ void body(const Params& p, Lds& L, LdsBias* X, int nk
   }
 }
 
+// Zeros at the padded entries of the gradients (mk, mq: valid keys and queries), so that the caller needs no fill:
+// five launches, nine with a bias (forward and backward of 128 molecules of up to 29 atoms, 8 heads of 32: 138 -> 122
+// us).  Called after the
+// operand loads have arrived: a load that waits behind stores waits for them too.
+template <bool BIAS>
+__device__ __forceinline__ void zero_padding(const Params& p, unsigned long long mk, unsigned long long mq, size_t rbase) {
+  const int N = p.N, D = p.D;
+  const int row = threadIdx.x / (DP / 4), c = 4 * (threadIdx.x % (DP / 4));
+  if (row < N && c < D) {
+    const size_t o = (rbase + row) * D + c;
+    if (!((mq >> row) & 1u)) *reinterpret_cast<float4*>(p.dq + o) = float4{0.f, 0.f, 0.f, 0.f};
+    if (!((mk >> row) & 1u)) {
+      *reinterpret_cast<float4*>(p.dk2 + o) = float4{0.f, 0.f, 0.f, 0.f};
+      *reinterpret_cast<float4*>(p.dv2 + o) = float4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) p.dk1[o + e] = p.dv1[o + e] = 0.0f;  // (these two may be unaligned)
+    }
+  }
+  if constexpr (BIAS) {
+    for (int u = threadIdx.x; u < N * N; u += kThreads) {
+      const int a = u / N, e = u % N;
+      const size_t o = rbase * N + u;
+      const bool k = (mk >> e) & 1u, q = k && ((mq >> a) & 1u), j = k && ((mk >> a) & 1u);
+      if (p.du != nullptr && !q) p.du[o] = 0.0f;
+      if (p.dvb != nullptr && !q) p.dvb[o] = 0.0f;
+      if (p.dw != nullptr && !j) p.dw[o] = 0.0f;
+    }
+    if (p.dgate != nullptr && int(threadIdx.x) < N && !((mq >> threadIdx.x) & 1u)) p.dgate[rbase + threadIdx.x] = 0.0f;
+  }
+}
+
 template <bool BIAS>
 __global__ void __launch_bounds__(kThreads, 2) pair_f32_bwd_kernel(Params p) {
   __shared__ __attribute__((aligned(16))) Lds L;
@@ -412,7 +443,10 @@ __global__ void __launch_bounds__(kThreads, 2) pair_f32_bwd_kernel(Params p) {
   const bool vq = lane < N && p.qv[size_t(b) * N + min(lane, N - 1)] != 0;
   const unsigned long long mk = __ballot(vk), mq = __ballot(vq);
   const int nk = __popcll(mk), nq = __popcll(mq);
-  if (nk == 0 || nq == 0) return;
+  if (nk == 0 || nq == 0) {  // no pair or no query: every gradient is zero
+    zero_padding<BIAS>(p, 0ull, 0ull, rbase);
+    return;
+  }
   const unsigned long long below = (1ull << lane) - 1ull;
   if (vk) L.kidx[__popcll(mk & below)] = lane;  // (every wave writes the same lists)
   if (vq) L.qidx[__popcll(mq & below)] = lane;
@@ -473,6 +507,7 @@ __global__ void __launch_bounds__(kThreads, 2) pair_f32_bwd_kernel(Params p) {
     }
   }
   __syncthreads();
+  zero_padding<BIAS>(p, mk, mq, rbase);
   if (nq > 16) {
     if (nk > 16) body<2, 2, BIAS>(p, L, X, nk, nq, rbase);
     else body<2, 1, BIAS>(p, L, X, nk, nq, rbase);

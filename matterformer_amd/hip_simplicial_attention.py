@@ -399,7 +399,8 @@ def _kernel_backward(grad_out, q, k1, v1, k2, v2, out, lse, query_valid, pair_ke
                           message_left, message_right, message_basis)
     # bf16 operands, grad_out and leaves, no low-rank term: the library writes every element of bf16 gradients (no
     # fill, no cast); so it does for an fp32 bias in the pair kernel's range (64 molecules of 44 atoms padded to
-    # 181, 8 heads: 495 -> 406 us); otherwise fp32 gradients, zero-filled here and cast to the leaves' dtypes
+    # 181, 8 heads: 495 -> 406 us); otherwise fp32 gradients, cast to the leaves' dtypes, zero-filled here
+    # unless the library writes every element of those too (fp32 calls of small molecules)
     g16 = (dt == torch.bfloat16 and gdt == torch.bfloat16 and ext.angle is None and ext.message is None
            and D % 8 == 0 and N <= 4096 and all(t.dtype == torch.bfloat16 for t in (q, k1, v1, k2, v2)))
     leaf = False
@@ -407,17 +408,13 @@ def _kernel_backward(grad_out, q, k1, v1, k2, v2, out, lse, query_valid, pair_ke
         g16 = leaf = (allow_leaf and D == 64 and N <= 512
                       and all(t.dtype == torch.float32 for t in (u, v_bias, w, gate)))
     bdt = torch.float32 if leaf else torch.bfloat16
-    if g16:
-        grads = [torch.empty(B, H, N, D, device=dev, dtype=torch.bfloat16) for _ in range(5)]
-    else:
-        grads = [torch.zeros(B, H, N, D, device=dev, dtype=torch.float32) for _ in range(5)]
+    grads = [torch.empty(B, H, N, D, device=dev, dtype=torch.bfloat16 if g16 else torch.float32) for _ in range(5)]
     bias_grads = [None] * 4
     if ext.bias is not None:
         for idx, (name, shape) in enumerate((("need_du", (B, H, N, N)), ("need_dv_bias", (B, H, N, N)),
                                              ("need_dw", (B, H, N, N)), ("need_dgate", (B, H, N)))):
             if flags[name]:
-                bias_grads[idx] = (torch.empty(shape, device=dev, dtype=bdt) if g16 else
-                                   torch.zeros(shape, device=dev, dtype=torch.float32))
+                bias_grads[idx] = torch.empty(shape, device=dev, dtype=bdt if g16 else torch.float32)
     # low-rank gradients: (dangle_left, dangle_right, dangle_gate), (dmessage_left, dmessage_right, dmessage_basis)
     lr_grads: list[torch.Tensor | None] = [None] * 6
     if ext.angle is not None:
@@ -459,6 +456,10 @@ def _kernel_backward(grad_out, q, k1, v1, k2, v2, out, lse, query_valid, pair_ke
         dmessage_right=_native.ptr(lr_grads[4]), dmessage_basis=_native.ptr(lr_grads[5]),
         workspace=_native.ptr(workspace), workspace_bytes=0 if workspace is None else workspace.numel())
     lib = _native.lib()
+    if not g16 and not lib.mf_simplicial_bwd_writes_all(args):
+        for t in (*grads, *bias_grads):
+            if t is not None:
+                t.zero_()
     with torch.cuda.device(dev):
         status = (lib.mf_simplicial_bwd_leaf if leaf else lib.mf_simplicial_bwd)(args, _native.current_stream(dev))
     if status == _native.MF_ERR_UNSUPPORTED:

@@ -71,3 +71,62 @@ def test_large_and_masking_scale_logits(cuda):
     assert torch.equal(out, out32)
     assert not out[2:].any() and not lse[2:].any()
     assert not out[1, :, 20:].any() and not lse[1, :, 20:].any()
+
+
+@pytest.mark.parametrize("wanted", [(True, True, True, True), (False, True, False, False)], ids=["all", "dv"])
+@pytest.mark.parametrize("counts,N,D", [([1, 3], 4, 4), ([16, 9, 0], 17, 20), ([32, 5], 32, 32), ([29, 12], 29, 32)])
+def test_gradients_are_written_in_full(cuda, counts, N, D, wanted):
+    """Over buffers that held NaN, every padded entry of the fp32 gradients is zero and the others are those of the
+    same call into zero-filled buffers, bit for bit (the sums do not depend on what the buffers held); queries and
+    keys padded differently, a molecule without either."""
+    import matterformer_amd.hip_simplicial_attention as hsa
+
+    B, H = len(counts), 2
+    q, k1, v1, k2, v2, qv, pkv, _ = random_simplicial(B, H, N, D, seed=N, counts=counts, std=logit_std(D))
+    qv = qv.clone()
+    qv[0, counts[0] // 2:] = False
+    if B > 1:
+        qv[1, 0] = True  # a query past the keys' count too when there are no keys
+    gen = torch.Generator().manual_seed(N)
+    ops = [t.to(cuda) for t in (q, k1, v1, k2, v2)]
+    go = torch.randn(B, H, N, D, generator=gen).to(cuda)
+    bias = [torch.randn(s, generator=gen).to(cuda) for s in [(B, H, N, N)] * 3 + [(B, H, N)]]
+    masks = (qv.to(cuda), pkv.to(cuda), None)
+    kw = dict(zip(("query_valid", "pair_key_valid", "pair_valid"), masks))
+    flags = dict.fromkeys([f"need_d{n}" for n in ("u", "v_bias", "w", "gate", "angle_left", "angle_right", "angle_gate",
+                                                  "message_left", "message_right", "message_basis")], False)
+    flags.update(zip(("need_du", "need_dv_bias", "need_dw", "need_dgate"), wanted))
+    for b in (bias, [None] * 4):
+        _, lse, out32 = hip_simplicial_attention_forward(*ops, **kw, u=b[0], v_bias=b[1], w=b[2], gate=b[3],
+                                                         precision="ieee_fp32")
+        call = (go, *ops, out32, lse, *masks, *b, *[None] * 6, flags)
+        results = []
+        for fill in (0.0, float("nan")):
+            real = torch.empty
+            with pytest.MonkeyPatch.context() as mp:
+                mp.setattr(hsa.torch, "empty", lambda *a, **k: real(*a, **k).fill_(fill)
+                           if k.get("dtype") == torch.float32 else real(*a, **k))
+                results.append(hsa._kernel_backward(*call))
+        for want, got in zip(*results):
+            assert (got is None) == (want is None)
+            if got is not None:
+                assert torch.equal(got, want)
+        qp, kp = ~masks[0][:, None, :].expand(B, H, N), ~masks[1][:, None, :].expand(B, H, N)
+        for g, pad in zip(results[1][:5], (qp, kp, kp, kp, kp)):
+            assert not g[pad].any()
+
+
+def test_writes_all_follows_the_route():
+    """Only calls of the small fp32 kernel report that they write every element."""
+    from matterformer_amd import _native
+
+    lib = _native.lib()
+    names = ("q", "k1", "v1", "k2", "v2", "grad_out", "out", "lse", "query_valid", "pair_key_valid", "dq", "dk1",
+             "dv1", "dk2", "dv2")
+    base = dict.fromkeys(names, 4096) | dict(batch=2, heads=2, tokens=32, head_dim=32, dtype=_native.MF_DTYPE_F32,
+                                             grad_dtype=_native.MF_DTYPE_F32, grads_dtype=_native.MF_DTYPE_F32)
+    for change, want in ((dict(), 1), (dict(tokens=33), 0), (dict(head_dim=36), 0), (dict(head_dim=30), 0),
+                         (dict(dtype=_native.MF_DTYPE_BF16), 0), (dict(grad_dtype=_native.MF_DTYPE_BF16), 0),
+                         (dict(dq=4100), 0), (dict(dk1=4100, dv1=4100), 1), (dict(angle_left=4096), 0),
+                         (dict(message_left=4096), 0), (dict(dv2=None), 0)):
+        assert lib.mf_simplicial_bwd_writes_all(_native.MfSimplicialBwdArgs(**(base | change))) == want, change
