@@ -7,7 +7,7 @@
 // kernel (simplicial_fwd.hip) gives every query its own nk x nk slab of 16 x 16
 // tiles.  Everything is fp32: fp32 MFMA 16x16x4, fp32 softmax and sums.
 //
-//   S^T[pair][query] = sum_d W[pair][d] (q log2 e)[query][d]   pairs (j, k0 + 0..15), A = W formed in
+//   S^T[pair][query] = sum_d W[pair][d] q[query][d]   pairs (j, k0 + 0..15), A = W formed in
 //       registers; the K index of step c of lane group g is d = (DP / 4) g + c, so a lane's d are
 //       contiguous in LDS
 //   O^T[d][query]   += sum_pair Z[pair][d] P[pair][query]      accumulator r of S^T (pair 4 g + r) is the
@@ -148,14 +148,22 @@ __device__ __forceinline__ void pair_loop(const float* smem, const unsigned long
 #pragma unroll
         for (int t = 0; t < NT; ++t) uj[t] = uT[j * UI + 16 * t + r16];
       }
-      mf_f32x4 s[NT];
+      // natural logits, in two chains of NC / 2 steps: log2 e enters with the offset, in one fma, and not as a
+      // rounding of every q
+      mf_f32x4 s[NT], sb[NT];
 #pragma unroll
-      for (int t = 0; t < NT; ++t) s[t] = mf_f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int t = 0; t < NT; ++t) s[t] = sb[t] = mf_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        s[0] = mma(wz[c], qf[0][c], s[0]);
-        if constexpr (NT > 1) s[1] = mma(wz[c], qf[1][c], s[1]);
-      }
+      for (int c = 0; c < NC / 2; ++c)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          s[t] = mma(wz[c], qf[t][c], s[t]);
+          sb[t] = mma(wz[NC / 2 + c], qf[t][NC / 2 + c], sb[t]);
+        }
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s[t][r] += sb[t][r];
       if constexpr (BIAS) {
         const float wk[4] = {w4.x, w4.y, w4.z, w4.w};
 #pragma unroll
@@ -177,12 +185,12 @@ __device__ __forceinline__ void pair_loop(const float* smem, const unsigned long
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
         top[t] = fmaxf(fmaxf(s[t][0], s[t][1]), fmaxf(s[t][2], s[t][3]));
-        over = over || top[t] > M[t] + kRescaleSlack;
+        over = over || fmaf(top[t], kLog2e, -M[t]) > kRescaleSlack;
       }
       if (__any(over)) {
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-          const float x = max_groups(top[t]);
+          const float x = max_groups(top[t]) * kLog2e;
           if (x > M[t] + kRescaleSlack) {
             const float alpha = M[t] == -INFINITY ? 0.0f : fast_exp2(M[t] - x);
             M[t] = x;
@@ -198,30 +206,30 @@ __device__ __forceinline__ void pair_loop(const float* smem, const unsigned long
       for (int t = 0; t < NT; ++t) {
         const float m = M[t] == -INFINITY ? 0.0f : M[t];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) s[t][r] = fast_exp2(s[t][r] - m);
+        for (int r = 0; r < 4; ++r) s[t][r] = fast_exp2(fmaf(s[t][r], kLog2e, -m));
         lsum[t] += (s[t][0] + s[t][1]) + (s[t][2] + s[t][3]);
       }
-      // the tile's 16 pairs are summed on their own, then added: sums of 16 and of the wave's tiles, not one long
-      // chain (error against 64 bits 1.2e-7 instead of 1.8e-7, at no measured cost)
-      mf_f32x4 ot[NT][ND];
+      // the tile's pairs are summed on their own, in two chains of 8, then added: not one long chain (error against
+      // 64 bits 1.13e-7 instead of 1.8e-7, 1.2e-7 with one chain of 16 and one of logits, at no measured cost)
+      mf_f32x4 ot[2][NT][ND];
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int dt = 0; dt < ND; ++dt) ot[t][dt] = mf_f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int dt = 0; dt < ND; ++dt) ot[0][t][dt] = ot[1][t][dt] = mf_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int r = 0; r < 4; ++r)
 #pragma unroll
         for (int dt = 0; dt < ND; ++dt) {
           const float z = v1[dt] * v2[r][dt];
 #pragma unroll
-          for (int t = 0; t < NT; ++t) ot[t][dt] = mma(z, s[t][r], ot[t][dt]);
+          for (int t = 0; t < NT; ++t) ot[r & 1][t][dt] = mma(z, s[t][r], ot[r & 1][t][dt]);
         }
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int dt = 0; dt < ND; ++dt)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) oa[t][dt][r] += ot[t][dt][r];
+          for (int r = 0; r < 4; ++r) oa[t][dt][r] += ot[0][t][dt][r] + ot[1][t][dt][r];
     }
   }
 }
@@ -320,7 +328,7 @@ __global__ void __launch_bounds__(kThreads, DP == 32 ? 4 : 2) simplicial_pair_f3
       wS[j * (NP + 4) + k] = load_any(p.w, (rbase + s_k[j]) * N + s_k[min(k, nk - 1)], p.bias_dtype);
     }
   }
-  // ---- the queries' operand: q log2 e of query 16 t + r16 at d = NC g + c (zero past nqb and D) ----
+  // ---- the queries' operand: q of query 16 t + r16 at d = NC g + c (zero past nqb and D) ----
   float qf[QT][NC], gq[QT];
 #pragma unroll
   for (int t = 0; t < QT; ++t) {
@@ -330,13 +338,13 @@ __global__ void __launch_bounds__(kThreads, DP == 32 ? 4 : 2) simplicial_pair_f3
     for (int c = 0; c < NC; c += 4) {
       const int d = NC * g + c;
       const float4 x = *reinterpret_cast<const float4*>(p.q + row * D + min(d, D - 4));
-      const float f = i < nqb && d < D ? kLog2e : 0.0f;
-      qf[t][c] = i < nqb && d < D ? x.x * f : 0.0f;
-      qf[t][c + 1] = i < nqb && d < D ? x.y * f : 0.0f;
-      qf[t][c + 2] = i < nqb && d < D ? x.z * f : 0.0f;
-      qf[t][c + 3] = i < nqb && d < D ? x.w * f : 0.0f;
+      const bool on = i < nqb && d < D;
+      qf[t][c] = on ? x.x : 0.0f;
+      qf[t][c + 1] = on ? x.y : 0.0f;
+      qf[t][c + 2] = on ? x.z : 0.0f;
+      qf[t][c + 3] = on ? x.w : 0.0f;
     }
-    gq[t] = BIAS ? load_any(p.gate, row, p.bias_dtype) * kLog2e : 0.0f;
+    gq[t] = BIAS ? load_any(p.gate, row, p.bias_dtype) : 0.0f;
   }
   __syncthreads();
 
