@@ -77,8 +77,11 @@
 //     exact (the product of two bf16 values has at most 16 significant
 //     bits), since dP - go . out cancels when one pair dominates the softmax
 //     (the reference's dP contraction is fp32, :611-645);
-//   dS (scaled by 2^-es, es chosen from the operand scales so that
-//     |dS| < 2^15 always) and P as MFMA operands: rounded once to fp16;
+//   dS (scaled by 2^-es) and P as MFMA operands: rounded once to fp16.  es is
+//     chosen per block triple so that |dS 2^-es| < 2^15 P: from the scales of
+//     go, v1 and v2, which bound |dP| in the block, and from the largest
+//     |go . out| of its queries, which sums over every key of the molecule
+//     and may be far larger;
 //   softmax, dS, every accumulator and every bias sum fp32; the scales are
 //   undone, exactly, before block triples are added.
 //
@@ -258,9 +261,19 @@ __device__ __forceinline__ uint32_t absmax_bits8(const uint4 r) {
   return max(a, b);
 }
 
-// Exponent of the largest magnitude (its bf16 pattern), 0 for an all-zero operand: scaling by 2^-e puts the
+// Exponent of the largest magnitude (its bf16 pattern), -127 for an all-zero operand: scaling by 2^-e puts the
 // largest magnitude in [1, 2).
-__device__ __forceinline__ int scale_exp(uint32_t bits) { return bits == 0u ? 0 : int((bits >> 7) & 0xffu) - 127; }
+__device__ __forceinline__ int scale_exp(uint32_t bits) { return int((bits >> 7) & 0xffu) - 127; }
+
+// 2^e for a uniform e (held to the normal range), by scalar operations.
+__device__ __forceinline__ float pow2(int e) { return __uint_as_float(uint32_t(min(max(e, -126), 127) + 127) << 23); }
+
+// The exponent of dS, dS 2^-es in fp16.  dP is a sum of 64 products of magnitude below 2^(eg + f1 + f2 + 3), so
+// |dP 2^-es| < 2^14 from es = eg + f1 + f2 - 5 on; |go . out| < 2^(ed + 1) needs es = ed - 13 for the same bound.
+// Held where 2^-es and 2^es are finite (gradients past either end leave the fp32 range themselves).
+__device__ __forceinline__ int ds_exp(int eg, int f1, int f2, int ed) {
+  return min(max(max(eg + f1 + f2 - 5, ed - 13), -110), 110);
+}
 
 // Eight bf16 times 2^-e (exact) as fp16 (exact in the normal fp16 range).
 __device__ __forceinline__ uint4 to_f16x8(const uint4 r, float scale) {
@@ -489,7 +502,7 @@ __device__ __forceinline__ int opaque_tid() {
 // (compacted positions), the scale exponents of its operands.
 struct Triple {
   int bh, part, q0, nq, j0, nj, k0, nk;
-  int eq, eg, e1, e2, f1, f2;       // exponents of q, go, k1, k2, v1, v2
+  int eq, eg, e1, e2, f1, f2, ed;   // exponents of q, go, k1, k2, v1, v2 and of the largest |go . out|
   bool direct;                      // the molecule's only triple: gradients written here, not to the slab
   bool first_q, first_k;            // the unit's first triple with these queries (dq) / these keys (dk2, dv2)
   bool first_t;                     // the unit's first triple with these (queries, keys): dv_bias
@@ -559,11 +572,11 @@ __device__ __forceinline__ void triple_body(const Params& p, unsigned char* smem
   const uint32_t* pvb = reinterpret_cast<const uint32_t*>(smem + Ly::pvb);
   const int* kidx = reinterpret_cast<const int*>(smem + Ly::kidx);
   const int* qidx = reinterpret_cast<const int*>(smem + Ly::qidx);
-  // dS is carried as dS 2^-es, |dS 2^-es| < 2^15:  S log2 e = S_c cS,  dS 2^-es = P (dP_c cP - delta 2^-es)
-  const int es = c.eg + c.f1 + c.f2 - 5;
+  // dS is carried as dS 2^-es, |dS 2^-es| < 2^15 P:  S log2 e = S_c cS,  dS 2^-es = P (dP_c cP - delta 2^-es)
+  const int es = ds_exp(c.eg, c.f1, c.f2, c.ed);
   const float cS = ldexpf(kLog2e, c.eq + c.e1 + c.e2);
-  constexpr float cP = 32.0f;  // 2^(eg + f1 + f2 - es)
-  const float uD = ldexpf(1.0f, es);
+  const float cP = pow2(c.eg + c.f1 + c.f2 - es);
+  const float uD = pow2(es);
   const float fk1 = ldexpf(1.0f, c.e2 + es + c.eq), fv1 = ldexpf(1.0f, c.f2 + c.eg);
 
   const int nkt = (c.nk + 15) / 16;
@@ -1025,23 +1038,38 @@ __global__ void __launch_bounds__(kThreads, 2) pair_bwd_kernel(Params p) {
           }
           if (r0 + 32 * i >= c.nk) b2[i] = d2[i] = zero;
         }
-        // largest magnitude of each operand over the block: per thread, per wave, then over the four waves
-        uint32_t mx[6] = {max(absmax_bits8(bq[0]), absmax_bits8(bq[1])), max(absmax_bits8(bg[0]), absmax_bits8(bg[1])),
-                          absmax_bits8(b1), max(absmax_bits8(b2[0]), absmax_bits8(b2[1])), absmax_bits8(d1),
-                          max(absmax_bits8(d2[0]), absmax_bits8(d2[1]))};
+        // go . out of the thread's query rows (in the eight threads of a row)
+        float go[2];
 #pragma unroll
-        for (int t = 0; t < 6; ++t) {
+        for (int i = 0; i < 2; ++i) {
+          float s = bf_lo(bg[i].x) * o0[i].x;
+          s = fmaf(bf_hi(bg[i].x), o0[i].y, s); s = fmaf(bf_lo(bg[i].y), o0[i].z, s);
+          s = fmaf(bf_hi(bg[i].y), o0[i].w, s); s = fmaf(bf_lo(bg[i].z), o1[i].x, s);
+          s = fmaf(bf_hi(bg[i].z), o1[i].y, s); s = fmaf(bf_lo(bg[i].w), o1[i].z, s);
+          s = fmaf(bf_hi(bg[i].w), o1[i].w, s);
+          go[i] = sum8(s);
+        }
+        // largest magnitude of each operand over the block, and of go . out (its bf16 bits: the exponent is what
+        // counts, one that is not finite leaves the others' scale alone): per thread, per wave, then over the four waves
+        const uint32_t da = __float_as_uint(go[0]) << 1 >> 17, db = __float_as_uint(go[1]) << 1 >> 17;
+        uint32_t mx[7] = {max(absmax_bits8(bq[0]), absmax_bits8(bq[1])), max(absmax_bits8(bg[0]), absmax_bits8(bg[1])),
+                          absmax_bits8(b1), max(absmax_bits8(b2[0]), absmax_bits8(b2[1])), absmax_bits8(d1),
+                          max(absmax_bits8(d2[0]), absmax_bits8(d2[1])),
+                          max(da < 0x7f80u ? da : 0u, db < 0x7f80u ? db : 0u)};
+#pragma unroll
+        for (int t = 0; t < 7; ++t) {
           mx[t] = wave_max_u32(mx[t]);
           if (lane == 0) red[wave * 8 + t] = mx[t];
         }
         lds_barrier();
-        int ex[6];
+        int ex[7];
 #pragma unroll
-        for (int t = 0; t < 6; ++t)
+        for (int t = 0; t < 7; ++t)
           ex[t] = __builtin_amdgcn_readfirstlane(scale_exp(max(max(red[t], red[8 + t]), max(red[16 + t], red[24 + t]))));
         if (do_q) {
           c.eq = ex[0];
           c.eg = ex[1];
+          c.ed = ex[6];
         }
         if (do_j) {
           c.e1 = ex[2];
@@ -1051,24 +1079,18 @@ __global__ void __launch_bounds__(kThreads, 2) pair_bwd_kernel(Params p) {
           c.e2 = ex[3];
           c.f2 = ex[5];
         }
-        const float dscale = ldexpf(1.0f, -(c.eg + c.f1 + c.f2 - 5));
+        const float dscale = pow2(-ds_exp(c.eg, c.f1, c.f2, c.ed));
         if (do_q) {
           const float sq = ldexpf(1.0f, -ex[0]), sg = ldexpf(1.0f, -ex[1]);
 #pragma unroll
           for (int i = 0; i < 2; ++i) {
             const int r = r0 + 32 * i;
-            float s = bf_lo(bg[i].x) * o0[i].x;
-            s = fmaf(bf_hi(bg[i].x), o0[i].y, s); s = fmaf(bf_lo(bg[i].y), o0[i].z, s);
-            s = fmaf(bf_hi(bg[i].y), o0[i].w, s); s = fmaf(bf_lo(bg[i].z), o1[i].x, s);
-            s = fmaf(bf_hi(bg[i].z), o1[i].y, s); s = fmaf(bf_lo(bg[i].w), o1[i].z, s);
-            s = fmaf(bf_hi(bg[i].w), o1[i].w, s);
-            s = sum8(s);
             if (r < QM) {
               *reinterpret_cast<uint4*>(Qs + r * KS + 8 * ch) = to_f16x8(bq[i], sq);
               *reinterpret_cast<uint4*>(Gs + r * KS + 8 * ch) = to_f16x8(bg[i], sg);
               if (ch == 0) {
-                dlt[r] = r < c.nq ? s : 0.0f;
-                dls[r] = r < c.nq ? s * dscale : 0.0f;
+                dlt[r] = r < c.nq ? go[i] : 0.0f;
+                dls[r] = r < c.nq ? go[i] * dscale : 0.0f;
                 lse2[r] = lv[i];
                 qidx[r] = iq[i];
               }

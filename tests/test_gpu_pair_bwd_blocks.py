@@ -45,6 +45,58 @@ def test_block_edges(cuda, counts, bias_dtype):
         assert torch.isfinite(g).all(), name
 
 
+@pytest.mark.parametrize("factor", [2.0 ** -16, 2.0 ** -40, 0.0], ids=["2^-16", "2^-40", "zero"])
+@pytest.mark.parametrize("bias_dtype", [None, torch.float32], ids=["none", "fp32"])
+@pytest.mark.parametrize("n", [48, 100])
+def test_value_rows_of_one_block_far_below_the_others(cuda, n, bias_dtype, factor):
+    """The first 24 rows of v1 (or of v2) `factor` times the others: go . out, which sums over every key, is then far
+    larger than any dP of a block that holds only such rows, and dS there is -P go . out.  Logits of std 5.7 let some
+    of those pairs weigh in.  Bar: W rounded to fp16 moves a logit by 2^-11 of itself, |S| up to 17 (3 std) with
+    random signs over d (1 / sqrt(3) and less): P off by 3e-3 where it is largest, beside the 1.7e-3 of the results'
+    rounding: 6e-3, the small rows' key gradients by themselves too."""
+    B, H, N, D = 1, 2, n, 64
+    q, k1, v1, k2, v2, qv, pkv, _ = random_simplicial(B, H, N, D, seed=n, counts=[n], std=logit_std(D))
+    q = q * 2.85
+    gen = torch.Generator().manual_seed(n + 1)
+    go = torch.randn(B, H, N, D, generator=gen).to(torch.bfloat16)
+    bias = None
+    if bias_dtype is not None:
+        bias = [torch.randn(B, H, N, N, generator=gen) * 0.5 for _ in range(3)] + [torch.rand(B, H, N, generator=gen)]
+    for small in (1, 2):
+        w1, w2 = v1.clone(), v2.clone()
+        (w1 if small == 1 else w2)[:, :, :24] *= factor
+        ops = [t.to(torch.bfloat16) for t in (q, k1, w1, k2, w2)]
+        _, got = hip_grads([t.to(cuda) for t in ops], qv.to(cuda), pkv.to(cuda), None, go.to(cuda), "bf16_tc",
+                           bias=None if bias is None else [t.to(cuda) for t in bias])
+        _, ref = fp64_grads(ops, qv, pkv, None, go, bias=bias)
+        for name, g, r in zip(GRAD_NAMES, got, ref):
+            g = g.float().cpu().numpy()
+            assert rel_err(g, r) <= 6e-3, (small, name, rel_err(g, r))
+            if name == f"dk{small}":
+                e = rel_err(g[:, :, :24], r[:, :, :24])
+                assert e <= 6e-3, (small, name, "small rows", e)
+
+
+def test_gradients_below_the_fp32_range_are_zero_not_nan(cuda):
+    """go of 1e-6 and v1 of 2^-110: dS is below 2^-126, so dq, dk1 and dk2 vanish; dv1 does not.  (2^-es of such a
+    block, unbounded, is infinite, and infinity times the zeros of dropped pairs was NaN.)"""
+    B, H, N, D = 1, 2, 48, 64
+    q, k1, v1, k2, v2, qv, pkv, pv = random_simplicial(B, H, N, D, seed=9, counts=[48], pair_drop=0.2, std=logit_std(D))
+    pv = pv | (torch.arange(N) < 2)[None, None, :]
+    go = torch.randn(B, H, N, D, generator=torch.Generator().manual_seed(10)) * 1e-6
+    ops = [t.to(torch.bfloat16) for t in (q, k1, v1 * 2.0 ** -110, k2, v2)]
+    go = go.to(torch.bfloat16)
+    _, got = hip_grads([t.to(cuda) for t in ops], qv.to(cuda), pkv.to(cuda), pv.to(cuda), go.to(cuda), "bf16_tc")
+    _, ref = fp64_grads(ops, qv, pkv, pv, go)
+    for name, g, r in zip(GRAD_NAMES, got, ref):
+        g = g.float().cpu()
+        assert torch.isfinite(g).all(), name
+        if name in ("dq", "dk1", "dk2", "dv2"):
+            assert float(g.abs().max()) <= 2.0 ** -110, name
+        else:
+            assert rel_err(g.numpy(), r) <= 4e-3, (name, rel_err(g.numpy(), r))
+
+
 def test_queries_and_keys_of_different_counts(cuda):
     """More queries than keys and the reverse (70 / 20 and 20 / 70 valid rows): blocks of one side only."""
     B, H, N, D = 2, 2, 75, 64
