@@ -162,6 +162,7 @@ struct Params {
   int NP;       // N rounded up to 64: LDS list capacity
   int OB;       // workgroups per (b, h, role)
   int vec;      // q/k/v/go/out rows 4-element loads are aligned (D % 4 == 0, aligned bases)
+  int halves;   // fp32 S and dP as two sums of half of d each, as the forward of these calls forms them
   // low-rank terms (LR instantiations): factors [B*H, N, N, R] fp32, gates [B*H, N], basis [H, Rm, D]
   const float* al;
   const float* ar;
@@ -624,14 +625,29 @@ __device__ __forceinline__ void run_role(const Params& p, unsigned char* smem, i
         if (kt < nkt) {
           const float* cs = CS + (kt * 16 + r16) * D4 + 4 * g;
           const float* cp = CP + (kt * 16 + r16) * D4 + 4 * g;
+          mf_f32x4 s1 = sv[kt], d1 = dv[kt];  // halves: the sums of the first half of d
 #pragma unroll
           for (int t = 0; t < NT; ++t) {
+            if constexpr (!LR) {
+              if (t == NT / 2 && p.halves) {  // uniform
+                s1 = sv[kt];
+                d1 = dv[kt];
+                sv[kt] = dv[kt] = mf_f32x4{0.f, 0.f, 0.f, 0.f};
+              }
+            }
             const float4 as = *reinterpret_cast<const float4*>(cs + 16 * t);
             const float4 ap = *reinterpret_cast<const float4*>(cp + 16 * t);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
               sv[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(f4(as, e), f4(rs[t], e) * f4(oS[t], e), sv[kt], 0, 0, 0);
               dv[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(f4(ap, e), f4(rp[t], e) * f4(oP[t], e), dv[kt], 0, 0, 0);
+            }
+          }
+          if constexpr (!LR) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              sv[kt][r] += s1[r];
+              dv[kt][r] += d1[r];
             }
           }
         }
@@ -1211,6 +1227,7 @@ static int simplicial_bwd_impl(const mf_simplicial_bwd_args* a, bool bias32, voi
   vec = vec && reinterpret_cast<uintptr_t>(a->grad_out) % (a->grad_dtype == MF_DTYPE_F32 ? 16 : 8) == 0;
   vec = vec && reinterpret_cast<uintptr_t>(a->out) % 16 == 0;
   prm.vec = vec ? 1 : 0;
+  prm.halves = a->dtype == MF_DTYPE_F32 && a->tokens <= 64 && a->head_dim <= 64 && a->head_dim % 4 == 0 ? 1 : 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const bool has_pv = a->pair_valid != nullptr;
   const int D = a->head_dim;

@@ -199,11 +199,16 @@ __device__ __forceinline__ void body(const Params& p, Lds& L, LdsBias* X, int nk
       const int k0 = 16 * kt;
       const bool ok = (bits >> (k0 + r16)) & 1u;
       // B operands: W, Z of pair (j, k0 + r16) at d = NC g + c
-      mf_f32x4 s[NT], dp[NT];
+      // (two sums of half of d each, S in the forward's own order, so that P = exp(S - lse) is its P)
+      mf_f32x4 sh[2][NT], dph[2][NT], s[NT], dp[NT];
 #pragma unroll
-      for (int t = 0; t < NT; ++t) s[t] = dp[t] = mf_f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int t = 0; t < NT; ++t) sh[0][t] = sh[1][t] = dph[0][t] = dph[1][t] = mf_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int c = 0; c < NC; c += 4) {
+        constexpr int kHalf = NC / 2;
+        static_assert(kHalf % 4 == 0, "whole steps");
+        mf_f32x4(&sc)[NT] = sh[c / kHalf];
+        mf_f32x4(&dc)[NT] = dph[c / kHalf];
         const float4 x = *reinterpret_cast<const float4*>(K2 + (k0 + r16) * KS + NC * g + c);
         const float4 y = *reinterpret_cast<const float4*>(V2 + (k0 + r16) * KS + NC * g + c);
         const float wv[4] = {x.x * k1a[c], x.y * k1a[c + 1], x.z * k1a[c + 2], x.w * k1a[c + 3]};
@@ -213,21 +218,28 @@ __device__ __forceinline__ void body(const Params& p, Lds& L, LdsBias* X, int nk
           for (int t = 0; t < NT; ++t) {
             float4 q4, g4;
             rows_of(t, c, q4, g4);
-            s[t] = mma(q4.x, wv[0], s[t]); dp[t] = mma(g4.x, zv[0], dp[t]);
-            s[t] = mma(q4.y, wv[1], s[t]); dp[t] = mma(g4.y, zv[1], dp[t]);
-            s[t] = mma(q4.z, wv[2], s[t]); dp[t] = mma(g4.z, zv[2], dp[t]);
-            s[t] = mma(q4.w, wv[3], s[t]); dp[t] = mma(g4.w, zv[3], dp[t]);
+            sc[t] = mma(q4.x, wv[0], sc[t]); dc[t] = mma(g4.x, zv[0], dc[t]);
+            sc[t] = mma(q4.y, wv[1], sc[t]); dc[t] = mma(g4.y, zv[1], dc[t]);
+            sc[t] = mma(q4.z, wv[2], sc[t]); dc[t] = mma(g4.z, zv[2], dc[t]);
+            sc[t] = mma(q4.w, wv[3], sc[t]); dc[t] = mma(g4.w, zv[3], dc[t]);
           }
         } else {
 #pragma unroll
           for (int e = 0; e < 4; ++e)
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
-              s[t] = mma(qf[t][c + e], wv[e], s[t]);
-              dp[t] = mma(gf[t][c + e], zv[e], dp[t]);
+              sc[t] = mma(qf[t][c + e], wv[e], sc[t]);
+              dc[t] = mma(gf[t][c + e], zv[e], dc[t]);
             }
         }
       }
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          s[t][r] = sh[0][t][r] + sh[1][t][r];
+          dp[t][r] = dph[0][t][r] + dph[1][t][r];
+        }
       float dwj = 0.0f;
 #pragma unroll
       for (int t = 0; t < NT; ++t) {

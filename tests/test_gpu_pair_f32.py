@@ -45,6 +45,23 @@ def test_fp32_tile_edges(cuda, counts, D, bias_dtype):
         assert rel_err(g.float().cpu().numpy(), r) <= bar, name
 
 
+@pytest.mark.parametrize("n,D,bar", [(29, 32, 7.5e-7), (29, 64, 1.05e-6), (48, 64, 1.1e-6)])
+def test_backward_sums_the_logits_as_the_forward_does(cuda, n, D, bar):
+    """Gradients of calls whose forward runs in pair form, over 8 molecules of 4 heads.  The matrix cores' fp32 sums
+    err to one side along a chain, so lse and the backward's S have to sum in chains of the same length: with S in
+    one chain of D / 4 steps and the forward's lse from two, the errors were 9.5e-7 .. 1.1e-6 (29 tokens, head_dim
+    32), 1.1e-6 .. 1.25e-6 (head_dim 64) and 1.2e-6 .. 1.4e-6 (48, 64).  The rounding of lse (8 .. 9, 2.8e-7 rms), of
+    lse log2 e and of exp2's argument (2e-7 each) make 4e-7, which adds to the chains' 4e-7 at D = 32 and 8e-7 at 64."""
+    B, H = 8, 4
+    q, k1, v1, k2, v2, qv, pkv, _ = random_simplicial(B, H, n, D, seed=n + D, counts=[n] * B, std=logit_std(D))
+    go = torch.randn(B, H, n, D, generator=torch.Generator().manual_seed(D))
+    ops = [q, k1, v1, k2, v2]
+    _, got = hip_grads([t.to(cuda) for t in ops], qv.to(cuda), pkv.to(cuda), None, go.to(cuda), "ieee_fp32")
+    _, ref = fp64_grads(ops, qv, pkv, None, go)
+    for name, g, r in zip(GRAD_NAMES, got, ref):
+        assert rel_err(g.cpu().numpy(), r) <= bar, (name, rel_err(g.cpu().numpy(), r))
+
+
 def test_large_and_masking_scale_logits(cuda):
     """Logits far past the first tile's maximum in both directions (the offset moves many times) and bias terms of
     -30000 beside ordinary ones; padded queries, a molecule without keys and one without queries give zeros."""
