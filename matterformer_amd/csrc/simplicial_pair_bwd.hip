@@ -77,7 +77,11 @@
 //     exact (the product of two bf16 values has at most 16 significant
 //     bits), since dP - go . out cancels when one pair dominates the softmax
 //     (the reference's dP contraction is fp32, :611-645);
-//   dS (scaled by 2^-es) and P as MFMA operands: rounded once to fp16.  es is
+//   dS (scaled by 2^-es) and P (by 2^kPScale) as MFMA operands: rounded once
+//     to fp16, to nearest: a softmax spread over n^2 pairs has P near n^-2,
+//     below fp16's normal range from 128 atoms on, and truncation's one-sided
+//     error does not average out in dv1 and dv2 (512 atoms, flat logits: 8.7e-3
+//     unscaled and truncated, 1.7e-3 so).  es is
 //     chosen per block triple so that |dS 2^-es| < 2^15 P: from the scales of
 //     go, v1 and v2, which bound |dP| in the block, and from the largest
 //     |go . out| of its queries, which sums over every key of the molecule
@@ -107,6 +111,7 @@ constexpr int PS = DP + 4;        // fp32 row stride of the waves' partial sums
 constexpr int kMaxTokens = 512;
 constexpr int kMaxPlanBatch = 2048;
 constexpr int kPlanThreads = 1024;
+constexpr int kPScale = 12;       // P 2^12: exact to fp16's 11 bits down to 2^-26, room to 2^4 above
 
 struct Params {
   const __bf16* q;
@@ -210,7 +215,7 @@ struct Lay {
   static constexpr size_t gt = vt + (BIAS ? size_t(KM) * KU * 4 : 0);           // BIAS: [QM] f32 gate log2 e
   static constexpr size_t lse2 = gt + (BIAS ? QM * 4 : 0);                      // [QM] f32
   static constexpr size_t dlt = lse2 + QM * 4;                                  // [QM] f32 go . out
-  static constexpr size_t dls = dlt + QM * 4;                                   // [QM] f32 go . out 2^-es
+  static constexpr size_t dls = dlt + QM * 4;                                   // [QM] f32 go . out 2^(-es - kPScale)
   static constexpr size_t pvb = dls + QM * 4;                                   // [JM][8] bytes: pair bits
   static constexpr size_t jidx = pvb + JM * 8;                                  // [JM] i32
   static constexpr size_t kidx = jidx + JM * 4;                                 // [KM] i32
@@ -264,6 +269,16 @@ __device__ __forceinline__ uint32_t absmax_bits8(const uint4 r) {
 // Exponent of the largest magnitude (its bf16 pattern), -127 for an all-zero operand: scaling by 2^-e puts the
 // largest magnitude in [1, 2).
 __device__ __forceinline__ int scale_exp(uint32_t bits) { return int((bits >> 7) & 0xffu) - 127; }
+
+typedef __attribute__((__vector_size__(2 * sizeof(float)))) float mf_f32x2;
+typedef __attribute__((__vector_size__(2 * sizeof(_Float16)))) _Float16 mf_f16x2;
+
+// Two fp16, rounded to nearest.
+__device__ __forceinline__ uint32_t pack_f16(float a, float b) {
+  uint32_t r;
+  asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
 
 // 2^e for a uniform e (held to the normal range), by scalar operations.
 __device__ __forceinline__ float pow2(int e) { return __uint_as_float(uint32_t(min(max(e, -126), 127) + 127) << 23); }
@@ -572,12 +587,13 @@ __device__ __forceinline__ void triple_body(const Params& p, unsigned char* smem
   const uint32_t* pvb = reinterpret_cast<const uint32_t*>(smem + Ly::pvb);
   const int* kidx = reinterpret_cast<const int*>(smem + Ly::kidx);
   const int* qidx = reinterpret_cast<const int*>(smem + Ly::qidx);
-  // dS is carried as dS 2^-es, |dS 2^-es| < 2^15 P:  S log2 e = S_c cS,  dS 2^-es = P (dP_c cP - delta 2^-es)
+  // dS is carried as dS 2^-es, |dS 2^-es| < 2^15 P, P as P 2^kPScale (staged with lse):  S log2 e = S_c cS,
+  // dS 2^-es = P 2^kPScale (dP_c cP - delta 2^(-es - kPScale))
   const int es = ds_exp(c.eg, c.f1, c.f2, c.ed);
   const float cS = ldexpf(kLog2e, c.eq + c.e1 + c.e2);
-  const float cP = pow2(c.eg + c.f1 + c.f2 - es);
+  const float cP = pow2(c.eg + c.f1 + c.f2 - es - kPScale);
   const float uD = pow2(es);
-  const float fk1 = ldexpf(1.0f, c.e2 + es + c.eq), fv1 = ldexpf(1.0f, c.f2 + c.eg);
+  const float fk1 = ldexpf(1.0f, c.e2 + es + c.eq), fv1 = ldexpf(1.0f, c.f2 + c.eg - kPScale);
 
   const int nkt = (c.nk + 15) / 16;
   const int njp = (c.nj + 1) / 2;
@@ -667,10 +683,8 @@ __device__ __forceinline__ void triple_body(const Params& p, unsigned char* smem
             dva[t][r] += dsv[r];
           }
         }
-        dsw[jn][t] = uint2{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(dsv[0], dsv[1])),
-                           __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(dsv[2], dsv[3]))};
-        pw[jn][t] = uint2{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(pp[0], pp[1])),
-                          __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(pp[2], pp[3]))};
+        dsw[jn][t] = uint2{pack_f16(dsv[0], dsv[1]), pack_f16(dsv[2], dsv[3])};
+        pw[jn][t] = uint2{pack_f16(pp[0], pp[1]), pack_f16(pp[2], pp[3])};
         // dS [pair (jn, key)][query] into the tile's slot of the wave's scratch
         *reinterpret_cast<uint2*>(scr + t * 32 * SS + (jn * 16 + r16) * SS + 4 * g) = dsw[jn][t];
       };
@@ -821,7 +835,7 @@ __device__ __forceinline__ void triple_body(const Params& p, unsigned char* smem
       lds_barrier();
       const int kk = tid / 16, d4 = 4 * (tid % 16);
       if (k0 + kk < c.nk) {
-        const float4 s = sum_partials(slot, kk, d4, which ? ldexpf(1.0f, c.f1 + c.eg) : ldexpf(1.0f, c.e1 + es + c.eq));
+        const float4 s = sum_partials(slot, kk, d4, which ? ldexpf(1.0f, c.f1 + c.eg - kPScale) : ldexpf(1.0f, c.e1 + es + c.eq));
         if (c.direct) {
           store_grad4(which ? p.dv2 : p.dk2, (rbase + kidx[k0 + kk]) * DP + d4, s, p.gout16);
         } else {
@@ -935,6 +949,9 @@ __global__ void __launch_bounds__(kThreads, 2) pair_bwd_kernel(Params p) {
   int* qidx = reinterpret_cast<int*>(smem + Lk::qidx);
   uint32_t* red = reinterpret_cast<uint32_t*>(smem + Lk::red);
 
+  // FP16_OVFL: fp16 results past the range become the largest fp16 (P where a saturated bias left lse far too small).
+  // (Here, after the addresses: at the kernel's top the bias instantiations spilled 45 registers instead of 16.)
+  asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 23, 1), 1");
   for (int jb = 0; jb < njb; ++jb) {
     c.j0 = ju0 + jb * jrows;
     c.nj = min(ju1 - c.j0, jrows);
@@ -948,7 +965,7 @@ __global__ void __launch_bounds__(kThreads, 2) pair_bwd_kernel(Params p) {
         c.first_k = jb == 0 && qb == 0;
         c.first_t = jb == 0;
         // ---- stage the rows that changed (compacted, zero past the counts) as fp16 scaled by 2^-e per
-        // operand, lse log2 e and go . out of each query (+inf / 0 on the padding rows: P = 0 there).  A
+        // operand, lse log2 e (less kPScale) and go . out of each query (+inf / 0 on the padding rows: P = 0 there).  A
         // thread has a 16-byte piece of row tid / 8 and, for q and k blocks, of row 32 + tid / 8; every
         // global load is issued before the first LDS store, rows past a count load its last row. ----
         const bool do_j = qb == 0 && kb == 0, do_q = kb == 0, do_k = nkb > 1 || do_j;
@@ -979,7 +996,7 @@ __global__ void __launch_bounds__(kThreads, 2) pair_bwd_kernel(Params p) {
             bg[i] = *reinterpret_cast<const uint4*>(p.go + row * DP + 8 * ch);
             o0[i] = *reinterpret_cast<const float4*>(p.out + row * DP + 8 * ch);
             o1[i] = *reinterpret_cast<const float4*>(p.out + row * DP + 8 * ch + 4);
-            lv[i] = p.lse[row] * kLog2e;
+            lv[i] = fmaf(p.lse[row], kLog2e, -float(kPScale));
           }
         }
         if (do_k) {
@@ -1079,7 +1096,7 @@ __global__ void __launch_bounds__(kThreads, 2) pair_bwd_kernel(Params p) {
           c.e2 = ex[3];
           c.f2 = ex[5];
         }
-        const float dscale = pow2(-ds_exp(c.eg, c.f1, c.f2, c.ed));
+        const float dscale = pow2(-ds_exp(c.eg, c.f1, c.f2, c.ed) - kPScale);
         if (do_q) {
           const float sq = ldexpf(1.0f, -ex[0]), sg = ldexpf(1.0f, -ex[1]);
 #pragma unroll

@@ -11,6 +11,10 @@ fp16: 2^-11 of |S| < 4, so P is off by 2e-3 of itself at most, 6e-4 over random 
 import pytest
 import torch
 
+from matterformer_amd.hip_simplicial_attention import (
+    hip_simplicial_attention_backward,
+    hip_simplicial_attention_forward,
+)
 from matterformer_amd.workloads import random_simplicial
 from test_gpu_simplicial_bwd import GRAD_NAMES, fp64_grads, hip_grads, logit_std, rel_err
 
@@ -75,6 +79,40 @@ def test_value_rows_of_one_block_far_below_the_others(cuda, n, bias_dtype, facto
             if name == f"dk{small}":
                 e = rel_err(g[:, :, :24], r[:, :, :24])
                 assert e <= 6e-3, (small, name, "small rows", e)
+
+
+@pytest.mark.parametrize("n", [128, 384, 512])
+def test_flat_softmax_of_a_large_molecule(cuda, n):
+    """Logits of std 0.2 over n^2 pairs: every P is near n^-2 (2^-18 at 512 tokens), below fp16's normal range unless
+    it is scaled, and only rounding to nearest averages out in dv1 and dv2 (unscaled and truncated: 8.7e-3).  Bar:
+    the bf16 result's 1.7e-3 with the fp16 roundings of W, P and dS (2.8e-4 rms each) below it: 2.2e-3.  The float64
+    reference runs on the GPU."""
+    H, D = 1, 64
+    q, k1, v1, k2, v2, *_ = random_simplicial(1, H, n, D, seed=n, counts=[n], std=logit_std(D))
+    go = torch.randn(1, H, n, D, generator=torch.Generator().manual_seed(n)).to(torch.bfloat16).to(cuda)
+    ops = [t.to(torch.bfloat16).to(cuda) for t in (q * 0.1, k1, v1, k2, v2)]
+    valid = torch.ones(1, n, dtype=torch.bool, device=cuda)
+    _, got = hip_grads(ops, valid, valid, None, go, "bf16_tc")
+    leaves = [t[0].double().requires_grad_(True) for t in ops]
+    a, b, c, d, e = leaves
+    logits = torch.matmul((a[:, :, None] * b[:, None]).reshape(H, n * n, D), d.transpose(1, 2).contiguous())
+    p = torch.softmax(logits.view(H, n, n * n), dim=-1).view(H, n * n, n)
+    out = (torch.matmul(p, e).view(H, n, n, D) * c[:, None]).sum(2)
+    for name, g, r in zip(GRAD_NAMES, got, torch.autograd.grad(out, leaves, go[0].double())):
+        assert rel_err(g[0].float().cpu().numpy(), r.cpu().numpy()) <= 2.2e-3, name
+
+
+def test_lse_far_too_small_gives_large_gradients_not_nan(cuda):
+    """A forward that saturated its bias terms returns an lse below the backward's own logits: P up to e^10 leaves
+    fp16, where it becomes the largest fp16."""
+    n = 40
+    q, k1, v1, k2, v2, *_ = random_simplicial(1, 2, n, 64, seed=1, counts=[n], std=logit_std(64))
+    ops = [t.to(torch.bfloat16).to(cuda) for t in (q, k1, v1, k2, v2)]
+    masks = dict.fromkeys(("query_valid", "pair_key_valid"), torch.ones(1, n, dtype=torch.bool, device=cuda))
+    masks["pair_valid"] = None
+    _, lse, out32 = hip_simplicial_attention_forward(*ops, **masks)
+    for g in hip_simplicial_attention_backward(ops[0], *ops, out32, lse - 10.0, **masks)[:5]:
+        assert torch.isfinite(g).all()
 
 
 def test_gradients_below_the_fp32_range_are_zero_not_nan(cuda):
