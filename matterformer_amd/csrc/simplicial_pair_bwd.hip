@@ -666,10 +666,11 @@ __device__ __forceinline__ void triple_body(const Params& p, unsigned char* smem
           const float4 u4 = *reinterpret_cast<const float4*>(uT + (ja + jn) * KU + t * 16 + 4 * g);
           const float4 v4 = *reinterpret_cast<const float4*>(vT + (k0 + r16) * KU + t * 16 + 4 * g);
           cl[0] = c4.x; cl[1] = c4.y; cl[2] = c4.z; cl[3] = c4.w;
-          base[0] = (u4.x + v4.x) + wj;
-          base[1] = (u4.y + v4.y) + wj;
-          base[2] = (u4.z + v4.z) + wj;
-          base[3] = (u4.w + v4.w) + wj;
+          // (0 at a dropped pair: dS is 0 there, but the terms may be -inf or NaN)
+          base[0] = ok[jn] ? (u4.x + v4.x) + wj : 0.0f;
+          base[1] = ok[jn] ? (u4.y + v4.y) + wj : 0.0f;
+          base[2] = ok[jn] ? (u4.z + v4.z) + wj : 0.0f;
+          base[3] = ok[jn] ? (u4.w + v4.w) + wj : 0.0f;
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -1132,7 +1133,8 @@ __global__ void __launch_bounds__(kThreads, 2) pair_bwd_kernel(Params p) {
         }
         if (do_bits) (smem + Lk::pvb)[(tid / (KM / 8)) * 8 + tid % (KM / 8)] = uint8_t(bits);
         if constexpr (BIAS != 0) {
-          if (do_q && tid < QM) cgs[tid] = tid < c.nq ? ga * kLog2e : 0.0f;
+          // (1 on the padding rows: there lse = inf makes P = 0 whatever finite or -inf terms it multiplies)
+          if (do_q && tid < QM) cgs[tid] = tid < c.nq ? ga * kLog2e : 1.0f;
 #pragma unroll
           for (int t = 0; t < kT; ++t) {
             if (do_q) {

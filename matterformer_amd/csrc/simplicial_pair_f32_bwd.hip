@@ -253,8 +253,9 @@ __device__ __forceinline__ void body(const Params& p, Lds& L, LdsBias* X, int nk
           const float4 v4 = *reinterpret_cast<const float4*>(X->vt + (k0 + r16) * KS + 16 * t + 4 * g);
           const float wjk = X->w[j * KS + k0 + r16];
           gt[0] = g4.x; gt[1] = g4.y; gt[2] = g4.z; gt[3] = g4.w;
-          base[0] = (u4.x + v4.x) + wjk; base[1] = (u4.y + v4.y) + wjk;
-          base[2] = (u4.z + v4.z) + wjk; base[3] = (u4.w + v4.w) + wjk;
+          // (0 at a dropped pair: dS is 0 there, but the terms may be -inf or NaN)
+          base[0] = ok ? (u4.x + v4.x) + wjk : 0.0f; base[1] = ok ? (u4.y + v4.y) + wjk : 0.0f;
+          base[2] = ok ? (u4.z + v4.z) + wjk : 0.0f; base[3] = ok ? (u4.w + v4.w) + wjk : 0.0f;
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -515,7 +516,8 @@ __global__ void __launch_bounds__(kThreads, 2) pair_f32_bwd_kernel(Params p) {
         X->vt[e * KS + a] = load_any(p.v, qk, p.bias_dtype);
         X->w[a * KS + e] = load_any(p.w, (rbase + L.kidx[min(a, nk - 1)]) * N + L.kidx[min(e, nk - 1)], p.bias_dtype);
       }
-      if (tid < MN) X->gate[tid] = tid < nq ? load_any(p.gate, rbase + L.qidx[tid], p.bias_dtype) : 0.0f;
+      // (1 on the padding rows: there lse = inf makes P = 0 whatever finite or -inf terms it multiplies)
+      if (tid < MN) X->gate[tid] = tid < nq ? load_any(p.gate, rbase + L.qidx[tid], p.bias_dtype) : 1.0f;
     }
   }
   __syncthreads();

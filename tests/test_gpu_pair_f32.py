@@ -90,6 +90,45 @@ def test_large_and_masking_scale_logits(cuda):
     assert not out[1, :, 20:].any() and not lse[1, :, 20:].any()
 
 
+# operands, bias, head_dim, tokens, bars of the operand and bias gradients (bf16 operands: the bars of the block tests)
+INFINITE = [(torch.float32, torch.float32, 32, 20, 4e-6, 4e-6), (torch.float32, torch.float32, 64, 20, 4e-6, 4e-6),
+            (torch.bfloat16, torch.bfloat16, 64, 20, 4e-3, 4e-3), (torch.bfloat16, torch.float32, 64, 20, 4e-3, 2e-3),
+            (torch.bfloat16, torch.float32, 64, 90, 4e-3, 2e-3)]
+
+
+@pytest.mark.parametrize("dtype,bias_dtype,D,n,bar,bias_bar", INFINITE,
+                         ids=lambda v: str(v).replace("torch.", "") if not isinstance(v, float) else None)
+@pytest.mark.parametrize("term", ["-inf dropped", "nan dropped", "-inf kept"])
+def test_bias_terms_that_are_not_finite(cuda, dtype, bias_dtype, D, n, bar, bias_bar, term):
+    """-inf or NaN terms at pairs that pair_valid drops count for nothing; -inf at pairs that it keeps is a mask of
+    its own (P = 0 for every query), and every gradient but dgate, whose sum has 0 * -inf, is finite.  20 and 90
+    tokens leave padding rows in the last query tile."""
+    B, H = 1, 2
+    q, k1, v1, k2, v2, qv, pkv, _ = random_simplicial(B, H, n, D, seed=n + D, counts=[n], std=logit_std(D))
+    gen = torch.Generator().manual_seed(n)
+    pv = torch.rand(B, n, n, generator=gen) < 0.8
+    pv[:, :, :2] = True
+    go = torch.randn(B, H, n, D, generator=gen).to(dtype)
+    ops = [t.to(dtype) for t in (q, k1, v1, k2, v2)]
+    bias = [(torch.randn(B, H, n, n, generator=gen) * 0.5).to(bias_dtype) for _ in range(3)] + \
+           [(torch.rand(B, H, n, generator=gen) + 0.5).to(bias_dtype)]
+    at = ~pv[:, None].expand(B, H, n, n)
+    bias[2][at] = 0.0
+    plain = [t.clone() for t in bias]
+    bias[2][at] = float(term.split()[0])
+    kept = term.endswith("kept")
+    mask = None if kept else pv
+    _, got = hip_grads([t.to(cuda) for t in ops], qv.to(cuda), pkv.to(cuda), None if kept else pv.to(cuda), go.to(cuda),
+                       "ieee_fp32" if dtype == torch.float32 else "bf16_tc", bias=[t.to(cuda) for t in bias])
+    _, ref = fp64_grads(ops, qv, pkv, mask, go, bias=bias if kept else plain)
+    for name, g, r in zip(GRAD_NAMES, got, ref):
+        if kept and name == "dgate":
+            continue
+        assert torch.isfinite(g).all(), name
+        e = rel_err(g.float().cpu().numpy(), r)
+        assert e <= (bias_bar if name in GRAD_NAMES[5:] else bar), (name, e)
+
+
 @pytest.mark.parametrize("wanted", [(True, True, True, True), (False, True, False, False)], ids=["all", "dv"])
 @pytest.mark.parametrize("counts,N,D", [([1, 3], 4, 4), ([16, 9, 0], 17, 20), ([32, 5], 32, 32), ([29, 12], 29, 32)])
 def test_gradients_are_written_in_full(cuda, counts, N, D, wanted):
