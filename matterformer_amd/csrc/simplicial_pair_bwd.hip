@@ -96,6 +96,7 @@
 // wave's j), dgate and dw all come from the fp32 dS.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "mf_common.h"
 
@@ -259,11 +260,18 @@ __device__ __forceinline__ void store_grad(void* base, size_t i, float v, int bf
   else static_cast<float*>(base)[i] = v;
 }
 
-// Largest magnitude of eight bf16 (as the 15-bit pattern: for positive values bit order is value order).
+// Largest magnitude of eight bf16 (as the 15-bit pattern: for positive values bit order is value order); FINITE
+// leaves infinities and NaN out.
+template <bool FINITE>
 __device__ __forceinline__ uint32_t absmax_bits8(const uint4 r) {
-  const uint32_t a = max(max(r.x & 0x7fffu, (r.x >> 16) & 0x7fffu), max(r.y & 0x7fffu, (r.y >> 16) & 0x7fffu));
-  const uint32_t b = max(max(r.z & 0x7fffu, (r.z >> 16) & 0x7fffu), max(r.w & 0x7fffu, (r.w >> 16) & 0x7fffu));
-  return max(a, b);
+  uint32_t m = 0u;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t w = i == 0 ? r.x : (i == 1 ? r.y : (i == 2 ? r.z : r.w));
+    const uint32_t lo = w & 0x7fffu, hi = (w >> 16) & 0x7fffu;
+    m = max(m, max(FINITE && lo >= 0x7f80u ? 0u : lo, FINITE && hi >= 0x7f80u ? 0u : hi));
+  }
+  return m;
 }
 
 // Exponent of the largest magnitude (its bf16 pattern), -127 for an all-zero operand: scaling by 2^-e puts the
@@ -1070,10 +1078,20 @@ __global__ void __launch_bounds__(kThreads, 2) pair_bwd_kernel(Params p) {
         // largest magnitude of each operand over the block, and of go . out (its bf16 bits: the exponent is what
         // counts, one that is not finite leaves the others' scale alone): per thread, per wave, then over the four waves
         const uint32_t da = __float_as_uint(go[0]) << 1 >> 17, db = __float_as_uint(go[1]) << 1 >> 17;
-        uint32_t mx[7] = {max(absmax_bits8(bq[0]), absmax_bits8(bq[1])), max(absmax_bits8(bg[0]), absmax_bits8(bg[1])),
-                          absmax_bits8(b1), max(absmax_bits8(b2[0]), absmax_bits8(b2[1])), absmax_bits8(d1),
-                          max(absmax_bits8(d2[0]), absmax_bits8(d2[1])),
-                          max(da < 0x7f80u ? da : 0u, db < 0x7f80u ? db : 0u)};
+        uint32_t mx[7];
+        auto magnitudes = [&](auto finite) {
+          auto am = [](const uint4& r) { return absmax_bits8<decltype(finite)::value>(r); };
+          mx[0] = max(am(bq[0]), am(bq[1]));
+          mx[1] = max(am(bg[0]), am(bg[1]));
+          mx[2] = am(b1);
+          mx[3] = max(am(b2[0]), am(b2[1]));
+          mx[4] = am(d1);
+          mx[5] = max(am(d2[0]), am(d2[1]));
+        };
+        magnitudes(std::false_type{});
+        // (infinities and NaN stay what they are under any scale and must not decide that of the other rows)
+        if (max(max(max(mx[0], mx[1]), max(mx[2], mx[3])), max(mx[4], mx[5])) >= 0x7f80u) magnitudes(std::true_type{});
+        mx[6] = max(da < 0x7f80u ? da : 0u, db < 0x7f80u ? db : 0u);
 #pragma unroll
         for (int t = 0; t < 7; ++t) {
           mx[t] = wave_max_u32(mx[t]);

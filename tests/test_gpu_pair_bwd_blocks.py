@@ -102,6 +102,32 @@ def test_flat_softmax_of_a_large_molecule(cuda, n):
         assert rel_err(g[0].float().cpu().numpy(), r.cpu().numpy()) <= 2.2e-3, name
 
 
+@pytest.mark.parametrize("value", [float("nan"), float("inf")], ids=["nan", "inf"])
+@pytest.mark.parametrize("which", ["q", "go"])
+@pytest.mark.parametrize("n", [20, 90, 150])
+def test_a_row_that_is_not_finite_leaves_the_other_queries_alone(cuda, n, which, value):
+    """NaN or infinity in one row of q or grad_out: dq, du, dv_bias and dgate of the other queries are those of the
+    call without it (the sums over queries are NaN, as they should be)."""
+    B, H, D, bad = 1, 2, 64, 3
+    q, k1, v1, k2, v2, qv, pkv, _ = random_simplicial(B, H, n, D, seed=n, counts=[n], std=logit_std(D))
+    gen = torch.Generator().manual_seed(n)
+    go = torch.randn(B, H, n, D, generator=gen).to(torch.bfloat16)
+    ops = [t.to(torch.bfloat16) for t in (q, k1, v1, k2, v2)]
+    for bias in (None, [torch.randn(B, H, n, n, generator=gen) * 0.5 for _ in range(3)] +
+                 [torch.rand(B, H, n, generator=gen)]):
+        _, ref = fp64_grads(ops, qv, pkv, None, go, bias=bias)
+        x = [t.clone() for t in (*ops, go)]
+        x[0 if which == "q" else 5][:, :, bad, 7] = value
+        _, got = hip_grads([t.to(cuda) for t in x[:5]], qv.to(cuda), pkv.to(cuda), None, x[5].to(cuda), "bf16_tc",
+                           bias=None if bias is None else [t.to(cuda) for t in bias])
+        others = [i for i in range(n) if i != bad]
+        for name, g, r in zip(GRAD_NAMES, got, ref):
+            if name in ("dq", "du", "dv_bias", "dgate") and g is not None:
+                bar = 2e-3 if g.dtype == torch.float32 else 4e-3
+                e = rel_err(g.float().cpu().numpy()[:, :, others], r[:, :, others])
+                assert e <= bar, (name, e)
+
+
 def test_lse_far_too_small_gives_large_gradients_not_nan(cuda):
     """A forward that saturated its bias terms returns an lse below the backward's own logits: P up to e^10 leaves
     fp16, where it becomes the largest fp16."""
