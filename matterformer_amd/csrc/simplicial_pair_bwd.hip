@@ -54,8 +54,8 @@
 // waves per SIMD cannot cover.
 //
 // Schedule.  The prepare launch's first workgroup counts every molecule's
-// valid keys and queries, picks the j per unit (24, 12 or 6, with a bias 16, 8 or 4: fewer when more
-// leaves the chip without two units per CU) and writes the unit list longest
+// valid keys and queries, picks the j per unit (24, 12 or 6, with a bias 16, 8 or 4: by the
+// time its units take on two slots per CU) and writes the unit list longest
 // first (LPT); its other workgroups write the zero rows of 16-bit gradients.
 // The units of a molecule own their dk1 / dv1 rows; where a molecule has more
 // than one block triple, dq, dk2 and dv2 are summed in the unit's slab of the
@@ -192,6 +192,7 @@ struct PlanParams {
   void* dv2;
   int B, H, N, cap;
   int jm;           // j per unit at most
+  int bias;
 };
 
 // LDS layout (bytes).  A block has at most QM query, JM j and KM k rows: 64, 24 and 64 without a bias; the bias
@@ -227,23 +228,35 @@ struct Lay {
   static_assert(!BIAS || size_t(kWaves) * QM * 16 * 4 <= scr_bytes, "the waves' dv_bias partials of a key tile fit");
 };
 
+// ceil(n / d), n below 2^12: (n + d - 1/2) / d is at least 1 / (2 d) from a whole number, far past the rounding of
+// the reciprocal.  (An integer division is some forty instructions; the plan makes a chain of them per molecule.)
+__device__ __forceinline__ int ceil_div_small(int n, int d) {
+  return int((float(n + d) - 0.5f) * __builtin_amdgcn_rcpf(float(d)));
+}
 // j keys per unit and units of a molecule: `jt` j per unit, at most `cap` units, whole key pairs.
 __device__ __forceinline__ int parts_of(int nk, int jt, int cap) {
-  const int pairs = (nk + 1) / 2, most = min(cap, (nk + jt - 1) / jt);
-  const int per = (pairs + most - 1) / most;
-  return (pairs + per - 1) / per;
+  const int pairs = (nk + 1) / 2, most = min(cap, ceil_div_small(nk, jt));
+  return ceil_div_small(pairs, ceil_div_small(pairs, most));
 }
-__device__ __forceinline__ int unit_rows(int nk, int parts) { return 2 * (((nk + 1) / 2 + parts - 1) / parts); }
+__device__ __forceinline__ int unit_rows(int nk, int parts) { return 2 * ceil_div_small((nk + 1) / 2, parts); }
 // Blocks of a run of n rows, at most m rows (a multiple of 16) each, cut at multiples of 16.
 __device__ __forceinline__ int blocks_of(int n, int m) { return (n + m - 1) / m; }
 __device__ __forceinline__ int block_rows(int n, int blocks) { return 16 * (((n + 15) / 16 + blocks - 1) / blocks); }
 
-// Relative cost of one unit: rounds of key pairs x key tiles x (fixed work per query block + query tiles), and
-// the staging.
-__device__ __forceinline__ uint32_t unit_cost(int nk, int nq, int jt, int cap) {
-  const int jr = unit_rows(nk, parts_of(nk, jt, cap));
-  const int nqt = (nq + 15) / 16, nkt = (nk + 15) / 16, nqb = blocks_of(nq, 64);
-  return uint32_t((jr / 2 + kWaves - 1) / kWaves) * uint32_t(nkt) * uint32_t(6 * nqb + 2 * nqt) + 24u;
+// Relative cost of one unit: per key tile the sums that end it, for each query block, and the rounds of four key
+// pairs (fixed work per query block, and the query tiles); without a bias, staging and slab sums of further block
+// triples.  Two units to a CU take about 0.25 us of it without a bias (22 rows of 44 tokens: 42 us, of 64: 59; of 128:
+// 197 in three rounds, 104 in one), 0.5 us with one (12 rows of 24: 25 us, 16 of 48: 45, 16 of 64: 100; 16 of
+// 192: 700, 8 of 192: 530).
+__device__ __forceinline__ uint32_t unit_cost(int nk, int nq, int parts, const PlanParams& pp) {
+  const int rounds = (unit_rows(nk, parts) + 2 * kWaves - 1) / (2 * kWaves);
+  const int nqt = (nq + 15) / 16, nkt = (nk + 15) / 16;
+  if (pp.bias) {
+    const int nqb = blocks_of(nq, Lay<true>::QM);
+    return uint32_t(nkt * (14 * nqb + rounds * (nqb + 2 * nqt)));
+  }
+  const int nqb = blocks_of(nq, Lay<false>::QM), nkb = blocks_of(nk, Lay<false>::KM);
+  return uint32_t(nkt * (8 * nqb + rounds * (6 * nqb + 2 * nqt)) + 25 * (nqb * nkb - 1));
 }
 
 typedef __attribute__((__vector_size__(4 * sizeof(_Float16)))) _Float16 mf_f16x4;
@@ -410,7 +423,8 @@ __global__ void __launch_bounds__(kPlanThreads) pair_bwd_prepare(PlanParams pp) 
   __shared__ uint32_t s_cost[kMaxPlanBatch];
   __shared__ int s_units[kMaxPlanBatch];
   __shared__ int s_count[2 * kMaxPlanBatch];
-  __shared__ int s_total, s_level[3];
+  __shared__ int s_total;
+  __shared__ float s_level[kPlanThreads / 64][3][3];  // units, largest cost, sum of costs at each j per unit, by wave
   const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
   const int B = pp.B, H = pp.H, N = pp.N;
   if (blockIdx.x > 0) {
@@ -467,22 +481,66 @@ __global__ void __launch_bounds__(kPlanThreads) pair_bwd_prepare(PlanParams pp) 
     }
   }
   if (tid == 0) s_total = 0;
-  if (tid < 3) s_level[tid] = 0;
   lds_barrier();
-  // units at jm, jm / 2 and jm / 4 j per unit; the largest j that still gives two units per CU (512), else jm / 4
-  for (int b = tid; b < B; b += kPlanThreads) {
-    const int nk = s_count[2 * b], nq = s_count[2 * b + 1];
-    if (nk <= 0 || nq <= 0) continue;
+  // jm, jm / 2 or jm / 4 j per unit: the one whose units finish first on 512 slots (two per CU; 256 units or fewer
+  // left for the last round have a CU each and take 0.5 to 0.8 of their time), in rounds of the mean cost, or by the
+  // longest unit; of equals the larger, whose fewer parts are added sooner.  (By the largest j that gives 512 units,
+  // 16 molecules of 72 tokens, 8 heads, ran 768 units of 12 rows, 179 us; 384 of 24 rows take one round: 148.)
+  {
+    // thread 4 b + l: molecule b at jm >> l
+    const int l = tid & 3;
+    float units = 0.0f, most = 0.0f, sum = 0.0f;
+    for (int b = tid >> 2; b < B; b += kPlanThreads / 4) {
+      const int nk = s_count[2 * b], nq = s_count[2 * b + 1];
+      if (nk <= 0 || nq <= 0 || l == 3) continue;
+      const int parts = parts_of(nk, pp.jm >> l, pp.cap);
+      const float u = float(H * parts), c = float(unit_cost(nk, nq, parts, pp));
+      units += u;
+      most = fmaxf(most, c);
+      sum += u * c;
+    }
+    if (16 * wave < B) {
 #pragma unroll
-    for (int l = 0; l < 3; ++l) atomicAdd(&s_level[l], H * parts_of(nk, pp.jm >> l, pp.cap));
+      for (int off = 4; off < 64; off <<= 1) {
+        units += __shfl_xor(units, off, 64);
+        most = fmaxf(most, __shfl_xor(most, off, 64));
+        sum += __shfl_xor(sum, off, 64);
+      }
+      if (lane < 3) {
+        s_level[wave][lane][0] = units;
+        s_level[wave][lane][1] = most;
+        s_level[wave][lane][2] = sum;
+      }
+    }
   }
   lds_barrier();
-  const int jt = s_level[0] >= 512 ? pp.jm : (s_level[1] >= 512 ? pp.jm / 2 : pp.jm / 4);
+  int jt = pp.jm;
+  {
+    float least = INFINITY;
+#pragma unroll
+    for (int l = 0; l < 3; ++l) {
+      float units = 0.0f, most = 0.0f, sum = 0.0f;
+      for (int w = 0; w < min(kPlanThreads / 64, (B + 15) / 16); ++w) {
+        units += s_level[w][l][0];
+        most = fmaxf(most, s_level[w][l][1]);
+        sum += s_level[w][l][2];
+      }
+      if (units == 0.0f) continue;
+      const float full = floorf(units / 512.0f), rest = units - 512.0f * full;
+      const float last = rest == 0.0f ? 0.0f : (rest <= 256.0f ? 0.5f + 0.3f / 256.0f * rest : 1.0f);
+      const float t = fmaxf((full + last) * (sum / units), full == 0.0f ? last * most : most);
+      if (t < least) {
+        least = t;
+        jt = pp.jm >> l;
+      }
+    }
+  }
   for (int b = tid; b < B; b += kPlanThreads) {
     const int nk = s_count[2 * b], nq = s_count[2 * b + 1];
     const bool work = nk > 0 && nq > 0;
-    s_cost[b] = work ? unit_cost(nk, nq, jt, pp.cap) : 0u;
-    s_units[b] = work ? H * parts_of(nk, jt, pp.cap) : 0;
+    const int parts = work ? parts_of(nk, jt, pp.cap) : 0;
+    s_cost[b] = work ? unit_cost(nk, nq, parts, pp) : 0u;
+    s_units[b] = H * parts;
     pp.counts[b] = int2{nk, nq};
   }
   lds_barrier();
@@ -934,7 +992,8 @@ __global__ void __launch_bounds__(kThreads, 2) pair_bwd_kernel(Params p) {
   const uint16_t* klist = p.lists + size_t(2 * b) * N;
   const uint16_t* qlist = klist + N;
   const int njb = blocks_of(ju1 - ju0, JM), nqb = blocks_of(nq, QM), nkb = blocks_of(nk, KM);
-  const int jrows = 2 * (((ju1 - ju0 + 1) / 2 + njb - 1) / njb);
+  // (whole rounds of four key pairs in every block but the last)
+  const int jrows = 2 * kWaves * (((ju1 - ju0 + 2 * kWaves - 1) / (2 * kWaves) + njb - 1) / njb);
   const int qrows = block_rows(nq, nqb), krows = block_rows(nk, nkb);
   c.direct = parts == 1 && njb == 1 && nqb == 1 && nkb == 1;
 
@@ -1228,7 +1287,7 @@ __global__ void __launch_bounds__(kThreads, 2) pair_bwd_kernel(Params p) {
 // workgroups per (molecule, head); a separate launch, so the stream orders it after the units without any
 // cross-workgroup fence.
 constexpr int kCombineSplit = 2;
-__global__ void __launch_bounds__(kThreads) pair_bwd_combine(Params p, int qm, int jm) {
+__device__ __forceinline__ void combine(const Params& p, int split, int qm, int jm) {
   const int bh = blockIdx.x;
   const int b = bh / p.H;
   const int2 nkq = p.counts[b];
@@ -1244,7 +1303,7 @@ __global__ void __launch_bounds__(kThreads) pair_bwd_combine(Params p, int qm, i
   // rows: dq of the nq queries, then dk2 and dv2 of the nk keys, 16 float4 each; kAt per thread at a time
   constexpr int kAt = 4;
   const int total = (nq + 2 * nk) * 16;
-  for (int u0 = blockIdx.y * kAt * kThreads; u0 < total; u0 += kCombineSplit * kAt * kThreads) {
+  for (int u0 = split * kAt * kThreads; u0 < total; u0 += kCombineSplit * kAt * kThreads) {
     float4 a[kAt];
     size_t so[kAt], dst[kAt];
     void* base[kAt];
@@ -1277,7 +1336,7 @@ __global__ void __launch_bounds__(kThreads) pair_bwd_combine(Params p, int qm, i
 // units).  kFinishSplit workgroups per (molecule, head), each thread kFinishAt entries at a time.
 constexpr int kFinishSplit = 4, kFinishAt = 4;
 template <int BIAS>
-__global__ void __launch_bounds__(kThreads) pair_bwd_bias_finish(Params p) {
+__device__ __forceinline__ void bias_finish(const Params& p, int split) {
   const int bh = blockIdx.x;
   const int b = bh / p.H;
   const int2 nkq = p.counts[b];
@@ -1292,7 +1351,7 @@ __global__ void __launch_bounds__(kThreads) pair_bwd_bias_finish(Params p) {
   if (p.dvb != nullptr) {
     const float* dvp = p.dvpart + size_t(bh) * p.cap * N * N;
     const int n = nq * nk, step = kThreads * kFinishSplit;
-    for (int u0 = blockIdx.y * kThreads + tid; u0 < n; u0 += kFinishAt * step) {
+    for (int u0 = split * kThreads + tid; u0 < n; u0 += kFinishAt * step) {
       float sv[kFinishAt], gate[kFinishAt];
       size_t e[kFinishAt], o[kFinishAt];
 #pragma unroll
@@ -1312,7 +1371,7 @@ __global__ void __launch_bounds__(kThreads) pair_bwd_bias_finish(Params p) {
         if (u0 + t * step < n) store_grad(p.dvb, o[t], gate[t] * sv[t], p.bout16);
     }
   }
-  if (p.dgate != nullptr && blockIdx.y == 0) {
+  if (p.dgate != nullptr && split == 0) {
     const float* gp = p.dgpart + size_t(bh) * p.cap * N;
     for (int i = tid; i < nq; i += kThreads) {
       float s = gp[i];
@@ -1320,6 +1379,15 @@ __global__ void __launch_bounds__(kThreads) pair_bwd_bias_finish(Params p) {
       store_grad(p.dgate, rbase + qlist[i], s, p.bout16);
     }
   }
+}
+
+// Both in one launch, side by side: workgroups 0 .. kCombineSplit - 1 of a (molecule, head) combine, the others (with
+// a bias) finish its gradients (one molecule of 56 tokens, fp32 bias, 8 heads: 7 + 6 us as two launches).
+template <int BIAS>
+__global__ void __launch_bounds__(kThreads) pair_bwd_finish(Params p) {
+  const int y = blockIdx.y;
+  if (y < kCombineSplit) combine(p, y, Lay<BIAS != 0>::QM, Lay<BIAS != 0>::JM);
+  else if constexpr (BIAS != 0) bias_finish<BIAS>(p, y - kCombineSplit);
 }
 
 }  // namespace pbwd
@@ -1358,15 +1426,10 @@ static int launch_units(const pbwd::Params& p, int blocks, int bh, hipStream_t s
   if (st != MF_OK) return st;
   hipLaunchKernelGGL(pair_bwd_kernel<BIAS>, dim3(unsigned(blocks)), dim3(kThreads), lds, stream, p);
   MF_HIP_CHECK(hipGetLastError());
-  hipLaunchKernelGGL(pair_bwd_combine, dim3(unsigned(bh), kCombineSplit), dim3(kThreads), 0, stream, p,
-                     Lay<BIAS != 0>::QM, Lay<BIAS != 0>::JM);
+  const bool finish = BIAS != 0 && (p.dvb != nullptr || p.dgate != nullptr);
+  hipLaunchKernelGGL(pair_bwd_finish<BIAS>, dim3(unsigned(bh), kCombineSplit + (finish ? kFinishSplit : 0)), dim3(kThreads),
+                     0, stream, p);
   MF_HIP_CHECK(hipGetLastError());
-  if constexpr (BIAS != 0) {
-    if (p.dvb != nullptr || p.dgate != nullptr) {
-      hipLaunchKernelGGL(pair_bwd_bias_finish<BIAS>, dim3(unsigned(bh), kFinishSplit), dim3(kThreads), 0, stream, p);
-      MF_HIP_CHECK(hipGetLastError());
-    }
-  }
   return MF_OK;
 }
 
@@ -1387,7 +1450,8 @@ int simplicial_pair_bwd_launch(const mf_simplicial_bwd_args* a, bool bias16, hip
   pp.H = a->heads;
   pp.N = a->tokens;
   pp.cap = ws.cap;
-  pp.jm = a->bias_u != nullptr ? Lay<true>::JM : Lay<false>::JM;
+  pp.bias = a->bias_u != nullptr ? 1 : 0;
+  pp.jm = pp.bias ? Lay<true>::JM : Lay<false>::JM;
   Params p{};
   p.head = pp.head;
   p.units = pp.units;

@@ -16,7 +16,7 @@ from matterformer_amd.hip_simplicial_attention import (
     hip_simplicial_attention_forward,
 )
 from matterformer_amd.workloads import random_simplicial
-from test_gpu_simplicial_bwd import GRAD_NAMES, fp64_grads, hip_grads, logit_std, rel_err
+from test_gpu_simplicial_bwd import GRAD_NAMES, abi_bwd, fp64_grads, hip_grads, logit_std, rel_err
 
 pytestmark = pytest.mark.gpu
 
@@ -159,6 +159,32 @@ def test_gradients_below_the_fp32_range_are_zero_not_nan(cuda):
             assert float(g.abs().max()) <= 2.0 ** -110, name
         else:
             assert rel_err(g.numpy(), r) <= 4e-3, (name, rel_err(g.numpy(), r))
+
+
+def _plan(counts, heads, bias_dtype, device):
+    """(units, j per unit) of the plan that mf_simplicial_bwd leaves at the start of its workspace."""
+    B, N = len(counts), max(counts)
+    valid = torch.arange(N)[None, :] < torch.tensor(counts)[:, None]
+    ops = [torch.zeros(B, heads, N, 64, device=device, dtype=torch.bfloat16) for _ in range(5)]
+    bias = None
+    if bias_dtype is not None:
+        bias = [torch.zeros(s, device=device, dtype=bias_dtype) for s in [(B, heads, N, N)] * 3 + [(B, heads, N)]]
+    out32, lse = torch.zeros(B, heads, N, 64, device=device), torch.zeros(B, heads, N, device=device)
+    *_, ws = abi_bwd(ops, ops[0], out32, lse, valid.to(device), valid.to(device), torch.float32, bias=bias)
+    units, j = ws[:8].view(torch.int32).tolist()
+    return units, j
+
+
+@pytest.mark.parametrize("counts,heads,bias_dtype,want", [
+    ([72] * 16, 8, None, (384, 24)),               # one round; not 768 units of 12 rows
+    ([64], 8, torch.float32, (64, 8)),             # half the parts to add for the same round
+    ([192] * 4, 12, torch.bfloat16, (576, 16)),    # 64 units left for the second round, not 1152 of 8 rows
+    ([128] * 16, 8, None, (768, 24)),              # not 2048 of 8 rows, whose staging is most of their time
+    ([256], 8, None, (344, 6)), ([44] * 64, 8, None, (1024, 24)), ([44, 9, 30], 2, None, (30, 6)),
+], ids=lambda v: str(v) if isinstance(v, int) else None)
+def test_rows_per_unit(cuda, counts, heads, bias_dtype, want):
+    """The schedule takes the j per unit whose units finish first on the chip's 512 slots."""
+    assert _plan(counts, heads, bias_dtype, cuda) == want
 
 
 def test_queries_and_keys_of_different_counts(cuda):

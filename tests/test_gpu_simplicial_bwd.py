@@ -253,10 +253,10 @@ def test_low_rank_terms_run_on_the_kernel(cuda):
     assert res[9] is not None and res[11] is not None
 
 
-def _abi_bwd(ops, go, out32, lse, qv, pkv, grads_dtype, bias=None):
+def abi_bwd(ops, go, out32, lse, qv, pkv, grads_dtype, bias=None):
     """mf_simplicial_bwd through the C ABI; gradient buffers filled with NaN (bf16) or zeros (fp32, the
-    caller's fill that the fp32 contract asks for); with a bf16 factorized bias also du, dv_bias, dw, dgate
-    (the same dtype and fill)."""
+    caller's fill that the fp32 contract asks for); with a factorized bias also du, dv_bias, dw, dgate
+    (the same dtype and fill).  The gradients, then the workspace."""
     from matterformer_amd import _native
 
     B, H, N, D = ops[0].shape
@@ -292,7 +292,7 @@ def _abi_bwd(ops, go, out32, lse, qv, pkv, grads_dtype, bias=None):
     with torch.cuda.device(dev):
         _native.check(lib.mf_simplicial_bwd(args, _native.current_stream(dev)), "mf_simplicial_bwd")
     torch.cuda.synchronize()
-    return grads
+    return (*grads, ws)
 
 
 @pytest.mark.parametrize("with_bias", [False, True], ids=["nobias", "bias"])
@@ -319,8 +319,8 @@ def test_bf16_gradients_written_in_full(cuda, counts, with_bias):
         kw = dict(u=bias[0], v_bias=bias[1], w=bias[2], gate=bias[3])
     out, lse, out32 = hip_simplicial_attention_forward(*ops, query_valid=qv, pair_key_valid=pkv, pair_valid=None,
                                                        precision="bf16_tc", **kw)
-    g16 = _abi_bwd(ops, go, out32, lse, qv, pkv, torch.bfloat16, bias=bias)
-    g32 = _abi_bwd(ops, go, out32, lse, qv, pkv, torch.float32, bias=bias)
+    *g16, _ = abi_bwd(ops, go, out32, lse, qv, pkv, torch.bfloat16, bias=bias)
+    *g32, _ = abi_bwd(ops, go, out32, lse, qv, pkv, torch.float32, bias=bias)
     for name, a, r in zip(GRAD_NAMES, g16, g32):
         assert not torch.isnan(a).any(), name
         assert torch.equal(a, r.to(torch.bfloat16)), name
