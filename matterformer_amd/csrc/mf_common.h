@@ -45,8 +45,10 @@ size_t simplicial_pair_workspace_bytes(int batch, int tokens);
 int simplicial_pair_launch(const mf_simplicial_fwd_args* a, void* claims, int num_cus, hipStream_t stream);
 
 // Pair-formulation forward for fp32 operands of at most 64 tokens (simplicial_pair_f32.hip).
+// _range: the calls it takes when their rows are aligned and they have no rank terms.
+bool simplicial_pair_f32_range(int dtype, int64_t batch_heads, int tokens, int head_dim, bool bias);
 bool simplicial_pair_f32_serves(const mf_simplicial_fwd_args* a);
-int simplicial_pair_f32_launch(const mf_simplicial_fwd_args* a, hipStream_t stream);
+int simplicial_pair_f32_launch(const mf_simplicial_fwd_args* a, int num_cus, hipStream_t stream);
 // Its backward, at most 32 tokens and head_dim <= 32 (simplicial_pair_f32_bwd.hip).
 bool simplicial_pair_f32_bwd_serves(const mf_simplicial_bwd_args* a);
 int simplicial_pair_f32_bwd_launch(const mf_simplicial_bwd_args* a, hipStream_t stream);

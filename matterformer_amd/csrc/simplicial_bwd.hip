@@ -1227,7 +1227,8 @@ static int simplicial_bwd_impl(const mf_simplicial_bwd_args* a, bool bias32, voi
   vec = vec && reinterpret_cast<uintptr_t>(a->grad_out) % (a->grad_dtype == MF_DTYPE_F32 ? 16 : 8) == 0;
   vec = vec && reinterpret_cast<uintptr_t>(a->out) % 16 == 0;
   prm.vec = vec ? 1 : 0;
-  prm.halves = a->dtype == MF_DTYPE_F32 && a->tokens <= 64 && a->head_dim <= 64 && a->head_dim % 4 == 0 ? 1 : 0;
+  prm.halves =
+      simplicial_pair_f32_range(a->dtype, int64_t(a->batch) * a->heads, a->tokens, a->head_dim, a->bias_u != nullptr) ? 1 : 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const bool has_pv = a->pair_valid != nullptr;
   const int D = a->head_dim;

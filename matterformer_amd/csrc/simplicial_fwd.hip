@@ -993,7 +993,7 @@ static int simplicial_fwd_impl(const mf_simplicial_fwd_args* a, bool views, void
           return fail(MF_ERR_INVALID_ARGUMENT,
                       "mf_simplicial_fwd: operand strides must be non-negative multiples of 8 elements");
   }
-  if (simplicial_pair_f32_serves(a)) return simplicial_pair_f32_launch(a, s);
+  if (simplicial_pair_f32_serves(a)) return simplicial_pair_f32_launch(a, dev.num_cus, s);
   if (has_extras(a) && !(bias_only && pair_ok)) {
     st = check_shape(a->batch, a->heads, a->tokens, a->head_dim, a->dtype, has_pv, &lds);
     if (st != MF_OK) return st;

@@ -14,9 +14,10 @@
 //       B operand of K step r as it is; A = Z formed in registers
 //   S += gate_i (u_ij + v_ik + w_jk) in fp32 with a factorized bias
 //
-// One workgroup of four waves per (molecule, head, 32 queries).  The waves split the j rows; each keeps an
+// One workgroup of W waves per (molecule, head, 16 QT queries): four waves and two query tiles, or eight and one in
+// small calls.  The waves split the j rows; each keeps an
 // offset per query that follows its running maximum (moved only when a logit exceeds it by more than
-// kRescaleSlack, for the query's four lane groups together, so P <= 2^8), and the four partial (O, max, sum)
+// kRescaleSlack, for the query's four lane groups together, so P <= 2^8), and the partial (O, max, sum)
 // meet in LDS at the end.  MFMA-bound: an iteration (one j, 16 keys, 32 queries, head_dim 32) is 32 MFMA of 32
 // cycles against about 80 VALU instructions.  128 QM9-like molecules of 9-29 atoms, 8 heads, head_dim 32: 42 us at a
 // cold clock (134 us on the general kernel; 7.7 us of fp32 MFMA for the valid work, 13 with the tiles' padding, the
@@ -28,11 +29,9 @@
 namespace mf {
 namespace spf32 {
 
-constexpr int kWaves = 4;
-constexpr int kThreads = kWaves * 64;
 constexpr int kMaxN = 64;               // tokens
-constexpr int QT = 2;                   // query tiles per workgroup
 constexpr float kRescaleSlack = 8.0f;   // log2 units
+constexpr int kSmallGrid = 1;           // workgroups of one query tile per CU up to which they are taken
 
 struct Params {
   const float* q;
@@ -54,14 +53,14 @@ struct Params {
   int H, N, D, NP;   // NP: N rounded up to 16
 };
 
-// LDS (floats): the four key / value operands [NP][KS], then (BIAS) u^T [NP j][32 i + 4], v [32 i][NP + 4],
-// w [NP j][NP + 4]; the waves' partial outputs [4][32][DP + 4] reuse the operands' place.
-template <int DP, bool BIAS>
+// LDS (floats): the four key / value operands [NP][KS], then (BIAS) u^T [NP j][16 QT i + 4], v [16 QT i][NP + 4],
+// w [NP j][NP + 4]; the waves' partial outputs [W][16 QT][DP + 4] reuse the operands' place.
+template <int DP, bool BIAS, int QT, int W>
 struct Lay {
   static constexpr int KS = DP + 4;
   static constexpr int UI = 16 * QT + 4;
   __host__ __device__ static int operands(int NP) {
-    const int rows = 4 * NP * KS, parts = kWaves * 16 * QT * KS;
+    const int rows = 4 * NP * KS, parts = W * 16 * QT * KS;
     return rows > parts ? rows : parts;
   }
   __host__ __device__ static int floats(int NP) {
@@ -93,12 +92,12 @@ __device__ __forceinline__ mf_f32x4 mma(float a, float b, mf_f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// The pair tiles of the wave (j = wave, wave + 4, ...) against NT query tiles: offsets, sums and outputs in place.
-template <int DP, bool BIAS, int NT>
+// The pair tiles of the wave (j = wave, wave + W, ...) against NT query tiles: offsets, sums and outputs in place.
+template <int DP, bool BIAS, int QT, int W, int NT>
 __device__ __forceinline__ void pair_loop(const float* smem, const unsigned long long* s_bits, int nk, int NP,
                                           const float (&qf)[QT][DP / 4], const float (&gq)[QT], float (&M)[QT],
                                           float (&lsum)[QT], mf_f32x4 (&oa)[QT][DP / 16]) {
-  using L = Lay<DP, BIAS>;
+  using L = Lay<DP, BIAS, QT, W>;
   constexpr int KS = L::KS, UI = L::UI, NC = DP / 4, ND = DP / 16;
   const int lane = lane_id(), wave = wave_id();
   const int g = lane >> 4, r16 = lane & 15;
@@ -129,7 +128,7 @@ __device__ __forceinline__ void pair_loop(const float* smem, const unsigned long
         vb[t][0] = x.x; vb[t][1] = x.y; vb[t][2] = x.z; vb[t][3] = x.w;
       }
     }
-    for (int j = wave; j < nk; j += kWaves) {
+    for (int j = wave; j < nk; j += W) {
       const uint32_t bits = uint32_t(s_bits[j] >> k0) & 0xffffu;
       const bool whole = __builtin_amdgcn_readfirstlane(bits) == 0xffffu;
       float wz[NC];
@@ -234,9 +233,10 @@ __device__ __forceinline__ void pair_loop(const float* smem, const unsigned long
   }
 }
 
-template <int DP, bool BIAS>
-__global__ void __launch_bounds__(kThreads, DP == 32 ? 4 : 2) simplicial_pair_f32_kernel(Params p) {
-  using L = Lay<DP, BIAS>;
+template <int DP, bool BIAS, int QT, int W>
+__global__ void __launch_bounds__(W * 64, DP == 32 && W == 4 ? 4 : 2) simplicial_pair_f32_kernel(Params p) {
+  constexpr int kWaves = W, kThreads = W * 64;
+  using L = Lay<DP, BIAS, QT, W>;
   constexpr int KS = L::KS, UI = L::UI;
   constexpr int NC = DP / 4;    // K steps of S, and a lane's contiguous d
   constexpr int ND = DP / 16;   // 16-d tiles of O
@@ -357,10 +357,10 @@ __global__ void __launch_bounds__(kThreads, DP == 32 ? 4 : 2) simplicial_pair_f3
 #pragma unroll
     for (int dt = 0; dt < ND; ++dt) oa[t][dt] = mf_f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  if (nqb > 16) pair_loop<DP, BIAS, 2>(smem, s_bits, nk, NP, qf, gq, M, lsum, oa);
-  else pair_loop<DP, BIAS, 1>(smem, s_bits, nk, NP, qf, gq, M, lsum, oa);
+  if (QT == 1 || nqb <= 16) pair_loop<DP, BIAS, QT, W, 1>(smem, s_bits, nk, NP, qf, gq, M, lsum, oa);
+  else pair_loop<DP, BIAS, QT, W, QT>(smem, s_bits, nk, NP, qf, gq, M, lsum, oa);
 
-  // ---- the four waves' partials: offsets and sums first, then the outputs scaled to the largest offset ----
+  // ---- the waves' partials: offsets and sums first, then the outputs scaled to the largest offset ----
 #pragma unroll
   for (int t = 0; t < QT; ++t) {
     const float l = sum_groups(lsum[t]);
@@ -374,7 +374,9 @@ __global__ void __launch_bounds__(kThreads, DP == 32 ? 4 : 2) simplicial_pair_f3
 #pragma unroll
   for (int t = 0; t < QT; ++t) {
     const int i = 16 * t + r16;
-    const float mx = fmaxf(fmaxf(s_m[0][i], s_m[1][i]), fmaxf(s_m[2][i], s_m[3][i]));
+    float mx = s_m[0][i];
+#pragma unroll
+    for (int w = 1; w < W; ++w) mx = fmaxf(mx, s_m[w][i]);
     const float f = M[t] == -INFINITY ? 0.0f : fast_exp2(M[t] - mx);
 #pragma unroll
     for (int dt = 0; dt < ND; ++dt)
@@ -384,7 +386,9 @@ __global__ void __launch_bounds__(kThreads, DP == 32 ? 4 : 2) simplicial_pair_f3
   __syncthreads();
   for (int u = tid; u < nqb * (D / 4); u += kThreads) {
     const int i = u / (D / 4), c = 4 * (u % (D / 4));
-    const float mx = fmaxf(fmaxf(s_m[0][i], s_m[1][i]), fmaxf(s_m[2][i], s_m[3][i]));
+    float mx = s_m[0][i];
+#pragma unroll
+    for (int w = 1; w < W; ++w) mx = fmaxf(mx, s_m[w][i]);
     float l = 0.0f;
     float4 o{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -403,24 +407,45 @@ __global__ void __launch_bounds__(kThreads, DP == 32 ? 4 : 2) simplicial_pair_f3
   }
 }
 
-template <int DP, bool BIAS>
+template <int DP, bool BIAS, int QT, int W>
 int launch(const Params& p, int bh, hipStream_t stream) {
-  const size_t lds = size_t(Lay<DP, BIAS>::floats(p.NP)) * 4;
-  const int st = ensure_dynamic_lds(reinterpret_cast<const void*>(simplicial_pair_f32_kernel<DP, BIAS>),
-                                    Lay<DP, BIAS>::floats(kMaxN) * 4);
+  using L = Lay<DP, BIAS, QT, W>;
+  const size_t lds = size_t(L::floats(p.NP)) * 4;
+  const int st = ensure_dynamic_lds(reinterpret_cast<const void*>(simplicial_pair_f32_kernel<DP, BIAS, QT, W>),
+                                    L::floats(kMaxN) * 4);
   if (st != MF_OK) return st;
-  hipLaunchKernelGGL((simplicial_pair_f32_kernel<DP, BIAS>), dim3(unsigned(bh), unsigned((p.N + 16 * QT - 1) / (16 * QT))),
-                     dim3(kThreads), lds, stream, p);
+  hipLaunchKernelGGL((simplicial_pair_f32_kernel<DP, BIAS, QT, W>),
+                     dim3(unsigned(bh), unsigned((p.N + 16 * QT - 1) / (16 * QT))), dim3(W * 64), lds, stream, p);
   MF_HIP_CHECK(hipGetLastError());
   return MF_OK;
 }
 
+// Two query tiles a workgroup of four waves share each W and Z; where that leaves CUs without work, one tile a
+// workgroup of eight waves: twice the workgroups of twice the waves.  8 heads, head_dim 32, one molecule of 32 / 48 /
+// 64 tokens 19 / 35 / 59 us -> 11 / 20 / 31; 16 of 32 tokens (256 workgroups) 20 -> 12, 16 of 64 (1024) 62 -> 55, 64
+// of 29 tokens (1024) 30 -> 31.  Sixteen waves: 12 / 20 / 30, the matrix cores of a workgroup's CU are busy.
+template <int DP, bool BIAS>
+int launch_for(const Params& p, int bh, int num_cus, hipStream_t stream) {
+  if (long(bh) * ((p.N + 15) / 16) <= kSmallGrid * num_cus) return launch<DP, BIAS, 1, 8>(p, bh, stream);
+  return launch<DP, BIAS, 2, 4>(p, bh, stream);
+}
+
 }  // namespace spf32
 
-// fp32 operands of at most 64 tokens, whole and aligned 16-byte rows, with or without a factorized bias.  (The
-// limit is the LDS that all keys of a molecule take; longer rows and the rank terms stay on the general kernel.)
+// fp32 operands of at most 64 tokens and head_dim 64, rows of whole 16-byte pieces, with or without a factorized bias.
+// (The limit is the LDS that all keys of a molecule take; longer rows and the rank terms stay on the general kernel.)
+// A few (molecule, head) of 49 .. 64 tokens without a bias do too: it spreads them over one wave per query where
+// the pair form has four workgroups each (8 heads, one molecule of 64 tokens, head_dim 32 / 64: 23 / 39 us
+// against 31 / 51; four of 56: 25 / 41 against 29 / 46; eight of 64, 45 / 80 against 32 / 52; 48 tokens 30 / 49 against
+// 20 / 31; with a bias, one of 64, 43 / 57 against 36 / 55).
+bool simplicial_pair_f32_range(int dtype, int64_t batch_heads, int tokens, int head_dim, bool bias) {
+  if (dtype != MF_DTYPE_F32 || tokens > spf32::kMaxN || head_dim > 64 || head_dim % 4 != 0) return false;
+  return bias || tokens <= 48 || batch_heads > 32;
+}
+
 bool simplicial_pair_f32_serves(const mf_simplicial_fwd_args* a) {
-  if (a->dtype != MF_DTYPE_F32 || a->tokens > spf32::kMaxN || a->head_dim > 64 || a->head_dim % 4 != 0) return false;
+  if (!simplicial_pair_f32_range(a->dtype, int64_t(a->batch) * a->heads, a->tokens, a->head_dim, a->bias_u != nullptr))
+    return false;
   if (a->angle_left != nullptr || a->message_left != nullptr) return false;
   if (int64_t(a->batch) * a->heads > 0x7fffffff) return false;
   for (const void* ptr : {a->q, a->k1, a->v1, a->k2, a->v2, (const void*)a->out, (const void*)a->out_f32})
@@ -428,7 +453,7 @@ bool simplicial_pair_f32_serves(const mf_simplicial_fwd_args* a) {
   return true;
 }
 
-int simplicial_pair_f32_launch(const mf_simplicial_fwd_args* a, hipStream_t stream) {
+int simplicial_pair_f32_launch(const mf_simplicial_fwd_args* a, int num_cus, hipStream_t stream) {
   using namespace spf32;
   Params p{};
   p.q = static_cast<const float*>(a->q);
@@ -443,8 +468,9 @@ int simplicial_pair_f32_launch(const mf_simplicial_fwd_args* a, hipStream_t stre
   p.H = a->heads; p.N = a->tokens; p.D = a->head_dim;
   p.NP = (a->tokens + 15) / 16 * 16;
   const int bh = a->batch * a->heads;
-  if (a->head_dim <= 32) return a->bias_u ? launch<32, true>(p, bh, stream) : launch<32, false>(p, bh, stream);
-  return a->bias_u ? launch<64, true>(p, bh, stream) : launch<64, false>(p, bh, stream);
+  if (a->head_dim <= 32)
+    return a->bias_u ? launch_for<32, true>(p, bh, num_cus, stream) : launch_for<32, false>(p, bh, num_cus, stream);
+  return a->bias_u ? launch_for<64, true>(p, bh, num_cus, stream) : launch_for<64, false>(p, bh, num_cus, stream);
 }
 
 }  // namespace mf

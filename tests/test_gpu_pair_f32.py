@@ -62,6 +62,39 @@ def test_backward_sums_the_logits_as_the_forward_does(cuda, n, D, bar):
         assert rel_err(g.cpu().numpy(), r) <= bar, (name, rel_err(g.cpu().numpy(), r))
 
 
+@pytest.mark.parametrize("with_bias", [False, True], ids=["none", "bias"])
+@pytest.mark.parametrize("B,H,n,D", [(32, 8, 16, 32), (33, 8, 16, 32), (16, 8, 31, 32), (17, 8, 32, 32), (40, 4, 33, 64),
+                                     (8, 8, 64, 64), (9, 8, 64, 20), (4, 8, 64, 32), (4, 8, 49, 64), (5, 8, 49, 32)])
+def test_both_workgroup_shapes_of_the_forward(cuda, B, H, n, D, with_bias):
+    """Calls on either side of the line between one query tile a workgroup of eight waves (one workgroup per CU at
+    most) and two tiles of four waves, and of the line past which few molecules of 49 tokens and more take the general
+    kernel (without a bias, 32 (molecule, head)): the same outputs as the molecules one by one, and as float64."""
+    counts = [n - b % 3 for b in range(B)]
+    q, k1, v1, k2, v2, qv, pkv, _ = random_simplicial(B, H, n, D, seed=B + n, counts=counts, std=logit_std(D))
+    gen = torch.Generator().manual_seed(B)
+    bias = None
+    if with_bias:
+        bias = [torch.randn(B, H, n, n, generator=gen) * 0.5 for _ in range(3)] + [torch.rand(B, H, n, generator=gen)]
+    ops = [t.to(cuda) for t in (q, k1, v1, k2, v2)]
+    masks = [qv.to(cuda), pkv.to(cuda)]
+
+    def forward(s):
+        kw = {} if bias is None else {k: t[s].to(cuda) for k, t in zip(("u", "v_bias", "w", "gate"), bias)}
+        return hip_simplicial_attention_forward(*[t[s] for t in ops], query_valid=masks[0][s], pair_key_valid=masks[1][s],
+                                                pair_valid=None, precision="ieee_fp32", **kw)
+
+    out, lse, _ = forward(slice(0, B))
+    for b in (0, B - 1):
+        s = slice(b, b + 1)
+        o1, l1, _ = forward(s)
+        assert rel_err(out[s].cpu().numpy(), o1.cpu().double().numpy()) <= 4e-6
+        assert rel_err(lse[s].cpu().numpy(), l1.cpu().double().numpy()) <= 4e-6
+        zero = torch.zeros(1, H, n, D)
+        want, _ = fp64_grads([t[s] for t in (q, k1, v1, k2, v2)], qv[s], pkv[s], None, zero,
+                             bias=None if bias is None else [t[s] for t in bias])
+        assert rel_err(out[s].cpu().numpy(), want) <= 4e-6
+
+
 def test_large_and_masking_scale_logits(cuda):
     """Logits far past the first tile's maximum in both directions (the offset moves many times) and bias terms of
     -30000 beside ordinary ones; padded queries, a molecule without keys and one without queries give zeros."""
