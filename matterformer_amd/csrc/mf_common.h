@@ -51,7 +51,7 @@ bool simplicial_pair_f32_serves(const mf_simplicial_fwd_args* a);
 int simplicial_pair_f32_launch(const mf_simplicial_fwd_args* a, int num_cus, hipStream_t stream);
 // Its backward, at most 32 tokens and head_dim <= 32 (simplicial_pair_f32_bwd.hip).
 bool simplicial_pair_f32_bwd_serves(const mf_simplicial_bwd_args* a);
-int simplicial_pair_f32_bwd_launch(const mf_simplicial_bwd_args* a, hipStream_t stream);
+int simplicial_pair_f32_bwd_launch(const mf_simplicial_bwd_args* a, int num_cus, hipStream_t stream);
 
 // Pair-formulation backward for bf16 operands and head_dim 64
 // (simplicial_pair_bwd.hip): every molecule of a call it serves, given

@@ -1086,6 +1086,13 @@ __global__ void __launch_bounds__(256) zero_rows_kernel(Params p) {
   }
 }
 
+// The n elements of each fp32 gradient of the operands.
+__global__ void __launch_bounds__(256) zero_grads_kernel(Params p, size_t n) {
+  const size_t i = size_t(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= n) return;
+  for (void* g : {p.dq, p.dk1, p.dv1, p.dk2, p.dv2}) static_cast<float*>(g)[i] = 0.0f;
+}
+
 // Bias gradients that are written in full: the four tensors are cleared first (one flat pass of 16-byte
 // stores, the last elements one by one), then the kernels write every valid entry.  plane and gates in 16-bit
 // units (twice the elements of fp32 gradients).
@@ -1290,7 +1297,20 @@ static int simplicial_bwd_impl(const mf_simplicial_bwd_args* a, bool bias32, voi
     }
   }
   if (pair) return simplicial_pair_bwd_launch(a, gout16 && !bias32, s);
-  if (simplicial_pair_f32_bwd_serves(a)) return simplicial_pair_f32_bwd_launch(a, s);
+  if (simplicial_pair_f32_bwd_serves(a)) {
+    // a few (molecule, head) of 25 .. 32 tokens without a bias keep one CU each busy there and spread over three roles
+    // of eight indices each here (8 heads, 32 tokens, fills included: one molecule 30 us against 24, four 31 against
+    // 36; 24 tokens 24 against 24; with a bias 39 against 40).  They come with unfilled gradients.
+    if (!has_bias && a->tokens > 24 && int64_t(a->batch) * a->heads <= 16) {
+      const size_t n = size_t(a->batch) * a->heads * a->tokens * D;
+      hipLaunchKernelGGL(zero_grads_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0, s, prm, n);
+      MF_HIP_CHECK(hipGetLastError());
+    } else {
+      DeviceInfo dev;
+      const int st = device_info(&dev);
+      return st != MF_OK ? st : simplicial_pair_f32_bwd_launch(a, dev.num_cus, s);
+    }
+  }
   // other bf16 operands with a bf16 grad_out: bf16 MFMA (K steps of 32 d), which stages grad_out rows as bf16
   // (exact only for a bf16 grad_out).  Everything else -- fp16 operands, or a grad_out of another dtype -- takes
   // the fp32 path, which reads every operand in its own dtype.

@@ -12,9 +12,9 @@
 //          operand of K step r as it is
 //   dq^T [d][query] += W^T [d][pair] dS^T [pair][query]: dS turned through a per-wave LDS scratch
 //   dk1_j = sum_k G_jk (.) k2_k, dk2_k = sum_j G_jk (.) k1_j (dv1, dv2 from H)
-// One workgroup of four waves per (molecule, head); a wave takes j = wave, wave + 4, ... with both key tiles of a
+// One workgroup of W = 4 or 8 waves per (molecule, head); a wave takes j = wave, wave + W, ... with both key tiles of a
 // molecule inside, so dk1_j / dv1_j are finished by one reduction over the lanes that hold the keys, and dq, dk2,
-// dv2 partials of the four waves are added in wave order at the end.  MFMA-bound: 80 MFMA of 32 cycles per (j, 16
+// dv2 partials of the waves are added in wave order at the end.  MFMA-bound: 80 MFMA of 32 cycles per (j, 16
 // keys) at two query tiles, with the rest (about 150 VALU and LDS instructions) beside them.
 #include <algorithm>
 
@@ -23,8 +23,6 @@
 namespace mf {
 namespace spf32b {
 
-constexpr int kWaves = 4;
-constexpr int kThreads = kWaves * 64;
 constexpr int MN = 32;        // tokens at most
 constexpr int DP = 32;        // head_dim at most
 constexpr int KS = DP + 4;    // row stride (floats)
@@ -61,18 +59,20 @@ struct Params {
   int H, N, D;
 };
 
-// LDS (floats)
+// LDS of W waves (floats)
+template <int W>
 struct Lds {
-  float op[6][MN * KS];                 // q, go, k1, v1, k2, v2 (compacted, zero past the counts); later the partials
-  float scr[kWaves][2][16 * SS];        // dS of a query tile, [pair][query]
+  float op[W > 6 ? W : 6][MN * KS];     // q, go, k1, v1, k2, v2 (compacted, zero past the counts); later the partials
+  float scr[W][2][16 * SS];             // dS of a query tile, [pair][query]
   float lse2[MN], dlt[MN];
   uint32_t bits[MN];                    // valid keys of each j
   int kidx[MN], qidx[MN];
 };
+template <int W>
 struct LdsBias {
   float ut[MN * KS], vt[MN * KS], w[MN * KS];  // u^T [j][i], v^T [k][i], w [j][k]
   float gate[MN];
-  float dg[kWaves][MN];
+  float dg[W][MN];
 };
 
 __device__ __forceinline__ float load_any(const void* p, size_t idx, int dtype) {
@@ -109,14 +109,15 @@ __device__ __forceinline__ float sum_groups(float x) {
   return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
-// Rows 0 .. n - 1 of the four waves' partials (row stride KS, wave stride MN KS) added in wave order into the rows
+// Rows 0 .. n - 1 of the waves' partials (row stride KS, wave stride MN KS) added in wave order into the rows
 // of `dst` that idx names.
+template <int W>
 __device__ __forceinline__ void write_rows(const float* part, float* dst, const int* idx, int n, int D, size_t rbase) {
-  for (int u = threadIdx.x; u < n * (D / 4); u += kThreads) {
+  for (int u = threadIdx.x; u < n * (D / 4); u += W * 64) {
     const int i = u / (D / 4), c = 4 * (u % (D / 4));
     float4 s = *reinterpret_cast<const float4*>(part + i * KS + c);
 #pragma unroll
-    for (int w = 1; w < kWaves; ++w) {
+    for (int w = 1; w < W; ++w) {
       const float4 x = *reinterpret_cast<const float4*>(part + w * MN * KS + i * KS + c);
       s.x += x.x; s.y += x.y; s.z += x.z; s.w += x.w;
     }
@@ -125,8 +126,9 @@ __device__ __forceinline__ void write_rows(const float* part, float* dst, const 
 }
 
 // NT query tiles, NK key tiles.
-template <int NT, int NK, bool BIAS>
-__device__ __forceinline__ void body(const Params& p, Lds& L, LdsBias* X, int nk, int nq, size_t rbase) {
+template <int NT, int NK, bool BIAS, int W>
+__device__ __forceinline__ void body(const Params& p, Lds<W>& L, LdsBias<W>* X, int nk, int nq, size_t rbase) {
+  constexpr int kThreads = W * 64;
   const int lane = lane_id(), wave = wave_id();
   const int g = lane >> 4, r16 = lane & 15;
   const int N = p.N, D = p.D;
@@ -171,7 +173,7 @@ __device__ __forceinline__ void body(const Params& p, Lds& L, LdsBias* X, int nk
     }
   }
 
-  for (int j = wave; j < nk; j += kWaves) {
+  for (int j = wave; j < nk; j += W) {
     const uint32_t bits = L.bits[j];
     float k1a[NC], v1a[NC];  // d = NC g + c
 #pragma unroll
@@ -358,8 +360,8 @@ __device__ __forceinline__ void body(const Params& p, Lds& L, LdsBias* X, int nk
     }
   }
 
-  // ---- the four waves' partials ----
-  float* part = &L.op[0][0];  // [4][MN][KS] over the operands
+  // ---- the waves' partials ----
+  float* part = &L.op[0][0];  // [W][MN][KS] over the operands
   __syncthreads();
 #pragma unroll
   for (int t = 0; t < NT; ++t)
@@ -368,7 +370,7 @@ __device__ __forceinline__ void body(const Params& p, Lds& L, LdsBias* X, int nk
       *reinterpret_cast<float4*>(part + wave * MN * KS + (16 * t + r16) * KS + 16 * dt + 4 * g) =
           float4{dqa[t][dt][0], dqa[t][dt][1], dqa[t][dt][2], dqa[t][dt][3]};
   __syncthreads();
-  write_rows(part, p.dq, L.qidx, nq, D, rbase);
+  write_rows<W>(part, p.dq, L.qidx, nq, D, rbase);
 #pragma unroll
   for (int which = 0; which < 2; ++which) {
     __syncthreads();
@@ -381,7 +383,7 @@ __device__ __forceinline__ void body(const Params& p, Lds& L, LdsBias* X, int nk
             float4{a[0], a[1], a[2], a[3]};
       }
     __syncthreads();
-    write_rows(part, which ? p.dv2 : p.dk2, L.kidx, nk, D, rbase);
+    write_rows<W>(part, which ? p.dv2 : p.dk2, L.kidx, nk, D, rbase);
   }
   if constexpr (BIAS) {
     __syncthreads();
@@ -401,13 +403,18 @@ __device__ __forceinline__ void body(const Params& p, Lds& L, LdsBias* X, int nk
     if (p.dvb != nullptr) {
       for (int u = threadIdx.x; u < nq * nk; u += kThreads) {
         const int i = u / nk, k = u % nk, o = k * KS + i;
-        const float s = ((part[o] + part[MN * KS + o]) + part[2 * MN * KS + o]) + part[3 * MN * KS + o];
+        float s = part[o];
+#pragma unroll
+        for (int w = 1; w < W; ++w) s += part[w * MN * KS + o];
         p.dvb[(rbase + L.qidx[i]) * N + L.kidx[k]] = X->gate[i] * s;
       }
     }
     if (p.dgate != nullptr && int(threadIdx.x) < nq) {
       const int i = threadIdx.x;
-      p.dgate[rbase + L.qidx[i]] = ((X->dg[0][i] + X->dg[1][i]) + X->dg[2][i]) + X->dg[3][i];
+      float s = X->dg[0][i];
+#pragma unroll
+      for (int w = 1; w < W; ++w) s += X->dg[w][i];
+      p.dgate[rbase + L.qidx[i]] = s;
     }
   }
 }
@@ -416,7 +423,7 @@ __device__ __forceinline__ void body(const Params& p, Lds& L, LdsBias* X, int nk
 // five launches, nine with a bias (forward and backward of 128 molecules of up to 29 atoms, 8 heads of 32: 138 -> 122
 // us).  Called after the
 // operand loads have arrived: a load that waits behind stores waits for them too.
-template <bool BIAS>
+template <bool BIAS, int W>
 __device__ __forceinline__ void zero_padding(const Params& p, unsigned long long mk, unsigned long long mq, size_t rbase) {
   const int N = p.N, D = p.D;
   const int row = threadIdx.x / (DP / 4), c = 4 * (threadIdx.x % (DP / 4));
@@ -431,7 +438,7 @@ __device__ __forceinline__ void zero_padding(const Params& p, unsigned long long
     }
   }
   if constexpr (BIAS) {
-    for (int u = threadIdx.x; u < N * N; u += kThreads) {
+    for (int u = threadIdx.x; u < N * N; u += W * 64) {
       const int a = u / N, e = u % N;
       const size_t o = rbase * N + u;
       const bool k = (mk >> e) & 1u, q = k && ((mq >> a) & 1u), j = k && ((mk >> a) & 1u);
@@ -443,11 +450,13 @@ __device__ __forceinline__ void zero_padding(const Params& p, unsigned long long
   }
 }
 
-template <bool BIAS>
-__global__ void __launch_bounds__(kThreads, 2) pair_f32_bwd_kernel(Params p) {
-  __shared__ __attribute__((aligned(16))) Lds L;
+template <bool BIAS, int W>
+__global__ void __launch_bounds__(W * 64, 2) pair_f32_bwd_kernel(Params p) {
+  constexpr int kThreads = W * 64;
   extern __shared__ __attribute__((aligned(16))) unsigned char dyn[];
-  LdsBias* X = reinterpret_cast<LdsBias*>(dyn);
+  Lds<W>& L = *reinterpret_cast<Lds<W>*>(dyn);
+  LdsBias<W>* X = reinterpret_cast<LdsBias<W>*>(dyn + sizeof(Lds<W>));
+  static_assert(sizeof(Lds<W>) % 16 == 0, "16-byte rows");
   const int N = p.N, D = p.D;
   const int tid = threadIdx.x, lane = lane_id();
   const int bh = blockIdx.x, b = bh / p.H;
@@ -457,16 +466,17 @@ __global__ void __launch_bounds__(kThreads, 2) pair_f32_bwd_kernel(Params p) {
   const unsigned long long mk = __ballot(vk), mq = __ballot(vq);
   const int nk = __popcll(mk), nq = __popcll(mq);
   if (nk == 0 || nq == 0) {  // no pair or no query: every gradient is zero
-    zero_padding<BIAS>(p, 0ull, 0ull, rbase);
+    zero_padding<BIAS, W>(p, 0ull, 0ull, rbase);
     return;
   }
   const unsigned long long below = (1ull << lane) - 1ull;
   if (vk) L.kidx[__popcll(mk & below)] = lane;  // (every wave writes the same lists)
   if (vq) L.qidx[__popcll(mq & below)] = lane;
   __syncthreads();
-  // ---- stage the six operands (row u / 8, 16-byte piece u % 8: one row per eight threads) and go . out ----
-  {
-    static_assert(kThreads == MN * (DP / 4), "one pass");
+  // ---- stage the six operands (row u / 8, 16-byte piece u % 8: one row per eight threads, the first 256) and
+  // go . out ----
+  static_assert(kThreads >= MN * (DP / 4) && MN * (DP / 4) % 64 == 0, "one pass of whole waves");
+  if (tid < MN * (DP / 4)) {
     const int row = tid / (DP / 4), c = 4 * (tid % (DP / 4)), cc = min(c, D - 4);
     const size_t oq = (rbase + L.qidx[min(row, nq - 1)]) * D + cc, ok = (rbase + L.kidx[min(row, nk - 1)]) * D + cc;
     float4 x[6], o;
@@ -508,27 +518,43 @@ __global__ void __launch_bounds__(kThreads, 2) pair_f32_bwd_kernel(Params p) {
     bits |= __float_as_uint(dpp<kXor2>(__uint_as_float(bits)));
     bits |= __float_as_uint(dpp<0x141>(__uint_as_float(bits)));
     if (c == 0) L.bits[j] = bits;
-    if constexpr (BIAS) {
-      for (int u = tid; u < MN * MN; u += kThreads) {
-        const int a = u / MN, e = u % MN;
-        const size_t qk = (rbase + L.qidx[min(a, nq - 1)]) * N + L.kidx[min(e, nk - 1)];
-        X->ut[e * KS + a] = load_any(p.u, qk, p.bias_dtype);
-        X->vt[e * KS + a] = load_any(p.v, qk, p.bias_dtype);
-        X->w[a * KS + e] = load_any(p.w, (rbase + L.kidx[min(a, nk - 1)]) * N + L.kidx[min(e, nk - 1)], p.bias_dtype);
-      }
-      // (1 on the padding rows: there lse = inf makes P = 0 whatever finite or -inf terms it multiplies)
-      if (tid < MN) X->gate[tid] = tid < nq ? load_any(p.gate, rbase + L.qidx[tid], p.bias_dtype) : 1.0f;
+  }
+  if constexpr (BIAS) {
+    for (int u = tid; u < MN * MN; u += kThreads) {
+      const int a = u / MN, e = u % MN;
+      const size_t qk = (rbase + L.qidx[min(a, nq - 1)]) * N + L.kidx[min(e, nk - 1)];
+      X->ut[e * KS + a] = load_any(p.u, qk, p.bias_dtype);
+      X->vt[e * KS + a] = load_any(p.v, qk, p.bias_dtype);
+      X->w[a * KS + e] = load_any(p.w, (rbase + L.kidx[min(a, nk - 1)]) * N + L.kidx[min(e, nk - 1)], p.bias_dtype);
     }
+    // (1 on the padding rows: there lse = inf makes P = 0 whatever finite or -inf terms it multiplies)
+    if (tid < MN) X->gate[tid] = tid < nq ? load_any(p.gate, rbase + L.qidx[tid], p.bias_dtype) : 1.0f;
   }
   __syncthreads();
-  zero_padding<BIAS>(p, mk, mq, rbase);
+  zero_padding<BIAS, W>(p, mk, mq, rbase);
   if (nq > 16) {
-    if (nk > 16) body<2, 2, BIAS>(p, L, X, nk, nq, rbase);
-    else body<2, 1, BIAS>(p, L, X, nk, nq, rbase);
+    if (nk > 16) body<2, 2, BIAS, W>(p, L, X, nk, nq, rbase);
+    else body<2, 1, BIAS, W>(p, L, X, nk, nq, rbase);
   } else {
-    if (nk > 16) body<1, 2, BIAS>(p, L, X, nk, nq, rbase);
-    else body<1, 1, BIAS>(p, L, X, nk, nq, rbase);
+    if (nk > 16) body<1, 2, BIAS, W>(p, L, X, nk, nq, rbase);
+    else body<1, 1, BIAS, W>(p, L, X, nk, nq, rbase);
   }
+}
+
+template <bool BIAS, int W>
+int launch(const Params& p, int bh, hipStream_t stream) {
+  constexpr size_t lds = sizeof(Lds<W>) + (BIAS ? sizeof(LdsBias<W>) : 0);
+  const int st = ensure_dynamic_lds(reinterpret_cast<const void*>(pair_f32_bwd_kernel<BIAS, W>), int(lds));
+  if (st != MF_OK) return st;
+  hipLaunchKernelGGL((pair_f32_bwd_kernel<BIAS, W>), dim3(unsigned(bh)), dim3(W * 64), lds, stream, p);
+  MF_HIP_CHECK(hipGetLastError());
+  return MF_OK;
+}
+
+// Four waves a (molecule, head), two of its workgroups to a CU; eight where every workgroup has a CU to itself.
+template <bool BIAS>
+int launch_for(const Params& p, int bh, int num_cus, hipStream_t stream) {
+  return bh <= num_cus ? launch<BIAS, 8>(p, bh, stream) : launch<BIAS, 4>(p, bh, stream);
 }
 
 }  // namespace spf32b
@@ -548,7 +574,7 @@ bool simplicial_pair_f32_bwd_serves(const mf_simplicial_bwd_args* a) {
   return true;
 }
 
-int simplicial_pair_f32_bwd_launch(const mf_simplicial_bwd_args* a, hipStream_t stream) {
+int simplicial_pair_f32_bwd_launch(const mf_simplicial_bwd_args* a, int num_cus, hipStream_t stream) {
   using namespace spf32b;
   Params p{};
   p.q = static_cast<const float*>(a->q);
@@ -572,13 +598,8 @@ int simplicial_pair_f32_bwd_launch(const mf_simplicial_bwd_args* a, hipStream_t 
   p.dgate = static_cast<float*>(a->dgate);
   p.bias_dtype = a->bias_dtype;
   p.H = a->heads; p.N = a->tokens; p.D = a->head_dim;
-  const dim3 grid(unsigned(a->batch * a->heads));
-  if (a->bias_u != nullptr)
-    hipLaunchKernelGGL(pair_f32_bwd_kernel<true>, grid, dim3(kThreads), sizeof(LdsBias), stream, p);
-  else
-    hipLaunchKernelGGL(pair_f32_bwd_kernel<false>, grid, dim3(kThreads), 0, stream, p);
-  MF_HIP_CHECK(hipGetLastError());
-  return MF_OK;
+  const int bh = a->batch * a->heads;
+  return a->bias_u != nullptr ? launch_for<true>(p, bh, num_cus, stream) : launch_for<false>(p, bh, num_cus, stream);
 }
 
 }  // namespace mf

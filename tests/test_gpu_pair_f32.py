@@ -95,6 +95,26 @@ def test_both_workgroup_shapes_of_the_forward(cuda, B, H, n, D, with_bias):
         assert rel_err(out[s].cpu().numpy(), want) <= 4e-6
 
 
+@pytest.mark.parametrize("with_bias", [False, True], ids=["none", "bias"])
+@pytest.mark.parametrize("B,n,D", [(64, 17, 32), (65, 17, 32), (65, 32, 20), (66, 9, 32)])
+def test_both_workgroup_shapes_of_the_backward(cuda, B, n, D, with_bias):
+    """Eight waves a (molecule, head) up to one workgroup per CU (256), four past it; bar as above."""
+    H = 4
+    counts = [n - b % 4 for b in range(B)]
+    q, k1, v1, k2, v2, qv, pkv, _ = random_simplicial(B, H, n, D, seed=B + n, counts=counts, std=logit_std(D))
+    gen = torch.Generator().manual_seed(B)
+    go = torch.randn(B, H, n, D, generator=gen)
+    bias = None
+    if with_bias:
+        bias = [torch.randn(B, H, n, n, generator=gen) * 0.5 for _ in range(3)] + [torch.rand(B, H, n, generator=gen)]
+    ops = [q, k1, v1, k2, v2]
+    _, got = hip_grads([t.to(cuda) for t in ops], qv.to(cuda), pkv.to(cuda), None, go.to(cuda), "ieee_fp32",
+                       bias=None if bias is None else [t.to(cuda) for t in bias])
+    _, ref = fp64_grads(ops, qv, pkv, None, go, bias=bias)
+    for name, g, r in zip(GRAD_NAMES, got, ref):
+        assert rel_err(g.cpu().numpy(), r) <= 4e-6, name
+
+
 def test_large_and_masking_scale_logits(cuda):
     """Logits far past the first tile's maximum in both directions (the offset moves many times) and bias terms of
     -30000 beside ordinary ones; padded queries, a molecule without keys and one without queries give zeros."""
