@@ -69,6 +69,7 @@ struct Params {
   float* out[3];
   QueueSize queue;
   int B, N, R, hidden, heads;
+  int splits, cols;  // items per row, columns of one (a multiple of 64)
   // periodic features (PER instantiations): nf Fourier frequencies, the molecule's 6 global features
   int nf;
   const float* freqs;
@@ -123,8 +124,8 @@ __device__ __forceinline__ void scan_row(long long s, int B, int& b, int& i) {
   b = int((unsigned(r) + (unsigned(i) * 0x9E3779B1u >> 8) % unsigned(B)) % unsigned(B));
 }
 
-// Valid columns of (b, i) from j0: one ballot per 64 columns.
-__device__ __forceinline__ void row_bits(const uint8_t* mask, int N, int b, int i, int j0, int groups, int lane,
+// Valid columns of (b, i) from j0 to j1 - 1: one ballot per 64 columns.
+__device__ __forceinline__ void row_bits(const uint8_t* mask, int N, int b, int i, int j0, int j1, int groups, int lane,
                                          unsigned long long (&bal)[kSegGroups]) {
   uint8_t v[kSegGroups];
 #pragma unroll
@@ -133,7 +134,7 @@ __device__ __forceinline__ void row_bits(const uint8_t* mask, int N, int b, int 
 #pragma unroll
   for (int c = 0; c < kSegGroups; ++c) {
     const int j = j0 + 64 * c + lane;
-    bal[c] = __ballot(c < groups && j < N && j != i && v[c] != 0);
+    bal[c] = __ballot(c < groups && j < j1 && j != i && v[c] != 0);
   }
 }
 
@@ -262,10 +263,10 @@ __global__ void __launch_bounds__(kThreads, PER ? 1 : 4) pair_mlp_kernel(Params 
   __shared__ int counts[kWaves];
   const int wave = tid >> 6;
   const int sw = 64 * p.queue.seg_groups;  // columns scanned at a time
-  const long long rows = (long long)B * N;
+  const long long items = (long long)B * N * p.splits;
   const long long stride = (long long)gridDim.x * kWaves;
   int pending = 0;
-  // the first `tiles` tiles of the queue (the last one may be short): features, MLPs, stores
+  // the tiles of the queue's first n pairs (the last one may be short): features, MLPs, stores
   auto run_tiles = [&](int n) {
     for (int t0 = wave * kTile; t0 < n; t0 += kBatch) {
       bool pv[2];
@@ -333,18 +334,25 @@ __global__ void __launch_bounds__(kThreads, PER ? 1 : 4) pair_mlp_kernel(Params 
       }
     }
   };
-  for (long long s0 = (long long)blockIdx.x; s0 < rows; s0 += stride) {
+  for (long long s0 = (long long)blockIdx.x; s0 < items; s0 += stride) {
     const long long s = s0 + (long long)wave * gridDim.x;
-    const bool on = s < rows;
-    int b = 0, i = 0;
-    if (on) scan_row(s, B, b, i);
-    for (int j0 = 0; j0 < N; j0 += sw) {
+    const bool on = s < items;
+    int b = 0, i = 0, begin = 0, end = 0;
+    if (on) {
+      scan_row(s, B, b, i);  // i: item i % splits of row i / splits
+      const int part = i % p.splits;
+      i /= p.splits;
+      begin = part * p.cols;
+      end = min(N, begin + p.cols);
+    }
+    for (int jo = 0; jo < p.cols; jo += sw) {
+      const int j0 = begin + jo;
       unsigned long long bal[kSegGroups];
 #pragma unroll
       for (int c = 0; c < kSegGroups; ++c) bal[c] = 0ull;
       int mine = 0;
       if (on) {
-        row_bits(p.mask, N, b, i, j0, p.queue.seg_groups, lane, bal);
+        row_bits(p.mask, N, b, i, j0, end, p.queue.seg_groups, lane, bal);
 #pragma unroll
         for (int c = 0; c < kSegGroups; ++c) mine += __popcll(bal[c]);
       }
@@ -368,7 +376,7 @@ __global__ void __launch_bounds__(kThreads, PER ? 1 : 4) pair_mlp_kernel(Params 
 #pragma unroll
             for (int c = 0; c < kSegGroups; ++c) {
               const int j = 64 * c + lane;
-              if (c < p.queue.seg_groups && j0 + j < N && !((bal[c] >> lane) & 1ull)) dst[j] = 0.0f;
+              if (c < p.queue.seg_groups && j0 + j < end && !((bal[c] >> lane) & 1ull)) dst[j] = 0.0f;
             }
           }
       }
@@ -409,8 +417,16 @@ int launch(Params p, int num_cus, int max_lds, hipStream_t s) {
   const int st = ensure_dynamic_lds(reinterpret_cast<const void*>(pair_mlp_kernel<KS, KP, PER>),
                                     max_lds - int(sizeof(int)) * kWaves);
   if (st != MF_OK) return st;
+  // items: whole rows, or pieces of 64 columns and more as long as a CU does not get a second workgroup of eight (each
+  // stages the weights).  Hidden 128: one molecule of 181 / 256 atoms 165 / 201 us in whole rows, 89 / 86 in pieces
+  // (111 / 113 on the kernel that dealt out 64-column groups); four of 256 215 -> 138; four of 400 (200 workgroups
+  // of whole rows) 323, in halves 372.
   const long long rows = (long long)p.B * p.N;
-  const int grid = int(std::min<long long>((rows + 7) / 8, (long long)num_cus * 2));
+  const int groups = (p.N + 63) / 64;
+  const long long want = std::max(1LL, (long long)num_cus * kWaves / rows);
+  p.cols = 64 * int((groups + std::min<long long>(want, groups) - 1) / std::min<long long>(want, groups));
+  p.splits = (p.N + p.cols - 1) / p.cols;
+  const int grid = int(std::min<long long>((rows * p.splits + kWaves - 1) / kWaves, (long long)num_cus * 2));
   hipLaunchKernelGGL((pair_mlp_kernel<KS, KP, PER>), dim3(grid), dim3(kThreads), lds, s, p);
   MF_HIP_CHECK(hipGetLastError());
   return MF_OK;
@@ -601,7 +617,7 @@ __global__ void __launch_bounds__(kBwdThreads, 2) pair_mlp_bwd_kernel(BwdParams 
       for (int c = 0; c < kSegGroups; ++c) bal[c] = 0ull;
       int mine = 0;
       if (on) {
-        row_bits(p.mask, N, b, i, j0, p.queue.seg_groups, lane, bal);
+        row_bits(p.mask, N, b, i, j0, N, p.queue.seg_groups, lane, bal);
 #pragma unroll
         for (int c = 0; c < kSegGroups; ++c) mine += __popcll(bal[c]);
       }

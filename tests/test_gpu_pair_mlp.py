@@ -228,10 +228,11 @@ def test_periodic_features_match_torch(cuda, n_freqs, R):
 
 
 @pytest.mark.parametrize("B,N,hidden,H,R", [(1, 2, 16, 1, 4), (2, 65, 48, 8, 16), (2, 257, 256, 4, 29),
-                                            (70, 3, 128, 16, 28)])
+                                            (70, 3, 128, 16, 28), (1, 181, 128, 8, 16), (3, 129, 64, 4, 12)])
 def test_queue_edges_match_torch(cuda, B, N, hidden, H, R):
     """The queues of valid pairs at their edges: almost no pair, rows of one column past a 64-column group, more than
-    one scan of a row with weights that leave the smaller queue, many tiny molecules; forward and, where it is
+    one scan of a row with weights that leave the smaller queue, many tiny molecules, few molecules whose rows are
+    scanned in pieces (whole pieces and a last one of a single column); forward and, where it is
     served, the weight gradients; padded atoms passed beside the pair mask come out zero.  Both sides read the same
     features (the rbf turn an ulp of d_norm into 1e-4 of a term at 28 centres).  Bar 1e-5 of the largest term of
     the tensor and 5e-7 beside it: the two pairs of a two-atom molecule may hold one small output, the cancelling
