@@ -269,7 +269,11 @@ int mf_simplicial_bwd_writes_all(const mf_simplicial_bwd_args* args);
 /* Bytes of workspace the backward uses (0: none).  With a message term, per */
 /* query the message coefficients dc = basis . go and sum_jk P ML MR; at     */
 /* head_dim 64, the pair kernel's plan and partial sums (a smaller or NULL   */
-/* workspace there is accepted and the general kernel runs).                 */
+/* workspace there is accepted and the general kernel runs).  _bytes: of     */
+/* these arguments (sizes, types and which terms and gradients are given;    */
+/* the workspace fields are not read); _size: enough for any call of the     */
+/* shape, the partial sums of every bias gradient included.                  */
+uint64_t mf_simplicial_bwd_workspace_bytes(const mf_simplicial_bwd_args* args);
 uint64_t mf_simplicial_bwd_workspace_size(int32_t batch, int32_t heads, int32_t tokens,
                                           int32_t head_dim, int32_t message_rank);
 

@@ -42,6 +42,7 @@ EXPORTED_SYMBOLS = (
     "mf_simplicial_bwd",
     "mf_simplicial_bwd_leaf",
     "mf_simplicial_bwd_writes_all",
+    "mf_simplicial_bwd_workspace_bytes",
     "mf_simplicial_bwd_workspace_size",
     "mf_knn",
     "mf_knn_mask",
@@ -270,6 +271,8 @@ def _load() -> ctypes.CDLL | None:
     lib.mf_simplicial_fwd_workspace_size.restype = ctypes.c_uint64
     lib.mf_simplicial_bwd_writes_all.argtypes = [ctypes.POINTER(MfSimplicialBwdArgs)]
     lib.mf_simplicial_bwd_writes_all.restype = ctypes.c_int
+    lib.mf_simplicial_bwd_workspace_bytes.argtypes = [ctypes.POINTER(MfSimplicialBwdArgs)]
+    lib.mf_simplicial_bwd_workspace_bytes.restype = ctypes.c_uint64
     lib.mf_simplicial_bwd_workspace_size.argtypes = [ctypes.c_int32] * 5
     lib.mf_simplicial_bwd_workspace_size.restype = ctypes.c_uint64
     if getattr(lib, "mf_pair_mlp_bias_bwd_workspace_size", None) is not None:

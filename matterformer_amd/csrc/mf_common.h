@@ -58,7 +58,8 @@ int simplicial_pair_f32_bwd_launch(const mf_simplicial_bwd_args* a, int num_cus,
 // simplicial_pair_bwd_workspace_bytes() of 256-byte aligned workspace (a plan
 // of units, atom lists and partial sums).
 bool simplicial_pair_bwd_serves(const mf_simplicial_bwd_args* a);
-size_t simplicial_pair_bwd_workspace_bytes(int batch, int heads, int tokens);
+size_t simplicial_pair_bwd_workspace_bytes(int batch, int heads, int tokens);  // of any call of the shape
+size_t simplicial_pair_bwd_workspace_bytes(const mf_simplicial_bwd_args* a);   // of this call
 // (bias16: the bias gradients are bf16, else fp32)
 int simplicial_pair_bwd_launch(const mf_simplicial_bwd_args* a, bool bias16, hipStream_t stream);
 

@@ -1339,6 +1339,12 @@ extern "C" int mf_simplicial_bwd_leaf(const mf_simplicial_bwd_args* a, void* str
   return simplicial_bwd_impl(a, true, stream);
 }
 
+extern "C" uint64_t mf_simplicial_bwd_workspace_bytes(const mf_simplicial_bwd_args* a) {
+  if (a == nullptr) return 0;
+  if (a->message_left != nullptr) return message_workspace_bytes(a->batch, a->heads, a->tokens, a->message_rank);
+  return uint64_t(mf::simplicial_pair_bwd_workspace_bytes(a));
+}
+
 extern "C" uint64_t mf_simplicial_bwd_workspace_size(int32_t batch, int32_t heads, int32_t tokens, int32_t head_dim,
                                                      int32_t message_rank) {
   if (batch <= 0 || heads <= 0 || tokens <= 0) return 0;

@@ -152,30 +152,20 @@ struct Params {
   int H, N, cap;
 };
 
-// Workspace of the pair path (16-byte aligned regions).
-constexpr size_t kWsTarget = size_t(16) << 30;  // bytes; calls past kWsLimit take the ownership kernel
-constexpr size_t kWsLimit = size_t(48) << 30;
+// Workspace of the pair path (16-byte aligned regions): what the call uses, no more.  The partial sums of the bias
+// gradients are laid out for those that are wanted (dw's only where a molecule can have a second query block).
+constexpr size_t kWsTarget = size_t(1) << 30;                   // bytes that any call may take, and per (molecule,
+constexpr size_t kWsPerHead = 420 << 10, kWsPerHeadBias = 1 << 20;  // head) what a large one may
+constexpr size_t kWsLimit = size_t(48) << 30;                   // calls past it take the ownership kernel
 struct Ws {
   int cap;  // units per (molecule, head) at most
+  bool dv, dg, dw;
   size_t units, counts, lists, slab, dvpart, dgpart, dwpart, bytes;
-  Ws(int B, int H, int N) {
-    const size_t bh = size_t(B) * H, n = size_t(N);
-    // a few units per CU are enough: large batches get three per (molecule, head), small ones as many as give
-    // 2048 units (4 j each at the least); fewer where the partial sums would pass kWsTarget
-    cap = int(std::min<size_t>(std::min<size_t>(std::max<size_t>(3, 2048 / bh), (n + 3) / 4), 64));
-    while (layout(B, bh, n) > kWsTarget && cap > 1) --cap;
-  }
-  size_t layout(int B, size_t bh, size_t n) {
-    units = 16;
-    counts = units + ((bh * cap * 4 + 15) & ~size_t(15));
-    lists = counts + size_t(B) * 8;
-    slab = (lists + size_t(B) * 2 * n * 2 + 255) & ~size_t(255);
-    dvpart = slab + bh * cap * 3 * n * DP * 4;
-    dgpart = dvpart + bh * cap * n * n * 4;
-    dwpart = (dgpart + bh * cap * n * 4 + 15) & ~size_t(15);
-    bytes = dwpart + bh * n * n * 4;
-    return bytes;
-  }
+  Ws(int B, int H, int N, bool bias, bool dv_, bool dg_, bool dw_);
+  explicit Ws(const mf_simplicial_bwd_args* a)
+      : Ws(a->batch, a->heads, a->tokens, a->bias_u != nullptr, a->dv_bias != nullptr, a->dgate != nullptr,
+           a->dw != nullptr) {}
+  size_t layout(int B, size_t bh, size_t n);
 };
 
 struct PlanParams {
@@ -233,6 +223,27 @@ struct Lay {
 __device__ __forceinline__ int ceil_div_small(int n, int d) {
   return int((float(n + d) - 0.5f) * __builtin_amdgcn_rcpf(float(d)));
 }
+inline Ws::Ws(int B, int H, int N, bool bias, bool dv_, bool dg_, bool dw_)
+    : dv(dv_), dg(dg_), dw(dw_ && N > Lay<true>::QM) {
+  const size_t bh = size_t(B) * H, n = size_t(N);
+  // a few units per CU are enough: large batches get three per (molecule, head), small ones as many as give 2048 units
+  // (4 j each at the least); fewer where the partial sums would pass the target
+  const size_t target = std::max(kWsTarget, bh * (bias ? kWsPerHeadBias : kWsPerHead));
+  cap = int(std::min<size_t>(std::min<size_t>(std::max<size_t>(3, 2048 / bh), (n + 3) / 4), 64));
+  while (layout(B, bh, n) > target && cap > 1) --cap;
+}
+inline size_t Ws::layout(int B, size_t bh, size_t n) {
+  units = 16;
+  counts = units + ((bh * cap * 4 + 15) & ~size_t(15));
+  lists = counts + size_t(B) * 8;
+  slab = (lists + size_t(B) * 2 * n * 2 + 255) & ~size_t(255);
+  dvpart = slab + bh * cap * 3 * n * DP * 4;
+  dgpart = dvpart + (dv ? bh * cap * n * n * 4 : 0);
+  dwpart = (dgpart + (dg ? bh * cap * n * 4 : 0) + 15) & ~size_t(15);
+  bytes = dwpart + (dw ? bh * n * n * 4 : 0);
+  return bytes;
+}
+
 // j keys per unit and units of a molecule: `jt` j per unit, at most `cap` units, whole key pairs.
 __device__ __forceinline__ int parts_of(int nk, int jt, int cap) {
   const int pairs = (nk + 1) / 2, most = min(cap, ceil_div_small(nk, jt));
@@ -1392,24 +1403,34 @@ __global__ void __launch_bounds__(kThreads) pair_bwd_finish(Params p) {
 
 }  // namespace pbwd
 
+static size_t within_limit(size_t bytes) { return bytes <= pbwd::kWsLimit ? bytes : 0; }
+
 size_t simplicial_pair_bwd_workspace_bytes(int batch, int heads, int tokens) {
   if (batch <= 0 || heads <= 0 || tokens <= 0 || batch > pbwd::kMaxPlanBatch || tokens > pbwd::kMaxTokens) return 0;
-  const size_t bytes = pbwd::Ws(batch, heads, tokens).bytes;
-  return bytes <= pbwd::kWsLimit ? bytes : 0;
+  // (with fewer bias gradients there may be more units per molecule)
+  size_t most = 0;
+  for (int w = 0; w < 9; ++w)
+    most = std::max(most, within_limit(pbwd::Ws(batch, heads, tokens, w < 8, w & 1, w & 2, w & 4).bytes));
+  return most;
+}
+
+// Bytes that this call uses, 0 when it is not one of the pair kernel's (its buffers' alignment aside).
+size_t simplicial_pair_bwd_workspace_bytes(const mf_simplicial_bwd_args* a) {
+  if (a->dtype != MF_DTYPE_BF16 || a->grad_dtype != MF_DTYPE_BF16 || a->head_dim != pbwd::DP) return 0;
+  if (a->batch <= 0 || a->heads <= 0 || a->tokens <= 0 || a->batch > pbwd::kMaxPlanBatch || a->tokens > pbwd::kMaxTokens)
+    return 0;
+  if (a->angle_left != nullptr || a->message_left != nullptr) return 0;
+  if (a->bias_u != nullptr && a->bias_dtype != MF_DTYPE_BF16 && a->bias_dtype != MF_DTYPE_F32) return 0;
+  return within_limit(pbwd::Ws(a).bytes);
 }
 
 bool simplicial_pair_bwd_serves(const mf_simplicial_bwd_args* a) {
-  if (a->dtype != MF_DTYPE_BF16 || a->grad_dtype != MF_DTYPE_BF16 || a->head_dim != pbwd::DP) return false;
-  const size_t need = simplicial_pair_bwd_workspace_bytes(a->batch, a->heads, a->tokens);
+  const size_t need = simplicial_pair_bwd_workspace_bytes(a);
   if (need == 0 || a->workspace == nullptr || reinterpret_cast<uintptr_t>(a->workspace) % 256 != 0 ||
       a->workspace_bytes < need)
     return false;
   if (int64_t(a->batch) * a->heads >= (1 << 26)) return false;  // unit codes are 32 bits
-  if (a->angle_left != nullptr || a->message_left != nullptr) return false;
-  if (a->bias_u != nullptr) {
-    if (a->bias_dtype != MF_DTYPE_BF16 && a->bias_dtype != MF_DTYPE_F32) return false;
-    if (!a->bias_v || !a->bias_w || !a->bias_gate) return false;
-  }
+  if (a->bias_u != nullptr && (!a->bias_v || !a->bias_w || !a->bias_gate)) return false;
   if (!a->dq || !a->dk1 || !a->dv1 || !a->dk2 || !a->dv2) return false;
   for (const void* ptr : {(const void*)a->q, (const void*)a->k1, (const void*)a->v1, (const void*)a->k2,
                           (const void*)a->v2, (const void*)a->grad_out, (const void*)a->out, (const void*)a->dq,
@@ -1435,7 +1456,7 @@ static int launch_units(const pbwd::Params& p, int blocks, int bh, hipStream_t s
 
 int simplicial_pair_bwd_launch(const mf_simplicial_bwd_args* a, bool bias16, hipStream_t stream) {
   using namespace pbwd;
-  const Ws ws(a->batch, a->heads, a->tokens);
+  const Ws ws(a);
   unsigned char* wsp = static_cast<unsigned char*>(a->workspace);
   const bool g16 = a->grads_dtype == MF_DTYPE_BF16;
   PlanParams pp{};

@@ -424,7 +424,6 @@ def _kernel_backward(grad_out, q, k1, v1, k2, v2, out, lse, query_valid, pair_ke
                                              ("need_dangle_gate", (B, H, N)))):
             if flags[name]:
                 lr_grads[idx] = torch.zeros(shape, device=dev, dtype=torch.float32)
-    rm = 0
     if ext.message is not None:
         rm = int(ext.message[0].shape[-1])
         for idx, (name, shape) in enumerate((("need_dmessage_left", (B, H, N, N, rm)),
@@ -432,9 +431,6 @@ def _kernel_backward(grad_out, q, k1, v1, k2, v2, out, lse, query_valid, pair_ke
                                              ("need_dmessage_basis", (H, rm, D)))):
             if flags[name]:
                 lr_grads[3 + idx] = torch.zeros(shape, device=dev, dtype=torch.float32)
-    # the message term's coefficients, or the pair kernel's plan and partial sums (bf16, head_dim 64)
-    nbytes = int(_native.lib().mf_simplicial_bwd_workspace_size(B, H, N, D, rm))
-    workspace = torch.empty(nbytes, device=dev, dtype=torch.uint8) if nbytes > 0 else None
     f = ext.fields()
     args = _native.MfSimplicialBwdArgs(
         q=ops[0].data_ptr(), k1=ops[1].data_ptr(), v1=ops[2].data_ptr(), k2=ops[3].data_ptr(), v2=ops[4].data_ptr(),
@@ -453,9 +449,18 @@ def _kernel_backward(grad_out, q, k1, v1, k2, v2, out, lse, query_valid, pair_ke
         message_basis=f.get("message_basis"),
         dangle_left=_native.ptr(lr_grads[0]), dangle_right=_native.ptr(lr_grads[1]),
         dangle_gate=_native.ptr(lr_grads[2]), dmessage_left=_native.ptr(lr_grads[3]),
-        dmessage_right=_native.ptr(lr_grads[4]), dmessage_basis=_native.ptr(lr_grads[5]),
-        workspace=_native.ptr(workspace), workspace_bytes=0 if workspace is None else workspace.numel())
+        dmessage_right=_native.ptr(lr_grads[4]), dmessage_basis=_native.ptr(lr_grads[5]))
     lib = _native.lib()
+    # the message term's coefficients, or the pair kernel's plan and partial sums (bf16, head_dim 64)
+    nbytes = int(lib.mf_simplicial_bwd_workspace_bytes(args))
+    if nbytes > 0:
+        try:
+            workspace = torch.empty(nbytes, device=dev, dtype=torch.uint8)
+            args.workspace, args.workspace_bytes = workspace.data_ptr(), nbytes
+        except torch.OutOfMemoryError:
+            if ext.message is not None:
+                raise
+            # without it the call takes the ownership kernel, which needs none
     if not g16 and not lib.mf_simplicial_bwd_writes_all(args):
         for t in (*grads, *bias_grads):
             if t is not None:

@@ -149,5 +149,42 @@ def test_backward_low_rank_arguments_are_validated_before_any_device_call():
     need = lib.mf_simplicial_bwd_workspace_size(2, 2, 8, 16, 8)
     assert need == 2 * 2 * 2 * 8 * 8 * 4
     assert lib.mf_simplicial_bwd_workspace_size(2, 2, 8, 16, 0) == 0
+    assert lib.mf_simplicial_bwd_workspace_bytes(a) == need
     a.workspace, a.workspace_bytes = fake, need - 4
     assert lib.mf_simplicial_bwd(a, None) == _native.MF_ERR_INVALID_ARGUMENT and "workspace" in _native.last_error()
+
+
+def test_backward_workspace_is_what_the_call_uses():
+    """mf_simplicial_bwd_workspace_bytes: nothing for calls that do not reach the pair kernel; the bias gradients'
+    partial sums only where they are wanted; per (molecule, head) of a large call at most 420 KB without a bias and
+    1 MB with one; never more than mf_simplicial_bwd_workspace_size, and 64-bit where it is large."""
+    from itertools import product
+
+    from matterformer_amd import _native
+
+    lib = _native.lib()
+    bf16, f32, fake = _native.MF_DTYPE_BF16, _native.MF_DTYPE_F32, 4096
+
+    def need(B, H, N, D=64, dtype=bf16, grad_dtype=bf16, **given):
+        return lib.mf_simplicial_bwd_workspace_bytes(_native.MfSimplicialBwdArgs(
+            batch=B, heads=H, tokens=N, head_dim=D, dtype=dtype, grad_dtype=grad_dtype, **given))
+
+    bias = dict.fromkeys(("bias_u", "bias_v", "bias_w", "bias_gate"), fake) | dict(bias_dtype=f32)
+    for none in (dict(dtype=f32), dict(grad_dtype=f32), dict(D=32), dict(N=513), dict(B=2049), dict(angle_left=fake),
+                 bias | dict(bias_dtype=_native.MF_DTYPE_F16)):
+        assert need(**(dict(B=2, H=8, N=181) | none)) == 0, none
+    plain = need(64, 8, 181)
+    assert need(64, 8, 181, **bias) == plain  # a bias without gradients adds nothing
+    dv, dw = need(64, 8, 181, **bias, dv_bias=fake), need(64, 8, 181, **bias, dw=fake)
+    assert plain < dw < dv < need(64, 8, 181, **bias, dv_bias=fake, dw=fake, dgate=fake, du=fake)
+    assert need(64, 8, 48, **bias, dw=fake) == need(64, 8, 48, **bias)  # one query block: dw is written at once
+    for B, H, N in ((512, 8, 181), (2048, 8, 29), (512, 8, 512), (2048, 16, 512), (1024, 12, 200)):
+        assert need(B, H, N) <= B * H * (420 << 10) + (2 << 20), (B, H, N)
+    for B, H, N in ((512, 8, 181), (2048, 8, 29), (2048, 8, 100)):
+        every = need(B, H, N, **bias, dv_bias=fake, dw=fake, dgate=fake)
+        assert every <= B * H * (1 << 20) + (2 << 20), (B, H, N)
+    for B, H, N in ((1, 1, 1), (4, 12, 192), (64, 8, 181), (4, 8, 512), (512, 8, 181)):
+        size = lib.mf_simplicial_bwd_workspace_size(B, H, N, 64, 0)
+        for grads in product((None, fake), repeat=4):
+            assert 0 < need(B, H, N, **bias, **dict(zip(("du", "dv_bias", "dw", "dgate"), grads))) <= size
+        assert need(B, H, N) <= size

@@ -206,6 +206,46 @@ def test_queries_and_keys_of_different_counts(cuda):
         assert rel_err(g.float().cpu().numpy(), r) <= bar, (name, rel_err(g.float().cpu().numpy(), r))
 
 
+@pytest.mark.parametrize("bias_dtype", [None, torch.bfloat16, torch.float32], ids=["none", "bf16", "fp32"])
+def test_without_memory_for_the_workspace(cuda, bias_dtype, monkeypatch):
+    """When the workspace cannot be allocated the call runs on the ownership kernel (bf16 products, 2e-2 as in its
+    own tests), with an fp32 bias after the entry that writes the leaves' dtypes has refused it."""
+    import matterformer_amd.hip_simplicial_attention as hsa
+
+    B, H, N, D = 2, 2, 70, 64
+    q, k1, v1, k2, v2, qv, pkv, pv = random_simplicial(B, H, N, D, seed=11, counts=[70, 33], pair_drop=0.1,
+                                                       std=logit_std(D))
+    pv = pv | (torch.arange(N) < 2)[None, None, :]
+    gen = torch.Generator().manual_seed(12)
+    go = torch.randn(B, H, N, D, generator=gen).to(torch.bfloat16)
+    ops = [t.to(torch.bfloat16) for t in (q, k1, v1, k2, v2)]
+    bias = None
+    if bias_dtype is not None:
+        bias = [(torch.randn(B, H, N, N, generator=gen) * 0.5).to(bias_dtype) for _ in range(3)] + \
+               [torch.rand(B, H, N, generator=gen).to(bias_dtype)]
+    args = [[t.to(cuda) for t in ops], qv.to(cuda), pkv.to(cuda), pv.to(cuda), go.to(cuda), "bf16_tc"]
+    dbias = None if bias is None else [t.to(cuda) for t in bias]
+    _, usual = hip_grads(*args, bias=dbias)
+    real, refused = torch.empty, []
+
+    def empty(*a, **k):
+        if k.get("dtype") == torch.uint8:
+            refused.append(a)
+            raise torch.OutOfMemoryError("no memory")
+        return real(*a, **k)
+
+    monkeypatch.setattr(hsa.torch, "empty", empty)
+    _, got = hip_grads(*args, bias=dbias)
+    monkeypatch.undo()
+    assert len(refused) == (2 if bias_dtype == torch.float32 else 1)
+    _, ref = fp64_grads(ops, qv, pkv, pv, go, bias=bias)
+    for name, g, u, r in zip(GRAD_NAMES, got, usual, ref):
+        assert g.dtype == u.dtype
+        assert rel_err(g.float().cpu().numpy(), r) <= 2e-2, name
+        pad = torch.from_numpy(r == 0.0).to(cuda)
+        assert not g[pad].any(), name
+
+
 @pytest.mark.parametrize("wanted", [(True, True, True, True), (False, True, False, False)], ids=["all", "dv"])
 @pytest.mark.parametrize("B,N", [(1, 9), (3, 45), (2, 130)])
 def test_gradients_in_the_leaves_dtypes_are_written_in_full(cuda, B, N, wanted):
