@@ -226,10 +226,12 @@ __device__ __forceinline__ int ceil_div_small(int n, int d) {
 inline Ws::Ws(int B, int H, int N, bool bias, bool dv_, bool dg_, bool dw_)
     : dv(dv_), dg(dg_), dw(dw_ && N > Lay<true>::QM) {
   const size_t bh = size_t(B) * H, n = size_t(N);
-  // a few units per CU are enough: large batches get three per (molecule, head), small ones as many as give 2048 units
-  // (4 j each at the least); fewer where the partial sums would pass the target
+  // a few units per CU are enough: large batches get four per (molecule, head) (256 molecules of 80 tokens, 8 heads,
+  // 1983 us in three of 28 rows, 1850 in four of 20), with a bias, whose blocks of 16 j cost more than their rounds,
+  // three (3370 us, in four 3800); small ones as many as give 2048 units (4 j each at the least); fewer where the
+  // partial sums would pass the target
   const size_t target = std::max(kWsTarget, bh * (bias ? kWsPerHeadBias : kWsPerHead));
-  cap = int(std::min<size_t>(std::min<size_t>(std::max<size_t>(3, 2048 / bh), (n + 3) / 4), 64));
+  cap = int(std::min<size_t>(std::min<size_t>(std::max<size_t>(bias ? 3 : 4, 2048 / bh), (n + 3) / 4), 64));
   while (layout(B, bh, n) > target && cap > 1) --cap;
 }
 inline size_t Ws::layout(int B, size_t bh, size_t n) {
@@ -244,31 +246,44 @@ inline size_t Ws::layout(int B, size_t bh, size_t n) {
   return bytes;
 }
 
-// j keys per unit and units of a molecule: `jt` j per unit, at most `cap` units, whole key pairs.
+// Units of a molecule and their j: about `jt` j per unit, at most `cap` units, and no more than their rounds of four key
+// pairs ask for (a round takes its time with one pair too: 72 j in four units of 18 are twelve rounds, in three of
+// 24 nine); the pairs are shared out evenly.
+__device__ __forceinline__ int rounds_of(int pairs, int parts) { return (ceil_div_small(pairs, parts) + kWaves - 1) / kWaves; }
 __device__ __forceinline__ int parts_of(int nk, int jt, int cap) {
   const int pairs = (nk + 1) / 2, most = min(cap, ceil_div_small(nk, jt));
-  return ceil_div_small(pairs, ceil_div_small(pairs, most));
+  const int parts = ceil_div_small(pairs, kWaves * rounds_of(pairs, most));
+  return ceil_div_small(pairs, ceil_div_small(pairs, parts));
 }
 __device__ __forceinline__ int unit_rows(int nk, int parts) { return 2 * ceil_div_small((nk + 1) / 2, parts); }
 // Blocks of a run of n rows, at most m rows (a multiple of 16) each, cut at multiples of 16.
 __device__ __forceinline__ int blocks_of(int n, int m) { return (n + m - 1) / m; }
 __device__ __forceinline__ int block_rows(int n, int blocks) { return 16 * (((n + 15) / 16 + blocks - 1) / blocks); }
 
-// Relative cost of one unit: per key tile the sums that end it, for each query block, and the rounds of four key
-// pairs (fixed work per query block, and the query tiles); without a bias, staging and slab sums of further block
-// triples.  Two units to a CU take about 0.25 us of it without a bias (22 rows of 44 tokens: 42 us, of 64: 59; of 128:
-// 197 in three rounds, 104 in one), 0.5 us with one (12 rows of 24: 25 us, 16 of 48: 45, 16 of 64: 100; 16 of
-// 192: 700, 8 of 192: 530).
-__device__ __forceinline__ uint32_t unit_cost(int nk, int nq, int parts, const PlanParams& pp) {
-  const int rounds = (unit_rows(nk, parts) + 2 * kWaves - 1) / (2 * kWaves);
-  const int nqt = (nq + 15) / 16, nkt = (nk + 15) / 16;
-  if (pp.bias) {
-    const int nqb = blocks_of(nq, Lay<true>::QM);
-    return uint32_t(nkt * (14 * nqb + rounds * (nqb + 2 * nqt)));
+// Relative cost of one unit: for each j block, per key tile and query block the sums that end the tile, and without a
+// bias the staging and slab sums of further block triples; for each round of four key pairs, per key tile a fixed part
+// for each query block, and the query tiles.  Two units to a CU take about 0.25 us of it without a bias (22 rows of 44
+// tokens: 42 us, of 64: 59; of 128: 197 in three rounds, 104 in one), 0.5 us with one (12 rows of 24: 25 us, 16 of 48:
+// 45, 16 of 64: 100; 16 of 192: 700, 8 of 192: 530).
+struct UnitCost {
+  int block, round;
+  __device__ __forceinline__ UnitCost(int nk, int nq, int bias) {
+    const int nqt = (nq + 15) / 16, nkt = (nk + 15) / 16;
+    if (bias) {
+      const int nqb = blocks_of(nq, Lay<true>::QM);
+      block = nkt * 14 * nqb;
+      round = nkt * (nqb + 2 * nqt);
+    } else {
+      const int nqb = blocks_of(nq, Lay<false>::QM), nkb = blocks_of(nk, Lay<false>::KM);
+      block = nkt * 16 * nqb + 25 * (nqb * nkb - 1);
+      round = nkt * (6 * nqb + 2 * nqt);
+    }
   }
-  const int nqb = blocks_of(nq, Lay<false>::QM), nkb = blocks_of(nk, Lay<false>::KM);
-  return uint32_t(nkt * (8 * nqb + rounds * (6 * nqb + 2 * nqt)) + 25 * (nqb * nkb - 1));
-}
+  // a unit of that many rounds
+  __device__ __forceinline__ int unit(int rounds, int jm) const {
+    return ceil_div_small(rounds, jm / (2 * kWaves)) * block + rounds * round;
+  }
+};
 
 typedef __attribute__((__vector_size__(4 * sizeof(_Float16)))) _Float16 mf_f16x4;
 
@@ -505,7 +520,8 @@ __global__ void __launch_bounds__(kPlanThreads) pair_bwd_prepare(PlanParams pp) 
       const int nk = s_count[2 * b], nq = s_count[2 * b + 1];
       if (nk <= 0 || nq <= 0 || l == 3) continue;
       const int parts = parts_of(nk, pp.jm >> l, pp.cap);
-      const float u = float(H * parts), c = float(unit_cost(nk, nq, parts, pp));
+      const float u = float(H * parts);
+      const float c = float(UnitCost(nk, nq, pp.bias).unit(rounds_of((nk + 1) / 2, parts), pp.jm));
       units += u;
       most = fmaxf(most, c);
       sum += u * c;
@@ -550,7 +566,7 @@ __global__ void __launch_bounds__(kPlanThreads) pair_bwd_prepare(PlanParams pp) 
     const int nk = s_count[2 * b], nq = s_count[2 * b + 1];
     const bool work = nk > 0 && nq > 0;
     const int parts = work ? parts_of(nk, jt, pp.cap) : 0;
-    s_cost[b] = work ? unit_cost(nk, nq, parts, pp) : 0u;
+    s_cost[b] = work ? uint32_t(UnitCost(nk, nq, pp.bias).unit(rounds_of((nk + 1) / 2, parts), pp.jm)) : 0u;
     s_units[b] = H * parts;
     pp.counts[b] = int2{nk, nq};
   }
@@ -1135,9 +1151,10 @@ __global__ void __launch_bounds__(kThreads, 2) pair_bwd_kernel(Params p) {
           if (r0 + 32 * i >= c.nk) b2[i] = d2[i] = zero;
         }
         // go . out of the thread's query rows (in the eight threads of a row)
-        float go[2];
+        float go[2] = {0.0f, 0.0f};
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
+          if (!do_q) break;  // uniform
           float s = bf_lo(bg[i].x) * o0[i].x;
           s = fmaf(bf_hi(bg[i].x), o0[i].y, s); s = fmaf(bf_lo(bg[i].y), o0[i].z, s);
           s = fmaf(bf_hi(bg[i].y), o0[i].w, s); s = fmaf(bf_lo(bg[i].z), o1[i].x, s);

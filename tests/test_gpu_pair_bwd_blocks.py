@@ -179,8 +179,9 @@ def _plan(counts, heads, bias_dtype, device):
     ([72] * 16, 8, None, (384, 24)),               # one round; not 768 units of 12 rows
     ([64], 8, torch.float32, (64, 8)),             # half the parts to add for the same round
     ([192] * 4, 12, torch.bfloat16, (576, 16)),    # 64 units left for the second round, not 1152 of 8 rows
-    ([128] * 16, 8, None, (768, 24)),              # not 2048 of 8 rows, whose staging is most of their time
-    ([256], 8, None, (344, 6)), ([44] * 64, 8, None, (1024, 24)), ([44, 9, 30], 2, None, (30, 6)),
+    ([64] * 256, 8, None, (6144, 24)),             # many rounds: fewer, longer units
+    ([256], 8, None, (256, 6)),                    # whole rounds of four key pairs: 8 rows
+    ([128] * 16, 8, None, (1024, 12)), ([44] * 64, 8, None, (1024, 24)), ([44, 9, 30], 2, None, (24, 6)),
 ], ids=lambda v: str(v) if isinstance(v, int) else None)
 def test_rows_per_unit(cuda, counts, heads, bias_dtype, want):
     """The schedule takes the j per unit whose units finish first on the chip's 512 slots."""
