@@ -1,6 +1,6 @@
-"""The pair-formulation backward at the edges of its blocks: 16-row tiles, 24 / 16 j per unit, 64 / 48 query and
-key rows per block, and molecules whose units sum over several block triples, without a bias and with bf16 and fp32
-bias terms.
+"""The pair-formulation backward at the edges of its blocks: 16-row tiles, j blocks of 24 / 16 rows, query and key
+blocks of 64 / 48, the three sizes of a unit, and molecules whose units sum over several block triples, without a bias
+and with bf16 and fp32 bias terms; and with values that leave fp16, or are not finite.
 
 Bars, normwise per gradient against float64 autograd on the same rounded inputs.  bf16 gradients: the rounding of
 the result (2^-9 at most, 1.7e-3 over random mantissas) with the fp16 rounding of W, dS and P (2^-11 each, random
@@ -26,6 +26,7 @@ COUNTS = ([1, 2, 15], [16, 17, 24], [25, 47, 48], [49, 63, 64], [65, 80, 81], [9
 @pytest.mark.parametrize("bias_dtype", [None, torch.bfloat16, torch.float32], ids=["none", "bf16", "fp32"])
 @pytest.mark.parametrize("counts", COUNTS, ids=lambda c: "n" + "-".join(map(str, c)))
 def test_block_edges(cuda, counts, bias_dtype):
+    """One head and a few molecules: the smallest units (8 j at most), with one query and key block or several."""
     B, H, N, D = len(counts), 1, max(counts) + 3, 64
     # a key hole and dropped pairs in the larger molecules; every query has valid pairs
     holes = [(b, 3) for b, n in enumerate(counts) if n > 20]
@@ -47,6 +48,56 @@ def test_block_edges(cuda, counts, bias_dtype):
         bar = 2e-3 if g.dtype == torch.float32 else 4e-3
         assert rel_err(g.float().cpu().numpy(), r) <= bar, (name, rel_err(g.float().cpu().numpy(), r))
         assert torch.isfinite(g).all(), name
+
+
+def _plan(counts, heads, bias_dtype, device):
+    """(units, j per unit) of the plan that mf_simplicial_bwd leaves at the start of its workspace."""
+    B, N = len(counts), max(counts)
+    valid = torch.arange(N)[None, :] < torch.tensor(counts)[:, None]
+    ops = [torch.zeros(B, heads, N, 64, device=device, dtype=torch.bfloat16) for _ in range(5)]
+    bias = None
+    if bias_dtype is not None:
+        bias = [torch.zeros(s, device=device, dtype=bias_dtype) for s in [(B, heads, N, N)] * 3 + [(B, heads, N)]]
+    out32, lse = torch.zeros(B, heads, N, 64, device=device), torch.zeros(B, heads, N, device=device)
+    *_, ws = abi_bwd(ops, ops[0], out32, lse, valid.to(device), valid.to(device), torch.float32, bias=bias)
+    units, j = ws[:8].view(torch.int32).tolist()
+    return units, j
+
+
+@pytest.mark.parametrize("counts,bias_dtype,j,checked", [
+    ([200] + [23, 24, 25, 40] * 16, None, 24, (0, 1, 2, 3, 4)),
+    ([180] + [15, 16, 17, 33] * 16, torch.bfloat16, 16, (0, 1, 2, 3, 4)),
+    ([180] + [15, 16, 17, 33] * 16, torch.float32, 16, (0, 1, 2, 3, 4)),
+    ([128] * 16, None, 12, (7,)),
+    ([64], torch.float32, 8, (0,)), ([64], torch.bfloat16, 8, (0,)),
+], ids=["none-24", "bf16-16", "fp32-16", "none-12", "fp32-8", "bf16-8"])
+def test_units_of_every_size(cuda, counts, bias_dtype, j, checked):
+    """8 heads and enough molecules for units of 24 and 12 j (16 and 8 with a bias), whole and partial j blocks, beside
+    one molecule of 200 / 180 atoms whose few units walk several j blocks of several query and key blocks (their sums
+    in the slabs continue from one j block to the next).  The plan's j per unit is part of the test.  Float64 on the
+    first two heads of some molecules."""
+    H, D, B, N = 8, 64, len(counts), max(counts)
+    assert _plan(counts, H, bias_dtype, cuda)[1] == j
+    q, k1, v1, k2, v2, qv, pkv, _ = random_simplicial(B, H, N, D, seed=N, counts=counts, std=logit_std(D))
+    gen = torch.Generator().manual_seed(N + 1)
+    go = torch.randn(B, H, N, D, generator=gen).to(torch.bfloat16)
+    ops = [t.to(torch.bfloat16) for t in (q, k1, v1, k2, v2)]
+    bias = None
+    if bias_dtype is not None:
+        bias = [(torch.randn(B, H, N, N, generator=gen) * 0.5).to(bias_dtype) for _ in range(3)] + \
+               [torch.rand(B, H, N, generator=gen).to(bias_dtype)]
+    _, got = hip_grads([t.to(cuda) for t in ops], qv.to(cuda), pkv.to(cuda), None, go.to(cuda), "bf16_tc",
+                       bias=None if bias is None else [t.to(cuda) for t in bias])
+    for b in checked:
+        n = counts[b]
+        cut = lambda t: t[b:b + 1, :2, :n]  # noqa: E731
+        ones = torch.ones(1, n, dtype=torch.bool)
+        cbias = None if bias is None else [cut(t)[..., :n] for t in bias[:3]] + [cut(bias[3])]
+        _, ref = fp64_grads([cut(t) for t in ops], ones, ones, None, cut(go), bias=cbias)
+        for name, g, r in zip(GRAD_NAMES, got, ref):
+            g = cut(g)[..., :n] if name in ("du", "dv_bias", "dw") else cut(g)
+            bar = 2e-3 if g.dtype == torch.float32 else 4e-3
+            assert rel_err(g.float().cpu().numpy(), r) <= bar, (b, n, name, rel_err(g.float().cpu().numpy(), r))
 
 
 @pytest.mark.parametrize("factor", [2.0 ** -16, 2.0 ** -40, 0.0], ids=["2^-16", "2^-40", "zero"])
@@ -161,20 +212,6 @@ def test_gradients_below_the_fp32_range_are_zero_not_nan(cuda):
             assert rel_err(g.numpy(), r) <= 4e-3, (name, rel_err(g.numpy(), r))
 
 
-def _plan(counts, heads, bias_dtype, device):
-    """(units, j per unit) of the plan that mf_simplicial_bwd leaves at the start of its workspace."""
-    B, N = len(counts), max(counts)
-    valid = torch.arange(N)[None, :] < torch.tensor(counts)[:, None]
-    ops = [torch.zeros(B, heads, N, 64, device=device, dtype=torch.bfloat16) for _ in range(5)]
-    bias = None
-    if bias_dtype is not None:
-        bias = [torch.zeros(s, device=device, dtype=bias_dtype) for s in [(B, heads, N, N)] * 3 + [(B, heads, N)]]
-    out32, lse = torch.zeros(B, heads, N, 64, device=device), torch.zeros(B, heads, N, device=device)
-    *_, ws = abi_bwd(ops, ops[0], out32, lse, valid.to(device), valid.to(device), torch.float32, bias=bias)
-    units, j = ws[:8].view(torch.int32).tolist()
-    return units, j
-
-
 @pytest.mark.parametrize("counts,heads,bias_dtype,want", [
     ([72] * 16, 8, None, (384, 24)),               # one round; not 768 units of 12 rows
     ([64], 8, torch.float32, (64, 8)),             # half the parts to add for the same round
@@ -271,10 +308,11 @@ def test_gradients_in_the_leaves_dtypes_are_written_in_full(cuda, B, N, wanted):
     flags.update(zip(("need_du", "need_dv_bias", "need_dw", "need_dgate"), wanted))
     call = (go, *ops, out32, lse, *masks.values(), *bias, *[None] * 6, flags)
     want = hsa._kernel_backward(*call, allow_leaf=False)
-    poison = [torch.full((1 << 22,), float("nan"), device=cuda) for _ in range(4)]
-    poison += [torch.full((B * H * N * n,), float("nan"), device=cuda) for n in (1, D // 2, N) for _ in range(5)]
-    del poison  # the allocator hands these blocks out again
-    got = hsa._kernel_backward(*call)
+    real = torch.empty
+    with pytest.MonkeyPatch.context() as mp:
+        mp.setattr(hsa.torch, "empty", lambda *a, **k: real(*a, **k).fill_(float("nan"))
+                   if k.get("dtype") in (torch.float32, torch.bfloat16) else real(*a, **k))
+        got = hsa._kernel_backward(*call)
     for g, w in zip(got, want):
         assert (g is None) == (w is None)
         if w is not None:

@@ -166,8 +166,8 @@ def test_qm9_config_gradients_whole_batch(cuda):
 
 @pytest.mark.parametrize("with_bias", [False, True], ids=["nobias", "bias"])
 def test_geom_config_gradients_every_molecule(cuda, with_bias):
-    """Config 2 (bf16, 64 molecules of 10-72 atoms padded to 181), without a bias (the pair-formulation kernel)
-    and with a factorized bias (the ownership kernel): the batched HIP gradients of each molecule against
+    """Config 2 (bf16, 64 molecules of 10-72 atoms padded to 181), without a bias and with a factorized bias (both
+    the pair-formulation kernel): the batched HIP gradients of each molecule against
     float64 autograd over that molecule's atoms, 2e-2 per gradient."""
     w = simplicial_workload("geom")
     B, H, N, D = w.shape
@@ -253,10 +253,10 @@ def test_low_rank_terms_run_on_the_kernel(cuda):
     assert res[9] is not None and res[11] is not None
 
 
-def abi_bwd(ops, go, out32, lse, qv, pkv, grads_dtype, bias=None):
+def abi_bwd(ops, go, out32, lse, qv, pkv, grads_dtype, bias=None, workspace=True):
     """mf_simplicial_bwd through the C ABI; gradient buffers filled with NaN (bf16) or zeros (fp32, the
     caller's fill that the fp32 contract asks for); with a factorized bias also du, dv_bias, dw, dgate
-    (the same dtype and fill).  The gradients, then the workspace."""
+    (the same dtype and fill).  The gradients, then the workspace (workspace=False: NULL is passed)."""
     from matterformer_amd import _native
 
     B, H, N, D = ops[0].shape
@@ -288,21 +288,21 @@ def abi_bwd(ops, go, out32, lse, qv, pkv, grads_dtype, bias=None):
         grad_dtype=_native.dtype_code(torch.bfloat16), dq=grads[0].data_ptr(), dk1=grads[1].data_ptr(),
         dv1=grads[2].data_ptr(), dk2=grads[3].data_ptr(), dv2=grads[4].data_ptr(), batch=B, heads=H, tokens=N,
         head_dim=D, dtype=_native.dtype_code(torch.bfloat16), grads_dtype=_native.dtype_code(grads_dtype),
-        workspace=ws.data_ptr(), workspace_bytes=nbytes, **extra)
+        workspace=ws.data_ptr() if workspace else None, workspace_bytes=nbytes if workspace else 0, **extra)
     with torch.cuda.device(dev):
         _native.check(lib.mf_simplicial_bwd(args, _native.current_stream(dev)), "mf_simplicial_bwd")
     torch.cuda.synchronize()
     return (*grads, ws)
 
 
+@pytest.mark.parametrize("workspace", [True, False], ids=["pair", "ownership"])
 @pytest.mark.parametrize("with_bias", [False, True], ids=["nobias", "bias"])
-@pytest.mark.parametrize("counts", [[70, 41, 0, 12], [150, 64, 1, 33]], ids=["pair_only", "with_ownership"])
-def test_bf16_gradients_written_in_full(cuda, counts, with_bias):
+@pytest.mark.parametrize("counts", [[70, 41, 0, 12], [150, 64, 1, 33]], ids=["n70", "n150"])
+def test_bf16_gradients_written_in_full(cuda, counts, with_bias, workspace):
     """grads_dtype bf16: every element of the gradients (the bias gradients too) is written (buffers start as
     NaN; padded rows and entries, and a molecule without valid queries, come back 0), and the values are the
-    fp32-gradient call's rounded to bf16 (both paths form the same fp32 sums).  The second case has a 150-atom
-    molecule (ownership kernel) beside pair-kernel molecules, one of them split in two halves; the 70-atom
-    molecule runs its query tiles in two passes when there is a bias."""
+    fp32-gradient call's rounded to bf16 (both calls form the same fp32 sums).  With the workspace, the pair kernel
+    (molecules of one block and of several); without it, the ownership kernel."""
     B, H, N, D = len(counts), 2, max(counts) + 3, 64
     case = random_simplicial(B, H, N, D, seed=71, counts=counts, std=logit_std(D))
     q, k1, v1, k2, v2, qv, pkv, pv = case
@@ -319,8 +319,8 @@ def test_bf16_gradients_written_in_full(cuda, counts, with_bias):
         kw = dict(u=bias[0], v_bias=bias[1], w=bias[2], gate=bias[3])
     out, lse, out32 = hip_simplicial_attention_forward(*ops, query_valid=qv, pair_key_valid=pkv, pair_valid=None,
                                                        precision="bf16_tc", **kw)
-    *g16, _ = abi_bwd(ops, go, out32, lse, qv, pkv, torch.bfloat16, bias=bias)
-    *g32, _ = abi_bwd(ops, go, out32, lse, qv, pkv, torch.float32, bias=bias)
+    *g16, _ = abi_bwd(ops, go, out32, lse, qv, pkv, torch.bfloat16, bias=bias, workspace=workspace)
+    *g32, _ = abi_bwd(ops, go, out32, lse, qv, pkv, torch.float32, bias=bias, workspace=workspace)
     for name, a, r in zip(GRAD_NAMES, g16, g32):
         assert not torch.isnan(a).any(), name
         assert torch.equal(a, r.to(torch.bfloat16)), name
@@ -343,7 +343,7 @@ def test_bf16_gradients_written_in_full(cuda, counts, with_bias):
 def test_pair_path_bias_gradients_with_masking_scale_terms(cuda):
     """bf16 operands, pair formulation with a factorized bias whose w carries -30000 on a fifth of the pairs
     (positive gates: those pairs' P underflows to 0, as under an additive mask) beside ordinary terms; one
-    molecule of 70 atoms (split in two halves, query tiles in two passes) and one of 41.  Every gradient
+    molecule of 70 atoms (two query and two key blocks) and one of 41.  Every gradient
     against float64 autograd on the same rounded inputs, 2e-2."""
     B, H, N, D = 2, 2, 70, 64
     case = random_simplicial(B, H, N, D, seed=81, counts=[70, 41], std=logit_std(D))
