@@ -664,7 +664,7 @@ __device__ __forceinline__ void pair_loop(const unsigned char* smem, int nkj, in
             }
           }
         }
-        // Z^T operands: d = 16 dt + r16, keys 4g + r of row j0 (halves
+        // Z^T operands: d = ND r16 + dt, keys 4g + r of row j0 (halves
         // 0..3) and of row j0 + 1 (halves 4..7)
         uint4 z[ND];
 #pragma unroll

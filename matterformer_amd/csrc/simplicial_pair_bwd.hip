@@ -44,23 +44,25 @@
 // identical bits.
 //
 // Measured (64 GEOM-like molecules of mean 44 atoms, 8 heads, kernel time):
-// 109 us without a bias (191 us when one wave per SIMD held both j, the
+// 117 us without a bias (191 us when one wave per SIMD held both j, the
 // products' operands and all query tiles in 470 registers, and a unit had a
-// whole CU: 0.29 PFLOP/s of the five products now), 278 us with a fp32 or
-// bf16 bias (1.88 ms and 365 us on the kernels that served them before); four
-// molecules of 192 atoms, 12 heads, bf16 bias: 1.16 ms (5.47 ms on the
-// ownership kernel).  A variant with more spilled registers than the 8 of the
-// staging code doubled the loop's time: a spill waits on memory that two
-// waves per SIMD cannot cover.
+// whole CU), 219 us with a bf16 bias and 252 with a fp32 one (365 us and
+// 1.88 ms on the kernels that served them before); four molecules of 192
+// atoms, 12 heads, bf16 bias: 1.12 ms (5.47 ms on the ownership kernel).
+// Registers: a spill waits on memory that two waves per SIMD cannot cover (a
+// variant with many in the loop took twice the time); 2 of the 256 are spilled
+// without a bias, 11 with one, all in the staging code.
 //
 // Schedule.  The prepare launch's first workgroup counts every molecule's
-// valid keys and queries, picks the j per unit (24, 12 or 6, with a bias 16, 8 or 4: by the
-// time its units take on two slots per CU) and writes the unit list longest
-// first (LPT); its other workgroups write the zero rows of 16-bit gradients.
+// valid keys and queries, picks the j per unit (24, 12 or 6, with a bias 16, 8
+// or 4: by an estimate of the time the units take on the chip's 512 slots) and
+// writes the unit list longest first (LPT); its other workgroups write the
+// zero rows of 16-bit gradients.
 // The units of a molecule own their dk1 / dv1 rows; where a molecule has more
 // than one block triple, dq, dk2 and dv2 are summed in the unit's slab of the
-// workspace (read back by the thread that wrote it) and a combine launch adds
-// the slabs in unit order.  (Handing the sums over inside the kernel would
+// workspace (read back by the thread that wrote it) and a finish launch adds
+// the slabs, and the units' partial bias sums, in unit order.  (Handing the
+// sums over inside the kernel would
 // need a device-scope release and acquire per unit, which on this part write
 // back and invalidate the whole L2 of the XCD and held each workgroup's CU
 // for tens of microseconds.)
@@ -70,7 +72,8 @@
 // (bf16 values convert exactly; entries below 2^-14 of the largest lose low
 // bits as fp16 subnormals, which moves a dot product by at most 2^-24 of its
 // largest term), so that one v_pk_mul_f16 forms two pair products and the
-// MFMAs are 16x16x32 f16 with fp32 accumulation:
+// MFMAs are 16x16x32 f16 with fp32 accumulation.  Infinities and NaN stay what
+// they are and do not enter the scales:
 //   W for S and for dq: k1 k2 rounded to fp16 (the reference backward rounds
 //     the score products to bf16, triton_simplicial_attention.py:546-551);
 //   Z for dP: hi + lo, both fp16: hi = v1 v2 rounded, lo = fma(v1, v2, -hi),

@@ -1,6 +1,7 @@
 """The fp32 pair-formulation kernels at the edges of their tiles and of the range they serve (forward at most 64
-tokens and head_dim 64, backward 32 and 32; larger calls run the general kernels), with and without a factorized
-bias, against float64 on the same inputs.
+tokens and head_dim 64, backward 32 and 32; larger calls, and few molecules of 49 / 25 tokens and more without a bias,
+run the general kernels), in both shapes of their workgroups, with and without a factorized bias, against float64 on
+the same inputs.
 
 Bar, normwise per result: products and sums are fp32 over at most n^2 = 4096 terms in short chains; 2^-24 per
 rounding with random signs over the chains (about 20 roundings a term) gives below 1e-6, and the hardware exp2's

@@ -180,7 +180,7 @@ def test_16bit_terms_match_fp64(cuda, shape, terms, dtype):
                          ids=["one_block", "key_blocks"])
 def test_16bit_large_bias_takes_exact_offsets(cuda, shape):
     """Bias terms of several units in log2 units (beyond the one-pass bound and the shifted pass's cap): exact
-    offsets (running maxima in one key block, two passes over key blocks), every valid query row against
+    offsets (running maxima in one pass, over one key block and over several), every valid query row against
     float64."""
     B, H, N, D, counts, holes, drop = shape
     case = random_simplicial(B, H, N, D, seed=N + 11, counts=counts, holes=holes, pair_drop=drop,
