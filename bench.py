@@ -753,7 +753,7 @@ def measure_simplicial_extras(lib, w, wd) -> dict:
                          "peak": BF16_DENSE_PEAK_TFLOPS, "unit": "TFLOP/s",
                          "frac": round(bwd_flops / (bwd_ms * 1e-3) / 1e12 / BF16_DENSE_PEAK_TFLOPS, 5),
                          "kernel": "mf::pbwd::pair_bwd_kernel (pairs as keys, fp16 operands, LPT plan, "
-                                   "units of at most 24 j) with its plan, combine and zero-rows launches; "
+                                   "units of j blocks of at most 24) with its plan (and zero rows) and finish launches; "
                                    "deterministic, no atomics",
                          "kernel_ms": round(bwd_ms, 5),
                          "note": "hip_simplicial_attention_backward graph-replayed, bf16 gradients written by the "
@@ -785,7 +785,7 @@ def measure_simplicial_extras(lib, w, wd) -> dict:
     bias_bwd_ms = _graph_ms(bias_bwd_step, per_graph=10, replays=5)
     res["bias_bwd"] = {"ms": round(bias_bwd_ms, 5), "eager_ms": round(bias_bwd_eager_ms, 5),
                        "kernel": "mf::pbwd::pair_bwd_kernel<bias=1> (block triples of 48 / 16 / 48 rows) with "
-                                 "its plan, combine, bias finish and clearing launches; dq, dk1, dv1, dk2, dv2, du, "
+                                 "its plan, finish and clearing launches; dq, dk1, dv1, dk2, dv2, du, "
                                  "dv_bias, dw, dgate in bf16, written in full"}
 
     # C1: QM9 fp32
